@@ -4,13 +4,15 @@
  * Replaces the cuBLAS calls behind cudaGemm / cudaGemmBatched of the reference (src/gemm.cpp:25-209).  The batched
  * (N, T) form  M[b] = V[b] * U[b]^T  is the matrix-core stage of non-fused Winograd (app/CudaBackend.cu:417-418): both
  * operands are contiguous along k, so it runs on the shared MFMA engine with fp32 (int32 for int8) accumulation and the
- * result is rounded once, to nearest even, on store.  Every other operand form, and fp64, goes through a small LDS-tiled
- * kernel that exists for completeness of the API, not for speed.
+ * result is rounded once, to nearest even, on store.  The (T, N) form, the product of the weight gradient, has a matrix-core
+ * kernel of its own (gemm_tn.hip).  Every other operand form, and fp64, goes through a small LDS-tiled kernel that exists for
+ * completeness of the API, not for speed.
  * Unlike the reference there is a bf16 case, fp16 always accumulates in fp32, and the result of a 16-bit product may be
  * kept in fp32.
  */
 #include <type_traits>
 
+#include "gemm_tn.hpp"
 #include "mfma_core.hpp"
 #include "persistent_gemm.hpp"
 #include "resident_gemm.hpp"
@@ -518,26 +520,33 @@ extern "C" int avhip_gemm_batched(void *stream, int ab_dtype, int c_dtype, int o
 	if (batch > 65535)
 		return AVHIP_NOT_SUPPORTED;
 	hipStream_t s = static_cast<hipStream_t>(stream);
-	const bool nt = (opA == 0 && opB != 0);
+	const bool nt = (opA == 0 && opB != 0), tn = (opA != 0 && opB == 0);
 #define ARGS_MFMA s, A, B, C, batch, M, N, K, lda, ldb, ldc, strideA, strideB, strideC, alpha, beta
+#define TRY_TN(TE, TC) (tn && gemm_tn_launch<TE, TC>(s, A, B, C, batch, M, N, K, lda, ldb, ldc, strideA, strideB, strideC, static_cast<float>(alpha), static_cast<float>(beta)))
 #define ARGS_GEN s, A, B, C, batch, M, N, K, opA, opB, lda, ldb, ldc, strideA, strideB, strideC, alpha, beta
 	switch (ab_dtype)
 	{
 		case DT_FLOAT32:
 			if (c_dtype != DT_FLOAT32)
 				return AVHIP_UNSUPPORTED_DATATYPE;
+			if (TRY_TN(float, float))
+				return 0;
 			return nt ? launch_mfma<float, float>(ARGS_MFMA) : launch_generic<float, float, float>(ARGS_GEN);
 		case DT_FLOAT64:
 			if (c_dtype != DT_FLOAT64)
 				return AVHIP_UNSUPPORTED_DATATYPE;
 			return launch_generic<double, double, double>(ARGS_GEN);
 		case DT_FLOAT16:
+			if ((c_dtype == DT_FLOAT16 && TRY_TN(f16_t, f16_t)) || (c_dtype == DT_FLOAT32 && TRY_TN(f16_t, float)))
+				return 0;
 			if (c_dtype == DT_FLOAT16)
 				return nt ? launch_mfma<f16_t, f16_t>(ARGS_MFMA) : launch_generic<f16_t, f16_t, float>(ARGS_GEN);
 			if (c_dtype == DT_FLOAT32)
 				return nt ? launch_mfma<f16_t, float>(ARGS_MFMA) : launch_generic<f16_t, float, float>(ARGS_GEN);
 			return AVHIP_UNSUPPORTED_DATATYPE;
 		case DT_BFLOAT16:
+			if ((c_dtype == DT_BFLOAT16 && TRY_TN(bf16_t, bf16_t)) || (c_dtype == DT_FLOAT32 && TRY_TN(bf16_t, float)))
+				return 0;
 			if (c_dtype == DT_BFLOAT16)
 				return nt ? launch_mfma<bf16_t, bf16_t>(ARGS_MFMA) : launch_generic<bf16_val, bf16_val, float>(ARGS_GEN);
 			if (c_dtype == DT_FLOAT32)
@@ -551,5 +560,6 @@ extern "C" int avhip_gemm_batched(void *stream, int ab_dtype, int c_dtype, int o
 			return AVHIP_UNSUPPORTED_DATATYPE;
 	}
 #undef ARGS_MFMA
+#undef TRY_TN
 #undef ARGS_GEN
 }

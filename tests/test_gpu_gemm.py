@@ -85,6 +85,24 @@ def test_gemm_batched_other_forms(oracle, opA, opB):
     assert oracle.rel_l2(got, oracle.gemm_batched(A, B, C0, opA, opB, a, b)) < 2e-6
 
 
+@pytest.mark.parametrize("dtype,c_dtype", [("f32", "f32"), ("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"), ("bf16", "f32")])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 31, 33, 15), (3, 32, 64, 16), (1, 65, 63, 129), (5, 64, 2, 17), (36, 40, 24, 513),
+                                   (130, 64, 64, 130), (129, 63, 64, 127), (515, 60, 33, 33)])
+def test_gemm_batched_tn(oracle, dtype, c_dtype, shape):
+    """C[b] = A[b]^T B[b], the product of the weight gradient: 32 x 32 tiles for the small ones, 64 x 64 tiles from 128 (16-bit) or
+    512 (fp32) of them on, in pairs of elements where M and N are even; k below, at and above one stage of 16 rows and one round of the
+    eight wavefronts (128).  Bars as for the (N, T) form: one fp32 sum of at most 513 products, one rounding on store."""
+    g = h.rng(14)
+    batch, M, N, K = shape
+    A = h.rounded(oracle, g.standard_normal((batch, K, M)), dtype)
+    B = h.rounded(oracle, g.standard_normal((batch, K, N)), dtype)
+    C0 = h.rounded(oracle, g.standard_normal((batch, M, N)), c_dtype)
+    a, b = (float(np.float32(1.1)), float(np.float32(0.1))) if batch % 2 else (None, None)
+    got = h.gemm(A, B, C0, dtype, True, False, a, b, c_dtype=c_dtype, batched=True)
+    want = oracle.gemm_batched(A, B, C0, True, False, a if a is not None else 1.0, b if b is not None else 0.0)
+    assert oracle.rel_l2(got, want) < (TOL[c_dtype] if c_dtype != "f32" else 2e-6)
+
+
 @pytest.mark.parametrize("shape", [(64, 128, 1152), (100, 36, 68)])
 def test_gemm_int8_is_exact(oracle, shape):
     g = h.rng(13)
