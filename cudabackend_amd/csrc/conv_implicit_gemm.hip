@@ -662,8 +662,8 @@ namespace
 			}
 #undef AVHIP_PACKED
 		}
-		/* a problem of a few big tiles goes to the kernel with one 32 x 32 tile per wavefront */
-		if (fast && conv_small_launch<TE, Epi>(st, s, x, w, epi, static_cast<int64_t>(grid.x) * grid.y))
+		/* a problem that does not fill the chip with big tiles goes to the kernel with small ones and k shared by wavefronts */
+		if (fast_path_ok<TE>(s, flags, padding_value) && conv_small_launch<TE, Epi>(st, s, x, w, epi))
 			return 0;
 		/* one-tap filters are plain matrix products with a short k: a persistent kernel pipelines across tiles */
 		if (fast && s.R * s.S == 1 && conv_pointwise_launch<TE, Epi>(st, s, x, w, epi))
@@ -781,7 +781,7 @@ namespace
 	 * leaves most compute units idle for a long walk.  Estimates in microseconds (fitted to layers of 196 to 6272 pixels with
 	 * 1024 to 4608 elements of k): 4 + 0.7 per k-step for a workgroup of the plain gather kernel (less in the image-tile kernel); for the split, 10 for the two
 	 * launches and their prologues, 0.7 per step of a part, 0.25 per part and the parts read back at 4 TB/s in the reduction;
-	 * the one-wavefront-per-tile kernel by its own estimate where the launcher would use it. */
+	 * the small-tile kernel by its own estimate where the launcher would use it. */
 	struct SplitPlan
 	{
 		int splits, steps_per_split;
@@ -820,12 +820,8 @@ namespace
 		const double chip = sizeof(TE) == 4 ? 1.55e8 : 1.87e9;
 		const double flops = 2.0 * static_cast<double>(pixels) * s.K * s.C * s.R * s.S;
 		other = std::max(other, flops / (chip * std::min(1.0, static_cast<double>(plain_workgroups) / 256.0)));
-		if (s.R * s.S <= 32 && conv_small_preferred(s, static_cast<int>(sizeof(TE)), tiles))
-		{
-			const double wavefronts = static_cast<double>(((pixels + 31) / 32) * ((s.K + 31) / 32));
-			const double small = std::max(conv_small_estimate(s, static_cast<int>(sizeof(TE)), tiles).small_us, flops / (chip * std::min(1.0, wavefronts / 1024.0)));
-			other = std::min(other, small);
-		}
+		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true))
+			other = std::min(other, conv_small_plan(s, static_cast<int>(sizeof(TE))).us);
 		const double walk = std::max(0.7 * static_cast<double>(per_part), flops / (chip * std::min(1.0, static_cast<double>(tiles * parts) / 256.0)));
 		const double split = 10.0 + walk + 0.25 * static_cast<double>(parts) + plane_bytes * static_cast<double>(parts + 1) / 4.0e6;
 		if (split > 0.85 * other)

@@ -1,16 +1,22 @@
 /*
- * conv_small.hip -- implicit-GEMM convolution for problems too small to fill the chip with 128 x 128 workgroup tiles.
+ * conv_small.hip -- implicit-GEMM convolution for problems that do not fill the chip with 128 x 128 workgroup tiles.
  *
- * A batch of 8 images of 15 x 15 pixels with 64 filters is 15 tiles of 128 x 128: 15 of 256 compute units busy, each for the
- * whole k range.  This kernel cuts the same GEMM (rows = output pixels, columns = filters, k = (tap, channel)) into
- * 32 x 32 tiles, one per WAVEFRONT (workgroup = 64 work-items), several hundred of them for such a problem, and drops
- * everything a small problem does not need: no LDS staging, no barriers in the k loop.  Each lane fetches its own MFMA
- * operands straight from global memory in the operand layout (lane l: row l % 32 of the tile, 16-byte k-chunk l / 32 of a
- * 32-byte slab) with out-of-range buffer loads for padding and tails; the re-use of x and w between wavefronts is left to
- * L2, which holds a small problem entirely.  Loads run one group of four slabs ahead of the MFMAs.  The accumulator tile
- * leaves through 4 KB of LDS so that a lane stores four consecutive filters of a pixel, with the shared epilogue.
+ * The GEMM (rows = output pixels, columns = filters, k = (tap, channel)) is cut into tiles of 32 x 32 or 64 x 64 and the k range
+ * of a tile is shared by the one, four or eight wavefronts of a workgroup, so that a layer of a few hundred pixels still occupies
+ * the chip; the partial tiles are added through LDS in a fixed order.  There is no barrier in the k loop: each wavefront loads its
+ * own operands, 128 bytes of k of every row at a time, eight lanes to a row, and brings them into MFMA layout through its own
+ * part of LDS.  k runs over the 16-byte chunks of all taps in a row, so channel counts that are no multiple of 64 cost nothing.
+ *
+ * What bounds it: the 64 bytes per clock that a compute unit loads (128 clocks per stage of a 32 x 32 tile, 256 per stage of a
+ * 64 x 64 tile, which needs half as much per product), for fp32 the matrix cores, and for the smallest problems the latency of
+ * one launch.  Operands loaded straight in MFMA layout (32 lines per load instruction) took 55 to 60 clocks a kilobyte here, by
+ * rows 20.  Measured, before (that form, 128 x 128 gather kernel where it was preferred) and now: bf16 128 -> 128 3x3 on 2912
+ * pixels 12.5 -> 8.1 us, 256 -> 256 3x3 on 3800 pixels 18.1 -> 13.8 us, fp32 64 -> 218 5x5 on 1568 pixels 124 -> 23 us, fp16 72
+ * channels 3x3 with an ELU on 13520 pixels 25.3 -> 9.9 us, int8 128 -> 128 stride 2 on 6720 pixels 21.7 -> 9.8 us.
  */
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 
 #include "conv_small.hpp"
 #include "mfma_core.hpp"
@@ -20,161 +26,285 @@ namespace
 	using namespace avhip;
 
 	constexpr int SMALL_TILE = 32;
-	constexpr int GROUP = 4; /* 32-byte k-slabs fetched together */
-	constexpr int SMALL_PITCH = SMALL_TILE + 4; /* words per LDS row of the drain buffer */
 
 	struct SmallGeom
 	{
 		int H, W, C, K, R, S, Ho, Wo, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, flip;
-		int slabs_per_tap; /* 32-byte slabs covering the channels of one tap */
+		int chunks_per_tap; /* 16-byte chunks of the channels of one tap */
+		unsigned int by_chunks, by_s; /* ceil(2^32 / chunks_per_tap), ceil(2^16 / S): division by multiplication */
 		int pixels, images;
+		int pixels_first; /* order of the tiles: pixel tiles run fastest within an XCD (more weights than image), or filter tiles */
 	};
 
-	/* KW wavefronts share one tile: each takes a contiguous KW-th of the k range and the partial tiles are summed through LDS.
-	 * KW = 4 when even the 32 x 32 tiling leaves most SIMDs without a wavefront. */
-	template<typename TE, typename Epi, int KW>
-	__global__ __launch_bounds__(64 * KW) void k_conv_small(const TE *__restrict__ x, const TE *__restrict__ w, SmallGeom g, Epi epi)
+	/* LDS accesses of a wavefront to its own part stay in this order (the hardware does them in order, without a barrier) */
+	__device__ __forceinline__ void wave_order()
 	{
-		__shared__ __attribute__((aligned(16))) typename Epi::scalar_t sm[KW * SMALL_TILE * SMALL_PITCH];
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	}
+
+	/* T x T MFMA tiles of 32 x 32 per wavefront, KW wavefronts on one tile. */
+	template<typename TE, typename Epi, int T, int KW, int ACT>
+	__global__ __launch_bounds__(64 * KW, KW == 8 ? 2 : T == 1 ? 3 : 2) void k_conv_small(const TE *__restrict__ x, const TE *__restrict__ w, SmallGeom g, Epi epi)
+	{
 		constexpr unsigned int SZ = sizeof(TE);
+		constexpr int SIDE = SMALL_TILE * T;
+		constexpr int LOADS = 4 * T; /* loads of 8 rows each, per operand and stage */
+		constexpr int QUADS = SIDE / 4; /* runs of four filters of a pixel */
+		constexpr int PITCH = T == 1 ? SIDE + 2 : SIDE + 1; /* 16-byte slots between two runs of a pixel: conflict-free both ways */
+		constexpr int SLOTS = QUADS * PITCH > 2 * SIDE * 8 ? QUADS * PITCH : 2 * SIDE * 8;
+		constexpr int DEPTH = T == 1 ? 2 : 1; /* stages in flight */
+		constexpr bool VEC = ACT == ACT_SIMPLE;
+		typedef typename Epi::scalar_t scalar_t;
+		typedef Pack<scalar_t, 4> quad_t;
+		/* each wavefront its own part: rows of the stage being multiplied, then its partial tile */
+		__shared__ __attribute__((aligned(16))) uint4 lds[KW][SLOTS];
+
 		const int lane = threadIdx.x & 63;
-		const int wave = threadIdx.x >> 6;
-		const int r = lane & 31;
-		const unsigned int half = (lane >> 5) * 16;
-		/* neighbouring pixel tiles read overlapping windows: a contiguous run of them goes to one XCD and its L2 */
-		const int p0 = static_cast<int>(xcd_block(blockIdx.x, gridDim.x)) * SMALL_TILE, k0 = blockIdx.y * SMALL_TILE;
-		const int kcol = k0 + (threadIdx.x & 7) * 4;
-		typename Epi::Columns columns;
-		epi.load_columns(kcol, columns);
-
-		const __amdgpu_buffer_rsrc_t rx = make_buffer(x, static_cast<unsigned int>(g.images) * g.H * g.W * g.C * SZ);
-		const __amdgpu_buffer_rsrc_t rw = make_buffer(w, static_cast<unsigned int>(g.K) * g.R * g.S * g.C * SZ);
-		const unsigned int c_bytes = g.C * SZ;
-
-		/* this lane's row of A: one output pixel */
-		const int p = p0 + r;
-		const bool row_ok = p < g.pixels;
-		const int pp = row_ok ? p : 0;
-		const int line = pp / g.Wo, ow = pp - line * g.Wo;
-		const int n = line / g.Ho, oh = line - n * g.Ho;
-		const int ih0 = oh * g.stride_h + g.pad_h, iw0 = ow * g.stride_w + g.pad_w;
-		const unsigned int a_origin = static_cast<unsigned int>((n * g.H + ih0) * g.W + iw0) * c_bytes + half;
-		unsigned int inside = 0;
-		if (row_ok)
+		const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+		uint4 *mine = lds[wave];
+		/* Each XCD gets a contiguous run of the tiles, and within it the tiles that share the larger operand are neighbours, so
+		 * that its L2 fetches that operand once. */
+		unsigned int pixel_tile, filter_tile;
+		if (g.pixels_first)
 		{
-			unsigned int cols = 0;
-			for (int j = 0; j < g.S; j++)
-			{
-				const int iw = iw0 + (g.flip ? g.S - 1 - j : j) * g.dil_w;
-				if (iw >= 0 && iw < g.W)
-					cols |= 1u << j;
-			}
-			for (int i = 0; i < g.R; i++)
-			{
-				const int ih = ih0 + (g.flip ? g.R - 1 - i : i) * g.dil_h;
-				if (ih >= 0 && ih < g.H)
-					inside |= cols << (i * g.S);
-			}
+			const unsigned int t = xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+			filter_tile = t / gridDim.x;
+			pixel_tile = t - filter_tile * gridDim.x;
 		}
-		/* this lane's row of B: one filter */
-		const int kf = k0 + r;
-		const unsigned int b_origin = kf < g.K ? static_cast<unsigned int>(kf) * g.R * g.S * c_bytes + half : OUT_OF_RANGE;
+		else
+			xcd_tile(pixel_tile, filter_tile);
+		const int p0 = static_cast<int>(pixel_tile) * SIDE, k0 = static_cast<int>(filter_tile) * SIDE;
 
-		typename Mma<TE>::acc_t acc;
-#pragma unroll
-		for (int v = 0; v < 16; v++)
-			acc[v] = 0;
+		const unsigned int c_bytes = g.C * SZ, filter_bytes = g.R * g.S * c_bytes;
+		const __amdgpu_buffer_rsrc_t rx = make_buffer(x, static_cast<unsigned int>(g.images) * g.H * g.W * c_bytes);
+		const __amdgpu_buffer_rsrc_t rw = make_buffer(w, static_cast<unsigned int>(g.K) * filter_bytes);
 
-		/* k walks (tap, slab); everything about the position is wavefront-uniform */
-		const int taps = g.R * g.S;
-		const int groups_all = (taps * g.slabs_per_tap + GROUP - 1) / GROUP;
-		const int groups = (groups_all + KW - 1) / KW; /* groups of this wavefront: [wave * groups, (wave + 1) * groups) */
-		const int first_slab = wave * groups * GROUP;
-		int f_tap = first_slab / g.slabs_per_tap, f_slab = first_slab - f_tap * g.slabs_per_tap;
-		int f_i = f_tap / g.S, f_j = f_tap - f_i * g.S;
-		int left = groups * GROUP; /* slabs this wavefront may still fetch */
-		auto fetch = [&](uint4 (&a)[GROUP], uint4 (&b)[GROUP]) __attribute__((always_inline))
+		/* origin and border mask (bit = tap inside the image) of one pixel per lane, handed through LDS to the lanes that load it */
+		uint2 *pixel = reinterpret_cast<uint2*>(mine);
+		if (T == 2 || lane < SIDE)
 		{
-#pragma unroll
-			for (int q = 0; q < GROUP; q++)
+			const int p = p0 + lane;
+			const bool row_ok = p < g.pixels;
+			const int pp = row_ok ? p : 0;
+			const int line = pp / g.Wo, ow = pp - line * g.Wo;
+			const int n = line / g.Ho, oh = line - n * g.Ho;
+			const int ih0 = oh * g.stride_h + g.pad_h, iw0 = ow * g.stride_w + g.pad_w;
+			unsigned int inside = 0;
+			if (row_ok)
 			{
-				const int i = g.flip ? g.R - 1 - f_i : f_i, j = g.flip ? g.S - 1 - f_j : f_j;
-				const unsigned int cb = static_cast<unsigned int>(f_slab) * 32u;
-				const bool live = (left > 0) & (f_tap < taps) & (cb + half < c_bytes);
-				left--;
-				const unsigned int a_tap = static_cast<unsigned int>((i * g.dil_h) * g.W + j * g.dil_w) * c_bytes + cb;
-				const unsigned int b_tap = static_cast<unsigned int>(f_tap) * c_bytes + cb;
-				a[q] = buffer_fetch(rx, (live && ((inside >> (f_tap & 31)) & 1u)) ? a_origin + a_tap : OUT_OF_RANGE);
-				b[q] = buffer_fetch(rw, (live && b_origin != OUT_OF_RANGE) ? b_origin + b_tap : OUT_OF_RANGE);
-				if (++f_slab == g.slabs_per_tap)
+				unsigned int cols = 0;
+				for (int j = 0; j < g.S; j++)
 				{
-					f_slab = 0;
-					f_tap++;
-					if (++f_j == g.S)
-					{
-						f_j = 0;
-						f_i++;
-					}
+					const int iw = iw0 + (g.flip ? g.S - 1 - j : j) * g.dil_w;
+					if (iw >= 0 && iw < g.W)
+						cols |= 1u << j;
+				}
+				for (int i = 0; i < g.R; i++)
+				{
+					const int ih = ih0 + (g.flip ? g.R - 1 - i : i) * g.dil_h;
+					if (ih >= 0 && ih < g.H)
+						inside |= cols << (i * g.S);
 				}
 			}
+			pixel[lane] = make_uint2(static_cast<unsigned int>((n * g.H + ih0) * g.W + iw0) * c_bytes, inside);
+		}
+		wave_order();
+		/* this lane loads chunk (lane % 8) of the rows 8 i + lane / 8: eight lanes read the 128 bytes of a row together */
+		const int load_row = lane >> 3, load_chunk = lane & 7;
+		uint2 origin[LOADS];
+#pragma unroll
+		for (int i = 0; i < LOADS; i++)
+			origin[i] = pixel[8 * i + load_row];
+		wave_order();
+		const unsigned int w_origin = static_cast<unsigned int>(k0 + load_row) * filter_bytes; /* filters past the last lie outside the buffer */
+
+		typename Mma<TE>::acc_t acc[T][T]; /* [filters][pixels] */
+#pragma unroll
+		for (int i = 0; i < T; i++)
+#pragma unroll
+			for (int j = 0; j < T; j++)
+#pragma unroll
+				for (int v = 0; v < 16; v++)
+					acc[i][j][v] = 0;
+
+		/* k = the 16-byte chunks of (tap, channel) in a row, eight a stage; each wavefront takes a contiguous share of the stages */
+		const int chunks = g.R * g.S * g.chunks_per_tap;
+		const int stages = (chunks + 7) / 8;
+		const int share = (stages + KW - 1) / KW;
+		const int first = wave * share;
+		const int count = stages - first < share ? stages - first : share; /* may be negative: nothing left for this wavefront */
+		const unsigned int chunks_mine = count > 0 ? (chunks < 8 * (first + count) ? chunks : 8 * (first + count)) : 0;
+		unsigned int chunk = 8 * first + load_chunk;
+		auto fetch = [&](uint4 (&xs)[LOADS], uint4 (&ws)[LOADS]) __attribute__((always_inline))
+		{
+			const bool live = chunk < chunks_mine;
+			const unsigned int tap = __umulhi(chunk, g.by_chunks), c = chunk - tap * g.chunks_per_tap;
+			const unsigned int ti = (tap * g.by_s) >> 16, tj = tap - ti * g.S;
+			const unsigned int i = g.flip ? g.R - 1 - ti : ti, j = g.flip ? g.S - 1 - tj : tj;
+			const unsigned int x_tap = ((i * g.dil_h) * g.W + j * g.dil_w) * c_bytes + 16 * c;
+			const unsigned int bit = live ? 1u << (tap & 31) : 0u;
+			const unsigned int w_at = live ? w_origin + 16 * chunk : OUT_OF_RANGE;
+			chunk += 8;
+#pragma unroll
+			for (int q = 0; q < LOADS; q++)
+				xs[q] = buffer_fetch(rx, (origin[q].y & bit) ? origin[q].x + x_tap : OUT_OF_RANGE);
+#pragma unroll
+			for (int q = 0; q < LOADS; q++)
+				ws[q] = buffer_fetch(rw, live ? w_at + 8 * q * filter_bytes : OUT_OF_RANGE);
 		};
-		auto multiply = [&](const uint4 (&a)[GROUP], const uint4 (&b)[GROUP]) __attribute__((always_inline))
+		uint4 xs[DEPTH][LOADS], ws[DEPTH][LOADS];
+#pragma unroll
+		for (int d = 0; d < DEPTH; d++)
+			fetch(xs[d], ws[d]);
+
+		/* what the epilogue needs is requested behind the first operands and arrives with them */
+		constexpr int ROWS = 64 * KW / QUADS; /* pixels handed over in one pass of the workgroup */
+		constexpr int PASSES = (SIDE + ROWS - 1) / ROWS;
+		const int quad = static_cast<int>(threadIdx.x) % QUADS, row0 = static_cast<int>(threadIdx.x) / QUADS;
+		const int kcol = k0 + 4 * quad;
+		typename Epi::Columns columns;
+		epi.load_columns(kcol, columns);
+		typename Epi::template Residual<4> residual[PASSES];
+		if (VEC)
 		{
 #pragma unroll
-			for (int q = 0; q < GROUP; q++)
+			for (int pass = 0; pass < PASSES; pass++)
 			{
-				Chunk ca, cb;
-				ca.u = a[q];
-				cb.u = b[q];
-				Mma<TE>::run(ca, cb, acc);
+				const int row = row0 + ROWS * pass;
+				if (row < SIDE && p0 + row < g.pixels && kcol < g.K)
+					epi.template load_residual<4>(static_cast<int64_t>(p0 + row) * g.K + kcol, residual[pass]);
 			}
-		};
-		uint4 a0[GROUP], b0[GROUP], a1[GROUP], b1[GROUP];
-		fetch(a0, b0);
-		for (int s = 0; s < groups; s += 2)
-		{
-			fetch(a1, b1); /* zeros past the last slab */
-			multiply(a0, b0);
-			fetch(a0, b0);
-			multiply(a1, b1);
 		}
 
-		/* lane holds column r, rows 8 i + 4 (lane / 32) + j of its wavefront's partial tile; after the transpose through LDS a
-		 * work-item owns 4 consecutive columns of a row and adds up the KW partial tiles */
-		typename Epi::scalar_t *mine = sm + wave * (SMALL_TILE * SMALL_PITCH);
-#pragma unroll
-		for (int i = 0; i < 4; i++)
-#pragma unroll
-			for (int j = 0; j < 4; j++)
-				mine[(8 * i + 4 * (lane >> 5) + j) * SMALL_PITCH + r] = acc[4 * i + j];
-		__syncthreads();
-#pragma unroll
-		for (int it = 0; it < 4 / KW; it++)
+		/* LDS rows of 128 bytes, filters behind pixels; chunk c of row r lies in column c ^ (r / 2) % 8: conflict-free to write by rows
+		 * and to read by columns.  A wavefront's LDS accesses are done in their order and nobody else touches its part, so the next
+		 * stage may be written as soon as the reads of this one are issued: no barrier. */
+		const int put = load_row * 8 + (load_chunk ^ (load_row >> 1)); /* rows 8 i + load_row, i even; i odd: column ^ 4 */
+		const int r = lane & 31, half = lane >> 5;
+		for (int s = 0; s < count; s += DEPTH)
 		{
-			const int row = (static_cast<int>(threadIdx.x) >> 3) + 8 * KW * it;
-			typedef Pack<typename Epi::scalar_t, 4> P4;
-			P4 v = *reinterpret_cast<const P4*>(sm + row * SMALL_PITCH + (threadIdx.x & 7) * 4);
 #pragma unroll
-			for (int part = 1; part < KW; part++)
+			for (int d = 0; d < DEPTH; d++)
 			{
-				const P4 o = *reinterpret_cast<const P4*>(sm + part * (SMALL_TILE * SMALL_PITCH) + row * SMALL_PITCH + (threadIdx.x & 7) * 4);
 #pragma unroll
-				for (int q = 0; q < 4; q++)
-					v.v[q] += o.v[q];
+				for (int q = 0; q < LOADS; q++)
+				{
+					mine[64 * q + (q & 1 ? put ^ 4 : put)] = xs[d][q];
+					mine[8 * SIDE + 64 * q + (q & 1 ? put ^ 4 : put)] = ws[d][q];
+				}
+				wave_order();
+				fetch(xs[d], ws[d]); /* nothing behind the last stage */
+#pragma unroll
+				for (int slab = 0; slab < 4; slab++)
+				{
+					Chunk cw[T], cx[T];
+					const int get = r * 8 + ((2 * slab + half) ^ ((r >> 1) & 7));
+#pragma unroll
+					for (int t = 0; t < T; t++)
+					{
+						cx[t].u = mine[256 * t + get];
+						cw[t].u = mine[8 * SIDE + 256 * t + get];
+					}
+#pragma unroll
+					for (int i = 0; i < T; i++)
+#pragma unroll
+						for (int j = 0; j < T; j++)
+							Mma<TE>::run(cw[i], cx[j], acc[i][j]);
+				}
+				wave_order();
+			}
+		}
+
+		/* a lane holds, of pixel r of each pixel tile, the filters 8 v + 4 (lane / 32) .. + 3 of each filter tile */
+		quad_t *part = reinterpret_cast<quad_t*>(mine);
+#pragma unroll
+		for (int i = 0; i < T; i++)
+#pragma unroll
+			for (int j = 0; j < T; j++)
+#pragma unroll
+				for (int v = 0; v < 4; v++)
+				{
+					quad_t q;
+#pragma unroll
+					for (int e = 0; e < 4; e++)
+						q.v[e] = acc[i][j][4 * v + e];
+					part[(8 * i + 2 * v + half) * PITCH + 32 * j + r] = q;
+				}
+		__syncthreads();
+		auto hand_over = [&](int pass) __attribute__((always_inline))
+		{
+			const int row = row0 + ROWS * pass;
+			if (ROWS > SIDE && row >= SIDE)
+				return;
+			quad_t v = reinterpret_cast<const quad_t*>(lds[0])[quad * PITCH + row];
+#pragma unroll
+			for (int k = 1; k < KW; k++)
+			{
+				const quad_t o = reinterpret_cast<const quad_t*>(lds[k])[quad * PITCH + row];
+#pragma unroll
+				for (int e = 0; e < 4; e++)
+					v.v[e] += o.v[e];
 			}
 			if (p0 + row < g.pixels && kcol < g.K)
-				epi.template store<ACT_SIMPLE, true>(p0 + row, kcol, v.v, columns);
+				epi.template store_at<ACT, VEC, 4>(static_cast<int64_t>(p0 + row) * g.K + kcol, kcol, v.v, columns, VEC ? &residual[VEC ? pass : 0] : nullptr);
+		};
+		if constexpr (ACT == ACT_SIMPLE)
+		{
+#pragma unroll
+			for (int pass = 0; pass < PASSES; pass++)
+				hand_over(pass);
+		}
+		else
+		{
+#pragma unroll 1 /* the switch over the activations once, not once per pass */
+			for (int pass = 0; pass < PASSES; pass++)
+				hand_over(pass);
 		}
 	}
 }
 
 namespace
 {
-	/* below this many big workgroups most of the 256 compute units would idle */
+	/* only problems of fewer 128 x 128 tiles than this are candidates at all */
 	std::atomic<int>& small_problem_threshold()
 	{
-		static std::atomic<int> value(192);
+		static std::atomic<int> value(4096);
 		return value;
+	}
+	constexpr SmallPlan PLANS[] = { { 1, 1, 0.0 }, { 1, 4, 0.0 }, { 1, 8, 0.0 }, { 2, 4, 0.0 } };
+
+	struct Pace
+	{
+		double launch, chain, stage, tile;
+	};
+	/* Microseconds, fitted to 320 layers of all types (7 to 64 rows and columns, 16 to 512 channels and filters, 1x1 to 5x5, up to
+	 * 12 GFLOP; root mean square error 6 to 14 %): launch and first loads, one stage of a wavefront alone, one stage of a tile when its
+	 * compute unit is busy, and everything else about a tile.  Order of PLANS. */
+	constexpr Pace PACE_16[] = { { 4.99, 0.303, 0.107, 0.20 }, { 3.34, 0.409, 0.084, 0.90 }, { 2.64, 0.173, 0.091, 2.40 }, { 3.41, 0.88, 0.182, 1.86 } };
+	constexpr Pace PACE_32[] = { { 5.09, 0.662, 0.197, 0.27 }, { 3.62, 0.767, 0.164, 1.15 }, { 2.55, 0.162, 0.164, 3.24 }, { 1.66, 2.39, 0.528, 3.38 } };
+
+	/* What the kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles take, in microseconds, fitted to the same layers
+	 * (errors of 6 to 18 %).  `plain`: LINEAR or RELU and whole vectors of filters; everything else runs in the gather kernel, whose
+	 * hand-over is slow there. */
+	double workgroup_tiles_us(const avhipConvShape &s, int element_bytes, bool plain)
+	{
+		const bool fp32 = element_bytes == 4;
+		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
+		const double steps = static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 127) / 128);
+		const double tiles = std::ceil(pixels / 128.0) * ((s.K + 127) / 128), rounds = std::ceil(tiles / 512.0);
+		const bool dense = s.stride_h == 1 && s.stride_w == 1 && s.dil_h == 1 && s.dil_w == 1;
+		if (plain && dense && s.R * s.S > 1 && s.K % 8 == 0 && s.Ho * s.Wo >= 128)
+		{
+			/* image-tile kernel: a workgroup with a compute unit to itself, or sharing one */
+			const double workgroups = static_cast<double>(s.N) * ((s.K + 63) / 64) * ((s.Ho * s.Wo + 255) / 256);
+			const double pace = fp32 ? (workgroups <= 256.0 ? 2.0 : 3.3) : (workgroups <= 256.0 ? 0.47 : 0.68);
+			return std::ceil(workgroups / 512.0) * (3.6 + pace * steps);
+		}
+		if (plain && dense && s.R * s.S == 1 && steps <= 4.0) /* the persistent one-tap kernels */
+			return 4.5 + tiles * steps / 512.0 * (fp32 ? 6.0 : 1.4) + pixels * s.K * (element_bytes == 2 ? 2.0 : 4.0) / 6.0e6;
+		if (!plain)
+			return rounds * (18.0 + steps * (fp32 ? (tiles <= 256.0 ? 2.3 : 3.6) : (tiles <= 256.0 ? 0.70 : 0.85)));
+		return (fp32 ? 7.0 : 8.0) + rounds * steps * (fp32 ? (tiles <= 256.0 ? 2.1 : 3.0) : (tiles <= 256.0 ? 0.65 : 1.1));
 	}
 }
 
@@ -185,48 +315,58 @@ extern "C" int avhip_set_small_problem_threshold(int workgroups)
 
 namespace avhip
 {
-	/* Small in tiles is not enough: the problem must be short in k as well.  A wavefront fetches its own operands, one 32-byte
-	 * slab of both per MFMA with no re-use inside a workgroup: measured about 0.12 us per slab, plus 0.19 us per slab and
-	 * wavefront per SIMD as the tiles crowd L2 (a 3x3 layer of 256 channels on 32 images of 14 x 14 took 59 us here and 19 us in
-	 * the image-tile kernel with half the compute units idle).  The workgroup-tile kernels take about 0.7 us per 128-byte
-	 * k-step and 4 us around the loop, per round of 512 workgroups. */
-	SmallProblemEstimate conv_small_estimate(const avhipConvShape &s, int element_bytes, int64_t big_tile_workgroups)
+	/* Tile and number of wavefronts by the estimates above.  Where the lines lie: 1 wavefront for thousands of tiles with a short k
+	 * (bf16 1x1, 107632 pixels, one stage: 13.8 us against 20.0 with four), 64 x 64 tiles where they alone fill the chip (bf16 256 ->
+	 * 256 on 3800 pixels: 13.8 us against 19.2), 8 wavefronts for few tiles and a long k (fp32, 40 tiles, 325 stages: 56 us against
+	 * 68), otherwise 4. */
+	SmallPlan conv_small_plan(const avhipConvShape &s, int element_bytes)
 	{
-		const int64_t pixels = static_cast<int64_t>(s.N) * s.Ho * s.Wo;
-		const int64_t tiles = ((pixels + SMALL_TILE - 1) / SMALL_TILE) * ((static_cast<int64_t>(s.K) + SMALL_TILE - 1) / SMALL_TILE);
-		const int slabs_per_tap = (s.C * element_bytes + 31) / 32;
-		SmallProblemEstimate e;
-		/* fewer tiles than half the 1024 SIMDs of the chip, and enough k to share: four wavefronts per tile */
-		e.split_k = tiles < 512 && static_cast<int64_t>(s.R) * s.S * slabs_per_tap >= 4 * GROUP;
-		const double wavefronts = static_cast<double>(tiles) * (e.split_k ? 4 : 1);
-		const double slabs = static_cast<double>(s.R) * s.S * slabs_per_tap / (e.split_k ? 4 : 1);
-		e.small_us = 2.5 + slabs * (0.12 + 0.19 * wavefronts / 1024.0);
-		const double k_steps = static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 127) / 128);
-		e.workgroup_tiles_us = static_cast<double>((big_tile_workgroups + 511) / 512) * (0.7 * k_steps + 4.0);
-		return e;
+		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
+		const double stages = std::ceil(static_cast<double>(s.R) * s.S * s.C * element_bytes / 128.0);
+		SmallPlan best = { 0, 0, 0.0 };
+		for (int i = 0; i < 4; i++)
+		{
+			const int side = SMALL_TILE * PLANS[i].tiles;
+			const Pace &pace = element_bytes == 4 ? PACE_32[i] : PACE_16[i];
+			const double tiles = std::ceil(pixels / side) * ((s.K + side - 1) / side);
+			const double per_cu = tiles <= 1024.0 ? std::ceil(tiles / 256.0) : tiles / 256.0;
+			const double us = pace.launch + std::max(std::ceil(stages / PLANS[i].waves) * pace.chain, per_cu * stages * pace.stage) + per_cu * pace.tile;
+			if (best.tiles == 0 || us < best.us)
+				best = { PLANS[i].tiles, PLANS[i].waves, us };
+		}
+		return best;
 	}
-	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, int64_t big_tile_workgroups)
+	/* taps in a mask; exact division of a chunk's number by multiplication */
+	bool conv_small_possible(const avhipConvShape &s, int element_bytes)
 	{
-		const int64_t busy = small_problem_threshold().load(std::memory_order_relaxed);
-		if (busy < 0) /* asked for by name (tests): whatever the kernel can run */
-			return true;
-		if (big_tile_workgroups >= busy)
+		const int64_t chunks = static_cast<int64_t>(s.C) * element_bytes / 16;
+		return s.R * s.S <= 32 && chunks >= 2 && chunks <= 8192;
+	}
+	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, bool plain)
+	{
+		if (!conv_small_possible(s, element_bytes))
 			return false;
-		const SmallProblemEstimate e = conv_small_estimate(s, element_bytes, big_tile_workgroups);
-		return e.small_us <= e.workgroup_tiles_us;
+		const int threshold = small_problem_threshold().load(std::memory_order_relaxed);
+		if (threshold < 0) /* asked for by name (tests): whatever the kernel can run */
+			return true;
+		const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
+		return tiles < threshold && conv_small_plan(s, element_bytes).us < 0.95 * workgroup_tiles_us(s, element_bytes, plain);
 	}
 
 	template<typename TE, typename Epi>
-	bool conv_small_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi, int64_t big_tile_workgroups)
+	bool conv_small_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi)
 	{
+		constexpr int SZ = static_cast<int>(sizeof(TE));
 		const int64_t pixels = static_cast<int64_t>(s.N) * s.Ho * s.Wo;
-		if (!conv_small_preferred(s, static_cast<int>(sizeof(TE)), big_tile_workgroups) || !epi.vec || s.R * s.S > 32)
+		/* whole 4-filter vectors and LINEAR / RELU, or anything (the integer epilogues know no other activation) */
+		const bool simple = epi.vec && is_simple_activation(epi.activation);
+		if (!conv_small_preferred(s, SZ, simple))
 			return false;
-		const int64_t tiles = (pixels + SMALL_TILE - 1) / SMALL_TILE, filter_tiles = (static_cast<int64_t>(s.K) + SMALL_TILE - 1) / SMALL_TILE;
-		if (tiles > 0x7FFFFFFFll || filter_tiles > 65535 || pixels >= (1ll << 31) - SMALL_TILE)
+		const SmallPlan plan = conv_small_plan(s, SZ);
+		const int side = SMALL_TILE * plan.tiles;
+		const int64_t pixel_tiles = (pixels + side - 1) / side, filter_tiles = (static_cast<int64_t>(s.K) + side - 1) / side;
+		if (pixel_tiles > 0x7FFFFFFFll || filter_tiles > 65535 || pixel_tiles * filter_tiles > 0x7FFFFFFFll || pixels >= (1ll << 31) - side)
 			return false;
-		const int slabs_per_tap = (s.C * static_cast<int>(sizeof(TE)) + 31) / 32;
-		const bool split_k = conv_small_estimate(s, static_cast<int>(sizeof(TE)), big_tile_workgroups).split_k;
 		SmallGeom g;
 		g.H = s.H;
 		g.W = s.W;
@@ -243,19 +383,34 @@ namespace avhip
 		g.dil_h = s.dil_h;
 		g.dil_w = s.dil_w;
 		g.flip = s.mode != 0 ? 1 : 0;
-		g.slabs_per_tap = slabs_per_tap;
+		g.chunks_per_tap = s.C * SZ / 16;
+		g.by_chunks = static_cast<unsigned int>(((1ll << 32) + g.chunks_per_tap - 1) / g.chunks_per_tap);
+		g.by_s = (65536 + s.S - 1) / s.S;
 		g.pixels = static_cast<int>(pixels);
 		g.images = s.N;
-		const dim3 grid(static_cast<unsigned int>(tiles), static_cast<unsigned int>(filter_tiles));
-		/* fewer tiles than half the 1024 SIMDs of the chip, and enough k to share: four wavefronts per tile */
-		if (split_k)
-			hipLaunchKernelGGL((k_conv_small<TE, Epi, 4>), grid, dim3(256), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi);
+		g.pixels_first = static_cast<int64_t>(s.K) * s.R * s.S > static_cast<int64_t>(s.N) * s.H * s.W ? 1 : 0;
+		const dim3 grid(static_cast<unsigned int>(pixel_tiles), static_cast<unsigned int>(filter_tiles));
+#define AVHIP_SMALL(T, KW) \
+		do \
+		{ \
+			if (simple) \
+				hipLaunchKernelGGL((k_conv_small<TE, Epi, T, KW, ACT_SIMPLE>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
+			else \
+				hipLaunchKernelGGL((k_conv_small<TE, Epi, T, KW, ACT_ANY>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
+		} while (0)
+		if (plan.tiles == 2)
+			AVHIP_SMALL(2, 4);
+		else if (plan.waves == 8)
+			AVHIP_SMALL(1, 8);
+		else if (plan.waves == 4)
+			AVHIP_SMALL(1, 4);
 		else
-			hipLaunchKernelGGL((k_conv_small<TE, Epi, 1>), grid, dim3(64), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi);
+			AVHIP_SMALL(1, 1);
+#undef AVHIP_SMALL
 		return true;
 	}
 
-#define AVHIP_INSTANTIATE(TE, EPI) template bool conv_small_launch<TE, EPI>(hipStream_t, const avhipConvShape&, const void*, const void*, const EPI&, int64_t);
+#define AVHIP_INSTANTIATE(TE, EPI) template bool conv_small_launch<TE, EPI>(hipStream_t, const avhipConvShape&, const void*, const void*, const EPI&);
 	AVHIP_INSTANTIATE(float, FloatEpilogue<float>)
 	AVHIP_INSTANTIATE(f16_t, FloatEpilogue<f16_t>)
 	AVHIP_INSTANTIATE(bf16_t, FloatEpilogue<bf16_t>)

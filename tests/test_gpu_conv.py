@@ -16,8 +16,8 @@ BAR = {"f32": 1e-5, "f16": 2e-3, "bf16": 2e-3}
 
 @pytest.fixture(autouse=True, params=["wavefront_tiles", "workgroup_tiles"])
 def tiling(request):
-    """Every test runs twice: with the kernel that gives each wavefront one 32 x 32 tile forced for whatever it can run
-    (the launcher itself picks it for problems small in tiles and short in k), and with that kernel switched off, so that
+    """Every test runs twice: with the kernel of small tiles (32 x 32 or 64 x 64, k shared by wavefronts) forced for whatever it can run
+    (the launcher itself picks it for problems that do not fill the chip with large ones), and with that kernel switched off, so that
     the same geometry goes through the 128 x 128 gather kernel, the image-tile kernel or the few-channel kernels."""
     lib = cb.load_library()
     lib.avhip_set_small_problem_threshold.restype = int
@@ -43,6 +43,45 @@ def test_implicit_gemm_config1(oracle, dtype):
     err = oracle.rel_l2(got, want)
     print("implicit gemm %s rel-L2 = %.3e" % (dtype, err))
     assert err < BAR[dtype]
+
+
+SMALL_TILE_CASES = [
+    # the four forms of the kernel with small tiles (tile side, wavefronts that share k), as its estimates pick them
+    dict(x=(40, 36, 36, 32), w=(36, 1, 1, 32), dtype="bf16"),                                              # 32, 1: thousands of tiles, one stage
+    dict(x=(3, 31, 31, 136), w=(252, 3, 3, 136), pad=(-1, -1), dtype="f16", z=True, act="ELU"),            # 64, 4: ragged both ways, 20 stages
+    dict(x=(3, 31, 29, 136), w=(256, 3, 3, 136), pad=(-1, -1), dtype="i8"),
+    dict(x=(1, 9, 9, 200), w=(36, 5, 5, 200), pad=(-2, -2), dtype="f32", z=True),                          # 32, 8: long k, last wavefront short
+    dict(x=(5, 9, 7, 24), w=(23, 3, 2, 24), pad=(-1, 0), dtype="f32", act="TANH", z=True),                 # 32, 4: 3 chunks left in the last stage
+    dict(x=(5, 13, 11, 40), w=(64, 5, 5, 40), pad=(-4, -4), stride=(2, 1), dilation=(2, 2), mode=1, dtype="bf16", z=True),
+    dict(x=(2, 7, 7, 16), w=(8, 4, 8, 16), pad=(-3, -7), dtype="bf16", act="SIGMOID"),                     # 32 taps, 2 chunks each
+    dict(x=(1, 3, 3, 48), w=(4, 1, 1, 48), dtype="i8"),                                                    # less than one stage, 9 pixels
+]
+
+
+@pytest.mark.parametrize("case", range(len(SMALL_TILE_CASES)))
+def test_small_tile_forms(oracle, case):
+    """Bars as above (one fp32 sum per output, one rounding on store); integer sums bit-exact."""
+    c = SMALL_TILE_CASES[case]
+    g = h.rng(90 + case)
+    N, H, W, Cin = c["x"]
+    K, R, S, _ = c["w"]
+    geometry = {"pad": (0, 0), **{key: c[key] for key in ("pad", "stride", "dilation", "mode") if key in c}}
+    (ph, pw), (sh, sw), (dh, dw) = c.get("pad", (0, 0)), c.get("stride", (1, 1)), c.get("dilation", (1, 1))
+    ys = (N, (H - 2 * ph - ((R - 1) * dh + 1)) // sh + 1, (W - 2 * pw - ((S - 1) * dw + 1)) // sw + 1, K)
+    if c["dtype"] == "i8":
+        x, w = g.integers(-127, 128, c["x"], dtype=np.int8), g.integers(-127, 128, c["w"], dtype=np.int8)
+        b = g.integers(-2 ** 15, 2 ** 15, K).astype(np.int32)
+        got = h.conv_forward("implicit_gemm", x, w, ys, "i8", y_dtype="i32", bias=b, bias_dtype="i32", **geometry)
+        np.testing.assert_array_equal(got, oracle.conv2d_i8(x, w, b, **geometry))
+        return
+    x = h.rounded(oracle, g.standard_normal(c["x"]), c["dtype"])
+    w = he(g, c["w"], c["dtype"], oracle)
+    b = g.uniform(-0.1, 0.1, K).astype(np.float32).astype(np.float64)
+    z = h.rounded(oracle, g.standard_normal(ys), c["dtype"]) if c.get("z") else None
+    act = getattr(cb, "ACTIVATION_" + c.get("act", "RELU"))
+    got = h.conv_forward("implicit_gemm", x, w, ys, c["dtype"], bias=b, z=z, activation=act, **geometry)
+    want = oracle.conv2d(x, w, b, z, activation=act, **geometry)
+    assert oracle.rel_l2(got, want) < BAR[c["dtype"]]
 
 
 CASES = [
