@@ -629,6 +629,9 @@ namespace
 		 * at 64 (half a k-step per tap) the kernels below are the faster ones, measured on 3x3 layers of 64 int8 / 32 bf16 / 16 fp32
 		 * channels (12 against 28 us, 21 against 52 us, 82 against 113 us); at 48 and 32 bytes these are (16 against 22 us, 13 against 22 us) */
 		const int pixel_bytes = s.C * static_cast<int>(sizeof(TE));
+		/* channels that are no whole number of 16-byte chunks: of the kernels below the few-channel ones and that of small tiles take them.
+		 * (The latter before the packed gather: fp16 3 -> 32 3x3 stride 2 on 1152 pixels 16.7 us there, 6.0 here) */
+		const bool ragged = pixel_bytes % 16 != 0 && aligned_to(x, 16) && aligned_to(w, 16) && fast_path_ok<TE>(s, 1, padding_value);
 		if (pixel_bytes < STEP_BYTES / 2 && s.R * s.S > 1 && fast_path_ok<TE>(s, 1, padding_value, false) && is_simple_activation(epi.activation)
 				&& (flags & 2) != 0)
 		{
@@ -637,6 +640,8 @@ namespace
 				return 0;
 			/* the image tile in LDS, the operand gathered from there: filters of any number of taps */
 			if (conv_thin_launch<TE, Epi>(st, s, x, w, epi))
+				return 0;
+			if (ragged && conv_small_launch<TE, Epi>(st, s, x, w, epi))
 				return 0;
 			int pb = 16;
 			while (pb > 1 && (pixel_bytes % pb != 0 || !aligned_to(x, pb) || !aligned_to(w, pb)))
@@ -663,7 +668,7 @@ namespace
 #undef AVHIP_PACKED
 		}
 		/* a problem that does not fill the chip with big tiles goes to the kernel with small ones and k shared by wavefronts */
-		if (fast_path_ok<TE>(s, flags, padding_value) && conv_small_launch<TE, Epi>(st, s, x, w, epi))
+		if ((ragged || fast_path_ok<TE>(s, flags, padding_value)) && conv_small_launch<TE, Epi>(st, s, x, w, epi))
 			return 0;
 		/* one-tap filters are plain matrix products with a short k: a persistent kernel pipelines across tiles */
 		if (fast && s.R * s.S == 1 && conv_pointwise_launch<TE, Epi>(st, s, x, w, epi))

@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <type_traits>
 
 #include "conv_small.hpp"
 #include "mfma_core.hpp"
@@ -42,8 +43,50 @@ namespace
 		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 	}
 
+	/* What the rows of channels (one pixel, one tap of a filter) are known to be: whole 16-byte chunks; dwords; elements. */
+	constexpr int ROWS_OF_CHUNKS = 0, ROWS_OF_DWORDS = 1, ROWS_OF_ELEMENTS = 2;
+
+	/* 16 bytes on their way from memory, from any byte on if ROW is ROWS_OF_ELEMENTS: then they are the aligned dwords around them */
+	template<int ROW>
+	struct Piece
+	{
+		uint4 u;
+		__device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t rsrc, unsigned int offset)
+		{
+			u = buffer_fetch(rsrc, offset);
+		}
+		/* what belongs to the row: `left` bytes of it from the first one on */
+		__device__ __forceinline__ uint4 get(unsigned int, const uint4 &keep) const
+		{
+			if (ROW == ROWS_OF_CHUNKS)
+				return u;
+			return make_uint4(u.x & keep.x, u.y & keep.y, u.z & keep.z, u.w & keep.w);
+		}
+	};
+	template<>
+	struct Piece<ROWS_OF_ELEMENTS>
+	{
+		uint4 u;
+		unsigned int next;
+		__device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t rsrc, unsigned int offset)
+		{
+			u = buffer_fetch(rsrc, offset & ~3u);
+			next = __builtin_amdgcn_raw_buffer_load_b32(rsrc, static_cast<int>((offset & ~3u) + 16), 0, 0);
+		}
+		__device__ __forceinline__ uint4 get(unsigned int offset, const uint4 &keep) const
+		{
+			return make_uint4(__builtin_amdgcn_alignbyte(u.y, u.x, offset & 3) & keep.x, __builtin_amdgcn_alignbyte(u.z, u.y, offset & 3) & keep.y,
+					__builtin_amdgcn_alignbyte(u.w, u.z, offset & 3) & keep.z, __builtin_amdgcn_alignbyte(next, u.w, offset & 3) & keep.w);
+		}
+	};
+	/* which bits of a dword belong to a row that has `left` more bytes */
+	__device__ __forceinline__ unsigned int keep_bits(int left)
+	{
+		return left >= 4 ? ~0u : left <= 0 ? 0u : (1u << (8 * left)) - 1;
+	}
+
 	/* T x T MFMA tiles of 32 x 32 per wavefront, KW wavefronts on one tile. */
-	template<typename TE, typename Epi, int T, int KW, int ACT>
+	template<typename TE, typename Epi, int T, int KW, int ACT, int ROW = ROWS_OF_CHUNKS>
 	__global__ __launch_bounds__(64 * KW, KW == 8 ? 2 : T == 1 ? 3 : 2) void k_conv_small(const TE *__restrict__ x, const TE *__restrict__ w, SmallGeom g, Epi epi)
 	{
 		constexpr unsigned int SZ = sizeof(TE);
@@ -76,8 +119,8 @@ namespace
 		const int p0 = static_cast<int>(pixel_tile) * SIDE, k0 = static_cast<int>(filter_tile) * SIDE;
 
 		const unsigned int c_bytes = g.C * SZ, filter_bytes = g.R * g.S * c_bytes;
-		const __amdgpu_buffer_rsrc_t rx = make_buffer(x, static_cast<unsigned int>(g.images) * g.H * g.W * c_bytes);
-		const __amdgpu_buffer_rsrc_t rw = make_buffer(w, static_cast<unsigned int>(g.K) * filter_bytes);
+		const __amdgpu_buffer_rsrc_t rx = make_buffer(x, (static_cast<unsigned int>(g.images) * g.H * g.W * c_bytes + 3) & ~3u); /* a dword never crosses a page */
+		const __amdgpu_buffer_rsrc_t rw = make_buffer(w, (static_cast<unsigned int>(g.K) * filter_bytes + 3) & ~3u);
 
 		/* origin and border mask (bit = tap inside the image) of one pixel per lane, handed through LDS to the lanes that load it */
 		uint2 *pixel = reinterpret_cast<uint2*>(mine);
@@ -135,27 +178,41 @@ namespace
 		const int count = stages - first < share ? stages - first : share; /* may be negative: nothing left for this wavefront */
 		const unsigned int chunks_mine = count > 0 ? (chunks < 8 * (first + count) ? chunks : 8 * (first + count)) : 0;
 		unsigned int chunk = 8 * first + load_chunk;
-		auto fetch = [&](uint4 (&xs)[LOADS], uint4 (&ws)[LOADS]) __attribute__((always_inline))
+		struct Stage
+		{
+			Piece<ROW> xs[LOADS], ws[LOADS];
+			unsigned int x_tap, w_at; /* not whole chunks: where the pieces start (the lowest two bits are used) */
+			int left; /* and the bytes of the row from there */
+		};
+		auto fetch = [&](Stage &to) __attribute__((always_inline))
 		{
 			const bool live = chunk < chunks_mine;
-			const unsigned int tap = __umulhi(chunk, g.by_chunks), c = chunk - tap * g.chunks_per_tap;
+			/* (one chunk a tap: the factor would be 2^32) */
+			const unsigned int tap = ROW != ROWS_OF_CHUNKS && g.chunks_per_tap == 1 ? chunk : __umulhi(chunk, g.by_chunks);
+			const unsigned int c = chunk - tap * g.chunks_per_tap;
 			const unsigned int ti = (tap * g.by_s) >> 16, tj = tap - ti * g.S;
 			const unsigned int i = g.flip ? g.R - 1 - ti : ti, j = g.flip ? g.S - 1 - tj : tj;
 			const unsigned int x_tap = ((i * g.dil_h) * g.W + j * g.dil_w) * c_bytes + 16 * c;
 			const unsigned int bit = live ? 1u << (tap & 31) : 0u;
-			const unsigned int w_at = live ? w_origin + 16 * chunk : OUT_OF_RANGE;
+			const unsigned int w_at = w_origin + (ROW == ROWS_OF_CHUNKS ? 16 * chunk : tap * c_bytes + 16 * c);
+			if (ROW != ROWS_OF_CHUNKS)
+			{
+				to.x_tap = x_tap;
+				to.w_at = w_at;
+				to.left = static_cast<int>(c_bytes - 16 * c);
+			}
 			chunk += 8;
 #pragma unroll
 			for (int q = 0; q < LOADS; q++)
-				xs[q] = buffer_fetch(rx, (origin[q].y & bit) ? origin[q].x + x_tap : OUT_OF_RANGE);
+				to.xs[q].fetch(rx, (origin[q].y & bit) ? origin[q].x + x_tap : OUT_OF_RANGE);
 #pragma unroll
 			for (int q = 0; q < LOADS; q++)
-				ws[q] = buffer_fetch(rw, live ? w_at + 8 * q * filter_bytes : OUT_OF_RANGE);
+				to.ws[q].fetch(rw, live ? w_at + 8 * q * filter_bytes : OUT_OF_RANGE);
 		};
-		uint4 xs[DEPTH][LOADS], ws[DEPTH][LOADS];
+		Stage stage[DEPTH];
 #pragma unroll
 		for (int d = 0; d < DEPTH; d++)
-			fetch(xs[d], ws[d]);
+			fetch(stage[d]);
 
 		/* what the epilogue needs is requested behind the first operands and arrives with them */
 		constexpr int ROWS = 64 * KW / QUADS; /* pixels handed over in one pass of the workgroup */
@@ -186,14 +243,18 @@ namespace
 #pragma unroll
 			for (int d = 0; d < DEPTH; d++)
 			{
+				/* both operands, so that what lies behind a row (an infinity of the next pixel or tap) counts as nothing */
+				uint4 keep = make_uint4(0, 0, 0, 0);
+				if (ROW != ROWS_OF_CHUNKS)
+					keep = make_uint4(keep_bits(stage[d].left), keep_bits(stage[d].left - 4), keep_bits(stage[d].left - 8), keep_bits(stage[d].left - 12));
 #pragma unroll
 				for (int q = 0; q < LOADS; q++)
 				{
-					mine[64 * q + (q & 1 ? put ^ 4 : put)] = xs[d][q];
-					mine[8 * SIDE + 64 * q + (q & 1 ? put ^ 4 : put)] = ws[d][q];
+					mine[64 * q + (q & 1 ? put ^ 4 : put)] = stage[d].xs[q].get(origin[q].x + stage[d].x_tap, keep);
+					mine[8 * SIDE + 64 * q + (q & 1 ? put ^ 4 : put)] = stage[d].ws[q].get(stage[d].w_at + 8 * q * filter_bytes, keep);
 				}
 				wave_order();
-				fetch(xs[d], ws[d]); /* nothing behind the last stage */
+				fetch(stage[d]); /* nothing behind the last stage */
 #pragma unroll
 				for (int slab = 0; slab < 4; slab++)
 				{
@@ -322,7 +383,7 @@ namespace avhip
 	SmallPlan conv_small_plan(const avhipConvShape &s, int element_bytes)
 	{
 		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
-		const double stages = std::ceil(static_cast<double>(s.R) * s.S * s.C * element_bytes / 128.0);
+		const double stages = std::ceil(static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 15) / 16) / 8.0);
 		SmallPlan best = { 0, 0, 0.0 };
 		for (int i = 0; i < 4; i++)
 		{
@@ -336,11 +397,15 @@ namespace avhip
 		}
 		return best;
 	}
+	static bool whole_chunks(const avhipConvShape &s, int element_bytes)
+	{
+		return static_cast<int64_t>(s.C) * element_bytes % 16 == 0;
+	}
 	/* taps in a mask; exact division of a chunk's number by multiplication */
 	bool conv_small_possible(const avhipConvShape &s, int element_bytes)
 	{
-		const int64_t chunks = static_cast<int64_t>(s.C) * element_bytes / 16;
-		return s.R * s.S <= 32 && chunks >= 2 && chunks <= 8192;
+		const int64_t chunks = (static_cast<int64_t>(s.C) * element_bytes + 15) / 16;
+		return s.R * s.S <= 32 && (chunks >= 2 || !whole_chunks(s, element_bytes)) && chunks <= 8192;
 	}
 	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, bool plain)
 	{
@@ -349,6 +414,8 @@ namespace avhip
 		const int threshold = small_problem_threshold().load(std::memory_order_relaxed);
 		if (threshold < 0) /* asked for by name (tests): whatever the kernel can run */
 			return true;
+		if (!whole_chunks(s, element_bytes)) /* else such layers have the general gather kernel, element by element: 4 to 100 times slower */
+			return threshold != 0;
 		const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
 		return tiles < threshold && conv_small_plan(s, element_bytes).us < 0.95 * workgroup_tiles_us(s, element_bytes, plain);
 	}
@@ -383,30 +450,47 @@ namespace avhip
 		g.dil_h = s.dil_h;
 		g.dil_w = s.dil_w;
 		g.flip = s.mode != 0 ? 1 : 0;
-		g.chunks_per_tap = s.C * SZ / 16;
-		g.by_chunks = static_cast<unsigned int>(((1ll << 32) + g.chunks_per_tap - 1) / g.chunks_per_tap);
+		g.chunks_per_tap = (s.C * SZ + 15) / 16;
+		g.by_chunks = static_cast<unsigned int>(((1ll << 32) + g.chunks_per_tap - 1) / g.chunks_per_tap); /* 1: unused */
 		g.by_s = (65536 + s.S - 1) / s.S;
 		g.pixels = static_cast<int>(pixels);
 		g.images = s.N;
 		g.pixels_first = static_cast<int64_t>(s.K) * s.R * s.S > static_cast<int64_t>(s.N) * s.H * s.W ? 1 : 0;
 		const dim3 grid(static_cast<unsigned int>(pixel_tiles), static_cast<unsigned int>(filter_tiles));
-#define AVHIP_SMALL(T, KW) \
+#define AVHIP_SMALL_PLAN(T, KW, ROW) \
 		do \
 		{ \
 			if (simple) \
-				hipLaunchKernelGGL((k_conv_small<TE, Epi, T, KW, ACT_SIMPLE>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
+				hipLaunchKernelGGL((k_conv_small<TE, Epi, T, KW, ACT_SIMPLE, ROW>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
 			else \
-				hipLaunchKernelGGL((k_conv_small<TE, Epi, T, KW, ACT_ANY>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
+				hipLaunchKernelGGL((k_conv_small<TE, Epi, T, KW, ACT_ANY, ROW>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
 		} while (0)
-		if (plan.tiles == 2)
-			AVHIP_SMALL(2, 4);
-		else if (plan.waves == 8)
-			AVHIP_SMALL(1, 8);
-		else if (plan.waves == 4)
-			AVHIP_SMALL(1, 4);
+#define AVHIP_SMALL(ROW) \
+		do \
+		{ \
+			if (plan.tiles == 2) \
+				AVHIP_SMALL_PLAN(2, 4, ROW); \
+			else if (plan.waves == 8) \
+				AVHIP_SMALL_PLAN(1, 8, ROW); \
+			else if (plan.waves == 4) \
+				AVHIP_SMALL_PLAN(1, 4, ROW); \
+			else \
+				AVHIP_SMALL_PLAN(1, 1, ROW); \
+		} while (0)
+		if (!whole_chunks(s, SZ))
+		{
+			if (SZ == 4 || (SZ == 2 && s.C % 2 == 0))
+			{
+				if constexpr (SZ >= 2)
+					AVHIP_SMALL(ROWS_OF_DWORDS);
+			}
+			else if constexpr (SZ <= 2)
+				AVHIP_SMALL(ROWS_OF_ELEMENTS);
+		}
 		else
-			AVHIP_SMALL(1, 1);
+			AVHIP_SMALL(ROWS_OF_CHUNKS);
 #undef AVHIP_SMALL
+#undef AVHIP_SMALL_PLAN
 		return true;
 	}
 

@@ -10,7 +10,7 @@ namespace avhip
 {
 	/* Launches the kernel and returns true when its estimate for the problem is below that of the kernels with 128 x 128 (or
 	 * 256 x 64) workgroup tiles; returns false without side effects otherwise.  The caller has established the conditions of the
-	 * branch-free loaders (16-byte aligned tensors below 2 GiB, channels a multiple of the 16-byte chunk, zero padding value);
+	 * branch-free loaders (16-byte aligned tensors below 2 GiB, zero padding value);
 	 * any activation and number of filters. */
 	template<typename TE, typename Epi>
 	bool conv_small_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi);

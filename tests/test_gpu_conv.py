@@ -55,6 +55,18 @@ SMALL_TILE_CASES = [
     dict(x=(5, 13, 11, 40), w=(64, 5, 5, 40), pad=(-4, -4), stride=(2, 1), dilation=(2, 2), mode=1, dtype="bf16", z=True),
     dict(x=(2, 7, 7, 16), w=(8, 4, 8, 16), pad=(-3, -7), dtype="bf16", act="SIGMOID"),                     # 32 taps, 2 chunks each
     dict(x=(1, 3, 3, 48), w=(4, 1, 1, 48), dtype="i8"),                                                    # less than one stage, 9 pixels
+    # rows of channels that are no whole number of 16-byte chunks: dwords, then any element
+    dict(x=(3, 31, 31, 134), w=(252, 3, 3, 134), pad=(-1, -1), dtype="f16", z=True, act="ELU"),
+    dict(x=(3, 31, 31, 133), w=(250, 3, 3, 133), pad=(-1, -1), dtype="bf16", z=True),
+    dict(x=(2, 9, 9, 99), w=(36, 5, 5, 99), pad=(-2, -2), stride=(2, 2), dtype="f32"),
+    dict(x=(1, 9, 9, 201), w=(36, 5, 5, 201), pad=(-2, -2), dtype="f16", z=True),
+    dict(x=(5, 9, 7, 1), w=(23, 3, 2, 1), pad=(-1, 0), dtype="bf16", act="TANH", z=True),                  # one chunk a tap
+    dict(x=(5, 9, 7, 3), w=(22, 5, 6, 3), pad=(-4, -4), dilation=(2, 2), mode=1, dtype="f32"),
+    dict(x=(3, 5, 5, 9), w=(8, 1, 1, 9), dtype="f16", act="SIGMOID"),
+    dict(x=(1, 1, 3, 1), w=(1, 1, 1, 1), dtype="bf16"),
+    dict(x=(1, 1, 1, 17), w=(2, 1, 1, 17), dtype="i8"),
+    dict(x=(3, 15, 13, 131), w=(65, 3, 3, 131), pad=(-1, -1), dtype="i8"),
+    dict(x=(3, 15, 13, 6), w=(66, 3, 3, 6), pad=(-1, -1), dtype="i8"),
 ]
 
 
@@ -82,6 +94,18 @@ def test_small_tile_forms(oracle, case):
     got = h.conv_forward("implicit_gemm", x, w, ys, c["dtype"], bias=b, z=z, activation=act, **geometry)
     want = oracle.conv2d(x, w, b, z, activation=act, **geometry)
     assert oracle.rel_l2(got, want) < BAR[c["dtype"]]
+
+
+@pytest.mark.parametrize("dtype, c", [("f32", 35), ("f16", 38), ("bf16", 37)])
+def test_an_infinity_stays_with_its_pixel_and_filter(dtype, c):
+    """Rows of channels that end within a 16-byte chunk: what lies behind them (the next pixel, tap or filter) must not reach the sum."""
+    g = h.rng(c)
+    x, w = g.standard_normal((2, 6, 5, c)).astype(np.float32), g.standard_normal((9, 1, 1, c)).astype(np.float32)
+    x[0, 2, 3, 0], x[1, 0, 0, 1], w[4, 0, 0, 0] = np.inf, np.nan, -np.inf
+    finite = np.isfinite(h.conv_forward("implicit_gemm", x, w, (2, 6, 5, 9), dtype, pad=(0, 0)))
+    want = np.ones((2, 6, 5, 9), bool)
+    want[0, 2, 3] = want[1, 0, 0] = want[..., 4] = False
+    np.testing.assert_array_equal(finite, want)
 
 
 CASES = [
