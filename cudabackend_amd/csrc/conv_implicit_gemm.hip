@@ -791,6 +791,7 @@ namespace
 	{
 		int splits, steps_per_split;
 		int64_t bytes;
+		double us;
 	};
 	template<typename TE>
 	bool split_k_plan(const avhipConvShape &s, SplitPlan &plan)
@@ -825,8 +826,13 @@ namespace
 		const double chip = sizeof(TE) == 4 ? 1.55e8 : 1.87e9;
 		const double flops = 2.0 * static_cast<double>(pixels) * s.K * s.C * s.R * s.S;
 		other = std::max(other, flops / (chip * std::min(1.0, static_cast<double>(plain_workgroups) / 256.0)));
-		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true))
-			other = std::min(other, conv_small_plan(s, static_cast<int>(sizeof(TE))).us);
+		/* A wavefront on a 32 x 32 tile of its own, or four sharing its k: what decides which layers are offered a workspace (callers size
+		 * theirs by it).  Whether one is used is weighed again at the launch, against the small-tile kernel as it is. */
+		const double small_tiles = static_cast<double>((pixels + 31) / 32 * ((s.K + 31) / 32)), slabs = static_cast<double>(s.R) * s.S * ((s.C * sizeof(TE) + 31) / 32);
+		const double shared = small_tiles < 512.0 && slabs >= 16.0 ? 4.0 : 1.0;
+		const double small = 2.5 + slabs / shared * (0.12 + 0.19 * small_tiles * shared / 1024.0);
+		if (tiles < 192 && small <= 0.7 * static_cast<double>(steps) + 4.0)
+			other = std::min(other, std::max(small, flops / (chip * std::min(1.0, small_tiles / 1024.0))));
 		const double walk = std::max(0.7 * static_cast<double>(per_part), flops / (chip * std::min(1.0, static_cast<double>(tiles * parts) / 256.0)));
 		const double split = 10.0 + walk + 0.25 * static_cast<double>(parts) + plane_bytes * static_cast<double>(parts + 1) / 4.0e6;
 		if (split > 0.85 * other)
@@ -834,6 +840,7 @@ namespace
 		plan.splits = static_cast<int>(parts);
 		plan.steps_per_split = static_cast<int>(per_part);
 		plan.bytes = static_cast<int64_t>(plane_bytes) * parts;
+		plan.us = split;
 		return true;
 	}
 	template<typename TE>
@@ -845,6 +852,8 @@ namespace
 		if (!split_k_plan<TE>(s, plan) || !fast_path_ok<TE>(s, flags, padding_value) || (flags & 2) == 0 || workspace == nullptr
 				|| workspace_bytes < plan.bytes || !aligned_to(workspace, 16))
 			return AVHIP_NOT_SUPPORTED;
+		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true) && plan.us > 0.85 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us)
+			return AVHIP_NOT_SUPPORTED; /* fewer launches and no faster */
 		const ConvGeom g = make_geom<TE>(s);
 		const dim3 grid(ceil_div(g.pixels, BLOCK_M), ceil_div(s.K, BLOCK_N), static_cast<unsigned int>(plan.splits));
 		hipLaunchKernelGGL((k_conv_igemm_split<TE>), grid, dim3(256), 0, st, static_cast<const TE*>(x), static_cast<const TE*>(w), g, plan.steps_per_split,
