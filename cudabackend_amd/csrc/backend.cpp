@@ -27,6 +27,7 @@
 
 #include "../../include/avocado_hip_backend.h"
 #include "../../include/avocado_hip_kernels.h"
+#include "conv_winograd_f4.hpp"
 
 namespace
 {
@@ -482,7 +483,8 @@ namespace
 		av_int64 offset;
 		int K, C, dtype, mode, m; /* m: Winograd output tile, 2 = F(2x2,3x3) for the fused kernel, 4 = F(4x4,3x3) for the non-fused plan,
 		                           * 1 = F(2,3) along rows in the operand layout of the row-Winograd kernel, 3 = the weights themselves in the
-		                           * operand layout of the stride-2 kernel (no transform) */
+		                           * operand layout of the stride-2 kernel (no transform), 5 likewise of the pixel-block kernel, 6 = F(4x4,3x3) in the
+		                           * operand layout of the one-kernel plan */
 		bool operator<(const WeightKey &o) const
 		{
 			return std::tie(uid, offset, K, C, dtype, mode, m) < std::tie(o.uid, o.offset, o.K, o.C, o.dtype, o.mode, o.m);
@@ -648,6 +650,7 @@ namespace
 		const size_t bytes = m == 1 ? static_cast<size_t>(avhip_winograd_rows_weight_bytes(p.shape.K, p.shape.C))
 				: m == 3 ? static_cast<size_t>(avhip_conv2d_strided_weight_bytes(p.shape.K, p.shape.C))
 				: m == 5 ? static_cast<size_t>(avhip_conv2d_pointwise_block_weight_bytes(p.shape.K, p.shape.C))
+				: m == 6 ? static_cast<size_t>(avhip_winograd_f4_weight_bytes(p.shape.K, p.shape.C))
 				: static_cast<size_t>(t * t) * p.shape.K * p.shape.C * size_of(mat_dtype);
 		WeightCache &cache = weight_cache();
 		std::vector<WeightEntry> victims;
@@ -717,6 +720,7 @@ namespace
 				const int rc = m == 1 ? avhip_winograd_rows_weight_transform(ctx.stream, p.w_dtype, p.shape.mode, wm->data, e.U, p.shape.K, p.shape.C)
 						: m == 3 ? avhip_conv2d_strided_weight_layout(ctx.stream, p.w_dtype, p.shape.mode, wm->data, e.U, p.shape.K, p.shape.C)
 						: m == 5 ? avhip_conv2d_pointwise_block_weight_layout(ctx.stream, p.w_dtype, wm->data, e.U, p.shape.K, p.shape.C)
+						: m == 6 ? avhip_winograd_f4_weight_transform(ctx.stream, p.shape.mode, wm->data, e.U, p.shape.K, p.shape.C)
 						: avhip_winograd_weight_transform(ctx.stream, p.w_dtype, mat_dtype, m, 3, p.shape.mode, wm->data, e.U, p.shape.K, p.shape.C);
 				status = from_launcher(rc);
 				cache.transforms++;
@@ -1064,6 +1068,41 @@ namespace
 	bool nonfused_preferred(const ConvProblem &p, const NonFusedPlan &plan)
 	{
 		return plan.tiles >= 2048 && p.shape.C >= 64 && p.shape.K >= 64;
+	}
+	/* The same transform in one kernel (conv_winograd_f4.hip), weights in its operand layout from the cache (kind 6): for the layers of
+	 * the non-fused plan, so that the sums are those of F(4x4,3x3) where they were before.  A workgroup takes 32 tiles x 64 filters and a
+	 * compute unit for about 20 us (first loads, results) and 4.8 us per 16 channels, so it pays where the rounds of workgroups are full:
+	 * 256 x 15 x 15 x 128 -> 128 66 us against 95, 192 images 65 against 77, 64 channels 41 against 52; not with 128 workgroups of 128
+	 * channels (62 against 54) nor with a short second round (300 workgroups of 256 channels: 194 against 154).  The other side: its matrices
+	 * written and read at 5 TB/s and the products with filters filled up to 128, which holds within a fifth up to 128 channels and is too
+	 * low above. */
+	bool winograd_f4_pays(const ConvCall &c, const NonFusedPlan &plan, avActivationType_t activation)
+	{
+		const ConvProblem &p = c.problem;
+		const avhipConvShape &s = p.shape;
+		const char *x = c.x->data, *y = c.y->data;
+		const av_int64 x_bytes = static_cast<av_int64>(s.N) * s.H * s.W * s.C * 4, y_bytes = static_cast<av_int64>(s.N) * s.H * s.W * s.K * 4;
+		if (!p.conv->padding_value_is_zero() || c.beta != 0.0 || (activation != AVOCADO_ACTIVATION_LINEAR && activation != AVOCADO_ACTIVATION_RELU)
+				|| (x < y + y_bytes && y < x + x_bytes)) /* written while others still read: only the plan in three passes may work in place */
+			return false;
+		const av_int64 workgroups = (static_cast<av_int64>(plan.tiles) + 31) / 32 * ((s.K + 63) / 64);
+		const double one = static_cast<double>((workgroups + 255) / 256) * (20.0 + 4.8 * ((s.C + 15) / 16));
+		const double products = 2.0 * 36.0 * plan.tiles * s.C * ((s.K + 127) / 128 * 128.0);
+		const double three = 5.0 + (2.0 * static_cast<double>(plan.total) + static_cast<double>(x_bytes) + (c.z != nullptr ? 2.0 : 1.0) * static_cast<double>(y_bytes)) / 5.0e6
+				+ products / 2.5e8;
+		return one < 0.95 * three;
+	}
+	avStatus_t run_winograd_f4(const ConvCall &c, avMemoryDescriptor_t wMem, avMemoryDescriptor_t yMem, avActivationType_t activation)
+	{
+		const void *U = nullptr;
+		WeightLease lease;
+		const avStatus_t st = cached_winograd_weights(c.ctx, c.problem, wMem, 6, AVOCADO_DTYPE_FLOAT32, &U, lease);
+		if (st != AVOCADO_STATUS_SUCCESS)
+			return st;
+		const int rc = avhip_conv2d_winograd_f4(c.ctx.stream, &c.problem.shape, c.x->data, U, c.bias, c.z, c.y->data, c.alpha1, c.alpha2, c.beta, activation);
+		if (rc == 0)
+			touch(yMem);
+		return from_launcher(rc);
 	}
 	avStatus_t run_nonfused_winograd(const ConvCall &c, const NonFusedPlan &plan, Memory *ws, avMemoryDescriptor_t wMem, avMemoryDescriptor_t wsMem,
 			avMemoryDescriptor_t yMem, avActivationType_t activation)
@@ -2107,6 +2146,12 @@ namespace avocado
 			 * in the library's cache yet (nothing was launched): the implicit-GEMM plan needs none and takes over. */
 			if (nonfused_ready && nonfused_preferred(p, plan))
 			{
+				if (winograd_f4_pays(call, plan, activation))
+				{
+					const avStatus_t fs = run_winograd_f4(call, wMem, yMem, activation);
+					if (fs != AVOCADO_STATUS_NOT_SUPPORTED && fs != AVOCADO_STATUS_BAD_ALLOC)
+						return fs;
+				}
 				const avStatus_t ns = run_nonfused_winograd(call, plan, ws, wMem, workspaceMem, yMem, activation);
 				if (ns != AVOCADO_STATUS_BAD_ALLOC)
 					return ns;

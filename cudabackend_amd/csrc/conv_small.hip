@@ -6,13 +6,17 @@
  * the chip; the partial tiles are added through LDS in a fixed order.  There is no barrier in the k loop: each wavefront loads its
  * own operands, 128 bytes of k of every row at a time, eight lanes to a row, and brings them into MFMA layout through its own
  * part of LDS.  k runs over the 16-byte chunks of all taps in a row, so channel counts that are no multiple of 64 cost nothing.
+ * Where the channels of a tap are no whole number of chunks the last chunk of a tap is cut off in registers, and 16-bit or 8-bit
+ * rows that start between two dwords are loaded as the dwords around them and shifted.
  *
  * What bounds it: the 64 bytes per clock that a compute unit loads (128 clocks per stage of a 32 x 32 tile, 256 per stage of a
  * 64 x 64 tile, which needs half as much per product), for fp32 the matrix cores, and for the smallest problems the latency of
  * one launch.  Operands loaded straight in MFMA layout (32 lines per load instruction) took 55 to 60 clocks a kilobyte here, by
  * rows 20.  Measured, before (that form, 128 x 128 gather kernel where it was preferred) and now: bf16 128 -> 128 3x3 on 2912
  * pixels 12.5 -> 8.1 us, 256 -> 256 3x3 on 3800 pixels 18.1 -> 13.8 us, fp32 64 -> 218 5x5 on 1568 pixels 124 -> 23 us, fp16 72
- * channels 3x3 with an ELU on 13520 pixels 25.3 -> 9.9 us, int8 128 -> 128 stride 2 on 6720 pixels 21.7 -> 9.8 us.
+ * channels 3x3 with an ELU on 13520 pixels 25.3 -> 9.9 us, int8 128 -> 128 stride 2 on 6720 pixels 21.7 -> 9.8 us.  Against the general
+ * gather kernel, element by element: fp16 185 -> 160 3x3 on 8640 pixels 161 -> 25 us, fp16 370 -> 64 3x3 on 57876 pixels 418 -> 72 us,
+ * fp32 395 -> 32 5x5 stride 2 on 1170 pixels 1073 -> 62 us, bf16 90 -> 256 1x1 on 627200 pixels 493 -> 219 us.
  */
 #include <algorithm>
 #include <atomic>
@@ -414,7 +418,7 @@ namespace avhip
 		const int threshold = small_problem_threshold().load(std::memory_order_relaxed);
 		if (threshold < 0) /* asked for by name (tests): whatever the kernel can run */
 			return true;
-		if (!whole_chunks(s, element_bytes)) /* else such layers have the general gather kernel, element by element: 4 to 100 times slower */
+		if (!whole_chunks(s, element_bytes)) /* otherwise the general gather kernel, element by element: 2.2 to 17 times slower on all of 14 layers of 1152 to 627200 pixels */
 			return threshold != 0;
 		const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
 		return tiles < threshold && conv_small_plan(s, element_bytes).us < 0.95 * workgroup_tiles_us(s, element_bytes, plain);

@@ -3,6 +3,8 @@ the whole non-fused pipelines, through the C API,
 against the CPU oracle on identical seeded inputs.  Shapes follow the reference's own tests
 (test/test_winograd.cpp:28,32-38,174: x {12,13,14,135}, w {21,3,3,135} / {21,5,5,135}, alpha1 1.1, alpha2 1.2, beta 0.1,
 all four bias / residual combinations) plus channel counts that take the vectorised code path."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -209,3 +211,73 @@ def test_nonfused_pipeline_matches_direct_convolution(oracle, dtype, mat_dtype, 
     err = oracle.rel_l2(got, want)
     print("nonfused %s/%s F(%d,3) rel-L2 = %.3e" % (dtype, mat_dtype, m, err))
     assert err < tol
+
+
+class ConvShape(C.Structure):
+    """avhipConvShape of include/avocado_hip_kernels.h."""
+    _fields_ = [(name, C.c_int) for name in "N H W C K R S Ho Wo pad_h pad_w stride_h stride_w dil_h dil_w mode".split()]
+
+
+def f4_forward(x, w, bias, z, shape, alpha1=1.0, alpha2=1.0, activation=0, expect=0, beta=0.0):
+    with h.Call() as c:
+        lib = c.lib
+        lib.avhip_winograd_f4_weight_bytes.restype = C.c_int64
+        U = c.empty((lib.avhip_winograd_f4_weight_bytes(shape.K, shape.C) // 4,), "f32")
+        xt, wt, bt, zt = c.tensor(x, "f32"), c.tensor(w, "f32"), c.tensor(bias, "f32"), c.tensor(z, "f32")
+        y = c.empty((shape.N, shape.Ho, shape.Wo, shape.K), "f32")
+        p = lambda t: C.c_void_p(t.pointer()) if t is not None else None
+        stream = C.c_void_p(c.ctx.stream())
+        c.finish()
+        assert lib.avhip_winograd_f4_weight_transform(stream, shape.mode, p(wt), p(U), shape.K, shape.C) == 0
+        rc = lib.avhip_conv2d_winograd_f4(stream, C.byref(shape), p(xt), p(U), p(bt), p(zt), p(y), C.c_double(alpha1), C.c_double(alpha2), C.c_double(beta),
+                                          activation)
+        c.finish()
+        assert (rc == 0) == (expect == 0)
+        return y.download()
+
+
+@pytest.mark.parametrize("N, H, W, Cin, K, pad, use_bias, use_z, mode, act", [
+    (1, 1, 1, 1, 4, (-1, -1), True, True, 0, "RELU"),          # one tile of one pixel, one stage
+    (3, 13, 17, 67, 68, (-1, -1), True, True, 0, "RELU"),      # channels and filters that fill no block, 60 tiles
+    (2, 16, 16, 16, 64, (-1, -1), True, False, 1, "LINEAR"),   # 32 tiles: one whole workgroup, one stage
+    (11, 5, 6, 33, 132, (0, -2), False, True, 0, "LINEAR"),    # offsets other than the centre; three blocks of filters, the last nearly empty
+    (40, 9, 8, 128, 64, (-1, -1), False, False, 0, "RELU"),
+    (300, 4, 4, 48, 60, (-2, 0), True, True, 1, "RELU"),       # an image per tile
+])
+def test_f4_in_one_kernel(oracle, N, H, W, Cin, K, pad, use_bias, use_z, mode, act):
+    """Against the direct form; the bar of an fp32 F(4x4, 3x3) pipeline (its own error is 1e-6 to 3e-6)."""
+    g = h.rng(N + K)
+    x = h.rounded(oracle, g.standard_normal((N, H, W, Cin)), "f32")
+    w = h.rounded(oracle, g.standard_normal((K, 3, 3, Cin)) * np.sqrt(2.0 / (9 * Cin)), "f32")
+    bias = g.uniform(-0.1, 0.1, K).astype(np.float32).astype(np.float64) if use_bias else None
+    z = h.rounded(oracle, g.standard_normal((N, H, W, K)), "f32") if use_z else None
+    activation = getattr(h.cb, "ACTIVATION_" + act)
+    shape = ConvShape(N, H, W, Cin, K, 3, 3, H, W, *pad, 1, 1, 1, 1, mode)
+    got = f4_forward(x, w, bias, z, shape, alpha1=1.1, alpha2=1.2 if use_z else 0.0, activation=activation)
+    # zeros around the image, so that any offset gives an output of its size
+    wide = np.zeros((N, H + 4, W + 4, Cin))
+    wide[:, 2:-2, 2:-2] = x
+    corner = wide[:, 2 + pad[0]:2 + pad[0] + H + 2, 2 + pad[1]:2 + pad[1] + W + 2]
+    want = oracle.conv2d(np.ascontiguousarray(corner), w, bias, z, alpha1=1.1, alpha2=1.2 if use_z else 0.0, activation=activation, pad=(0, 0), mode=mode)
+    assert oracle.rel_l2(got, want) < 1e-5
+
+
+def test_f4_refuses_what_it_cannot_do(oracle):
+    x, w = np.zeros((1, 4, 4, 4)), np.zeros((6, 3, 3, 4))
+    f4_forward(x, w, None, None, ConvShape(1, 4, 4, 4, 6, 3, 3, 4, 4, -1, -1, 1, 1, 1, 1, 0), expect=1)  # filters in no runs of four
+    w = np.zeros((8, 3, 3, 4))
+    f4_forward(x, w, None, None, ConvShape(1, 4, 4, 4, 8, 3, 3, 2, 2, 0, 0, 1, 1, 1, 1, 0), expect=1)    # a smaller output
+    f4_forward(x, w, None, None, ConvShape(1, 4, 4, 4, 8, 3, 3, 4, 4, -1, -1, 1, 1, 1, 1, 0), beta=0.5, expect=1)
+
+
+def test_f4_through_the_dispatcher(oracle):
+    """A layer that goes there, with the workspace of the non-fused plan: first and last images."""
+    g = h.rng(77)
+    N, H, W, Cin = 200, 15, 15, 64
+    x = h.rounded(oracle, g.standard_normal((N, H, W, Cin)), "f32")
+    w = h.rounded(oracle, g.standard_normal((64, 3, 3, Cin)) * 0.06, "f32")
+    got = h.conv_forward("dispatch", x, w, (N, H, W, 64), "f32", workspace_bytes=1 << 28)
+    want = oracle.conv2d(x[:4], w, None, None, pad=(-1, -1))
+    assert oracle.rel_l2(got[:4], want) < 1e-5
+    want = oracle.conv2d(x[-2:], w, None, None, pad=(-1, -1))
+    assert oracle.rel_l2(got[-2:], want) < 1e-5
