@@ -831,7 +831,8 @@ namespace
 		const double small_tiles = static_cast<double>((pixels + 31) / 32 * ((s.K + 31) / 32)), slabs = static_cast<double>(s.R) * s.S * ((s.C * sizeof(TE) + 31) / 32);
 		const double shared = small_tiles < 512.0 && slabs >= 16.0 ? 4.0 : 1.0;
 		const double small = 2.5 + slabs / shared * (0.12 + 0.19 * small_tiles * shared / 1024.0);
-		if (tiles < 192 && small <= 0.7 * static_cast<double>(steps) + 4.0)
+		const int threshold = conv_small_threshold(); /* 0: that kernel is switched off and is nothing to compare with */
+		if (threshold < 0 || (tiles < std::min(threshold, 192) && small <= 0.7 * static_cast<double>(steps) + 4.0))
 			other = std::min(other, std::max(small, flops / (chip * std::min(1.0, small_tiles / 1024.0))));
 		const double walk = std::max(0.7 * static_cast<double>(per_part), flops / (chip * std::min(1.0, static_cast<double>(tiles * parts) / 256.0)));
 		const double split = 10.0 + walk + 0.25 * static_cast<double>(parts) + plane_bytes * static_cast<double>(parts + 1) / 4.0e6;

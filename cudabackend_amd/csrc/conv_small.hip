@@ -401,6 +401,10 @@ namespace avhip
 		}
 		return best;
 	}
+	int conv_small_threshold()
+	{
+		return small_problem_threshold().load(std::memory_order_relaxed);
+	}
 	static bool whole_chunks(const avhipConvShape &s, int element_bytes)
 	{
 		return static_cast<int64_t>(s.C) * element_bytes % 16 == 0;
@@ -415,7 +419,7 @@ namespace avhip
 	{
 		if (!conv_small_possible(s, element_bytes))
 			return false;
-		const int threshold = small_problem_threshold().load(std::memory_order_relaxed);
+		const int threshold = conv_small_threshold();
 		if (threshold < 0) /* asked for by name (tests): whatever the kernel can run */
 			return true;
 		if (!whole_chunks(s, element_bytes)) /* otherwise the general gather kernel, element by element: 2.2 to 17 times slower on all of 14 layers of 1152 to 627200 pixels */

@@ -21,6 +21,7 @@ namespace avhip
 		int tiles, waves;
 		double us;
 	};
+	int conv_small_threshold(); /* what avhip_set_small_problem_threshold set */
 	SmallPlan conv_small_plan(const avhipConvShape &s, int element_bytes);
 	/* Whether the launcher sends the layer to that kernel, given the conditions above.  `plain`: LINEAR or RELU, whole aligned
 	 * vectors of four filters. */
