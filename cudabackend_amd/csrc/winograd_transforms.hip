@@ -161,6 +161,18 @@ namespace
 		}
 	}
 
+	/* 4, 8 or 16 bytes through a buffer descriptor; zeros at OUT_OF_RANGE */
+	template<typename T, int V>
+	__device__ __forceinline__ Pack<T, V> fetch_pack(__amdgpu_buffer_rsrc_t rsrc, unsigned int offset)
+	{
+		if constexpr (sizeof(T) * V == 16)
+			return __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(offset), 0, 0));
+		else if constexpr (sizeof(T) * V == 8)
+			return __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b64(rsrc, static_cast<int>(offset), 0, 0));
+		else
+			return __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b32(rsrc, static_cast<int>(offset), 0, 0));
+	}
+
 	/* IDX is the integer type of the work-item and tile indices: 32 bits whenever the problem allows it (64-bit divisions
 	 * cost more than the transform itself).  V > 1 instances are launched only when every vector is complete and aligned:
 	 * they have no tail handling, and outside the image they load from a clamped address and select the padding value, so
@@ -181,7 +193,7 @@ namespace
 		const IDX CV = static_cast<IDX>((C + V - 1) / V);
 		const IDX tiles = static_cast<IDX>(N) * Th * Tw;
 		/* neighbouring tiles share input pixels: consecutive runs of tiles go to one XCD, whose L2 then serves the overlap */
-		const IDX gid = static_cast<IDX>(xcd_block(blockIdx.x, gridDim.x)) * 256 + threadIdx.x;
+		const IDX gid = static_cast<IDX>(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
 		const IDX tile = gid / CV;
 		const int cv = static_cast<int>(gid - tile * CV);
 		if (tile >= tiles)
@@ -210,12 +222,7 @@ namespace
 					const int ih = ih0 + a, iw = iw0 + b;
 					const bool inside = (static_cast<unsigned int>(ih) < static_cast<unsigned int>(H)) & (static_cast<unsigned int>(iw) < static_cast<unsigned int>(W));
 					const unsigned int offset = inside ? base + static_cast<unsigned int>((ih * W + iw) * C) * static_cast<unsigned int>(sizeof(T)) : OUT_OF_RANGE;
-					if constexpr (sizeof(T) * V == 16)
-						raw[a * t + b] = __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b128(rx, static_cast<int>(offset), 0, 0));
-					else if constexpr (sizeof(T) * V == 8)
-						raw[a * t + b] = __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b64(rx, static_cast<int>(offset), 0, 0));
-					else
-						raw[a * t + b] = __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b32(rx, static_cast<int>(offset), 0, 0));
+					raw[a * t + b] = fetch_pack<T, V>(rx, offset);
 				}
 #pragma unroll
 			for (int i = 0; i < t * t; i++)
@@ -340,26 +347,49 @@ namespace
 	}
 
 	/* Weight-gradient side, first transform: one M x M tile of dy (tiles do not overlap, positions past the border are zero)
-	 * becomes G' dy G'^T, a t x t tile of the matrices [t*t, tiles, K] (src/winograd_nonfused.cu:425-474). */
-	template<int M, int R, typename T, typename TM, int V>
+	 * becomes G' dy G'^T, a t x t tile of the matrices [t*t, tiles, K] (src/winograd_nonfused.cu:425-474).  IDX and BUF as in the input
+	 * transform: with 64-bit divisions and a branch around each load it waited for its loads one after the other.  Together with
+	 * group_size below: fp32 F(4x4, 3x3) gradient of 32 x 15 x 15 x 128 -> 128, all four launches, 29.8 -> 25.2 us. */
+	template<int M, int R, typename T, typename TM, int V, typename IDX, bool BUF = false>
 	__global__ __launch_bounds__(256) void k_gradient_transform(const T *__restrict__ dy, TM *__restrict__ Mx, int N, int H, int W, int K, int Th, int Tw)
 	{
 		typedef typename Traits<T>::compute CT;
 		constexpr int t = M + R - 1;
-		const size_t KV = static_cast<size_t>((K + V - 1) / V);
-		const size_t tiles = static_cast<size_t>(N) * Th * Tw;
-		const size_t gid = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-		const size_t tile = gid / KV;
+		constexpr bool FULL = V > 1;
+		const IDX KV = static_cast<IDX>((K + V - 1) / V);
+		const IDX tiles = static_cast<IDX>(N) * Th * Tw;
+		const IDX gid = static_cast<IDX>(blockIdx.x) * blockDim.x + threadIdx.x;
+		const IDX tile = gid / KV;
 		if (tile >= tiles)
 			return;
 		const int k = static_cast<int>(gid - tile * KV) * V;
-		const int valid = K - k;
-		const size_t row = tile / Tw;
+		const int valid = FULL ? V : K - k;
+		const IDX row = tile / static_cast<IDX>(Tw);
 		const int tw = static_cast<int>(tile - row * Tw);
-		const size_t n = row / Th;
+		const IDX n = row / static_cast<IDX>(Th);
 		const int th = static_cast<int>(row - n * Th);
 
 		CT d[M * M][V];
+		if constexpr (BUF)
+		{
+			const __amdgpu_buffer_rsrc_t rdy = make_buffer(dy, static_cast<unsigned int>(N) * H * W * K * static_cast<unsigned int>(sizeof(T)));
+			Pack<T, V> raw[M * M];
+#pragma unroll
+			for (int a = 0; a < M; a++)
+#pragma unroll
+				for (int b = 0; b < M; b++)
+				{
+					const int h = th * M + a, w = tw * M + b;
+					const unsigned int offset = (((static_cast<unsigned int>(n) * H + h) * W + w) * K + k) * static_cast<unsigned int>(sizeof(T));
+					raw[a * M + b] = fetch_pack<T, V>(rdy, (h < H) & (w < W) ? offset : OUT_OF_RANGE);
+				}
+#pragma unroll
+			for (int i = 0; i < M * M; i++)
+#pragma unroll
+				for (int v = 0; v < V; v++)
+					d[i][v] = Traits<T>::load(raw[i].v[v]);
+		}
+		else
 #pragma unroll
 		for (int a = 0; a < M; a++)
 #pragma unroll
@@ -367,7 +397,7 @@ namespace
 			{
 				const int h = th * M + a, w = tw * M + b;
 				if (h < H && w < W)
-					load_vec<T, V, CT>(dy + ((n * H + h) * W + w) * K + k, valid, d[a * M + b]);
+					load_vec<T, V, CT>(dy + ((static_cast<size_t>(n) * H + h) * W + w) * K + k, valid, d[a * M + b]);
 				else
 				{
 #pragma unroll
@@ -390,19 +420,21 @@ namespace
 
 	/* Weight-gradient side, last transform: dw[k, :, :, c] = alpha * U' m U'^T + beta * dw, m = the t x t tile of the matrices
 	 * [t*t, K, C] at (k, c) (src/winograd_nonfused.cu:475-519). */
-	template<int M, int R, typename T, typename TM, int V>
+	template<int M, int R, typename T, typename TM, int V, typename IDX>
 	__global__ __launch_bounds__(256) void k_update_transform(const TM *__restrict__ Mx, T *dw, int K, int C, typename Traits<T>::compute alpha,
 			typename Traits<T>::compute beta)
 	{
 		typedef typename Traits<T>::compute CT;
 		constexpr int t = M + R - 1;
-		const int CV = (C + V - 1) / V;
-		const size_t gid = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-		const int c = static_cast<int>(gid % CV) * V;
-		const size_t k = gid / CV;
-		if (k >= static_cast<size_t>(K))
+		constexpr bool FULL = V > 1;
+		const IDX CV = static_cast<IDX>((C + V - 1) / V);
+		const IDX gid = static_cast<IDX>(blockIdx.x) * blockDim.x + threadIdx.x;
+		const IDX row = gid / CV;
+		if (row >= static_cast<IDX>(K))
 			return;
-		const int valid = C - c;
+		const size_t k = row;
+		const int c = static_cast<int>(gid - row * CV) * V;
+		const int valid = FULL ? V : C - c;
 
 		CT m[t * t][V];
 #pragma unroll
@@ -457,6 +489,14 @@ namespace
 		return 1;
 	}
 
+	/* Work-items of a workgroup: one wavefront while workgroups of four would be fewer than two per compute unit.  What bounds a transform
+	 * that small is the latency of its loads, and workgroups of four leave compute units without any: 8192 work-items (update transform of
+	 * 128 x 128 filters) are 32 workgroups of 256 and 128 of 64. */
+	unsigned int group_size(size_t items)
+	{
+		return items < 2u * 256u * 256u ? 64 : 256;
+	}
+
 	template<typename T> typename Traits<T>::compute host_scalar(const void *p)
 	{
 		if (p == nullptr)
@@ -483,17 +523,18 @@ namespace
 		const int Th = (H + M - 1) / M, Tw = (W + M - 1) / M;
 		const int V = pick_vec<M, R, T, TM>(C, x, Vm);
 		const size_t items = static_cast<size_t>(N) * Th * Tw * ((C + V - 1) / V);
-		const dim3 grid(ceil_div(items, 256));
+		const unsigned int group = group_size(items);
+		const dim3 grid(ceil_div(items, group));
 		const typename Traits<T>::compute padv = host_scalar<T>(padding_value);
 		const bool narrow = items < (1ull << 31) && static_cast<uint64_t>(H) * W * C < (1ull << 31);
-#define AVHIP_LAUNCH_INPUT(WIDTH, IDX) hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, IDX>), grid, dim3(256), 0, s, static_cast<const T*>(x), \
+#define AVHIP_LAUNCH_INPUT(WIDTH, IDX) hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, IDX>), grid, dim3(group), 0, s, static_cast<const T*>(x), \
 		static_cast<TM*>(Vm), N, H, W, C, Th, Tw, pad_h, pad_w, padv)
 		const bool buffered = padv == static_cast<typename Traits<T>::compute>(0) && static_cast<uint64_t>(N) * H * W * C * sizeof(T) < (1ull << 31);
 		if (V > 1 && narrow && buffered)
 		{
 			constexpr int WIDTH = VecOf<M, R, T, TM>::value;
 			if constexpr (WIDTH > 1 && (sizeof(T) * WIDTH == 4 || sizeof(T) * WIDTH == 8 || sizeof(T) * WIDTH == 16))
-				hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, uint32_t, true>), grid, dim3(256), 0, s, static_cast<const T*>(x), static_cast<TM*>(Vm), N, H, W,
+				hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, uint32_t, true>), grid, dim3(group), 0, s, static_cast<const T*>(x), static_cast<TM*>(Vm), N, H, W,
 						C, Th, Tw, pad_h, pad_w, padv);
 			else
 				AVHIP_LAUNCH_INPUT(WIDTH, uint32_t);
@@ -560,13 +601,26 @@ namespace
 		const int Th = (H + M - 1) / M, Tw = (W + M - 1) / M;
 		const int V = pick_vec<M, R, T, TM>(K, dy, Mx);
 		const size_t items = static_cast<size_t>(N) * Th * Tw * ((K + V - 1) / V);
-		const dim3 grid(ceil_div(items, 256));
+		const unsigned int group = group_size(items);
+		const dim3 grid(ceil_div(items, group));
+		const bool narrow = items < (1ull << 31);
+		const bool buffered = static_cast<uint64_t>(N) * H * W * K * sizeof(T) < (1ull << 31);
+#define AVHIP_LAUNCH_GRADIENT(WIDTH, ...) hipLaunchKernelGGL((k_gradient_transform<M, R, T, TM, WIDTH, __VA_ARGS__>), grid, dim3(group), 0, s, \
+		static_cast<const T*>(dy), static_cast<TM*>(Mx), N, H, W, K, Th, Tw)
+		constexpr int WIDTH = VecOf<M, R, T, TM>::value;
+		if constexpr (WIDTH > 1 && (sizeof(T) * WIDTH == 4 || sizeof(T) * WIDTH == 8 || sizeof(T) * WIDTH == 16))
+			if (V > 1 && narrow && buffered)
+			{
+				AVHIP_LAUNCH_GRADIENT(WIDTH, uint32_t, true);
+				return 0;
+			}
 		if (V > 1)
-			hipLaunchKernelGGL((k_gradient_transform<M, R, T, TM, VecOf<M, R, T, TM>::value>), grid, dim3(256), 0, s, static_cast<const T*>(dy),
-					static_cast<TM*>(Mx), N, H, W, K, Th, Tw);
+			AVHIP_LAUNCH_GRADIENT(WIDTH, size_t);
+		else if (narrow)
+			AVHIP_LAUNCH_GRADIENT(1, uint32_t);
 		else
-			hipLaunchKernelGGL((k_gradient_transform<M, R, T, TM, 1>), grid, dim3(256), 0, s, static_cast<const T*>(dy), static_cast<TM*>(Mx), N, H, W, K, Th,
-					Tw);
+			AVHIP_LAUNCH_GRADIENT(1, size_t);
+#undef AVHIP_LAUNCH_GRADIENT
 		return 0;
 	}
 	template<int M, int R, typename T, typename TM>
@@ -575,13 +629,21 @@ namespace
 		typedef typename Traits<T>::compute CT;
 		const int V = pick_vec<M, R, T, TM>(C, Mx, dw);
 		const size_t items = static_cast<size_t>(K) * ((C + V - 1) / V);
-		const dim3 grid(ceil_div(items, 256));
-		if (V > 1)
-			hipLaunchKernelGGL((k_update_transform<M, R, T, TM, VecOf<M, R, T, TM>::value>), grid, dim3(256), 0, s, static_cast<const TM*>(Mx),
-					static_cast<T*>(dw), K, C, static_cast<CT>(alpha), static_cast<CT>(beta));
+		const unsigned int group = group_size(items);
+		const dim3 grid(ceil_div(items, group));
+#define AVHIP_LAUNCH_UPDATE(WIDTH, IDX) hipLaunchKernelGGL((k_update_transform<M, R, T, TM, WIDTH, IDX>), grid, dim3(group), 0, s, \
+		static_cast<const TM*>(Mx), static_cast<T*>(dw), K, C, static_cast<CT>(alpha), static_cast<CT>(beta))
+		constexpr int WIDTH = VecOf<M, R, T, TM>::value;
+		const bool narrow = items < (1ull << 31);
+		if (V > 1 && narrow)
+			AVHIP_LAUNCH_UPDATE(WIDTH, uint32_t);
+		else if (V > 1)
+			AVHIP_LAUNCH_UPDATE(WIDTH, size_t);
+		else if (narrow)
+			AVHIP_LAUNCH_UPDATE(1, uint32_t);
 		else
-			hipLaunchKernelGGL((k_update_transform<M, R, T, TM, 1>), grid, dim3(256), 0, s, static_cast<const TM*>(Mx), static_cast<T*>(dw), K, C,
-					static_cast<CT>(alpha), static_cast<CT>(beta));
+			AVHIP_LAUNCH_UPDATE(1, size_t);
+#undef AVHIP_LAUNCH_UPDATE
 		return 0;
 	}
 

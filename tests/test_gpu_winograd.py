@@ -130,6 +130,18 @@ def test_update_transform(oracle, dtype, m, r, C):
     assert oracle.rel_l2(got, want) < TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype,channels", [("f32", 64), ("bf16", 64), ("f16", 61)])
+def test_gradient_side_transforms_in_workgroups_of_four_wavefronts(oracle, dtype, channels):
+    """At least 131072 work-items, the last row and column of tiles cut off, with vectors and without; bars as above."""
+    g = h.rng(10)
+    dy = h.rounded(oracle, g.standard_normal((40, 29, 31, channels)), dtype)
+    got = h.winograd_gradient_transform(dy, (channels, 3, 3, 8), dtype, 2)
+    assert oracle.rel_l2(got, oracle.winograd_gradient_transform(dy, 2, 3)) < TOL[dtype]
+    M = h.rounded(oracle, g.standard_normal((16, 1024, 8 * channels + 32)), dtype)
+    got = h.winograd_update_transform(M, (1024, 3, 3, 8 * channels + 32), dtype, 2)
+    assert oracle.rel_l2(got, oracle.winograd_update_transform(M, 2, 3)) < TOL[dtype]
+
+
 @pytest.mark.parametrize("m,r", CASES)
 def test_weight_gradient_pipeline_matches_direct_correlation(oracle, m, r):
     """dw through the Winograd domain (input transform of x, gradient transform of dy, batched GEMM (T, N) over the tiles,
