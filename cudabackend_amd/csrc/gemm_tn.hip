@@ -286,7 +286,7 @@ namespace avhip
 		g.row_tiles = static_cast<int>(ceil_div(M, side));
 		g.col_tiles = static_cast<int>(ceil_div(N, side));
 		const int64_t tiles = static_cast<int64_t>(g.row_tiles) * g.col_tiles * batch;
-		if (tiles >= (1ll << 31))
+		if (tiles * 64 * WAVES >= (1ll << 32)) /* more work-items than a launch takes along one direction */
 			return false;
 		const dim3 grid(static_cast<unsigned int>(tiles)), block(64 * WAVES);
 		const TE *a = static_cast<const TE*>(A), *b = static_cast<const TE*>(B);

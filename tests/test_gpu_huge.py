@@ -82,3 +82,28 @@ def test_fp16_3x3_beyond_2gib(oracle):
         assert err < 2e-3
     for t in (x, y, wt, bt):
         t.close()
+
+
+def test_tn_product_of_more_tiles_than_one_launch_takes():
+    """65535 products 1 x 8193 over k = 1: 257 tiles of 32 columns (129 of 64) each are 16.8 (8.5) million workgroups of 512 work-items,
+    beyond the 2^32 work-items of one launch; the generic kernel, whose grid has three directions, has to take them.  One product per
+    output, rounded once: exact."""
+    batch, N, chunk = 65535, 8193, 4369
+    lib = cb.load_library()
+    ctx = lib.cudaGetDefaultContext(0)
+    a = ((np.arange(batch) % 61) * 0.25 - 7).astype(np.float16)
+    row = np.random.default_rng(14).standard_normal(N).astype(np.float16)
+    A = cb.DeviceTensor((batch, 1, 1), cb.DTYPE_FLOAT16, zero=False)
+    B, Y = (cb.DeviceTensor((batch, 1, N), cb.DTYPE_FLOAT16, zero=False) for _ in range(2))
+    cb.check(lib.cudaCopyMemoryFromHost(ctx, A.mem, 0, a.ctypes.data_as(C.c_void_p), a.nbytes), "upload")
+    rows = np.ascontiguousarray(np.broadcast_to(row, (chunk, N)))
+    for i in range(0, batch, chunk):
+        cb.check(lib.cudaCopyMemoryFromHost(ctx, B.mem, i * row.nbytes, rows.ctypes.data_as(C.c_void_p), rows.nbytes), "upload")
+    print("fp16 (T, N) product, 65535 x 1 x 8193", flush=True)
+    cb.check(lib.cudaGemmBatched(ctx, cb.GEMM_OPERATION_T, cb.GEMM_OPERATION_N, None, A.desc, A.mem, B.desc, B.mem, None, Y.desc, Y.mem), "cudaGemmBatched")
+    cb.check(lib.cudaSynchronizeWithContext(ctx), "sync")
+    for i in (0, 1, batch // 2, batch - 1):
+        want = (a[i].astype(np.float32) * row.astype(np.float32)).astype(np.float16)
+        np.testing.assert_array_equal(download_image(lib, ctx, Y, i, (N,), np.float16), want)
+    for t in (A, B, Y):
+        t.close()
