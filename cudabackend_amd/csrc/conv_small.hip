@@ -440,7 +440,8 @@ namespace avhip
 		const SmallPlan plan = conv_small_plan(s, SZ);
 		const int side = SMALL_TILE * plan.tiles;
 		const int64_t pixel_tiles = (pixels + side - 1) / side, filter_tiles = (static_cast<int64_t>(s.K) + side - 1) / side;
-		if (pixel_tiles > 0x7FFFFFFFll || filter_tiles > 65535 || pixel_tiles * filter_tiles > 0x7FFFFFFFll || pixels >= (1ll << 31) - side)
+		if (pixel_tiles * 64 * plan.waves >= (1ll << 32) /* work-items of a launch along one direction */ || filter_tiles > 65535
+				|| pixel_tiles * filter_tiles > 0x7FFFFFFFll || pixels >= (1ll << 31) - side)
 			return false;
 		SmallGeom g;
 		g.H = s.H;

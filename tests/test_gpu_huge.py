@@ -107,3 +107,32 @@ def test_tn_product_of_more_tiles_than_one_launch_takes():
         np.testing.assert_array_equal(download_image(lib, ctx, Y, i, (N,), np.float16), want)
     for t in (A, B, Y):
         t.close()
+
+
+def test_more_output_pixels_than_small_tiles_take_in_one_launch():
+    """540 million output pixels, all but four of them border: 16.9 million tiles of 32 pixels with four wavefronts each would be more
+    than 2^32 work-items.  The layer (1929 channels: no whole number of 16-byte chunks) has to be left to the gather kernel."""
+    lib = cb.load_library()
+    ctx = lib.cudaGetDefaultContext(0)
+    offset, Cin, K = 23240, 1929, 4
+    side = 2 + offset
+    assert (side * side + 31) // 32 * 256 >= 1 << 32
+    g = h.rng(71)
+    x, w = (g.standard_normal(s).astype(np.float16) for s in ((1, 2, 2, Cin), (K, 1, 1, Cin)))
+    xt, wt = cb.DeviceTensor.from_numpy(x, cb.DTYPE_FLOAT16), cb.DeviceTensor.from_numpy(w, cb.DTYPE_FLOAT16)
+    bias = np.array([0.5, -1.0, 2.0, 0.25])
+    bt = cb.DeviceTensor.from_numpy(bias, cb.DTYPE_FLOAT32)
+    y = cb.DeviceTensor((1, side, side, K), cb.DTYPE_FLOAT16)
+    conv = cb.ConvolutionDescriptor(padding=(-offset, -offset), dtype=cb.DTYPE_FLOAT16)
+    print("fp16 1x1 with 23240 rows and columns of border", flush=True)
+    cb.check(lib.cudaConvolutionImplicitGemmForward(ctx, conv.handle, None, xt.desc, xt.mem, wt.desc, wt.mem, bt.desc, bt.mem, None, 0, 0, None,
+                                                     y.desc, y.mem, cb.ACTIVATION_LINEAR), "conv")
+    cb.check(lib.cudaSynchronizeWithContext(ctx), "sync")
+    for row in (0, 1, side // 3, offset - 1, offset, offset + 1):
+        got = download_image(lib, ctx, y, row, (side, K), np.float16).astype(np.float64)
+        want = np.broadcast_to(bias, (side, K)).copy()
+        if offset <= row < offset + 2:
+            want[offset:offset + 2] += x[0, row - offset].astype(np.float64) @ w[:, 0, 0].astype(np.float64).T
+        np.testing.assert_allclose(got, want, rtol=2e-3, atol=2e-2)  # a sum of 1929 products of size 1 in fp32, rounded to fp16
+    for t in (xt, wt, bt, y):
+        t.close()
