@@ -285,6 +285,7 @@ namespace avhip
 	{
 		typedef int scalar_t;
 		static constexpr int wide = MODE == I8_REQUANT ? 8 : 4;
+		static constexpr int out_bytes = MODE == I8_REQUANT || MODE == I8_FLOAT_I8 ? 1 : 4;
 		template<int W> struct ColumnsT
 		{
 			int ibias[W];

@@ -853,7 +853,8 @@ namespace
 		if (!split_k_plan<TE>(s, plan) || !fast_path_ok<TE>(s, flags, padding_value) || (flags & 2) == 0 || workspace == nullptr
 				|| workspace_bytes < plan.bytes || !aligned_to(workspace, 16))
 			return AVHIP_NOT_SUPPORTED;
-		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true) && plan.us > 0.85 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us)
+		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true) && plan.us > 0.85 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
+				&& !in_place(s, x, sizeof(TE), y, sizeof(TE)))
 			return AVHIP_NOT_SUPPORTED; /* fewer launches and no faster */
 		const ConvGeom g = make_geom<TE>(s);
 		const dim3 grid(ceil_div(g.pixels, BLOCK_M), ceil_div(s.K, BLOCK_N), static_cast<unsigned int>(plan.splits));

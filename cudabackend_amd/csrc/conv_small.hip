@@ -435,7 +435,7 @@ namespace avhip
 		const int64_t pixels = static_cast<int64_t>(s.N) * s.Ho * s.Wo;
 		/* whole 4-filter vectors and LINEAR / RELU, or anything (the integer epilogues know no other activation) */
 		const bool simple = epi.vec && is_simple_activation(epi.activation);
-		if (!conv_small_preferred(s, SZ, simple))
+		if (!conv_small_preferred(s, SZ, simple) || in_place(s, x, SZ, epi.y, Epi::out_bytes))
 			return false;
 		const SmallPlan plan = conv_small_plan(s, SZ);
 		const int side = SMALL_TILE * plan.tiles;

@@ -11,9 +11,19 @@ namespace avhip
 	/* Launches the kernel and returns true when its estimate for the problem is below that of the kernels with 128 x 128 (or
 	 * 256 x 64) workgroup tiles; returns false without side effects otherwise.  The caller has established the conditions of the
 	 * branch-free loaders (16-byte aligned tensors below 2 GiB, zero padding value);
-	 * any activation and number of filters. */
+	 * any activation and number of filters.  Calls that work in place are left to the other kernels. */
 	template<typename TE, typename Epi>
 	bool conv_small_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi);
+
+	/* Whether the call writes y where x lies.  No header promises that, but it works where the sums are complete before the first result
+	 * is written (k split through the workspace, the three passes of non-fused Winograd) and where a workgroup alone reads the pixels that
+	 * it writes (one-tap filters, up to 128 filters in the kernels with 128 x 128 tiles).  Neither holds for tiles of 32 x 32 or 64 x 64. */
+	inline bool in_place(const avhipConvShape &s, const void *x, int x_size, const void *y, int y_size)
+	{
+		const int64_t x_bytes = static_cast<int64_t>(s.N) * s.H * s.W * s.C * x_size, y_bytes = static_cast<int64_t>(s.N) * s.Ho * s.Wo * s.K * y_size;
+		const char *in = static_cast<const char*>(x), *out = static_cast<const char*>(y);
+		return in < out + y_bytes && out < in + x_bytes;
+	}
 
 	/* tiles x tiles MFMA tiles of 32 x 32, `waves` wavefronts sharing the k range, and the estimated microseconds */
 	struct SmallPlan

@@ -748,3 +748,41 @@ def test_split_k_kernel_layer_entry(oracle, tiling, dtype, case):
         assert lib.avhip_conv2d_implicit_gemm_split_k(*args, space.pointer() + 4, need.value) == -1, "workspace not aligned for 16-byte accesses"
     want = oracle.conv2d(x, w, b, z, alpha2=float(np.float32(0.7)), activation=oracle.RELU, **kw)
     assert oracle.rel_l2(got, want) < BAR[dtype] * (3 if dtype == "f32" else 1)
+
+
+# ---- y written where x lies: works in the plans that complete their sums first, or whose workgroups alone read what they write -------
+@pytest.mark.parametrize("dtype, entry, N, H, W, Cin, R", [
+    ("f32", "dispatch", 2, 15, 15, 256, 3),      # k split, offered and taken with the workspace lent
+    ("bf16", "dispatch", 8, 15, 15, 384, 3),
+    ("f16", "dispatch", 4, 12, 12, 384, 5),
+    ("bf16", "implicit_gemm", 40, 15, 15, 36, 1),  # one tap: a workgroup per 128 pixels and all filters
+    ("f32", "implicit_gemm", 9, 20, 21, 101, 1),
+])
+def test_in_place(oracle, tiling, dtype, entry, N, H, W, Cin, R):
+    """The plan that the launcher picks by itself (default threshold of the kernel with small tiles, which cannot work in place)."""
+    if tiling != "workgroup_tiles":
+        pytest.skip("the threshold is set by the test itself")
+    lib = cb.load_library()
+    lib.avhip_set_small_problem_threshold(4096)
+    g = h.rng(46)
+    x = h.rounded(oracle, g.standard_normal((N, H, W, Cin)), dtype)
+    w = he(g, (Cin, R, R, Cin), dtype, oracle)
+    pad = (-(R // 2), -(R // 2))
+    with h.Call() as c:
+        conv = cb.ConvolutionDescriptor(padding=pad, dtype=h.DT[dtype])
+        xt, wt = c.tensor(x, dtype), c.tensor(w, dtype)
+        if entry == "dispatch":
+            need = C.c_int64(0)
+            cb.check(lib.cudaGetConvolutionWorkspaceSize(c.ctx.handle, conv.handle, xt.desc, wt.desc, 0, C.byref(need)), "workspace size")
+            assert need.value > 0
+            space = c.empty((need.value,), cb.DTYPE_UINT8)
+            st = lib.cudaConvolutionBiasActivationForward(c.ctx.handle, conv.handle, None, xt.desc, xt.mem, wt.desc, wt.mem, 0, 0, None, 0, 0, None, xt.desc, xt.mem,
+                                                          cb.ACTIVATION_RELU, space.mem)
+        else:
+            st = lib.cudaConvolutionImplicitGemmForward(c.ctx.handle, conv.handle, None, xt.desc, xt.mem, wt.desc, wt.mem, 0, 0, None, 0, 0, None, xt.desc, xt.mem,
+                                                        cb.ACTIVATION_RELU)
+        assert st == cb.STATUS_SUCCESS, cb.STATUS_NAMES[st]
+        c.finish()
+        got = xt.download()
+    want = oracle.conv2d(x, w, None, activation=oracle.RELU, pad=pad)
+    assert oracle.rel_l2(got, want) < BAR[dtype]
