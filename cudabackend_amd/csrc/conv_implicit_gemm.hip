@@ -853,9 +853,12 @@ namespace
 		if (!split_k_plan<TE>(s, plan) || !fast_path_ok<TE>(s, flags, padding_value) || (flags & 2) == 0 || workspace == nullptr
 				|| workspace_bytes < plan.bytes || !aligned_to(workspace, 16))
 			return AVHIP_NOT_SUPPORTED;
+		/* Where the kernel of small tiles is no slower the layer goes there, at once: told that it is declined, a caller would try the plans
+		 * that it keeps for layers that cannot be split (fp32 3x3 232 -> 244 on one image of 20 x 20: 31.6 us in three Winograd passes, 21.9 us
+		 * split, 16.7 by the small tiles' estimate) and an fp32 layer's sums would be of another kind. */
 		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true) && plan.us > 0.85 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
 				&& !in_place(s, x, sizeof(TE), y, sizeof(TE)))
-			return AVHIP_NOT_SUPPORTED; /* fewer launches and no faster */
+			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
 		const ConvGeom g = make_geom<TE>(s);
 		const dim3 grid(ceil_div(g.pixels, BLOCK_M), ceil_div(s.K, BLOCK_N), static_cast<unsigned int>(plan.splits));
 		hipLaunchKernelGGL((k_conv_igemm_split<TE>), grid, dim3(256), 0, st, static_cast<const TE*>(x), static_cast<const TE*>(w), g, plan.steps_per_split,

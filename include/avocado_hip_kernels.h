@@ -175,7 +175,8 @@ extern "C"
 	/* The implicit-GEMM forward with k split across workgroups, for layers with few output pixels and a long k (fewer than 256
 	 * tiles of 128 x 128 and a walk that is worth cutting, by the launcher's estimate): parts of the k range are summed in
 	 * fp32 into `workspace` ([parts][N * Ho * Wo][K] floats), a second kernel adds the parts and applies the same epilogue as
-	 * avhip_conv2d_implicit_gemm (any activation).  fp32 / fp16 / bf16 tensors, y of the type of x, fp32 bias.  Returns
+	 * avhip_conv2d_implicit_gemm (any activation).  Where the launcher's estimates find the kernel of small tiles no slower, the
+	 * layer runs there instead and the workspace is not touched.  fp32 / fp16 / bf16 tensors, y of the type of x, fp32 bias.  Returns
 	 * AVHIP_NOT_SUPPORTED, with nothing launched, when the layer is not worth splitting, the workspace is smaller than
 	 * avhip_conv2d_split_k_workspace() reports, or the tensors are not aligned for the branch-free loaders (the caller then
 	 * uses avhip_conv2d_implicit_gemm).  No counterpart in the reference, whose prototype has one tiling

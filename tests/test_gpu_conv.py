@@ -750,6 +750,27 @@ def test_split_k_kernel_layer_entry(oracle, tiling, dtype, case):
     assert oracle.rel_l2(got, want) < BAR[dtype] * (3 if dtype == "f32" else 1)
 
 
+@pytest.mark.parametrize("x, K, R", [((2, 15, 15, 256), 256, 3), ((16, 7, 7, 512), 512, 3), ((1, 20, 20, 232), 244, 3), ((4, 12, 12, 128), 128, 5)])
+def test_a_layer_that_small_tiles_take_from_split_k_stays_a_direct_sum(oracle, tiling, x, K, R):
+    """fp32 layers that are offered a workspace for split k (large enough for the non-fused Winograd plan as well) and that the kernel of
+    small tiles is estimated to run as fast: they must go to that kernel and not to Winograd.  Bit for bit what the implicit GEMM without
+    a workspace gives, and no weights transformed."""
+    if tiling != "workgroup_tiles":
+        pytest.skip("the threshold is set by the test itself")
+    lib = cb.load_library()
+    lib.avhip_set_small_problem_threshold(4096)
+    g = h.rng(47)
+    xv, w = h.rounded(oracle, g.standard_normal(x), "f32"), he(g, (K, R, R, x[3]), "f32", oracle)
+    pad, ys = (-(R // 2), -(R // 2)), x[:3] + (K,)
+    transforms = C.c_int64(0)
+    state = lambda: (lib.avhipGetWeightCacheState(C.byref(C.c_int64(0)), C.byref(C.c_int64(0)), C.byref(transforms)), transforms.value)[1]
+    before = state()
+    got = h.conv_forward("dispatch", xv, w, ys, "f32", activation=cb.ACTIVATION_RELU, pad=pad)
+    assert state() == before, "weights were transformed"
+    np.testing.assert_array_equal(got, h.conv_forward("implicit_gemm", xv, w, ys, "f32", activation=cb.ACTIVATION_RELU, pad=pad))
+    assert oracle.rel_l2(got, oracle.conv2d(xv, w, None, activation=oracle.RELU, pad=pad)) < BAR["f32"]
+
+
 # ---- y written where x lies: works in the plans that complete their sums first, or whose workgroups alone read what they write -------
 @pytest.mark.parametrize("dtype, entry, N, H, W, Cin, R", [
     ("f32", "dispatch", 2, 15, 15, 256, 3),      # k split, offered and taken with the workspace lent
