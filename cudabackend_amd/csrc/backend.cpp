@@ -1082,7 +1082,7 @@ namespace
 		const avhipConvShape &s = p.shape;
 		const char *x = c.x->data, *y = c.y->data;
 		const av_int64 x_bytes = static_cast<av_int64>(s.N) * s.H * s.W * s.C * 4, y_bytes = static_cast<av_int64>(s.N) * s.H * s.W * s.K * 4;
-		if (!p.conv->padding_value_is_zero() || c.beta != 0.0 || (activation != AVOCADO_ACTIVATION_LINEAR && activation != AVOCADO_ACTIVATION_RELU)
+		if (!p.conv->padding_value_is_zero() || !avhip::winograd_f4_takes(s, x, c.z, y, c.beta, activation)
 				|| (x < y + y_bytes && y < x + x_bytes)) /* written while others still read: only the plan in three passes may work in place */
 			return false;
 		const av_int64 workgroups = (static_cast<av_int64>(plan.tiles) + 31) / 32 * ((s.K + 63) / 64);

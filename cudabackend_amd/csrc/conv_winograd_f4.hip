@@ -343,6 +343,29 @@ namespace
 		return (static_cast<int64_t>(K) + FILTERS - 1) / FILTERS * FILTERS;
 	}
 	constexpr int64_t MOST_BYTES = 1ll << 29;
+	int64_t pixels_of(const avhipConvShape &s)
+	{
+		return static_cast<int64_t>(s.N) * s.H * s.W;
+	}
+	int64_t tiles_of(const avhipConvShape &s)
+	{
+		return static_cast<int64_t>(s.N) * ((s.H + 3) / 4) * ((s.W + 3) / 4);
+	}
+}
+
+namespace avhip
+{
+	bool winograd_f4_takes(const avhipConvShape &s, const void *x, const void *z, const void *y, double beta, int activation)
+	{
+		if (s.R != 3 || s.S != 3 || s.stride_h != 1 || s.stride_w != 1 || s.dil_h != 1 || s.dil_w != 1 || s.Ho != s.H || s.Wo != s.W
+				|| !is_simple_activation(activation) || beta != 0.0 || s.K % 4 != 0 || !aligned_to(x, 4) || !aligned_to(y, 16)
+				|| (z != nullptr && !aligned_to(z, 16)))
+			return false;
+		/* the output has the input's size, so every output pixel lies in a tile whatever the offset of the taps is */
+		const int64_t blocks = (tiles_of(s) + TILES - 1) / TILES * (padded_filters(s.K) / FILTERS);
+		return pixels_of(s) * s.C * 4 < MOST_BYTES && avhip_winograd_f4_weight_bytes(s.K, s.C) < MOST_BYTES && static_cast<int64_t>(s.C) * 4 * 8 < (1ll << 27)
+				&& blocks * 512 < (1ll << 32) && pixels_of(s) * s.K * 4 < (1ll << 31) && s.pad_h >= -8 && s.pad_h <= 8 && s.pad_w >= -8 && s.pad_w <= 8;
+	}
 }
 
 extern "C" int64_t avhip_winograd_f4_weight_bytes(int K, int C)
@@ -370,17 +393,10 @@ extern "C" int avhip_conv2d_winograd_f4(void *stream, const avhipConvShape *shap
 	const avhipConvShape &s = *shape;
 	if (s.N <= 0 || s.H <= 0 || s.W <= 0 || s.C <= 0 || s.K <= 0)
 		return AVHIP_BAD_PARAM;
-	if (s.R != 3 || s.S != 3 || s.stride_h != 1 || s.stride_w != 1 || s.dil_h != 1 || s.dil_w != 1 || s.Ho != s.H || s.Wo != s.W
-			|| !is_simple_activation(activation) || beta != 0.0 || s.K % 4 != 0 || !aligned_to(x, 4) || !aligned_to(U, 16) || !aligned_to(y, 16)
-			|| (z != nullptr && !aligned_to(z, 16)))
+	if (!winograd_f4_takes(s, x, z, y, beta, activation) || !aligned_to(U, 16))
 		return AVHIP_NOT_SUPPORTED;
-	/* the output has the input's size, so every output pixel lies in a tile whatever the offset of the taps is */
-	const int64_t pixels = static_cast<int64_t>(s.N) * s.H * s.W, x_bytes = pixels * s.C * 4, y_bytes = pixels * s.K * 4, u_bytes = avhip_winograd_f4_weight_bytes(s.K, s.C);
-	const int64_t tiles = static_cast<int64_t>(s.N) * ((s.H + 3) / 4) * ((s.W + 3) / 4);
+	const int64_t tiles = tiles_of(s);
 	const int64_t blocks = (tiles + TILES - 1) / TILES * (padded_filters(s.K) / FILTERS);
-	if (x_bytes >= MOST_BYTES || u_bytes >= MOST_BYTES || static_cast<int64_t>(s.C) * 4 * 8 >= (1ll << 27) || blocks >= (1ll << 31)
-			|| y_bytes >= (1ll << 31) || s.pad_h < -8 || s.pad_h > 8 || s.pad_w < -8 || s.pad_w > 8)
-		return AVHIP_NOT_SUPPORTED;
 	F4Geom g;
 	g.H = s.H;
 	g.W = s.W;
@@ -391,9 +407,9 @@ extern "C" int avhip_conv2d_winograd_f4(void *stream, const avhipConvShape *shap
 	g.tiles_w = (s.W + 3) / 4;
 	g.pad_h = s.pad_h;
 	g.pad_w = s.pad_w;
-	g.x_bytes = static_cast<unsigned int>(x_bytes);
-	g.u_bytes = static_cast<unsigned int>(u_bytes);
-	g.y_bytes = static_cast<unsigned int>(y_bytes);
+	g.x_bytes = static_cast<unsigned int>(pixels_of(s) * s.C * 4);
+	g.u_bytes = static_cast<unsigned int>(avhip_winograd_f4_weight_bytes(s.K, s.C));
+	g.y_bytes = static_cast<unsigned int>(pixels_of(s) * s.K * 4);
 	g.stages = static_cast<int>(padded_channels(s.C) / CHANNELS);
 	g.filter_blocks = static_cast<int>(padded_filters(s.K) / FILTERS);
 	const FloatEpilogue<float> epi { static_cast<const float*>(bias), static_cast<const float*>(z), static_cast<float*>(y), static_cast<float>(alpha1),

@@ -21,4 +21,10 @@ extern "C"
 	AVHIP_API int64_t avhip_winograd_f4_weight_bytes(int K, int C);
 }
 
+namespace avhip
+{
+	/* Whether avhip_conv2d_winograd_f4 takes the layer (U aligned to 16 bytes, y apart from x): to be asked before the weights are transformed. */
+	bool winograd_f4_takes(const avhipConvShape &s, const void *x, const void *z, const void *y, double beta, int activation);
+}
+
 #endif /* AVHIP_CONV_WINOGRAD_F4_HPP_ */

@@ -293,3 +293,26 @@ def test_f4_through_the_dispatcher(oracle):
     assert oracle.rel_l2(got[:4], want) < 1e-5
     want = oracle.conv2d(x[-2:], w, None, None, pad=(-1, -1))
     assert oracle.rel_l2(got[-2:], want) < 1e-5
+
+
+@pytest.mark.parametrize("K", [66, 126])
+def test_f4_matrices_are_not_made_for_a_layer_that_it_refuses(oracle, K):
+    """Filters in no runs of four on a layer large enough to pay: the three passes run it, and their matrices are all that is cached."""
+    lib = h.cb.load_library()
+    h.cb.check(lib.avhipInvalidateCaches(), "avhipInvalidateCaches")
+    g = h.rng(78)
+    x = h.rounded(oracle, g.standard_normal((256, 15, 15, 64)), "f32")
+    w = h.rounded(oracle, g.standard_normal((K, 3, 3, 64)) * 0.06, "f32")
+    with h.Call() as c:
+        conv = h.cb.ConvolutionDescriptor(padding=(-1, -1))
+        xt, wt, y = c.tensor(x, "f32"), c.tensor(w, "f32"), c.empty((256, 15, 15, K), "f32")
+        space = c.empty((1 << 28,), h.cb.DTYPE_UINT8)
+        counts = [C.c_int64(0) for _ in range(3)]
+        cached = lambda: (lib.avhipGetWeightCacheState(*[C.byref(n) for n in counts]), [n.value for n in counts])[1]
+        before = cached()
+        h.cb.check(lib.cudaConvolutionBiasActivationForward(c.ctx.handle, conv.handle, None, xt.desc, xt.mem, wt.desc, wt.mem, 0, 0, None, 0, 0, None, y.desc,
+                                                            y.mem, h.cb.ACTIVATION_RELU, space.mem), "conv")
+        c.finish()
+        assert [a - b for a, b in zip(cached(), before)] == [1, 36 * K * 64 * 4, 1]
+        got = y.download()
+    assert oracle.rel_l2(got[-2:], oracle.conv2d(x[-2:], w, None, activation=oracle.RELU, pad=(-1, -1))) < 1e-5
