@@ -2148,8 +2148,9 @@ namespace avocado
 			{
 				if (winograd_f4_pays(call, plan, activation))
 				{
+					/* (ALLOC_FAILED: no room for its matrices, nothing launched; those of the three passes may be there already) */
 					const avStatus_t fs = run_winograd_f4(call, wMem, yMem, activation);
-					if (fs != AVOCADO_STATUS_NOT_SUPPORTED && fs != AVOCADO_STATUS_BAD_ALLOC)
+					if (fs != AVOCADO_STATUS_NOT_SUPPORTED && fs != AVOCADO_STATUS_BAD_ALLOC && fs != AVOCADO_STATUS_ALLOC_FAILED)
 						return fs;
 				}
 				const avStatus_t ns = run_nonfused_winograd(call, plan, ws, wMem, workspaceMem, yMem, activation);

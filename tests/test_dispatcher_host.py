@@ -1,0 +1,87 @@
+"""The dispatcher's way from one plan to the next, on a machine without a GPU: backend.cpp linked with dispatcher_stubs.cpp, in which
+"device" memory is host memory and launchers count their calls.  What the plans compute is tested elsewhere."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+import cudabackend_amd as cb
+from cudabackend_amd import build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    out = tmp_path_factory.mktemp("dispatcher")
+    target = str(out / "libdispatcher.so")
+    for command in (["hipcc", *build.FLAGS, "-x", "hip", "-c", os.path.join(build.CSRC, "backend.cpp"), "-o", str(out / "backend.o")],
+                    ["g++", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-c", os.path.join(HERE, "dispatcher_stubs.cpp"), "-o",
+                     str(out / "stubs.o")],
+                    ["hipcc", "-shared", "-fPIC", "-Wl,-Bsymbolic", "-Wl,-z,defs", "--offload-arch=" + build.ARCH, "-o", target, str(out / "stubs.o"), str(out / "backend.o")]):
+        r = subprocess.run(command, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        assert r.returncode == 0, r.stdout[-4000:]
+    dll = C.CDLL(target)
+    for name, (res, args) in cb.api.PROTOTYPES.items():
+        fn = getattr(dll, name)
+        fn.restype, fn.argtypes = res, args
+    dll.stub_calls.argtypes = [C.c_char_p]
+    return dll
+
+
+class Layer:
+    """fp32 3x3 128 -> 128 on 256 images of 15 x 15, in a context of its own: one that the one-kernel F(4x4, 3x3) plan pays for."""
+
+    def __init__(self, lib):
+        self.lib = lib
+        lib.stub_set(0, 0)
+        self.context = self.made(lib.cudaCreateContextDescriptor, 0)
+        self.conv = self.made(lib.cudaCreateConvolutionDescriptor)
+        cb.check(lib.cudaSetConvolutionDescriptor(self.conv, cb.CONVOLUTION_MODE, 2, (C.c_int * 2)(-1, -1), None, None, 1, None))
+        self.x, self.y = self.tensor(256, 15, 15, 128), self.tensor(256, 15, 15, 128)
+        self.w = self.tensor(128, 3, 3, 128)
+        need = C.c_int64(0)
+        cb.check(lib.cudaGetConvolutionWorkspaceSize(self.context, self.conv, self.x[0], self.w[0], 0, C.byref(need)))
+        self.space = self.made(lib.cudaCreateMemoryDescriptor, 0, need.value)
+
+    def made(self, create, *args):
+        handle = C.c_int64(0)
+        cb.check(create(C.byref(handle), *args))
+        return handle.value
+
+    def tensor(self, *shape):
+        desc, size = self.made(self.lib.cudaCreateTensorDescriptor), 4
+        cb.check(self.lib.cudaSetTensorDescriptor(desc, cb.DTYPE_FLOAT32, 4, (C.c_int * 4)(*shape)))
+        for n in shape:
+            size *= n
+        return desc, self.made(self.lib.cudaCreateMemoryDescriptor, 0, size)
+
+    def forward(self, activation=cb.ACTIVATION_RELU, y=None, malloc_fails=False, capturing=False):
+        """Status and what was launched."""
+        self.lib.stub_set(int(malloc_fails), int(capturing))
+        y = y or self.y
+        status = self.lib.cudaConvolutionBiasActivationForward(self.context, self.conv, None, self.x[0], self.x[1], self.w[0], self.w[1], 0, 0, None, 0, 0, None,
+                                                               y[0], y[1], activation, self.space)
+        names = ("f4_weights", "f4", "weights", "input_transform", "gemm", "output_transform", "implicit_gemm")
+        return cb.STATUS_NAMES[status], [n for n in names if self.lib.stub_calls(n.encode())]
+
+
+F4, THREE_PASSES = ["f4"], ["input_transform", "gemm", "output_transform"]
+
+
+@pytest.fixture()
+def layer(lib):
+    return Layer(lib)
+
+
+def test_no_memory_for_the_one_kernel_plans_weights(layer):
+    assert layer.forward(cb.ACTIVATION_TANH) == ("SUCCESS", ["weights"] + THREE_PASSES)
+    assert layer.forward(malloc_fails=True) == ("SUCCESS", THREE_PASSES), "the plan whose matrices are there takes over"
+    assert layer.forward() == ("SUCCESS", ["f4_weights"] + F4)
+    assert layer.forward(malloc_fails=True) == ("SUCCESS", F4)
+
+
+def test_no_memory_for_any_plans_weights(layer):
+    assert layer.forward(malloc_fails=True) == ("ALLOC_FAILED", [])
+    assert layer.forward() == ("SUCCESS", ["f4_weights"] + F4)
