@@ -856,7 +856,8 @@ namespace
 		/* Where the kernel of small tiles is no slower the layer goes there, at once: told that it is declined, a caller would try the plans
 		 * that it keeps for layers that cannot be split (fp32 3x3 232 -> 244 on one image of 20 x 20: 31.6 us in three Winograd passes, 21.9 us
 		 * split, 16.7 by the small tiles' estimate) and an fp32 layer's sums would be of another kind. */
-		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true) && plan.us > 0.85 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
+		/* (at eight k-steps and more the one-tap kernels take nothing) */
+		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true, 0.0) && plan.us > 0.85 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
 				&& !in_place(s, x, sizeof(TE), y, sizeof(TE)))
 			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
 		const ConvGeom g = make_geom<TE>(s);

@@ -6,6 +6,8 @@
  * filter).  A 1x1 filter has a short k (C / 64 steps for 16-bit tensors) and x streams in from HBM once; the gather kernel's
  * one tile per workgroup leaves the matrix cores idle through every tile's first loads and drain.
  */
+#include <algorithm>
+
 #include "conv_pointwise.hpp"
 #include "persistent_gemm.hpp"
 #include "resident_gemm.hpp"
@@ -45,25 +47,68 @@ extern "C" int avhip_set_short_k_engine(int engine)
 
 namespace avhip
 {
+	static int64_t row_blocks_of(const avhipConvShape &s)
+	{
+		return (static_cast<int64_t>(s.N) * s.H * s.W + BLOCK_M - 1) / BLOCK_M;
+	}
+	static int64_t col_blocks_of(const avhipConvShape &s)
+	{
+		return (static_cast<int64_t>(s.K) + BLOCK_N - 1) / BLOCK_N;
+	}
+	static int64_t pointwise_tiles(const avhipConvShape &s)
+	{
+		return row_blocks_of(s) * col_blocks_of(s);
+	}
+	/* whole runs of Epi::wide filters leave with one vector store */
 	template<typename TE, typename Epi>
-	bool conv_pointwise_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi)
+	static bool pointwise_possible(const avhipConvShape &s, const Epi &epi)
 	{
 		if (s.R != 1 || s.S != 1 || s.stride_h != 1 || s.stride_w != 1 || s.pad_h != 0 || s.pad_w != 0 || s.Ho != s.H || s.Wo != s.W)
 			return false;
-		/* whole runs of Epi::wide filters leave with one vector store */
 		if (!epi.vec || s.K % Epi::wide != 0 || !aligned_to(epi.y, 16) || (epi.z != nullptr && !aligned_to(epi.z, 16)))
 			return false;
 		if (static_cast<size_t>(s.K) * sizeof(typename Epi::template ColumnsT<1>) > static_cast<size_t>(PERSISTENT_TABLE_BYTES))
 			return false;
 		const int64_t pixels = static_cast<int64_t>(s.N) * s.H * s.W;
-		const int64_t row_blocks = (pixels + BLOCK_M - 1) / BLOCK_M, col_blocks = (static_cast<int64_t>(s.K) + BLOCK_N - 1) / BLOCK_N;
-		const int64_t tiles = row_blocks * col_blocks;
-		if (pixels >= (1ll << 31) - BLOCK_M || tiles >= (1ll << 31) - 1024 || s.K >= (1 << 22))
+		return pixels < (1ll << 31) - BLOCK_M && pointwise_tiles(s) < (1ll << 31) - 1024 && s.K < (1 << 22);
+	}
+	template<typename TE, typename Epi>
+	static bool resident_possible(const avhipConvShape &s)
+	{
+		const unsigned int row_bytes = static_cast<unsigned int>(s.C) * static_cast<unsigned int>(sizeof(TE));
+		return short_k_engine().load(std::memory_order_relaxed) == 0 && (row_bytes + STEP_BYTES - 1) / STEP_BYTES <= RESIDENT_MAX_STEPS && row_bytes % 16 == 0
+				&& static_cast<size_t>(s.K) * sizeof(typename Epi::template ColumnsT<1>) <= static_cast<size_t>(RESIDENT_TABLE_BYTES);
+	}
+	/* a register set of x per step: longer rows stay with the gather kernel, whose k loop is long enough (int8 gets two
+	 * sets: its epilogue constants take the registers the other two would need) */
+	template<typename TE>
+	static constexpr int MAX_STEPS = sizeof(TE) == 1 ? 2 : PERSISTENT_MAX_STEPS;
+
+	/* Fitted to 290 layers of 16 to 512 channels (errors of 10 to 20 %): work at the rate of full rounds, but no less than the chain of one
+	 * tile, which for fp32 is long (one tile of 4 steps: 8.9 us, with a residual 12.6; of 1 step 5.2 and 6.0 to 9.3). */
+	template<typename TE, typename Epi>
+	double conv_pointwise_us(const avhipConvShape &s, const Epi &epi)
+	{
+		const int steps = static_cast<int>((static_cast<int64_t>(s.C) * sizeof(TE) + STEP_BYTES - 1) / STEP_BYTES);
+		if (!pointwise_possible<TE>(s, epi) || (!resident_possible<TE, Epi>(s) && steps > MAX_STEPS<TE>))
+			return 0.0;
+		const bool fp32 = sizeof(TE) == 4;
+		const double outputs = static_cast<double>(s.N) * s.H * s.W * s.K;
+		const double work = 4.5 + static_cast<double>(pointwise_tiles(s)) * steps / 512.0 * (fp32 ? 6.0 : 1.4) + outputs * (sizeof(TE) == 2 ? 2.0 : 4.0) / 6.0e6;
+		const int chain = steps <= 2 ? steps : 4;
+		return std::max(work, fp32 ? 4.2 + 1.1 * chain + (epi.z != nullptr ? 3.0 : 0.0) : 4.9 + 0.27 * chain + (epi.z != nullptr ? 0.3 : 0.0));
+	}
+
+	template<typename TE, typename Epi>
+	bool conv_pointwise_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi)
+	{
+		if (!pointwise_possible<TE>(s, epi))
 			return false;
+		const int64_t pixels = static_cast<int64_t>(s.N) * s.H * s.W;
+		const int64_t tiles = pointwise_tiles(s);
 		const unsigned int x_row_bytes = static_cast<unsigned int>(s.C) * static_cast<unsigned int>(sizeof(TE));
 		const int x_steps = static_cast<int>((x_row_bytes + STEP_BYTES - 1) / STEP_BYTES);
-		if (short_k_engine().load(std::memory_order_relaxed) == 0 && x_steps <= RESIDENT_MAX_STEPS && x_row_bytes % 16 == 0
-				&& static_cast<size_t>(s.K) * sizeof(typename Epi::template ColumnsT<1>) <= static_cast<size_t>(RESIDENT_TABLE_BYTES))
+		if (resident_possible<TE, Epi>(s))
 		{
 			ResidentGeom r;
 			r.rows = static_cast<int>(pixels);
@@ -91,10 +136,7 @@ namespace avhip
 		g.cols = s.K;
 		g.row_bytes = static_cast<unsigned int>(s.C) * static_cast<unsigned int>(sizeof(TE));
 		const int steps = static_cast<int>((g.row_bytes + STEP_BYTES - 1) / STEP_BYTES);
-		/* a register set of x per step: longer rows stay with the gather kernel, whose k loop is long enough (int8 gets two
-		 * sets: its epilogue constants take the registers the other two would need) */
-		constexpr int MAX_STEPS = sizeof(TE) == 1 ? 2 : PERSISTENT_MAX_STEPS;
-		if (steps > MAX_STEPS)
+		if (steps > MAX_STEPS<TE>)
 			return false;
 		g.a_pitch = g.b_pitch = g.row_bytes;
 		g.a_batch = g.b_batch = 0;
@@ -102,19 +144,20 @@ namespace avhip
 		g.b_bytes = static_cast<unsigned int>(s.K) * g.row_bytes;
 		g.c_batch = 0;
 		g.c_pitch = s.K;
-		g.row_blocks = static_cast<int>(row_blocks);
-		g.col_blocks = static_cast<int>(col_blocks);
+		g.row_blocks = static_cast<int>(row_blocks_of(s));
+		g.col_blocks = static_cast<int>(col_blocks_of(s));
 		g.tiles = static_cast<int>(tiles);
 		g.table_columns = s.K;
 		const dim3 grid(persistent_workgroups(tiles));
 		if (steps <= 2)
 			hipLaunchKernelGGL((k_conv_pointwise<TE, Epi, 2>), grid, dim3(256), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi);
-		else if constexpr (MAX_STEPS >= 4)
+		else if constexpr (MAX_STEPS<TE> >= 4)
 			hipLaunchKernelGGL((k_conv_pointwise<TE, Epi, 4>), grid, dim3(256), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi);
 		return true;
 	}
 
-#define AVHIP_INSTANTIATE(TE, EPI) template bool conv_pointwise_launch<TE, EPI>(hipStream_t, const avhipConvShape&, const void*, const void*, const EPI&);
+#define AVHIP_INSTANTIATE(TE, EPI) template bool conv_pointwise_launch<TE, EPI>(hipStream_t, const avhipConvShape&, const void*, const void*, const EPI&); \
+	template double conv_pointwise_us<TE, EPI>(const avhipConvShape&, const EPI&);
 	AVHIP_INSTANTIATE(float, FloatEpilogue<float>)
 	AVHIP_INSTANTIATE(f16_t, FloatEpilogue<f16_t>)
 	AVHIP_INSTANTIATE(bf16_t, FloatEpilogue<bf16_t>)

@@ -14,6 +14,9 @@ namespace avhip
 	 * chunk, LINEAR or RELU activation. */
 	template<typename TE, typename Epi>
 	bool conv_pointwise_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi);
+	/* The microseconds it is estimated to take, 0 where it does not take the layer (given the same conditions). */
+	template<typename TE, typename Epi>
+	double conv_pointwise_us(const avhipConvShape &s, const Epi &epi);
 }
 
 #endif /* AVHIP_CONV_POINTWISE_HPP_ */

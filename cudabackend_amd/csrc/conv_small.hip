@@ -23,6 +23,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "conv_pointwise.hpp"
 #include "conv_small.hpp"
 #include "mfma_core.hpp"
 
@@ -350,9 +351,13 @@ namespace
 
 	/* What the kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles take, in microseconds, fitted to the same layers
 	 * (errors of 6 to 18 %).  `plain`: LINEAR or RELU and whole vectors of filters; everything else runs in the gather kernel, whose
-	 * hand-over is slow there. */
-	double workgroup_tiles_us(const avhipConvShape &s, int element_bytes, bool plain)
+	 * hand-over is slow there.  `one_tap_us`: the estimate of the persistent one-tap kernels where they take the layer, or 0: what they
+	 * decline (filters in no whole runs of 16 bytes) is the gather kernel's and no less than 9 us (bf16 32 -> 20 on 8360 pixels, with a
+	 * residual: 11.6 us there, 5.0 in small tiles). */
+	double workgroup_tiles_us(const avhipConvShape &s, int element_bytes, bool plain, double one_tap_us)
 	{
+		if (plain && one_tap_us > 0.0)
+			return one_tap_us;
 		const bool fp32 = element_bytes == 4;
 		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
 		const double steps = static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 127) / 128);
@@ -365,8 +370,6 @@ namespace
 			const double pace = fp32 ? (workgroups <= 256.0 ? 2.0 : 3.3) : (workgroups <= 256.0 ? 0.47 : 0.68);
 			return std::ceil(workgroups / 512.0) * (3.6 + pace * steps);
 		}
-		if (plain && dense && s.R * s.S == 1 && steps <= 4.0) /* the persistent one-tap kernels */
-			return 4.5 + tiles * steps / 512.0 * (fp32 ? 6.0 : 1.4) + pixels * s.K * (element_bytes == 2 ? 2.0 : 4.0) / 6.0e6;
 		if (!plain)
 			return rounds * (18.0 + steps * (fp32 ? (tiles <= 256.0 ? 2.3 : 3.6) : (tiles <= 256.0 ? 0.70 : 0.85)));
 		return (fp32 ? 7.0 : 8.0) + rounds * steps * (fp32 ? (tiles <= 256.0 ? 2.1 : 3.0) : (tiles <= 256.0 ? 0.65 : 1.1));
@@ -415,7 +418,7 @@ namespace avhip
 		const int64_t chunks = (static_cast<int64_t>(s.C) * element_bytes + 15) / 16;
 		return s.R * s.S <= 32 && (chunks >= 2 || !whole_chunks(s, element_bytes)) && chunks <= 8192;
 	}
-	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, bool plain)
+	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, bool plain, double one_tap_us)
 	{
 		if (!conv_small_possible(s, element_bytes))
 			return false;
@@ -425,7 +428,7 @@ namespace avhip
 		if (!whole_chunks(s, element_bytes)) /* otherwise the general gather kernel, element by element: 2.2 to 17 times slower on all of 14 layers of 1152 to 627200 pixels */
 			return threshold != 0;
 		const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
-		return tiles < threshold && conv_small_plan(s, element_bytes).us < 0.95 * workgroup_tiles_us(s, element_bytes, plain);
+		return tiles < threshold && conv_small_plan(s, element_bytes).us < 0.95 * workgroup_tiles_us(s, element_bytes, plain, one_tap_us);
 	}
 
 	template<typename TE, typename Epi>
@@ -435,7 +438,7 @@ namespace avhip
 		const int64_t pixels = static_cast<int64_t>(s.N) * s.Ho * s.Wo;
 		/* whole 4-filter vectors and LINEAR / RELU, or anything (the integer epilogues know no other activation) */
 		const bool simple = epi.vec && is_simple_activation(epi.activation);
-		if (!conv_small_preferred(s, SZ, simple) || in_place(s, x, SZ, epi.y, Epi::out_bytes))
+		if (!conv_small_preferred(s, SZ, simple, simple ? conv_pointwise_us<TE>(s, epi) : 0.0) || in_place(s, x, SZ, epi.y, Epi::out_bytes))
 			return false;
 		const SmallPlan plan = conv_small_plan(s, SZ);
 		const int side = SMALL_TILE * plan.tiles;

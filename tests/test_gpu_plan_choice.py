@@ -38,3 +38,36 @@ def test_the_plan_taken_is_not_the_slower_one(case):
         ctx.close()
     print("%s: %.1f us with the plan, %.1f us without" % (layer[0], times[1], times[0]))
     assert times[1] <= 1.10 * times[0]
+
+
+# layers at which the estimates of the kernel of small tiles have to point the right way: name, dtype, x, w, padding, stride
+SMALL_OR_NOT = [
+    ("1x1 16->12, which the one-tap kernels decline", "bf16", (40, 12, 12, 16), (12, 1, 1, 16), 0, 1),
+    ("1x1 96->44, likewise", "f16", (7, 20, 20, 96), (44, 1, 1, 96), 0, 1),
+    ("1x1 116->44 in fp32: a chain of four steps in the one-tap kernels", "f32", (3, 12, 12, 116), (44, 1, 1, 116), 0, 1),
+    ("1x1 256->512: the one-tap kernels'", "bf16", (16, 28, 28, 256), (512, 1, 1, 256), 0, 1),
+    ("3x3 64->64 on few pixels", "f32", (8, 15, 15, 64), (64, 3, 3, 64), -1, 1),
+]
+
+
+@pytest.mark.parametrize("case", range(len(SMALL_OR_NOT)))
+def test_small_tiles_are_taken_where_they_are_the_faster_ones(case):
+    """Threshold of the kernel of small tiles: default, never, always.  The default must not be slower than either by more than a
+    quarter: the differences it has to tell apart here are factors of 1.4 to 2.5, and its estimates are off by up to 18 %."""
+    import bench
+    layer = SMALL_OR_NOT[case]
+    lib = cb.load_library()
+    lib.avhip_set_small_problem_threshold.restype = int
+    hip, ctx = bench.Hip(), cb.Context(0)
+    times = {}
+    previous = lib.avhip_set_small_problem_threshold(4096)
+    try:
+        for mode in (4096, 0, -1, 4096, 0, -1):
+            lib.avhip_set_small_problem_threshold(mode)
+            us = bench.other_configs(hip, ctx, 20, [layer])[layer[0]]["us"]
+            times[mode] = min(times.get(mode, us), us)
+    finally:
+        lib.avhip_set_small_problem_threshold(previous)
+        ctx.close()
+    print("%s: %.1f us, without small tiles %.1f, with %.1f" % (layer[0], times[4096], times[0], times[-1]))
+    assert times[4096] <= 1.25 * min(times[0], times[-1])
