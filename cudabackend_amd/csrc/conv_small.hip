@@ -345,9 +345,11 @@ namespace
 	};
 	/* Microseconds, fitted to 320 layers of all types (7 to 64 rows and columns, 16 to 512 channels and filters, 1x1 to 5x5, up to
 	 * 12 GFLOP; root mean square error 6 to 14 %): launch and first loads, one stage of a wavefront alone, one stage of a tile when its
-	 * compute unit is busy, and everything else about a tile.  Order of PLANS. */
+	 * compute unit is busy, and everything else about a tile.  Order of PLANS.  The first two of fp32 are of another fit, to 250 layers timed
+	 * with every plan, in which the first two stages of a wavefront, both in flight, do not cost as much as two later ones (52 -> 408 1x1
+	 * on 637 pixels: 7.2 us with four wavefronts, which the first fit chose, 5.5 with one). */
 	constexpr Pace PACE_16[] = { { 4.99, 0.303, 0.107, 0.20 }, { 3.34, 0.409, 0.084, 0.90 }, { 2.64, 0.173, 0.091, 2.40 }, { 3.41, 0.88, 0.182, 1.86 } };
-	constexpr Pace PACE_32[] = { { 5.09, 0.662, 0.197, 0.27 }, { 3.62, 0.767, 0.164, 1.15 }, { 2.55, 0.162, 0.164, 3.24 }, { 1.66, 2.39, 0.528, 3.38 } };
+	constexpr Pace PACE_32[] = { { 4.00, 0.654, 0.179, 0.35 }, { 3.40, 0.434, 0.174, 1.00 }, { 2.55, 0.162, 0.164, 3.24 }, { 1.66, 2.39, 0.528, 3.38 } };
 
 	/* What the kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles take, in microseconds, fitted to the same layers
 	 * (errors of 6 to 18 %).  `plain`: LINEAR or RELU and whole vectors of filters; everything else runs in the gather kernel, whose
