@@ -610,6 +610,34 @@ namespace
 				&& (!tap_mask || s.R * s.S <= 32); /* the gather kernel keeps one bit per tap: which taps of a pixel lie inside the image */
 	}
 
+	/* What the packed gather takes for a layer with pieces of `piece` bytes, in microseconds: fitted to 159 layers of 16-bit types and 71 of fp32
+	 * (700 to 700000 pixels, 36 to 508 filters, 3x3 and 5x5; root mean square error 8 to 12 %).  It packs k over the taps and has tiles of
+	 * 128 x 128, so it loses on few pixels (fp16 3 -> 32 3x3 stride 2 on 1152 pixels: 16.7 us, 6.0 in small tiles) and wins where it fills rounds
+	 * and rows of channels fill their chunks badly: fp16 12 -> 100 3x3 on 50176 pixels 15.4 against 19.4 us, bf16 28 -> 196 3x3 on 163072
+	 * pixels 74 against 102, fp32 5 -> 100 5x5 on 2789 images of 7 x 7 81 against 105. */
+	struct PackedPace
+	{
+		double launch, chain, step, tile, megabyte;
+	};
+	constexpr PackedPace PACKED_16[] = { { 6.6, 1.53, 1.0, 2.6, 0.2 }, { 9.8, 1.73, 1.29, 3.3, 0.2 }, { 10.8, 3.76, 3.0, 4.2, 0.2 } }; /* pieces of 8, 4 and 2 bytes */
+	constexpr PackedPace PACKED_32[] = { { 9.8, 2.66, 2.6, 3.1, 0.0 }, { 12.8, 2.73, 2.9, 5.1, 0.0 } };
+	double packed_us(const avhipConvShape &s, int element_bytes, int piece, bool residual)
+	{
+		const PackedPace &p = (element_bytes == 4 ? PACKED_32 : PACKED_16)[piece >= 8 ? 0 : piece == 4 ? 1 : 2];
+		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
+		const double steps = static_cast<double>((static_cast<int64_t>(s.R) * s.S * s.C * element_bytes + STEP_BYTES - 1) / STEP_BYTES);
+		const double rounds = std::ceil(pixels / BLOCK_M) * ((s.K + BLOCK_N - 1) / BLOCK_N) / 256.0;
+		return p.launch + std::max(p.chain * steps, rounds * p.step * steps) + rounds * p.tile + p.megabyte * pixels * s.K * element_bytes * 1.0e-6 * (residual ? 2.0 : 1.0);
+	}
+	/* Whether small tiles take a layer from the packed gather (pieces of `piece` bytes, 0: it cannot run it); int8 layers always.  Rows of
+	 * elements cost them a quarter more than their estimate, which is one of whole chunks. */
+	bool small_before_packed(const avhipConvShape &s, int element_bytes, int piece, bool residual)
+	{
+		if (piece == 0 || element_bytes == 1 || conv_small_threshold() < 0)
+			return true;
+		return conv_small_plan(s, element_bytes).us * (piece == 2 ? 1.25 : 1.0) < 0.95 * packed_us(s, element_bytes, piece, residual);
+	}
+
 	template<typename TE, typename Epi>
 	int launch(hipStream_t st, const avhipConvShape &s, const void *x, const void *w, const void *padding_value, int flags, const Epi &epi)
 	{
@@ -629,8 +657,7 @@ namespace
 		 * at 64 (half a k-step per tap) the kernels below are the faster ones, measured on 3x3 layers of 64 int8 / 32 bf16 / 16 fp32
 		 * channels (12 against 28 us, 21 against 52 us, 82 against 113 us); at 48 and 32 bytes these are (16 against 22 us, 13 against 22 us) */
 		const int pixel_bytes = s.C * static_cast<int>(sizeof(TE));
-		/* channels that are no whole number of 16-byte chunks: of the kernels below the few-channel ones and that of small tiles take them.
-		 * (The latter before the packed gather: fp16 3 -> 32 3x3 stride 2 on 1152 pixels 16.7 us there, 6.0 here) */
+		/* channels that are no whole number of 16-byte chunks: of the kernels below the few-channel ones and that of small tiles take them */
 		const bool ragged = pixel_bytes % 16 != 0 && aligned_to(x, 16) && aligned_to(w, 16) && fast_path_ok<TE>(s, 1, padding_value);
 		if (pixel_bytes < STEP_BYTES / 2 && s.R * s.S > 1 && fast_path_ok<TE>(s, 1, padding_value, false) && is_simple_activation(epi.activation)
 				&& (flags & 2) != 0)
@@ -641,12 +668,12 @@ namespace
 			/* the image tile in LDS, the operand gathered from there: filters of any number of taps */
 			if (conv_thin_launch<TE, Epi>(st, s, x, w, epi))
 				return 0;
-			if (ragged && conv_small_launch<TE, Epi>(st, s, x, w, epi))
-				return 0;
 			int pb = 16;
 			while (pb > 1 && (pixel_bytes % pb != 0 || !aligned_to(x, pb) || !aligned_to(w, pb)))
 				pb /= 2;
 			pb = (pb < static_cast<int>(sizeof(TE)) || s.R * s.S > 32) ? 0 : pb; /* the gather kernel's tap mask has 32 bits */
+			if (ragged && small_before_packed(s, sizeof(TE), pb, epi.z != nullptr) && conv_small_launch<TE, Epi>(st, s, x, w, epi))
+				return 0;
 #define AVHIP_PACKED(PB) hipLaunchKernelGGL((k_conv_igemm_packed<TE, PB, Epi>), grid, dim3(256), 0, st, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi)
 			switch (pb)
 			{

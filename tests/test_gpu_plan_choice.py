@@ -46,6 +46,8 @@ SMALL_OR_NOT = [
     ("1x1 96->44, likewise", "f16", (7, 20, 20, 96), (44, 1, 1, 96), 0, 1),
     ("1x1 116->44 in fp32: a chain of four steps in the one-tap kernels", "f32", (3, 12, 12, 116), (44, 1, 1, 116), 0, 1),
     ("1x1 256->512: the one-tap kernels'", "bf16", (16, 28, 28, 256), (512, 1, 1, 256), 0, 1),
+    ("3x3 28->196, packed gather", "bf16", (52, 56, 56, 28), (196, 3, 3, 28), -1, 1),
+    ("3x3 6->100 on few pixels, not the packed gather", "f16", (4, 28, 28, 6), (100, 3, 3, 6), -1, 1),
     ("3x3 64->64 on few pixels", "f32", (8, 15, 15, 64), (64, 3, 3, 64), -1, 1),
 ]
 
