@@ -33,12 +33,35 @@ namespace
 
 	constexpr int SMALL_TILE = 32;
 
+	/* n / d for n below 2^31 by a multiplication: with 2^shift >= d and factor = ceil(2^(31 + shift) / d), n * factor / 2^(31 + shift) is too
+	 * large by less than 1 / d.  A division by a number that only the launch knows is a chain of some twenty dependent instructions,
+	 * and three of them in a row stood before the first load of a workgroup: bf16 3x3 48 -> 48 on 3600 pixels 5.0 us a call with them, 4.4 without,
+	 * 4.6 in the kernel of one wavefront per tile that this one replaced (towers of twelve such layers; from a graph 4.3, 4.2). */
+	struct Divisor
+	{
+		unsigned int factor, shift;
+		__device__ __forceinline__ unsigned int of(unsigned int n) const
+		{
+			return __umulhi(2 * n, factor) >> shift;
+		}
+	};
+	Divisor divisor(unsigned int d)
+	{
+		Divisor result = { 0, 0 };
+		while ((1u << result.shift) < d)
+			result.shift++;
+		result.factor = static_cast<unsigned int>(((1ull << (31 + result.shift)) + d - 1) / d);
+		return result;
+	}
+
 	struct SmallGeom
 	{
 		int H, W, C, K, R, S, Ho, Wo, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, flip;
 		int chunks_per_tap; /* 16-byte chunks of the channels of one tap */
 		unsigned int by_chunks, by_s; /* ceil(2^32 / chunks_per_tap), ceil(2^16 / S): division by multiplication */
 		int pixels, images;
+		unsigned int pixel_tiles, filter_tiles;
+		Divisor by_wo, by_ho, by_tiles; /* by_tiles: of the faster of the two */
 		int pixels_first; /* order of the tiles: pixel tiles run fastest within an XCD (more weights than image), or filter tiles */
 	};
 
@@ -112,15 +135,9 @@ namespace
 		uint4 *mine = lds[wave];
 		/* Each XCD gets a contiguous run of the tiles, and within it the tiles that share the larger operand are neighbours, so
 		 * that its L2 fetches that operand once. */
-		unsigned int pixel_tile, filter_tile;
-		if (g.pixels_first)
-		{
-			const unsigned int t = xcd_block(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-			filter_tile = t / gridDim.x;
-			pixel_tile = t - filter_tile * gridDim.x;
-		}
-		else
-			xcd_tile(pixel_tile, filter_tile);
+		const unsigned int t = xcd_block(blockIdx.y * g.pixel_tiles + blockIdx.x, g.pixel_tiles * g.filter_tiles);
+		const unsigned int slow = g.by_tiles.of(t), fast = t - slow * (g.pixels_first ? g.pixel_tiles : g.filter_tiles);
+		const unsigned int pixel_tile = g.pixels_first ? fast : slow, filter_tile = g.pixels_first ? slow : fast;
 		const int p0 = static_cast<int>(pixel_tile) * SIDE, k0 = static_cast<int>(filter_tile) * SIDE;
 
 		const unsigned int c_bytes = g.C * SZ, filter_bytes = g.R * g.S * c_bytes;
@@ -134,8 +151,8 @@ namespace
 			const int p = p0 + lane;
 			const bool row_ok = p < g.pixels;
 			const int pp = row_ok ? p : 0;
-			const int line = pp / g.Wo, ow = pp - line * g.Wo;
-			const int n = line / g.Ho, oh = line - n * g.Ho;
+			const int line = static_cast<int>(g.by_wo.of(pp)), ow = pp - line * g.Wo;
+			const int n = static_cast<int>(g.by_ho.of(line)), oh = line - n * g.Ho;
 			const int ih0 = oh * g.stride_h + g.pad_h, iw0 = ow * g.stride_w + g.pad_w;
 			unsigned int inside = 0;
 			if (row_ok)
@@ -470,7 +487,12 @@ namespace avhip
 		g.pixels = static_cast<int>(pixels);
 		g.images = s.N;
 		g.pixels_first = static_cast<int64_t>(s.K) * s.R * s.S > static_cast<int64_t>(s.N) * s.H * s.W ? 1 : 0;
-		const dim3 grid(static_cast<unsigned int>(pixel_tiles), static_cast<unsigned int>(filter_tiles));
+		g.pixel_tiles = static_cast<unsigned int>(pixel_tiles);
+		g.filter_tiles = static_cast<unsigned int>(filter_tiles);
+		g.by_wo = divisor(s.Wo);
+		g.by_ho = divisor(s.Ho);
+		g.by_tiles = divisor(g.pixels_first ? g.pixel_tiles : g.filter_tiles);
+		const dim3 grid(g.pixel_tiles, g.filter_tiles);
 #define AVHIP_SMALL_PLAN(T, KW, ROW) \
 		do \
 		{ \
