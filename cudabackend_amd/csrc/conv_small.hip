@@ -360,13 +360,14 @@ namespace
 	{
 		double launch, chain, stage, tile;
 	};
-	/* Microseconds, fitted to 320 layers of all types (7 to 64 rows and columns, 16 to 512 channels and filters, 1x1 to 5x5, up to
-	 * 12 GFLOP; root mean square error 6 to 14 %): launch and first loads, one stage of a wavefront alone, one stage of a tile when its
-	 * compute unit is busy, and everything else about a tile.  Order of PLANS.  The first two of fp32 are of another fit, to 250 layers timed
-	 * with every plan, in which the first two stages of a wavefront, both in flight, do not cost as much as two later ones (52 -> 408 1x1
-	 * on 637 pixels: 7.2 us with four wavefronts, which the first fit chose, 5.5 with one). */
+	/* Microseconds: launch and first loads, one stage of a wavefront alone, one stage of a tile when its compute unit is busy, and everything
+	 * else about a tile.  Order of PLANS.  16-bit and 8-bit types: the larger of the two stage costs, fitted to 320 layers (7 to 64 rows and
+	 * columns, 16 to 512 channels and filters, 1x1 to 5x5, up to 12 GFLOP; root mean square error 6 to 14 %).  fp32: the root of the sum of
+	 * their squares, fitted to 222 layers timed with every plan (up to 6 GFLOP): the plan chosen is 0.5 % slower than the best of the four
+	 * on average and 15 % at most, with the larger of the two 1.2 % and 36 % (52 -> 408 1x1 on 637 pixels: 7.2 us with four wavefronts, which that chose,
+	 * 5.5 with one). */
 	constexpr Pace PACE_16[] = { { 4.99, 0.303, 0.107, 0.20 }, { 3.34, 0.409, 0.084, 0.90 }, { 2.64, 0.173, 0.091, 2.40 }, { 3.41, 0.88, 0.182, 1.86 } };
-	constexpr Pace PACE_32[] = { { 4.00, 0.654, 0.179, 0.35 }, { 3.40, 0.434, 0.174, 1.00 }, { 2.55, 0.162, 0.164, 3.24 }, { 1.66, 2.39, 0.528, 3.38 } };
+	constexpr Pace PACE_32[] = { { 3.80, 0.647, 0.143, 0.37 }, { 3.19, 0.490, 0.149, 1.00 }, { 2.34, 0.162, 0.165, 2.98 }, { 2.56, 1.48, 0.46, 2.79 } };
 
 	/* What the kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles take, in microseconds, fitted to the same layers
 	 * (errors of 6 to 18 %).  `plain`: LINEAR or RELU and whole vectors of filters; everything else runs in the gather kernel, whose
@@ -417,7 +418,8 @@ namespace avhip
 			const Pace &pace = element_bytes == 4 ? PACE_32[i] : PACE_16[i];
 			const double tiles = std::ceil(pixels / side) * ((s.K + side - 1) / side);
 			const double per_cu = tiles <= 1024.0 ? std::ceil(tiles / 256.0) : tiles / 256.0;
-			const double us = pace.launch + std::max(std::ceil(stages / PLANS[i].waves) * pace.chain, per_cu * stages * pace.stage) + per_cu * pace.tile;
+			const double alone = std::ceil(stages / PLANS[i].waves) * pace.chain, shared = per_cu * stages * pace.stage;
+			const double us = pace.launch + (element_bytes == 4 ? std::hypot(alone, shared) : std::max(alone, shared)) + per_cu * pace.tile;
 			if (best.tiles == 0 || us < best.us)
 				best = { PLANS[i].tiles, PLANS[i].waves, us };
 		}
