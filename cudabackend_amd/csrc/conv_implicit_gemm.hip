@@ -812,14 +812,25 @@ namespace
 	/* Whether to split k, into how many parts of how many steps, and the workspace that takes: worth it when the plain tiling
 	 * leaves most compute units idle for a long walk.  Estimates in microseconds (fitted to layers of 196 to 6272 pixels with
 	 * 1024 to 4608 elements of k): 4 + 0.7 per k-step for a workgroup of the plain gather kernel (less in the image-tile kernel); for the split, 10 for the two
-	 * launches and their prologues, 0.7 per step of a part, 0.25 per part and the parts read back at 4 TB/s in the reduction;
-	 * the small-tile kernel by its own estimate where the launcher would use it. */
+	 * launches and their prologues, 0.7 per step of a part, 0.25 per part and the parts read back at 4 TB/s in the reduction.
+	 * This decides which layers are offered a workspace, and callers size theirs by it, so it stays as it is; whether a layer
+	 * is split or goes to the kernel of small tiles is decided at the launch by split_us and that kernel's own estimate. */
 	struct SplitPlan
 	{
 		int splits, steps_per_split;
 		int64_t bytes;
-		double us;
 	};
+	/* What the two launches of the split take, in microseconds: fitted to 257 layers (186 of them fp32) that are offered a workspace and that the
+	 * kernel of small tiles may take, root mean square error 6 and 5 %.  A step of a part costs its latency until the tiles of all parts
+	 * outnumber the compute units. */
+	double split_us(const avhipConvShape &s, const SplitPlan &plan, int element_bytes)
+	{
+		const bool fp32 = element_bytes == 4;
+		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
+		const double rounds = std::ceil(pixels / BLOCK_M) * ((s.K + BLOCK_N - 1) / BLOCK_N) * plan.splits / 256.0;
+		const double step = fp32 ? std::max(1.77, 2.0 * rounds) : std::max(0.30, 0.48 * rounds);
+		return (fp32 ? 10.8 : 11.3) + step * plan.steps_per_split + 0.08 * plan.splits + (fp32 ? 0.41 : 0.29) * pixels * s.K * 4.0e-6 * (plan.splits + 1);
+	}
 	template<typename TE>
 	bool split_k_plan(const avhipConvShape &s, SplitPlan &plan)
 	{
@@ -853,8 +864,7 @@ namespace
 		const double chip = sizeof(TE) == 4 ? 1.55e8 : 1.87e9;
 		const double flops = 2.0 * static_cast<double>(pixels) * s.K * s.C * s.R * s.S;
 		other = std::max(other, flops / (chip * std::min(1.0, static_cast<double>(plain_workgroups) / 256.0)));
-		/* A wavefront on a 32 x 32 tile of its own, or four sharing its k: what decides which layers are offered a workspace (callers size
-		 * theirs by it).  Whether one is used is weighed again at the launch, against the small-tile kernel as it is. */
+		/* small tiles as they were when the offer was fixed: a wavefront on a 32 x 32 tile of its own, or four sharing its k */
 		const double small_tiles = static_cast<double>((pixels + 31) / 32 * ((s.K + 31) / 32)), slabs = static_cast<double>(s.R) * s.S * ((s.C * sizeof(TE) + 31) / 32);
 		const double shared = small_tiles < 512.0 && slabs >= 16.0 ? 4.0 : 1.0;
 		const double small = 2.5 + slabs / shared * (0.12 + 0.19 * small_tiles * shared / 1024.0);
@@ -868,7 +878,6 @@ namespace
 		plan.splits = static_cast<int>(parts);
 		plan.steps_per_split = static_cast<int>(per_part);
 		plan.bytes = static_cast<int64_t>(plane_bytes) * parts;
-		plan.us = split;
 		return true;
 	}
 	template<typename TE>
@@ -880,11 +889,12 @@ namespace
 		if (!split_k_plan<TE>(s, plan) || !fast_path_ok<TE>(s, flags, padding_value) || (flags & 2) == 0 || workspace == nullptr
 				|| workspace_bytes < plan.bytes || !aligned_to(workspace, 16))
 			return AVHIP_NOT_SUPPORTED;
-		/* Where the kernel of small tiles is no slower the layer goes there, at once: told that it is declined, a caller would try the plans
+		/* Where the kernel of small tiles is no slower (by the two estimates, of the 257 layers the slower one is taken for 17, 0.3 % on average over all and
+		 * 16 % at most) the layer goes there, at once: told that it is declined, a caller would try the plans
 		 * that it keeps for layers that cannot be split (fp32 3x3 232 -> 244 on one image of 20 x 20: 31.6 us in three Winograd passes, 21.9 us
-		 * split, 16.7 by the small tiles' estimate) and an fp32 layer's sums would be of another kind. */
+		 * split, 16.8 in small tiles) and an fp32 layer's sums would be of another kind. */
 		/* (at eight k-steps and more the one-tap kernels take nothing) */
-		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true, 0.0) && plan.us > 0.85 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
+		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true, 0.0) && split_us(s, plan, static_cast<int>(sizeof(TE))) > 0.95 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
 				&& !in_place(s, x, sizeof(TE), y, sizeof(TE)))
 			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
 		const ConvGeom g = make_geom<TE>(s);

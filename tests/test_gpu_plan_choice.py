@@ -48,6 +48,7 @@ SMALL_OR_NOT = [
     ("1x1 256->512: the one-tap kernels'", "bf16", (16, 28, 28, 256), (512, 1, 1, 256), 0, 1),
     ("3x3 28->196, packed gather", "bf16", (52, 56, 56, 28), (196, 3, 3, 28), -1, 1),
     ("3x3 6->100 on few pixels, not the packed gather", "f16", (4, 28, 28, 6), (100, 3, 3, 6), -1, 1),
+    ("3x3 484->92 on few pixels, offered a split of k", "f32", (1, 16, 16, 484), (92, 3, 3, 484), -1, 1),
     ("3x3 64->64 on few pixels", "f32", (8, 15, 15, 64), (64, 3, 3, 64), -1, 1),
 ]
 
