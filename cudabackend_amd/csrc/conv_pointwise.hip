@@ -85,7 +85,7 @@ namespace avhip
 	static constexpr int MAX_STEPS = sizeof(TE) == 1 ? 2 : PERSISTENT_MAX_STEPS;
 
 	/* Fitted to 290 layers of 16 to 512 channels (errors of 10 to 20 %): work at the rate of full rounds, but no less than the chain of one
-	 * tile, which for fp32 is long (one tile of 4 steps: 8.9 us, with a residual 12.6; of 1 step 5.2 and 6.0 to 9.3). */
+	 * tile, which for fp32 is long (one tile of 4 steps: 8.8 us, with a residual 12.6; of 2 steps 7.0, of 1 step 5.3 and 6.0 to 9.3). */
 	template<typename TE, typename Epi>
 	double conv_pointwise_us(const avhipConvShape &s, const Epi &epi)
 	{
@@ -95,8 +95,9 @@ namespace avhip
 		const bool fp32 = sizeof(TE) == 4;
 		const double outputs = static_cast<double>(s.N) * s.H * s.W * s.K;
 		const double work = 4.5 + static_cast<double>(pointwise_tiles(s)) * steps / 512.0 * (fp32 ? 6.0 : 1.4) + outputs * (sizeof(TE) == 2 ? 2.0 : 4.0) / 6.0e6;
-		const int chain = steps <= 2 ? steps : 4;
-		return std::max(work, fp32 ? 4.2 + 1.1 * chain + (epi.z != nullptr ? 3.0 : 0.0) : 4.9 + 0.27 * chain + (epi.z != nullptr ? 0.3 : 0.0));
+		const double chain = fp32 ? (steps == 1 ? 5.3 : steps == 2 ? 7.0 : 8.8) + (epi.z != nullptr ? 3.0 : 0.0)
+				: (steps == 1 ? 5.2 : steps == 2 ? 5.4 : 6.0) + (epi.z != nullptr ? 0.3 : 0.0);
+		return std::max(work, chain);
 	}
 
 	template<typename TE, typename Epi>
