@@ -85,3 +85,16 @@ def test_no_memory_for_the_one_kernel_plans_weights(layer):
 def test_no_memory_for_any_plans_weights(layer):
     assert layer.forward(malloc_fails=True) == ("ALLOC_FAILED", [])
     assert layer.forward() == ("SUCCESS", ["f4_weights"] + F4)
+
+
+def test_in_place_goes_through_the_workspace(layer):
+    """The one-kernel plan writes y while other workgroups still read x."""
+    assert layer.forward(y=layer.x) == ("SUCCESS", ["weights"] + THREE_PASSES)
+
+
+def test_capture_uses_what_is_cached(layer):
+    assert layer.forward(capturing=True) == ("SUCCESS", ["implicit_gemm"])
+    layer.forward(cb.ACTIVATION_TANH)
+    assert layer.forward(capturing=True) == ("SUCCESS", THREE_PASSES)
+    layer.forward()
+    assert layer.forward(capturing=True) == ("SUCCESS", F4)

@@ -67,6 +67,9 @@ SMALL_TILE_CASES = [
     dict(x=(1, 1, 1, 17), w=(2, 1, 1, 17), dtype="i8"),
     dict(x=(3, 15, 13, 131), w=(65, 3, 3, 131), pad=(-1, -1), dtype="i8"),
     dict(x=(3, 15, 13, 6), w=(66, 3, 3, 6), pad=(-1, -1), dtype="i8"),
+    dict(x=(40, 36, 36, 34), w=(36, 1, 1, 34), dtype="bf16", z=True),                                      # 32, 1 with rows of dwords
+    dict(x=(40, 36, 36, 33), w=(36, 1, 1, 33), dtype="f16", act="ELU"),                                    # 32, 1 with rows of elements
+    dict(x=(40, 36, 36, 7), w=(36, 1, 1, 7), dtype="f32"),
 ]
 
 
@@ -98,13 +101,26 @@ def test_small_tile_forms(oracle, case):
 
 @pytest.mark.parametrize("dtype, c", [("f32", 35), ("f16", 38), ("bf16", 37)])
 def test_an_infinity_stays_with_its_pixel_and_filter(dtype, c):
-    """Rows of channels that end within a 16-byte chunk: what lies behind them (the next pixel, tap or filter) must not reach the sum."""
+    """Rows of channels that end within a 16-byte chunk: what lies behind them (the next pixel or filter) must not reach the sum."""
     g = h.rng(c)
     x, w = g.standard_normal((2, 6, 5, c)).astype(np.float32), g.standard_normal((9, 1, 1, c)).astype(np.float32)
     x[0, 2, 3, 0], x[1, 0, 0, 1], w[4, 0, 0, 0] = np.inf, np.nan, -np.inf
     finite = np.isfinite(h.conv_forward("implicit_gemm", x, w, (2, 6, 5, 9), dtype, pad=(0, 0)))
     want = np.ones((2, 6, 5, 9), bool)
     want[0, 2, 3] = want[1, 0, 0] = want[..., 4] = False
+    np.testing.assert_array_equal(finite, want)
+
+
+@pytest.mark.parametrize("dtype, c", [("f32", 35), ("f16", 38), ("bf16", 37)])
+def test_an_infinity_stays_with_its_tap(dtype, c):
+    """The same with 3x3 filters: behind the last channel of a tap lie the weights of the next tap, and in the image the neighbouring pixel."""
+    g = h.rng(c + 1)
+    x, w = g.standard_normal((1, 7, 8, c)).astype(np.float32), g.standard_normal((9, 3, 3, c)).astype(np.float32)
+    x[0, 3, 4, 0], w[4, 1, 2, 0], w[6, 0, 0, 0] = np.inf, -np.inf, np.nan
+    finite = np.isfinite(h.conv_forward("implicit_gemm", x, w, (1, 7, 8, 9), dtype, pad=(-1, -1)))
+    want = np.ones((1, 7, 8, 9), bool)
+    want[0, 2:5, 3:6] = False       # the receptive field of the pixel
+    want[..., 4] = want[..., 6] = False  # everywhere, border included: there the tap multiplies the padding value, a zero
     np.testing.assert_array_equal(finite, want)
 
 
@@ -381,11 +397,30 @@ WALK_CASES = [
 ]
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "i8"])
+@pytest.mark.parametrize("case", WALK_CASES, ids=[str(i) for i in range(len(WALK_CASES))])
+def test_small_tiles_many_tiles(oracle, tiling, dtype, case):
+    """The same layers in the kernel of small tiles: thousands of them, in the order that shares the image and not the weights."""
+    if tiling != "wavefront_tiles":
+        pytest.skip("needs that kernel forced")
+    g = h.rng(45)
+    ys = out_shape(oracle, case)
+    if dtype == "i8":
+        x, w = g.integers(-127, 128, case["x"], dtype=np.int8), g.integers(-127, 128, case["w"], dtype=np.int8)
+        got = h.conv_forward("implicit_gemm", x, w, ys, "i8", y_dtype="i32", pad=case["pad"])
+        np.testing.assert_array_equal(got, oracle.conv2d_i8(x, w, None, pad=case["pad"]))
+        return
+    x, w = h.rounded(oracle, g.standard_normal(case["x"]), dtype), he(g, case["w"], dtype, oracle)
+    got = h.conv_forward("implicit_gemm", x, w, ys, dtype, activation=cb.ACTIVATION_RELU, pad=case["pad"])
+    want = oracle.conv2d(x, w, None, activation=oracle.RELU, pad=case["pad"])
+    assert max(oracle.rel_l2(got[i], want[i]) for i in range(ys[0])) < 2 * BAR[dtype]
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("case", WALK_CASES, ids=[str(i) for i in range(len(WALK_CASES))])
 def test_tile_kernel_many_tiles(oracle, tiling, dtype, case):
     if tiling != "workgroup_tiles":
-        pytest.skip("same kernel either way: the shape is far above the small-problem threshold")
+        pytest.skip("a test of the image-tile kernel; small tiles at many tiles: test_small_tiles_many_tiles")
     g = h.rng(42)
     x = h.rounded(oracle, g.standard_normal(case["x"]), dtype)
     w = he(g, case["w"], dtype, oracle)
@@ -403,7 +438,7 @@ def test_tile_kernel_many_tiles(oracle, tiling, dtype, case):
 @pytest.mark.parametrize("case", WALK_CASES, ids=[str(i) for i in range(len(WALK_CASES))])
 def test_tile_kernel_many_tiles_int8(oracle, tiling, case):
     if tiling != "workgroup_tiles":
-        pytest.skip("same kernel either way")
+        pytest.skip("a test of the image-tile kernel; small tiles at many tiles: test_small_tiles_many_tiles")
     g = h.rng(43)
     x = g.integers(-127, 128, case["x"], dtype=np.int8)
     w = g.integers(-127, 128, case["w"], dtype=np.int8)
@@ -676,7 +711,7 @@ SPLIT_CASES = [
 @pytest.mark.parametrize("case", SPLIT_CASES, ids=[str(i) for i in range(len(SPLIT_CASES))])
 def test_split_k_through_the_dispatcher(oracle, tiling, dtype, case):
     if tiling != "workgroup_tiles":
-        pytest.skip("with the one-wavefront-per-tile kernel available the plan leaves layers this small to it")
+        pytest.skip("forced small tiles leave nothing to split")
     g = h.rng(43)
     x = h.rounded(oracle, g.standard_normal(case["x"]), dtype)
     w = he(g, case["w"], dtype, oracle)
@@ -718,7 +753,7 @@ def test_split_k_kernel_layer_entry(oracle, tiling, dtype, case):
     """avhip_conv2d_implicit_gemm_split_k called directly: it must TAKE every one of these layers (return 0: the two split kernels ran,
     which the dispatcher test cannot tell from its fallback), and decline a workspace that is short or not aligned with nothing launched."""
     if tiling != "workgroup_tiles":
-        pytest.skip("with the one-wavefront-per-tile kernel available the plan leaves layers this small to it")
+        pytest.skip("forced small tiles leave nothing to split")
     lib = cb.load_library()
     g = h.rng(44)
     x = h.rounded(oracle, g.standard_normal(case["x"]), dtype)

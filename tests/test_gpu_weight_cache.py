@@ -232,6 +232,61 @@ def test_capture_with_a_cold_cache_allocates_nothing(oracle):
         t.close()
 
 
+def test_one_kernel_f4_weights_under_capture_and_rewritten(oracle):
+    """A layer that the one-kernel F(4x4, 3x3) plan pays for: captured with a cold cache it runs without matrices, captured with a warm one it is
+    the plan itself; weights rewritten are transformed again, into the same buffer, and the old graph replays with them."""
+    lib = cb.load_library()
+    hip = bench.Hip()
+    cb.check(lib.avhipInvalidateCaches(), "avhipInvalidateCaches")
+    lib.avhip_winograd_f4_weight_bytes.restype = C.c_int64
+    g = h.rng(94)
+    x, w, b = _problem(oracle, g, N=256, Cin=64, K=64)
+    some = slice(254, 256)
+    want = lambda weights: oracle.conv2d(x[some], weights, b, activation=oracle.RELU)
+    conv = cb.ConvolutionDescriptor(padding=(-1, -1))
+    xt, wt, bt = cb.DeviceTensor.from_numpy(x, cb.DTYPE_FLOAT32), cb.DeviceTensor.from_numpy(w, cb.DTYPE_FLOAT32), cb.DeviceTensor.from_numpy(b, cb.DTYPE_FLOAT32)
+    y = cb.DeviceTensor((256, 15, 15, 64), cb.DTYPE_FLOAT32)
+    need = C.c_int64(0)
+    with cb.Context(0) as ctx:
+        cb.check(lib.cudaGetConvolutionWorkspaceSize(ctx.handle, conv.handle, xt.desc, wt.desc, bt.desc, C.byref(need)), "workspace size")
+        ws = cb.DeviceTensor((need.value,), cb.DTYPE_UINT8)
+
+        def dispatch():
+            cb.check(lib.cudaConvolutionBiasActivationForward(ctx.handle, conv.handle, None, xt.desc, xt.mem, wt.desc, wt.mem, bt.desc, bt.mem, None, 0, 0,
+                                                              None, y.desc, y.mem, cb.ACTIVATION_RELU, ws.mem), "dispatch")
+
+        def replayed(exe):
+            cb.check(lib.cudaSetMemory(ctx.handle, y.mem, 0, y.nbytes, None, 0), "clear y")
+            hip.launch(exe, ctx.stream())
+            ctx.synchronize()
+            return y.download()
+        before = _state(lib)
+        exe = hip.capture(ctx.stream(), dispatch)
+        assert _state(lib) == before, "nothing allocated or transformed during capture"
+        assert oracle.rel_l2(replayed(exe)[some], want(w)) < 1e-5
+        hip.rt.hipGraphExecDestroy(exe)
+        dispatch()
+        ctx.synchronize()
+        eager = y.download()
+        warm = _state(lib)
+        assert warm == (before[0] + 1, before[1] + lib.avhip_winograd_f4_weight_bytes(64, 64), before[2] + 1)
+        exe = hip.capture(ctx.stream(), dispatch)
+        for _ in range(3):
+            np.testing.assert_array_equal(replayed(exe), eager)
+        assert _state(lib) == warm and oracle.rel_l2(eager[some], want(w)) < TOL
+        w2 = oracle.round_to(w[::-1] * 0.5, "f32")
+        wt.upload(w2)
+        dispatch()
+        ctx.synchronize()
+        eager = y.download()
+        assert _state(lib) == warm[:2] + (warm[2] + 1,) and oracle.rel_l2(eager[some], want(w2)) < TOL
+        np.testing.assert_array_equal(replayed(exe), eager)
+        hip.rt.hipGraphExecDestroy(exe)
+        ws.close()
+    for t in (xt, wt, bt, y):
+        t.close()
+
+
 def test_budget_never_frees_what_a_graph_holds(oracle):
     """With a budget that every insertion exceeds, the cache frees the least recently used matrices, but never those a captured graph
     was handed: the graph replays on valid memory after other weight tensors have gone through the cache."""

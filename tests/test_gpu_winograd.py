@@ -280,19 +280,46 @@ def test_f4_refuses_what_it_cannot_do(oracle):
     w = np.zeros((8, 3, 3, 4))
     f4_forward(x, w, None, None, ConvShape(1, 4, 4, 4, 8, 3, 3, 2, 2, 0, 0, 1, 1, 1, 1, 0), expect=1)    # a smaller output
     f4_forward(x, w, None, None, ConvShape(1, 4, 4, 4, 8, 3, 3, 4, 4, -1, -1, 1, 1, 1, 1, 0), beta=0.5, expect=1)
+    lib = h.cb.load_library()
+    stand_in = C.create_string_buffer(64)
+    aligned = C.c_void_p((C.addressof(stand_in) + 15) // 16 * 16)  # never read: tensors of these sizes are refused before a launch
+    for N, Cin, K in ((2 ** 20, 128, 4), (2 ** 17, 4, 4100), (2, 4096, 1024)):  # x of 512 MiB, y beyond 2 GiB, U beyond 512 MiB
+        shape = ConvShape(N, 1, 1, Cin, K, 3, 3, 1, 1, -1, -1, 1, 1, 1, 1, 0)
+        assert lib.avhip_conv2d_winograd_f4(None, C.byref(shape), aligned, aligned, None, None, aligned, C.c_double(1.0), C.c_double(0.0), C.c_double(0.0), 0) == -1
 
 
-def test_f4_through_the_dispatcher(oracle):
-    """A layer that goes there, with the workspace of the non-fused plan: first and last images."""
+@pytest.mark.parametrize("K, use_z, act", [(64, False, "LINEAR"), (128, True, "RELU"), (128, "in place of y", "LINEAR")])
+def test_f4_through_the_dispatcher(oracle, K, use_z, act):
+    """Layers that pay (256 images): bit for bit what the kernel's own entry gives, its matrices alone in the cache; first and last images
+    against the direct form.  A residual may lie where y is written: a work-item reads what it writes."""
     g = h.rng(77)
-    N, H, W, Cin = 200, 15, 15, 64
+    N, H, W, Cin = 256, 15, 15, 64
+    lib = h.cb.load_library()
+    h.cb.check(lib.avhipInvalidateCaches(), "avhipInvalidateCaches")
     x = h.rounded(oracle, g.standard_normal((N, H, W, Cin)), "f32")
-    w = h.rounded(oracle, g.standard_normal((64, 3, 3, Cin)) * 0.06, "f32")
-    got = h.conv_forward("dispatch", x, w, (N, H, W, 64), "f32", workspace_bytes=1 << 28)
-    want = oracle.conv2d(x[:4], w, None, None, pad=(-1, -1))
-    assert oracle.rel_l2(got[:4], want) < 1e-5
-    want = oracle.conv2d(x[-2:], w, None, None, pad=(-1, -1))
-    assert oracle.rel_l2(got[-2:], want) < 1e-5
+    w = h.rounded(oracle, g.standard_normal((K, 3, 3, Cin)) * 0.06, "f32")
+    bias = g.uniform(-0.1, 0.1, K).astype(np.float32).astype(np.float64)
+    z = h.rounded(oracle, g.standard_normal((N, H, W, K)), "f32") if use_z else None
+    activation = getattr(h.cb, "ACTIVATION_" + act)
+    with h.Call() as c:
+        conv = h.cb.ConvolutionDescriptor(padding=(-1, -1))
+        xt, wt, bt, zt = c.tensor(x, "f32"), c.tensor(w, "f32"), c.tensor(bias, "f32"), c.tensor(z, "f32")
+        y = zt if use_z == "in place of y" else c.empty((N, H, W, K), "f32")
+        need, counts = C.c_int64(0), [C.c_int64(0) for _ in range(3)]
+        h.cb.check(lib.cudaGetConvolutionWorkspaceSize(c.ctx.handle, conv.handle, xt.desc, wt.desc, bt.desc, C.byref(need)), "workspace size")
+        space = c.empty((need.value,), h.cb.DTYPE_UINT8)
+        h.cb.check(lib.cudaConvolutionBiasActivationForward(c.ctx.handle, conv.handle, None, xt.desc, xt.mem, wt.desc, wt.mem, bt.desc, bt.mem, None,
+                                                            zt.desc if zt else 0, zt.mem if zt else 0, None, y.desc, y.mem, activation, space.mem), "conv")
+        c.finish()
+        got = y.download()
+        lib.avhipGetWeightCacheState(*[C.byref(n) for n in counts])
+        lib.avhip_winograd_f4_weight_bytes.restype = C.c_int64
+        assert [n.value for n in counts[:2]] == [1, lib.avhip_winograd_f4_weight_bytes(K, Cin)]
+    shape = ConvShape(N, H, W, Cin, K, 3, 3, H, W, -1, -1, 1, 1, 1, 1, 0)
+    np.testing.assert_array_equal(got, f4_forward(x, w, bias, z, shape, activation=activation))
+    for images in (slice(0, 4), slice(N - 2, N)):
+        want = oracle.conv2d(x[images], w, bias, z[images] if use_z else None, activation=activation, pad=(-1, -1))
+        assert oracle.rel_l2(got[images], want) < 1e-5
 
 
 @pytest.mark.parametrize("K", [66, 126])
