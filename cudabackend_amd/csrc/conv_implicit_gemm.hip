@@ -892,9 +892,10 @@ namespace
 		/* Where the kernel of small tiles is no slower (by the two estimates, of the 257 layers the slower one is taken for 17, 0.3 % on average over all and
 		 * 16 % at most) the layer goes there, at once: told that it is declined, a caller would try the plans
 		 * that it keeps for layers that cannot be split (fp32 3x3 232 -> 244 on one image of 20 x 20: 31.6 us in three Winograd passes, 21.9 us
-		 * split, 16.8 in small tiles) and an fp32 layer's sums would be of another kind. */
+		 * split, 16.8 in small tiles) and an fp32 layer's sums would be of another kind (that layer's error against 64 bits: 2.1e-7 split, 3.1e-7 in
+		 * small tiles, 3.1e-6 through F(4x4, 3x3)). */
 		/* (at eight k-steps and more the one-tap kernels take nothing) */
-		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), true, 0.0) && split_us(s, plan, static_cast<int>(sizeof(TE))) > 0.95 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
+		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), HandOver::PLAIN, 0.0) && split_us(s, plan, static_cast<int>(sizeof(TE))) > 0.95 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
 				&& !in_place(s, x, sizeof(TE), y, sizeof(TE)))
 			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
 		const ConvGeom g = make_geom<TE>(s);

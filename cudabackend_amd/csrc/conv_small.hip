@@ -13,10 +13,10 @@
  * 64 x 64 tile, which needs half as much per product), for fp32 the matrix cores, and for the smallest problems the latency of
  * one launch.  Operands loaded straight in MFMA layout (32 lines per load instruction) took 55 to 60 clocks a kilobyte here, by
  * rows 20.  Measured, before (that form, 128 x 128 gather kernel where it was preferred) and now: bf16 128 -> 128 3x3 on 2912
- * pixels 12.5 -> 8.1 us, 256 -> 256 3x3 on 3800 pixels 18.1 -> 13.8 us, fp32 64 -> 218 5x5 on 1568 pixels 124 -> 23 us, fp16 72
- * channels 3x3 with an ELU on 13520 pixels 25.3 -> 9.9 us, int8 128 -> 128 stride 2 on 6720 pixels 21.7 -> 9.8 us.  Against the general
- * gather kernel, element by element: fp16 185 -> 160 3x3 on 8640 pixels 161 -> 25 us, fp16 370 -> 64 3x3 on 57876 pixels 418 -> 72 us,
- * fp32 395 -> 32 5x5 stride 2 on 1170 pixels 1073 -> 62 us, bf16 90 -> 256 1x1 on 627200 pixels 493 -> 219 us.
+ * pixels 11.8 -> 7.6 us, 256 -> 256 3x3 on 3800 pixels 17.3 -> 12.7 us, fp32 64 -> 218 5x5 on 1568 pixels 121 -> 23 us, fp16 72 -> 100
+ * channels 3x3 with an ELU and a residual on 13520 pixels 31.8 -> 12.9 us, int8 128 -> 128 stride 2 on 6720 pixels 21.7 -> 9.8 us.  Against the general
+ * gather kernel, element by element: fp16 185 -> 160 3x3 on 8640 pixels 157 -> 25 us, fp16 370 -> 64 3x3 on 57876 pixels 414 -> 66 us,
+ * fp32 395 -> 32 5x5 stride 2 on 1170 pixels 1068 -> 62 us, bf16 90 -> 256 1x1 on 627200 pixels 495 -> 214 us.
  */
 #include <algorithm>
 #include <atomic>
@@ -369,30 +369,39 @@ namespace
 	constexpr Pace PACE_16[] = { { 4.99, 0.303, 0.107, 0.20 }, { 3.34, 0.409, 0.084, 0.90 }, { 2.64, 0.173, 0.091, 2.40 }, { 3.41, 0.88, 0.182, 1.86 } };
 	constexpr Pace PACE_32[] = { { 3.80, 0.647, 0.143, 0.37 }, { 3.19, 0.490, 0.149, 1.00 }, { 2.34, 0.162, 0.165, 2.98 }, { 2.56, 1.48, 0.46, 2.79 } };
 
-	/* What the kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles take, in microseconds, fitted to the same layers
-	 * (errors of 6 to 18 %).  `plain`: LINEAR or RELU and whole vectors of filters; everything else runs in the gather kernel, whose
-	 * hand-over is slow there.  `one_tap_us`: the estimate of the persistent one-tap kernels where they take the layer, or 0: what they
+	/* The kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles: launch, a round of 512 workgroups (two to a compute unit), and
+	 * a k-step of one that has a compute unit to itself or shares it.  The last round, if it is of up to 256, goes at the pace of the former.
+	 * Microseconds, fitted to 448 layers (2000 to 130000 pixels, 16 to 512 channels and filters; root mean square error 6 to 13 %).  With every
+	 * round of the same length a 517th workgroup seemed to double the time: fp16 128 -> 128 3x3 on 129 images of 18 x 18 went to small tiles
+	 * and took 29.3 us, 25.5 in the image-tile kernel. */
+	struct TilePace
+	{
+		double launch, round, alone, shared;
+	};
+	enum { IMAGE_TILES, GATHER, GATHER_BY_ELEMENTS, GATHER_ACTIVATION };
+	constexpr TilePace TILES_16[] = { { 0.0, 4.0, 0.42, 0.68 }, { 1.7, 7.7, 0.70, 0.90 }, { 0.0, 13.5, 0.69, 0.96 }, { 4.4, 15.9, 0.67, 0.88 } };
+	constexpr TilePace TILES_32[] = { { 3.0, 4.1, 1.94, 3.84 }, { 2.0, 8.8, 2.17, 4.20 }, { 0.3, 17.3, 1.96, 4.04 }, { 4.7, 18.0, 2.07, 3.92 } };
+
+	/* What the layer takes in them.  `one_tap_us`: the estimate of the persistent one-tap kernels where they take the layer, or 0: what they
 	 * decline (filters in no whole runs of 16 bytes) is the gather kernel's and no less than 9 us (bf16 32 -> 20 on 8360 pixels, with a
 	 * residual: 11.6 us there, 5.0 in small tiles). */
-	double workgroup_tiles_us(const avhipConvShape &s, int element_bytes, bool plain, double one_tap_us)
+	double workgroup_tiles_us(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
 	{
-		if (plain && one_tap_us > 0.0)
+		if (hand_over == HandOver::PLAIN && one_tap_us > 0.0)
 			return one_tap_us;
-		const bool fp32 = element_bytes == 4;
 		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
 		const double steps = static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 127) / 128);
-		const double tiles = std::ceil(pixels / 128.0) * ((s.K + 127) / 128), rounds = std::ceil(tiles / 512.0);
 		const bool dense = s.stride_h == 1 && s.stride_w == 1 && s.dil_h == 1 && s.dil_w == 1;
-		if (plain && dense && s.R * s.S > 1 && s.K % 8 == 0 && s.Ho * s.Wo >= 128)
-		{
-			/* image-tile kernel: a workgroup with a compute unit to itself, or sharing one */
-			const double workgroups = static_cast<double>(s.N) * ((s.K + 63) / 64) * ((s.Ho * s.Wo + 255) / 256);
-			const double pace = fp32 ? (workgroups <= 256.0 ? 2.0 : 3.3) : (workgroups <= 256.0 ? 0.47 : 0.68);
-			return std::ceil(workgroups / 512.0) * (3.6 + pace * steps);
-		}
-		if (!plain)
-			return rounds * (18.0 + steps * (fp32 ? (tiles <= 256.0 ? 2.3 : 3.6) : (tiles <= 256.0 ? 0.70 : 0.85)));
-		return (fp32 ? 7.0 : 8.0) + rounds * steps * (fp32 ? (tiles <= 256.0 ? 2.1 : 3.0) : (tiles <= 256.0 ? 0.65 : 1.1));
+		const bool image_tiles = hand_over == HandOver::PLAIN && dense && s.R * s.S > 1 && s.K % 8 == 0 && s.Ho * s.Wo >= 128;
+		const int kernel = image_tiles ? IMAGE_TILES : hand_over == HandOver::PLAIN ? GATHER : hand_over == HandOver::ELEMENTS ? GATHER_BY_ELEMENTS : GATHER_ACTIVATION;
+		const TilePace &pace = (element_bytes == 4 ? TILES_32 : TILES_16)[kernel];
+		const double workgroups = image_tiles ? static_cast<double>(s.N) * ((s.K + 63) / 64) * ((s.Ho * s.Wo + 255) / 256)
+				: std::ceil(pixels / 128.0) * ((s.K + 127) / 128);
+		const double rounds = std::floor(workgroups / 512.0), rest = workgroups - 512.0 * rounds;
+		double us = pace.launch + rounds * (pace.round + pace.shared * steps);
+		if (rest > 0.0)
+			us += pace.round + (rest <= 256.0 ? pace.alone : pace.shared) * steps;
+		return us;
 	}
 }
 
@@ -439,7 +448,9 @@ namespace avhip
 		const int64_t chunks = (static_cast<int64_t>(s.C) * element_bytes + 15) / 16;
 		return s.R * s.S <= 32 && (chunks >= 2 || !whole_chunks(s, element_bytes)) && chunks <= 8192;
 	}
-	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, bool plain, double one_tap_us)
+	/* The small tiles' estimates are of the plain hand-over; the others cost them up to a fifth of the whole.  Against the one-tap kernels, whose
+	 * estimate is the coarsest, they have to be 5 % below. */
+	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
 	{
 		if (!conv_small_possible(s, element_bytes))
 			return false;
@@ -449,7 +460,8 @@ namespace avhip
 		if (!whole_chunks(s, element_bytes)) /* otherwise the general gather kernel, element by element: 2.2 to 17 times slower on all of 14 layers of 1152 to 627200 pixels */
 			return threshold != 0;
 		const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
-		return tiles < threshold && conv_small_plan(s, element_bytes).us < 0.95 * workgroup_tiles_us(s, element_bytes, plain, one_tap_us);
+		const double factor = hand_over != HandOver::PLAIN ? (element_bytes == 4 ? 1.1 : 1.2) : one_tap_us > 0.0 ? 1.05 : 1.0;
+		return tiles < threshold && factor * conv_small_plan(s, element_bytes).us < workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
 	}
 
 	template<typename TE, typename Epi>
@@ -459,7 +471,8 @@ namespace avhip
 		const int64_t pixels = static_cast<int64_t>(s.N) * s.Ho * s.Wo;
 		/* whole 4-filter vectors and LINEAR / RELU, or anything (the integer epilogues know no other activation) */
 		const bool simple = epi.vec && is_simple_activation(epi.activation);
-		if (!conv_small_preferred(s, SZ, simple, simple ? conv_pointwise_us<TE>(s, epi) : 0.0) || in_place(s, x, SZ, epi.y, Epi::out_bytes))
+		const HandOver hand_over = simple ? HandOver::PLAIN : is_simple_activation(epi.activation) ? HandOver::ELEMENTS : HandOver::ACTIVATION;
+		if (!conv_small_preferred(s, SZ, hand_over, simple ? conv_pointwise_us<TE>(s, epi) : 0.0) || in_place(s, x, SZ, epi.y, Epi::out_bytes))
 			return false;
 		const SmallPlan plan = conv_small_plan(s, SZ);
 		const int side = SMALL_TILE * plan.tiles;

@@ -33,9 +33,13 @@ namespace avhip
 	};
 	int conv_small_threshold(); /* what avhip_set_small_problem_threshold set */
 	SmallPlan conv_small_plan(const avhipConvShape &s, int element_bytes);
-	/* Whether the launcher sends the layer to that kernel, given the conditions above.  `plain`: LINEAR or RELU, whole aligned
-	 * vectors of four filters.  `one_tap_us`: conv_pointwise_us. */
-	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, bool plain, double one_tap_us);
+	/* How results leave: LINEAR or RELU in whole aligned vectors of four filters; those activations element by element; any activation */
+	enum class HandOver
+	{
+		PLAIN, ELEMENTS, ACTIVATION
+	};
+	/* Whether the launcher sends the layer to that kernel, given the conditions above.  `one_tap_us`: conv_pointwise_us. */
+	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us);
 }
 
 #endif /* AVHIP_CONV_SMALL_HPP_ */

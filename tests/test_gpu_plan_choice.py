@@ -49,6 +49,7 @@ SMALL_OR_NOT = [
     ("3x3 28->196, packed gather", "bf16", (52, 56, 56, 28), (196, 3, 3, 28), -1, 1),
     ("3x3 6->100 on few pixels, not the packed gather", "f16", (4, 28, 28, 6), (100, 3, 3, 6), -1, 1),
     ("3x3 484->92 on few pixels, offered a split of k", "f32", (1, 16, 16, 484), (92, 3, 3, 484), -1, 1),
+    ("3x3 128->128, four workgroups more than a round", "f16", (129, 18, 18, 128), (128, 3, 3, 128), -1, 1),
     ("3x3 64->64 on few pixels", "f32", (8, 15, 15, 64), (64, 3, 3, 64), -1, 1),
 ]
 
@@ -56,7 +57,8 @@ SMALL_OR_NOT = [
 @pytest.mark.parametrize("case", range(len(SMALL_OR_NOT)))
 def test_small_tiles_are_taken_where_they_are_the_faster_ones(case):
     """Threshold of the kernel of small tiles: default, never, always.  The default must not be slower than either by more than a
-    quarter: the differences it has to tell apart here are factors of 1.4 to 2.5, and its estimates are off by up to 18 %."""
+    quarter (but for the layer of one round and a bit, where that is the whole difference: a tenth): the differences it has to tell apart
+    here are factors of 1.15 to 2.5, and its estimates are off by 6 to 13 %."""
     import bench
     layer = SMALL_OR_NOT[case]
     lib = cb.load_library()
@@ -73,4 +75,4 @@ def test_small_tiles_are_taken_where_they_are_the_faster_ones(case):
         lib.avhip_set_small_problem_threshold(previous)
         ctx.close()
     print("%s: %.1f us, without small tiles %.1f, with %.1f" % (layer[0], times[4096], times[0], times[-1]))
-    assert times[4096] <= 1.25 * min(times[0], times[-1])
+    assert times[4096] <= (1.1 if "more than a round" in layer[0] else 1.25) * min(times[0], times[-1])
