@@ -1071,8 +1071,8 @@ namespace
 	}
 	/* The same transform in one kernel (conv_winograd_f4.hip), weights in its operand layout from the cache (kind 6): for the layers of
 	 * the non-fused plan, so that the sums are those of F(4x4,3x3) where they were before.  A workgroup takes 32 tiles x 64 filters and a
-	 * compute unit for about 20 us (first loads, results) and 4.8 us per 16 channels, so it pays where the rounds of workgroups are full:
-	 * 256 x 15 x 15 x 128 -> 128 66 us against 95, 192 images 65 against 77, 64 channels 41 against 52; not with 128 workgroups of 128
+	 * compute unit for about 20 us (first loads, results, spilled registers) and 4.8 us per 16 channels, so it pays where the rounds of
+	 * workgroups are full: 256 x 15 x 15 x 128 -> 128 61 us against 87, 192 images 58 against 68, 64 channels 36 against 49; not with 128 workgroups of 128
 	 * channels (62 against 54) nor with a short second round (300 workgroups of 256 channels: 194 against 154).  The other side: its matrices
 	 * written and read at 5 TB/s and the products with filters filled up to 128, which holds within a fifth up to 128 channels and is too
 	 * low above. */

@@ -189,8 +189,10 @@ extern "C"
 
 	/* Tuning knob without a counterpart in the reference.  The implicit-GEMM launcher sends a convolution to the kernel with
 	 * 32 x 32 or 64 x 64 tiles and k shared by wavefronts when its 128 x 128 tiling would yield fewer than this many workgroups
-	 * (default 4096) and that kernel is the faster one by the launcher's estimates; 0 never uses that kernel; a negative value
-	 * uses it for everything it can run (tests).  Returns the previous value.  Process-wide. */
+	 * (default 4096) and that kernel is the faster one by the launcher's estimates.  Channel counts that are no whole number of
+	 * 16-byte chunks go there whatever their size, unless the few-channel kernels or the packed gather take them or the call
+	 * works in place.  0 never uses that kernel, and such channel counts are then gathered element by element (2 to 17 times
+	 * slower); a negative value uses it for everything it can run (tests).  Returns the previous value.  Process-wide. */
 	AVHIP_API int avhip_set_small_problem_threshold(int workgroups);
 
 	/* Tuning knob without a counterpart in the reference.  Products with a short k (at most 512 bytes per operand row: 1x1

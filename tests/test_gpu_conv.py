@@ -789,7 +789,8 @@ def test_split_k_kernel_layer_entry(oracle, tiling, dtype, case):
 def test_a_layer_that_small_tiles_take_from_split_k_stays_a_direct_sum(oracle, tiling, x, K, R):
     """fp32 layers that are offered a workspace for split k (large enough for the non-fused Winograd plan as well) and that the kernel of
     small tiles is estimated to run as fast (the split at 1.04 times its microseconds or more, where the line lies at 0.95): they must go to that kernel and not to Winograd.  Bit for bit what the implicit GEMM without
-    a workspace gives, and no weights transformed."""
+    a workspace gives, no weights transformed, and an error that F(4x4, 3x3) does not reach (2.9e-6 and more on these layers; direct sums 2.1e-7 to
+    3.1e-7)."""
     if tiling != "workgroup_tiles":
         pytest.skip("the threshold is set by the test itself")
     lib = cb.load_library()
@@ -803,7 +804,7 @@ def test_a_layer_that_small_tiles_take_from_split_k_stays_a_direct_sum(oracle, t
     got = h.conv_forward("dispatch", xv, w, ys, "f32", activation=cb.ACTIVATION_RELU, pad=pad)
     assert state() == before, "weights were transformed"
     np.testing.assert_array_equal(got, h.conv_forward("implicit_gemm", xv, w, ys, "f32", activation=cb.ACTIVATION_RELU, pad=pad))
-    assert oracle.rel_l2(got, oracle.conv2d(xv, w, None, activation=oracle.RELU, pad=pad)) < BAR["f32"]
+    assert oracle.rel_l2(got, oracle.conv2d(xv, w, None, activation=oracle.RELU, pad=pad)) < 1e-6
 
 
 # ---- y written where x lies: works in the plans that complete their sums first, or whose workgroups alone read what they write -------
