@@ -19,7 +19,7 @@
  * known: every instance has 256 vector registers and spills (272 bytes of scratch a work-item, 292 with a residual: 36 to 38 MB a launch of
  * 256 workgroups, where x and y are 29.5), in front of the first loop, a few in every stage and in both passes of the output.
  * Measured, three passes before and now, one layer again and again from a graph: 256 x 15 x 15 x 128 -> 128 87 -> 61 us, with a residual 91 ->
- * 70 us (a tower of 20 of them in turn, 1925 -> 1422 us, is 69 and 77 us a layer), 64 channels 49 -> 36 us, 40 x 40 x 40 x 99 -> 128 118 -> 60 us,
+ * 70 us (a tower of 20 of them in turn, 1925 -> 1422 us, is 68 and 75 us a layer), 64 channels 49 -> 36 us, 40 x 40 x 40 x 99 -> 128 118 -> 60 us,
  * 32 x 56 x 56 x 64 -> 64 with residual 77 -> 47 us, 60 x 28 x 28 x 128 -> 128 68 -> 59 us.  Relative error against 64 bits 1.2e-6 to 2.9e-6 as
  * before (each within 3 % below).
  */
