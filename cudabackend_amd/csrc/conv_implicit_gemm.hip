@@ -23,6 +23,7 @@
 
 #include "conv_epilogue.hpp"
 #include "conv_pointwise.hpp"
+#include "conv_ring.hpp"
 #include "conv_small.hpp"
 #include "conv_stem.hpp"
 #include "conv_thin.hpp"
@@ -694,6 +695,10 @@ namespace
 			}
 #undef AVHIP_PACKED
 		}
+		/* operands through a ring of LDS buffers, where that is estimated to be faster than what follows */
+		if constexpr (sizeof(TE) < 4)
+			if (fast_path_ok<TE>(s, flags, padding_value) && conv_ring_launch<TE, Epi>(st, s, x, w, epi))
+				return 0;
 		/* a problem that does not fill the chip with big tiles goes to the kernel with small ones and k shared by wavefronts */
 		if ((ragged || fast_path_ok<TE>(s, flags, padding_value)) && conv_small_launch<TE, Epi>(st, s, x, w, epi))
 			return 0;
@@ -897,6 +902,10 @@ namespace
 		/* (at eight k-steps and more the one-tap kernels take nothing) */
 		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), HandOver::PLAIN, 0.0) && split_us(s, plan, static_cast<int>(sizeof(TE))) > 0.95 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
 				&& !in_place(s, x, sizeof(TE), y, sizeof(TE)))
+			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
+		/* Nor is it where the ring kernel is: bf16 480 -> 128 5x5 stride 2 on 155 images of 9 x 9, 34.5 us in nine parts. */
+		const double ring = is_simple_activation(activation) ? conv_ring_us(s, static_cast<int>(sizeof(TE)), static_cast<int>(sizeof(TE)), HandOver::PLAIN, 0.0, z != nullptr) : 0.0;
+		if (ring > 0.0 && ring < 0.9 * split_us(s, plan, static_cast<int>(sizeof(TE))) && !in_place(s, x, sizeof(TE), y, sizeof(TE)))
 			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
 		const ConvGeom g = make_geom<TE>(s);
 		const dim3 grid(ceil_div(g.pixels, BLOCK_M), ceil_div(s.K, BLOCK_N), static_cast<unsigned int>(plan.splits));

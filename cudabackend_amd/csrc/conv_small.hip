@@ -33,27 +33,6 @@ namespace
 
 	constexpr int SMALL_TILE = 32;
 
-	/* n / d for n below 2^31 by a multiplication: with 2^shift >= d and factor = ceil(2^(31 + shift) / d), n * factor / 2^(31 + shift) is too
-	 * large by less than 1 / d.  A division by a number that only the launch knows is a chain of some twenty dependent instructions,
-	 * and three of them in a row stood before the first load of a workgroup: bf16 3x3 48 -> 48 on 3600 pixels 5.0 us a call with them, 4.4 without,
-	 * 4.6 in the kernel of one wavefront per tile that this one replaced (towers of twelve such layers; from a graph 4.3, 4.2). */
-	struct Divisor
-	{
-		unsigned int factor, shift;
-		__device__ __forceinline__ unsigned int of(unsigned int n) const
-		{
-			return __umulhi(2 * n, factor) >> shift;
-		}
-	};
-	Divisor divisor(unsigned int d)
-	{
-		Divisor result = { 0, 0 };
-		while ((1u << result.shift) < d)
-			result.shift++;
-		result.factor = static_cast<unsigned int>(((1ull << (31 + result.shift)) + d - 1) / d);
-		return result;
-	}
-
 	struct SmallGeom
 	{
 		int H, W, C, K, R, S, Ho, Wo, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, flip;
@@ -450,6 +429,10 @@ namespace avhip
 	}
 	/* The small tiles' estimates are of the plain hand-over; the others cost them up to a fifth of the whole.  Against the one-tap kernels, whose
 	 * estimate is the coarsest, they have to be 5 % below. */
+	static double small_factor(int element_bytes, HandOver hand_over, double one_tap_us)
+	{
+		return hand_over != HandOver::PLAIN ? (element_bytes == 4 ? 1.1 : 1.2) : one_tap_us > 0.0 ? 1.05 : 1.0;
+	}
 	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
 	{
 		if (!conv_small_possible(s, element_bytes))
@@ -460,8 +443,13 @@ namespace avhip
 		if (!whole_chunks(s, element_bytes)) /* otherwise the general gather kernel, element by element: 2.2 to 17 times slower on all of 14 layers of 1152 to 627200 pixels */
 			return threshold != 0;
 		const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
-		const double factor = hand_over != HandOver::PLAIN ? (element_bytes == 4 ? 1.1 : 1.2) : one_tap_us > 0.0 ? 1.05 : 1.0;
-		return tiles < threshold && factor * conv_small_plan(s, element_bytes).us < workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
+		return tiles < threshold && small_factor(element_bytes, hand_over, one_tap_us) * conv_small_plan(s, element_bytes).us
+				< workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
+	}
+	double conv_without_ring_us(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
+	{
+		return conv_small_preferred(s, element_bytes, hand_over, one_tap_us) ? small_factor(element_bytes, hand_over, 0.0) * conv_small_plan(s, element_bytes).us
+				: workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
 	}
 
 	template<typename TE, typename Epi>

@@ -8,6 +8,27 @@
 
 namespace avhip
 {
+	/* n / d for n below 2^31 by a multiplication: with 2^shift >= d and factor = ceil(2^(31 + shift) / d), n * factor / 2^(31 + shift) is too
+	 * large by less than 1 / d.  A division by a number that only the launch knows is a chain of some twenty dependent instructions,
+	 * and three of them in a row stood before the first load of a workgroup: bf16 3x3 48 -> 48 on 3600 pixels 5.0 us a call with them, 4.4 without,
+	 * 4.6 in the kernel of one wavefront per tile that this one replaced (towers of twelve such layers; from a graph 4.3, 4.2). */
+	struct Divisor
+	{
+		unsigned int factor, shift;
+		__device__ __forceinline__ unsigned int of(unsigned int n) const
+		{
+			return __umulhi(2 * n, factor) >> shift;
+		}
+	};
+	inline Divisor divisor(unsigned int d)
+	{
+		Divisor result = { 0, 0 };
+		while ((1u << result.shift) < d)
+			result.shift++;
+		result.factor = static_cast<unsigned int>(((1ull << (31 + result.shift)) + d - 1) / d);
+		return result;
+	}
+
 	/* Launches the kernel and returns true when its estimate for the problem is below that of the kernels with 128 x 128 (or
 	 * 256 x 64) workgroup tiles; returns false without side effects otherwise.  The caller has established the conditions of the
 	 * branch-free loaders (16-byte aligned tensors below 2 GiB, zero padding value);
@@ -32,6 +53,7 @@ namespace avhip
 		double us;
 	};
 	int conv_small_threshold(); /* what avhip_set_small_problem_threshold set */
+	bool conv_small_possible(const avhipConvShape &s, int element_bytes); /* taps and chunks of a tap within the kernel's arithmetic */
 	SmallPlan conv_small_plan(const avhipConvShape &s, int element_bytes);
 	/* How results leave: LINEAR or RELU in whole aligned vectors of four filters; those activations element by element; any activation */
 	enum class HandOver
@@ -40,6 +62,8 @@ namespace avhip
 	};
 	/* Whether the launcher sends the layer to that kernel, given the conditions above.  `one_tap_us`: conv_pointwise_us. */
 	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us);
+	/* What the layer is estimated to take in that kernel or, where it is not preferred, in those with large tiles: microseconds. */
+	double conv_without_ring_us(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us);
 }
 
 #endif /* AVHIP_CONV_SMALL_HPP_ */
