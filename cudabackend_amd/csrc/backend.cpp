@@ -27,6 +27,7 @@
 
 #include "../../include/avocado_hip_backend.h"
 #include "../../include/avocado_hip_kernels.h"
+#include "conv_ring_plan.hpp"
 #include "conv_winograd_f4.hpp"
 
 namespace
@@ -976,9 +977,24 @@ namespace
 		return from_launcher(rc);
 	}
 
+	/* Whether the implicit-GEMM kernel with a ring of LDS buffers (conv_ring.hip) is estimated to need less than `us` for a 16-bit layer.  A kernel
+	 * with one workgroup per compute unit and fixed tiles pays a whole round for the first workgroup beyond the last full one. */
+	bool ring_is_faster(const ConvCall &c, double us)
+	{
+		const avhipConvShape &s = c.problem.shape;
+		const char *x = static_cast<const char*>(c.x->data), *y = static_cast<const char*>(c.y->data);
+		const int64_t x_bytes = 2ll * s.N * s.H * s.W * s.C, y_bytes = 2ll * s.N * s.Ho * s.Wo * s.K;
+		if (x < y + y_bytes && y < x + x_bytes) /* it takes no calls in place */
+			return false;
+		return avhip::ring_choice(s, 2, 2, 0, c.z != nullptr).us < us;
+	}
+
 	/* 3x3 stride-2 layers of 16-bit tensors through the parity-plane kernel (conv_strided.hip), weights in its operand layout from
 	 * the cache.  Worth it from 96 workgroups (one per compute unit, 256 filters each) on: 56 x 56 x 128 -> 256 in bf16 takes 23.5
-	 * us against 28.2 us in the gather kernel at 24 images (96 workgroups), 22.7 against 22.7 at 16. */
+	 * us against 28.2 us in the gather kernel at 24 images (96 workgroups), 22.7 against 22.7 at 16.  Of those, the layers that do not fill
+	 * its rounds go to the ring kernel: here 3.5 us and 8.0 per 64 channels in every round of 256 workgroups, 0.14 per megabyte of input and output, 1.7
+	 * less in all (110 layers of 9 to 64 rows, root mean square error 6 %); with the ring kernel 10 % below that, 59 of the 110 go there, 1.22 times as
+	 * fast on average and none slower (bf16 192 -> 512 on 24 images of 34 x 34: 29.2 against 17.2 us, 256 -> 256 on 75: 42.3 against 30.4). */
 	bool strided_kernel_pays(const ConvCall &c, avActivationType_t activation)
 	{
 		const ConvProblem &p = c.problem;
@@ -989,7 +1005,14 @@ namespace
 		int workgroups = 0, rows_used = 0;
 		if (avhip_conv2d_strided_plan(p.x_dtype, &p.shape, &workgroups, &rows_used) != 0)
 			return false;
-		return avhip_set_conv_strided(-1) == 2 || (workgroups >= 96 && rows_used >= 144);
+		if (avhip_set_conv_strided(-1) == 2)
+			return true;
+		if (workgroups < 96 || rows_used < 144)
+			return false;
+		const avhipConvShape &s = p.shape;
+		const double megabytes = 2.0e-6 * s.N * (static_cast<double>(s.H) * s.W * s.C + static_cast<double>(s.Ho) * s.Wo * s.K);
+		const double us = std::ceil(workgroups / 256.0) * (3.5 + 8.0 * s.C / 64.0) - 1.7 + 0.14 * megabytes;
+		return !ring_is_faster(c, 0.9 * us);
 	}
 	avStatus_t run_strided_kernel(const ConvCall &c, avMemoryDescriptor_t wMem, avMemoryDescriptor_t yMem, avActivationType_t activation)
 	{
