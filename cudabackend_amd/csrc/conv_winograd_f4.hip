@@ -5,23 +5,25 @@
  * M in memory: for 256 images of 15 x 15 with 128 channels these are 75 MB each, written and read once, and that traffic and not the
  * 4.8 GFLOP of the products was what bounded the plan (16 + 56 + 18 us).
  *
+ * The products run on the bf16 matrix cores, which are sixteen times as fast as the fp32 ones: every value is cut into three bf16 pieces that
+ * add up to it exactly (8 + 8 + 8 bits of the 24), and of the nine products of pieces the six that matter in 32 bits are taken.
+ *
  *   workgroup = 32 tiles (of 4 x 4 output pixels, in the order of the images) x 64 filters, eight wavefronts: four groups of nine
  *               transform points x two halves of the filters; a wavefront keeps its nine 32 x 32 products in 144 registers over the
  *               whole of k.  4096 tiles x 128 filters are 256 workgroups, one per compute unit;
  *   input     : per stage of 16 channels a work-item loads the 6 x 6 pixels of one tile and channel, transforms them in registers and
- *               writes 36 dwords of V to LDS (two buffers of 72 KB, one barrier a stage).  Wavefronts 0 to 3 do this before their
- *               products and 4 to 7 behind them: one of each kind shares a SIMD, so the vector ALU works under the other's MFMAs;
- *   weights   : U in operand order (avhip_winograd_f4_weight_transform), one contiguous kilobyte per load, six loads ahead;
+ *               writes them to LDS in pieces, two rows of points (a third) at a time into one of two buffers, in portions between the products of
+ *               the third before;
+ *   weights   : U in pieces and operand order (avhip_winograd_f4_weight_transform), one contiguous kilobyte per load, nine loads ahead;
  *   output    : M through LDS, 32 filters at a time, A^T M A in registers, the shared epilogue.
  *
- * What bounds it: the matrix cores during the stages (3.8 us for 36 x 32 x 64 x 16 products at 256 flop a clock, 4.8 measured), and
- * around them some 20 us in which all compute units load their first tiles and write their results.  How much of those is the HBM's is not
- * known: every instance has 256 vector registers and spills (272 bytes of scratch a work-item, 292 with a residual: 36 to 38 MB a launch of
- * 256 workgroups, where x and y are 29.5), in front of the first loop, a few in every stage and in both passes of the output.
- * Measured, three passes before and now, one layer again and again from a graph: 256 x 15 x 15 x 128 -> 128 87 -> 61 us, with a residual 91 ->
- * 70 us (a tower of 20 of them in turn, 1925 -> 1422 us, is 68 and 75 us a layer), 64 channels 49 -> 36 us, 40 x 40 x 40 x 99 -> 128 118 -> 60 us,
- * 32 x 56 x 56 x 64 -> 64 with residual 77 -> 47 us, 60 x 28 x 28 x 128 -> 128 68 -> 59 us.  Relative error against 64 bits 1.2e-6 to 2.9e-6 as
- * before (each within 3 % below).
+ * What bounds it: a stage takes 4.1 us and its parts 1.6 (products, 3456 clocks), 1.4 (500 vector instructions of each of two wavefronts on a SIMD), 1.3
+ * (LDS) and 2.2 (63 loads per wavefront) of them, one more in the way of the other than they should be with two wavefronts per SIMD;
+ * around the stages 13 us of first loads and results.  All instructions of a stage must find their registers: one value in scratch makes every
+ * load in flight be waited for (in-order counter), which cost a fifth.  The two passes of the output are a loop because straight-line code
+ * of that length comes from memory instruction by instruction (written out: 8 us more).
+ * Measured, fp32 products and now, one layer again and again: 256 x 15 x 15 x 128 -> 128 61 -> 46 us (three passes through memory 87), 64 channels 36 -> 24 us,
+ * a tower of 20 of them in turn 1425 -> 950 us.  Relative error against 64 bits 1.1e-6 to 2.4e-6, with fp32 products 1.2e-6 to 2.9e-6.
  */
 #include <type_traits>
 
@@ -38,9 +40,11 @@ namespace
 	constexpr int FILTERS = 64;
 	constexpr int CHANNELS = 16; /* of a stage */
 	constexpr int MY_POINTS = 9; /* of a wavefront */
-	constexpr int STEPS = MY_POINTS * CHANNELS / 8; /* loads of U per wavefront and stage */
-	constexpr int AHEAD = 6; /* of them in flight */
-	static_assert(STEPS % AHEAD == 0, "the slots of the loads in flight are the same in every stage");
+	constexpr int PARTS = 3; /* of a stage: two rows of six points each, three of the twelve a wavefront's */
+	constexpr int PART_POINTS = POINTS / PARTS, MY_PART = MY_POINTS / PARTS;
+	/* V in LDS: [point of the part][piece][half of the channels][tile][channel of the half], bf16.  The halves lie 64 bytes more than their size apart,
+	 * so that the sixteen channels of a tile go to different banks. */
+	constexpr int V_HALF = TILES * 16 + 64, V_PIECE = 2 * V_HALF, V_POINT = 3 * V_PIECE, V_PART = PART_POINTS * V_POINT;
 
 	struct F4Geom
 	{
@@ -49,8 +53,8 @@ namespace
 		int stages, filter_blocks;
 	};
 
-	/* offsets beyond every tensor the launcher accepts (below 2^29 bytes), alone and added up */
-	constexpr unsigned int NO_ROW = 0x80000000u, NO_COLUMN = 0x40000000u, NO_CHANNEL = 0x20000000u;
+	/* an offset beyond every tensor the launcher accepts (below 2^29 bytes), with the offset of a pixel added too */
+	constexpr unsigned int NO_PIXEL = 0x80000000u;
 
 	/* B^T d along one direction: [1 0 -5/4 0 1/4 0; 0 1 1 -1/4 -1/4 0; 0 -1 1 1/4 -1/4 0; 0 -1 -1/2 1 1/2 0; 0 1 -1/2 -1 1/2 0; 0 1 0 -5/4 0 1/4] */
 	__device__ __forceinline__ void input_line(float &d0, float &d1, float &d2, float &d3, float &d4, float &d5)
@@ -77,15 +81,15 @@ namespace
 	template<bool RELU, bool RESIDUAL>
 	__global__ __launch_bounds__(512, 2) void k_winograd_f4(const float *__restrict__ x, const float *__restrict__ U, F4Geom g, FloatEpilogue<float> epi)
 	{
-		/* V: [point][quad of channels][tile][channel of the quad]; M: [point][quad of filters][tile][filter of the quad], tiles in
-		 * the order tile ^ 4 * quad: conflict-free for the work-items of neighbouring quads and for those of neighbouring tiles */
-		constexpr int V_FLOATS = POINTS * CHANNELS * TILES;
-		static_assert(2 * V_FLOATS == POINTS * 32 * TILES, "the products of half of the filters take the place of the two stages");
-		__shared__ __attribute__((aligned(16))) float lds[2 * V_FLOATS];
+		/* two parts of V; behind the loop M: [point][quad of filters][tile][filter of the quad], tiles in the order tile ^ 4 * quad: conflict-free
+		 * for the work-items of neighbouring quads and for those of neighbouring tiles */
+		constexpr int M_BYTES = POINTS * 32 * TILES * 4;
+		static_assert(2 * V_PART <= M_BYTES, "the products of half of the filters take the place of the two parts");
+		__shared__ __attribute__((aligned(16))) char lds[M_BYTES];
 
 		const int tid = threadIdx.x, lane = tid & 63;
 		const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-		const int first_point = MY_POINTS * (wave & 3), my_half = wave >> 2;
+		const int my_points = MY_PART * (wave & 3), my_half = wave >> 2; /* point q of part j is 12 j + my_points + q */
 		/* the filter blocks of a tile block are neighbours: their input comes from one L2 */
 		const unsigned int block = xcd_block(blockIdx.x, gridDim.x);
 		const unsigned int tile_block = block / g.filter_blocks, filter_block = block - tile_block * g.filter_blocks;
@@ -100,55 +104,110 @@ namespace
 		const int t = t0 + tile;
 		const int line = t / g.tiles_w, tw = t - line * g.tiles_w;
 		const int image = line / g.tiles_h, th = line - image * g.tiles_h;
-		unsigned int row[6], column[6];
+		/* which rows and columns of the tile exist: lane masks in scalar registers, of which there are enough */
+		const unsigned int top = static_cast<unsigned int>(((image * g.H + 4 * th + g.pad_h) * g.W + 4 * tw + g.pad_w) * g.C + channel) * 4u;
+		bool row[6], column[6];
 #pragma unroll
 		for (int a = 0; a < 6; a++)
 		{
 			const int ih = 4 * th + g.pad_h + a, iw = 4 * tw + g.pad_w + a;
-			row[a] = t < g.tiles && ih >= 0 && ih < g.H
-					? static_cast<unsigned int>(((image * g.H + ih) * g.W + 4 * tw + g.pad_w) * g.C + channel) * 4u : NO_ROW;
-			column[a] = iw >= 0 && iw < g.W ? static_cast<unsigned int>(a * g.C) * 4u : NO_COLUMN;
+			row[a] = t < g.tiles && ih >= 0 && ih < g.H;
+			column[a] = iw >= 0 && iw < g.W;
 		}
+		const unsigned int pixel_bytes = static_cast<unsigned int>(g.C) * 4u, row_bytes = static_cast<unsigned int>(g.W) * pixel_bytes;
+		const int last = g.stages - 1;
+		const bool in_last = CHANNELS * last + channel < g.C;
 		float d[36];
-		auto load_input = [&](int stage) __attribute__((always_inline))
+		auto load_row = [&](int stage, int a) __attribute__((always_inline))
 		{
-			const unsigned int at = 64u * stage + (CHANNELS * stage + channel < g.C ? 0u : NO_CHANNEL);
-#pragma unroll
-			for (int a = 0; a < 6; a++)
-			{
-				unsigned int line = row[a] + at;
-				asm volatile("" : "+v"(line)); /* or 36 sums of row and column are kept over the loop, more than there are registers */
-#pragma unroll
-				for (int b = 0; b < 6; b++)
-					d[6 * a + b] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, static_cast<int>(line + column[b]), 0, 0));
-				__builtin_amdgcn_sched_barrier(0); /* six offsets at a time */
-			}
-		};
-		const int put = (channel >> 2) * (TILES * 4) + (tile ^ (channel & ~3)) * 4 + (channel & 3);
-		auto transform_input = [&](int buffer) __attribute__((always_inline))
-		{
-			float *to = lds + buffer * V_FLOATS + put;
+			const bool exists = row[a] && (stage < last || (stage == last && in_last)); /* (the stages behind the last: zeros) */
+			unsigned int line = exists ? top + a * row_bytes + 64u * stage : NO_PIXEL;
+			asm volatile("" : "+v"(line)); /* or 36 offsets are kept over the loop, more than there are registers */
 #pragma unroll
 			for (int b = 0; b < 6; b++)
-				input_line(d[b], d[6 + b], d[12 + b], d[18 + b], d[24 + b], d[30 + b]);
+				d[6 * a + b] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, static_cast<int>(column[b] ? line + b * pixel_bytes : NO_PIXEL), 0, 0));
+		};
+		/* (the sixteen channels of a tile are in the order 0, 8, 1, 9, .. in V and U) */
+		const int put = ((channel & 7) >> 2) * V_HALF + tile * 16 + (channel & 3) * 4 + (channel >> 3) * V_POINT;
+		auto transform_column = [&](int b) __attribute__((always_inline))
+		{
+			input_line(d[b], d[6 + b], d[12 + b], d[18 + b], d[24 + b], d[30 + b]);
+		};
+		auto transform_row = [&](int a) __attribute__((always_inline))
+		{
+			input_line(d[6 * a], d[6 * a + 1], d[6 * a + 2], d[6 * a + 3], d[6 * a + 4], d[6 * a + 5]);
+		};
+		/* Two values of V, in pieces: the sixteen highest bits of a float are a bf16, and these are stored of v, of v less that, and of the rest.
+		 * (med3: no rest of an infinity, and not NaN.)  Eight lanes beside the eight that have the first eight channels have the others of the
+		 * same tile: they exchange values, so that each has both channels of a pair for one of the points, and write dwords: stores of single
+		 * pieces took the LDS longer than the products take the matrix cores. */
+		auto store_pieces = [&](int part, int buffer, int e) __attribute__((always_inline))
+		{
+			constexpr int ROW_ROTATE_8 = 0x128;
+			const int e0 = __builtin_bit_cast(int, d[12 * part + e]), e1 = __builtin_bit_cast(int, d[12 * part + e + 1]);
+			unsigned int value[2] = { static_cast<unsigned int>(__builtin_amdgcn_update_dpp(e0, e1, ROW_ROTATE_8, 15, 12, false)),
+					static_cast<unsigned int>(__builtin_amdgcn_update_dpp(e1, e0, ROW_ROTATE_8, 15, 3, false)) };
+			unsigned int *to = reinterpret_cast<unsigned int*>(lds + buffer * V_PART + put + e * V_POINT);
 #pragma unroll
-			for (int a = 0; a < 6; a++)
+			for (int piece = 0; piece < 3; piece++)
 			{
-				input_line(d[6 * a], d[6 * a + 1], d[6 * a + 2], d[6 * a + 3], d[6 * a + 4], d[6 * a + 5]);
+				to[piece * V_PIECE / 4] = __builtin_amdgcn_perm(value[1], value[0], 0x07060302u);
 #pragma unroll
-				for (int b = 0; b < 6; b++)
-					to[(6 * a + b) * (CHANNELS * TILES)] = d[6 * a + b];
+				for (int i = 0; i < 2; i++)
+				{
+					const float rest = __builtin_bit_cast(float, value[i]) - __builtin_bit_cast(float, value[i] & 0xFFFF0000u);
+					value[i] = __builtin_bit_cast(unsigned int, piece == 0 ? __builtin_amdgcn_fmed3f(rest, rest, 0.0f) : rest);
+				}
+			}
+		};
+		/* A part is two rows of V: made in 18 pieces of work, one in front of each product of the part before; then their places in the
+		 * registers are loaded with pixels of the next stage.  (Columns are transformed for the first part, as late as its work allows: its last
+		 * pixels were requested a part ago.) */
+		constexpr int SLOTS = 6 * MY_PART;
+		static_assert(SLOTS == 18, "the work below");
+		auto produce = [&](int slot, int part, int buffer, int next_stage) __attribute__((always_inline))
+		{
+			const int a = 2 * part;
+			if (part == 0)
+			{
+				if (slot >= 4 && slot < 10)
+					transform_column(slot - 4);
+				if (slot == 10 || slot == 14)
+					transform_row(a + (slot == 14 ? 1 : 0));
+				if ((slot >= 11 && slot < 14) || slot >= 15)
+				{
+					const int e = slot < 14 ? 2 * (slot - 11) : 6 + 2 * (slot - 15);
+					store_pieces(part, buffer, e);
+				}
+				if (slot == 14)
+					load_row(next_stage, a);
+				if (slot == 17)
+					load_row(next_stage, a + 1);
+			}
+			else
+			{
+				if (slot == 0 || slot == 7)
+					transform_row(a + (slot == 7 ? 1 : 0));
+				if (slot < 7 && slot % 2 == 1)
+					store_pieces(part, buffer, slot - 1);
+				if (slot > 7 && slot < 14 && slot % 2 == 0)
+					store_pieces(part, buffer, slot - 2);
+				if (slot == 7)
+					load_row(next_stage, a);
+				if (slot == 14)
+					load_row(next_stage, a + 1);
 			}
 		};
 
-		/* U: [block of 32 filters][point][8 channels][lane][4 channels]; step i of a stage: point i / 2, half i % 2 of its channels */
-		const int slabs = 2 * g.stages;
-		const int u_first = ((2 * static_cast<int>(filter_block) + my_half) * POINTS + first_point) * slabs;
-		uint4 u[AHEAD];
-		auto load_weights = [&](int step, int stage) __attribute__((always_inline))
+		/* U: [block of 32 filters][point][16 channels][piece][lane][8 channels] */
+		const int u_first = ((2 * static_cast<int>(filter_block) + my_half) * POINTS + my_points) * g.stages;
+		Chunk u[MY_PART][3];
+		auto load_weights = [&](int stage, int part, int q) __attribute__((always_inline))
 		{
-			const int slab = u_first + (step >> 1) * slabs + 2 * stage + (step & 1);
-			u[step % AHEAD] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ru, lane * 16, slab * 1024, 0));
+			const int at = (u_first + (PART_POINTS * part + q) * g.stages + stage) * 3072;
+#pragma unroll
+			for (int piece = 0; piece < 3; piece++)
+				u[q][piece].u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ru, lane * 16, at + 1024 * piece, 0));
 		};
 		Mma<float>::acc_t acc[MY_POINTS]; /* [filters][tiles] */
 #pragma unroll
@@ -157,63 +216,60 @@ namespace
 			for (int v = 0; v < 16; v++)
 				acc[p][v] = 0;
 		const int r = lane & 31, half = lane >> 5;
-		auto multiply = [&](int stage, int next) __attribute__((always_inline))
+		const int get = my_points * V_POINT + half * V_HALF + r * 16;
+		/* One part: its products, v w of the pieces h + m + l with the smallest products first (what is left out, m l and below, is less than 2^-22 of
+		 * the whole), and between them the work on the next part. */
+		auto step = [&](int stage, int part, int buffer) __attribute__((always_inline))
 		{
-			const uint4 *from = reinterpret_cast<const uint4*>(lds + (stage & 1) * V_FLOATS) + first_point * (CHANNELS / 4 * TILES);
-			Chunk cx[2];
-			auto read = [&](int i) __attribute__((always_inline))
+			constexpr int V_OF[6] = { 2, 1, 1, 0, 0, 0 }, U_OF[6] = { 0, 1, 0, 2, 1, 0 };
+			const int next_part = (part + 1) % PARTS, next = part == PARTS - 1 ? stage + 1 : stage;
+			const int weights_of = next < last ? next : last; /* (behind the last: its own once more) */
+			__syncthreads(); /* this part of V is complete, the one before has been read */
+			const char *from = lds + buffer * V_PART + get;
+			Chunk cx[3];
+			auto read = [&](int q, int piece) __attribute__((always_inline))
 			{
-				const int quad = 2 * (i & 1) + half;
-				cx[i & 1].u = from[((i >> 1) * (CHANNELS / 4) + quad) * TILES + (r ^ (4 * quad))];
+				cx[piece].u = *reinterpret_cast<const uint4*>(from + q * V_POINT + piece * V_PIECE);
 			};
-			read(0);
+			read(0, 2);
+			read(0, 1);
+			read(0, 0);
 #pragma unroll
-			for (int i = 0; i < STEPS; i++)
+			for (int slot = 0; slot < SLOTS; slot++)
 			{
-				if (i + 1 < STEPS)
-					read(i + 1);
-				Chunk cw;
-				cw.u = u[i % AHEAD];
-				Mma<float>::run(cw, cx[i & 1], acc[i >> 1]);
-				if (i + AHEAD < STEPS)
-					load_weights(i + AHEAD, stage);
-				else
-					load_weights(i + AHEAD - STEPS, next);
-				/* without it the loads are moved down to their use and every step waits for its own */
+				const int q = slot / 6, i = slot - 6 * q;
+				produce(slot, next_part, buffer ^ 1, next + 1); /* (pixels behind the last channel: zeros) */
+				__builtin_amdgcn_sched_barrier(0);
+				Mma<bf16_t>::run(u[q][U_OF[i]], cx[V_OF[i]], acc[MY_PART * part + q]);
+				__builtin_amdgcn_sched_barrier(0);
+				if (q + 1 < MY_PART && (i == 0 || i == 2 || i == 5))
+					read(q + 1, V_OF[i]);
+				if (i == 5)
+					load_weights(weights_of, next_part, q);
 				__builtin_amdgcn_sched_barrier(0);
 			}
 		};
 
-		load_input(0);
 #pragma unroll
-		for (int i = 0; i < AHEAD; i++)
-			load_weights(i, 0);
-		transform_input(0);
-		load_input(1); /* (behind the last channel: zeros) */
-		const int last = g.stages - 1;
-		if (wave < 4)
-			for (int s = 0; s < last; s++)
-			{
-				__syncthreads(); /* V of this stage is complete, that of the one before has been read */
-				transform_input((s + 1) & 1);
-				load_input(s + 2);
-				multiply(s, s + 1);
-			}
-		else
-			for (int s = 0; s < last; s++)
-			{
-				__syncthreads();
-				multiply(s, s + 1);
-				transform_input((s + 1) & 1);
-				load_input(s + 2);
-			}
-		__syncthreads();
-		multiply(last, last); /* (the loads ahead: its own weights once more) */
+		for (int a = 0; a < 6; a++)
+			load_row(0, a);
+#pragma unroll
+		for (int q = 0; q < MY_PART; q++)
+			load_weights(0, 0, q);
+#pragma unroll
+		for (int slot = 0; slot < SLOTS; slot++)
+			produce(slot, 0, 0, 1);
+		for (int s = 0, odd = 0; s <= last; s++, odd ^= 1)
+		{
+			step(s, 0, odd);
+			step(s, 1, odd ^ 1);
+			step(s, 2, odd);
+		}
 
 		/* two filters of a tile per work-item: its place among 16 neighbours is the pair, so that runs of 128 bytes leave */
 		const int pair = tid & 15;
 		float4 *products = reinterpret_cast<float4*>(lds);
-#pragma unroll
+#pragma unroll 1
 		for (int pass = 0; pass < 2; pass++)
 		{
 			const int k = k0 + 32 * pass + 2 * pair;
@@ -245,7 +301,7 @@ namespace
 					for (int v = 0; v < 4; v++)
 					{
 						const int quad = 2 * v + half;
-						products[((first_point + p) * 8 + quad) * TILES + (r ^ (4 * quad))] = make_float4(acc[p][4 * v], acc[p][4 * v + 1], acc[p][4 * v + 2], acc[p][4 * v + 3]);
+						products[((PART_POINTS * (p / MY_PART) + my_points + p % MY_PART) * 8 + quad) * TILES + (r ^ (4 * quad))] = make_float4(acc[p][4 * v], acc[p][4 * v + 1], acc[p][4 * v + 2], acc[p][4 * v + 3]);
 					}
 			}
 			__syncthreads();
@@ -305,7 +361,7 @@ namespace
 		u[4] = q - m;
 		u[5] = 2.0f * g2;
 	}
-	__global__ __launch_bounds__(256) void k_f4_weights(const float *__restrict__ w, float *__restrict__ U, int K, int C, int padded_c, int work, int invert)
+	__global__ __launch_bounds__(256) void k_f4_weights(const float *__restrict__ w, unsigned short *__restrict__ U, int K, int C, int padded_c, int work, int invert)
 	{
 		const int id = blockIdx.x * 256 + threadIdx.x;
 		if (id >= work)
@@ -324,8 +380,8 @@ namespace
 #pragma unroll
 		for (int j = 0; j < 3; j++)
 			weight_line(taps[0][j], taps[1][j], taps[2][j], columns[j]);
-		const int slabs = padded_c / 8;
-		float *to = U + (static_cast<int64_t>(k >> 5) * POINTS * slabs + (c >> 3)) * 256 + ((c & 7) >> 2) * 128 + (k & 31) * 4 + (c & 3);
+		const int slabs = padded_c / CHANNELS, place = 2 * (c & 7) + ((c >> 3) & 1); /* in the order 0, 8, 1, 9, .. */
+		unsigned short *to = U + (static_cast<int64_t>(k >> 5) * POINTS * slabs + c / CHANNELS) * 1536 + ((place >> 3) * 256) + (k & 31) * 8 + (place & 7);
 #pragma unroll
 		for (int i = 0; i < 6; i++)
 		{
@@ -333,7 +389,20 @@ namespace
 			weight_line(columns[0][i], columns[1][i], columns[2][i], u);
 #pragma unroll
 			for (int j = 0; j < 6; j++)
-				to[static_cast<int64_t>(6 * i + j) * slabs * 256] = u[j];
+			{
+				unsigned short *piece = to + static_cast<int64_t>(6 * i + j) * slabs * 1536;
+				float rest = u[j];
+#pragma unroll
+				for (int n = 0; n < 3; n++)
+				{
+					unsigned int bits = __builtin_bit_cast(unsigned int, rest);
+					rest = fabsf(rest) < INFINITY ? rest - __builtin_bit_cast(float, bits & 0xFFFF0000u) : 0.0f;
+					/* no piece is zero where u is not (and large against what takes the zero's place): the product with an infinity stays one */
+					if (bits << 1 == 0 && fabsf(u[j]) > 0x1p-80f)
+						bits = (__builtin_bit_cast(unsigned int, u[j]) & 0x80000000u) | 0x00800000u;
+					piece[512 * n] = static_cast<unsigned short>(bits >> 16);
+				}
+			}
 		}
 	}
 
@@ -345,7 +414,7 @@ namespace
 	{
 		return (static_cast<int64_t>(K) + FILTERS - 1) / FILTERS * FILTERS;
 	}
-	constexpr int64_t MOST_BYTES = 1ll << 29;
+	constexpr int64_t MOST_BYTES = 1ll << 29, MOST_WEIGHT_BYTES = 3ll << 28;
 	int64_t pixels_of(const avhipConvShape &s)
 	{
 		return static_cast<int64_t>(s.N) * s.H * s.W;
@@ -366,25 +435,25 @@ namespace avhip
 			return false;
 		/* the output has the input's size, so every output pixel lies in a tile whatever the offset of the taps is */
 		const int64_t blocks = (tiles_of(s) + TILES - 1) / TILES * (padded_filters(s.K) / FILTERS);
-		return pixels_of(s) * s.C * 4 < MOST_BYTES && avhip_winograd_f4_weight_bytes(s.K, s.C) < MOST_BYTES && static_cast<int64_t>(s.C) * 4 * 8 < (1ll << 27)
+		return pixels_of(s) * s.C * 4 < MOST_BYTES && avhip_winograd_f4_weight_bytes(s.K, s.C) < MOST_WEIGHT_BYTES && static_cast<int64_t>(s.C) * 4 * 8 < (1ll << 27)
 				&& blocks * 512 < (1ll << 32) && pixels_of(s) * s.K * 4 < (1ll << 31) && s.pad_h >= -8 && s.pad_h <= 8 && s.pad_w >= -8 && s.pad_w <= 8;
 	}
 }
 
 extern "C" int64_t avhip_winograd_f4_weight_bytes(int K, int C)
 {
-	return POINTS * padded_filters(K) * padded_channels(C) * 4;
+	return POINTS * padded_filters(K) * padded_channels(C) * 6;
 }
 
 extern "C" int avhip_winograd_f4_weight_transform(void *stream, int invert, const void *w, void *U, int K, int C)
 {
 	if (w == nullptr || U == nullptr || K <= 0 || C <= 0)
 		return AVHIP_BAD_PARAM;
-	if (avhip_winograd_f4_weight_bytes(K, C) >= MOST_BYTES)
+	if (avhip_winograd_f4_weight_bytes(K, C) >= MOST_WEIGHT_BYTES)
 		return AVHIP_NOT_SUPPORTED;
 	const int padded_c = static_cast<int>(padded_channels(C)), work = static_cast<int>(padded_filters(K)) * padded_c;
 	hipLaunchKernelGGL(k_f4_weights, dim3(ceil_div(work, 256)), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const float*>(w),
-			static_cast<float*>(U), K, C, padded_c, work, invert != 0 ? 1 : 0);
+			static_cast<unsigned short*>(U), K, C, padded_c, work, invert != 0 ? 1 : 0);
 	return 0;
 }
 
