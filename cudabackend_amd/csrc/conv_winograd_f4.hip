@@ -19,9 +19,9 @@
  *
  * What bounds it: a stage takes 4.1 us and its parts 1.6 (products, 3456 clocks), 1.4 (500 vector instructions of each of two wavefronts on a SIMD), 1.3
  * (LDS) and 2.2 (63 loads per wavefront) of them, one more in the way of the other than they should be with two wavefronts per SIMD;
- * around the stages 13 us of first loads and results.  All instructions of a stage must find their registers: one value in scratch makes every
- * load in flight be waited for (in-order counter), which cost a fifth.  The two passes of the output are a loop because straight-line code
- * of that length comes from memory instruction by instruction (written out: 8 us more).
+ * around the stages 13 us of first loads and results.  All values of a stage must stay in registers: one in scratch makes every load in flight be
+ * waited for (in-order counter), which cost a fifth.  The two passes of the output are a loop, for the same reason: written out they kept 24
+ * registers in scratch and the kernel took 8 us longer.
  * Measured, fp32 products and now, one layer again and again: 256 x 15 x 15 x 128 -> 128 61 -> 46 us (three passes through memory 87), 64 channels 36 -> 24 us,
  * a tower of 20 of them in turn 1425 -> 950 us.  Relative error against 64 bits 1.1e-6 to 2.4e-6, with fp32 products 1.2e-6 to 2.9e-6.
  */
