@@ -161,7 +161,7 @@ namespace
 		}
 	}
 
-	/* 4, 8 or 16 bytes through a buffer descriptor; zeros at OUT_OF_RANGE */
+	/* 2, 4, 8 or 16 bytes through a buffer descriptor; zeros at OUT_OF_RANGE */
 	template<typename T, int V>
 	__device__ __forceinline__ Pack<T, V> fetch_pack(__amdgpu_buffer_rsrc_t rsrc, unsigned int offset)
 	{
@@ -169,27 +169,32 @@ namespace
 			return __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(offset), 0, 0));
 		else if constexpr (sizeof(T) * V == 8)
 			return __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b64(rsrc, static_cast<int>(offset), 0, 0));
-		else
+		else if constexpr (sizeof(T) * V == 4)
 			return __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b32(rsrc, static_cast<int>(offset), 0, 0));
+		else
+			return __builtin_bit_cast(Pack<T, V>, __builtin_amdgcn_raw_buffer_load_b16(rsrc, static_cast<int>(offset), 0, 0));
 	}
+	template<typename T, int V>
+	constexpr bool buffer_run = sizeof(T) <= 4 && (sizeof(T) * V == 2 || sizeof(T) * V == 4 || sizeof(T) * V == 8 || sizeof(T) * V == 16);
 
 	/* IDX is the integer type of the work-item and tile indices: 32 bits whenever the problem allows it (64-bit divisions
 	 * cost more than the transform itself).  V > 1 instances are launched only when every vector is complete and aligned:
 	 * they have no tail handling, and outside the image they load from a clamped address and select the padding value, so
 	 * the whole work-item is branch-free and all its loads are in flight together. */
-	/* BUF instances (complete vectors of 4, 8 or 16 bytes, zero padding value, x below 2 GiB) fetch through a buffer descriptor: a pixel outside the image is
+	/* BUF instances (complete vectors of 2 to 16 bytes, zero padding value, x below 2 GiB) fetch through a buffer descriptor: a pixel outside the image is
 	 * asked for at an out-of-range offset and comes back as zeros, so every load of the work-item is unconditional.  With ordinary
 	 * loads the compiler turns "load at a clamped address, then select the padding value" back into a branch around each load,
 	 * and where the element conversion is an instruction of its own (fp16) it ends up behind the branch with a wait in front of it: the
-	 * sixteen loads of a tile then run one after the other (the fp16 instance was 13 % slower than the bf16 one on the same bytes). */
+	 * sixteen loads of a tile then run one after the other (the fp16 instance was 13 % slower than the bf16 one on the same bytes).  Single
+	 * channels (odd counts) likewise: bf16 159 channels on 85 images of 15 x 14 13.5 -> 9.3 us. */
 	template<int M, int R, typename T, typename TM, int V, typename IDX, bool BUF = false>
 	__global__ __launch_bounds__(256) void k_input_transform(const T *__restrict__ x, TM *__restrict__ Vm, int N, int H, int W, int C, int Th, int Tw,
 			int pad_h, int pad_w, typename Traits<T>::compute padv)
 	{
 		typedef typename Traits<T>::compute CT;
 		constexpr int t = M + R - 1;
-		constexpr bool FULL = V > 1;
-		static_assert(!BUF || (FULL && (sizeof(T) * V == 4 || sizeof(T) * V == 8 || sizeof(T) * V == 16) && sizeof(IDX) == 4), "whole 4-, 8- or 16-byte vectors, 32-bit offsets");
+		constexpr bool FULL = V > 1 || BUF;
+		static_assert(!BUF || (buffer_run<T, V> && sizeof(IDX) == 4), "runs of 2 to 16 bytes, 32-bit offsets");
 		const IDX CV = static_cast<IDX>((C + V - 1) / V);
 		const IDX tiles = static_cast<IDX>(N) * Th * Tw;
 		/* neighbouring tiles share input pixels: consecutive runs of tiles go to one XCD, whose L2 then serves the overlap */
@@ -355,7 +360,7 @@ namespace
 	{
 		typedef typename Traits<T>::compute CT;
 		constexpr int t = M + R - 1;
-		constexpr bool FULL = V > 1;
+		constexpr bool FULL = V > 1 || BUF;
 		const IDX KV = static_cast<IDX>((K + V - 1) / V);
 		const IDX tiles = static_cast<IDX>(N) * Th * Tw;
 		const IDX gid = static_cast<IDX>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -381,7 +386,7 @@ namespace
 				{
 					const int h = th * M + a, w = tw * M + b;
 					const unsigned int offset = (((static_cast<unsigned int>(n) * H + h) * W + w) * K + k) * static_cast<unsigned int>(sizeof(T));
-					raw[a * M + b] = fetch_pack<T, V>(rdy, (h < H) & (w < W) ? offset : OUT_OF_RANGE);
+					raw[a * M + b] = fetch_pack<T, V>(rdy, ((h < H) & (w < W)) ? offset : OUT_OF_RANGE);
 				}
 #pragma unroll
 			for (int i = 0; i < M * M; i++)
@@ -497,6 +502,16 @@ namespace
 		return items < 2u * 256u * 256u ? 64 : 256;
 	}
 
+	/* Channels per work-item of the input and gradient transforms: `widest` (what pick_vec allows), or half of it, dwords at least, where that leaves
+	 * fewer than two wavefronts per SIMD, each of which would do its loads, its arithmetic and its stores one after the other (fp32 F(2x2, 3x3)
+	 * gradient of 41 images of 12 x 12, 240 -> 32, all four launches: 32.7 -> 31.1 us; of 61 x 21 x 24, 96 -> 140: 65.3 -> 61.9). */
+	constexpr size_t TWO_WAVES_PER_SIMD = 2 * 4 * 256 * 64;
+	template<int M, int R, typename T, typename TM>
+	int run_of_items(int widest, size_t elements)
+	{
+		return widest > 1 && sizeof(T) * widest > 4 && elements / widest < TWO_WAVES_PER_SIMD ? widest / 2 : widest;
+	}
+
 	template<typename T> typename Traits<T>::compute host_scalar(const void *p)
 	{
 		if (p == nullptr)
@@ -522,24 +537,32 @@ namespace
 	{
 		const int Th = (H + M - 1) / M, Tw = (W + M - 1) / M;
 		const int V = pick_vec<M, R, T, TM>(C, x, Vm);
+		const bool narrow = static_cast<size_t>(N) * Th * Tw * ((C + V - 1) / V) < (1ull << 31) && static_cast<uint64_t>(H) * W * C < (1ull << 31);
+		const typename Traits<T>::compute padv = host_scalar<T>(padding_value);
+		const bool buffered = padv == static_cast<typename Traits<T>::compute>(0) && static_cast<uint64_t>(N) * H * W * C * sizeof(T) < (1ull << 31);
+		if constexpr (buffer_run<T, 1>)
+			if (narrow && buffered)
+			{
+				const int width = run_of_items<M, R, T, TM>(V, static_cast<size_t>(N) * Th * Tw * C);
+				const size_t items = static_cast<size_t>(N) * Th * Tw * (C / width);
+				const unsigned int group = group_size(items);
+#define AVHIP_LAUNCH_INPUT_BUFFER(WIDTH) hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, uint32_t, true>), dim3(ceil_div(items, group)), dim3(group), 0, s, \
+		static_cast<const T*>(x), static_cast<TM*>(Vm), N, H, W, C, Th, Tw, pad_h, pad_w, padv)
+				if (width == 1)
+					AVHIP_LAUNCH_INPUT_BUFFER(1);
+				else if (width == VecOf<M, R, T, TM>::value)
+					AVHIP_LAUNCH_INPUT_BUFFER((VecOf<M, R, T, TM>::value));
+				else
+					AVHIP_LAUNCH_INPUT_BUFFER(2);
+#undef AVHIP_LAUNCH_INPUT_BUFFER
+				return 0;
+			}
 		const size_t items = static_cast<size_t>(N) * Th * Tw * ((C + V - 1) / V);
 		const unsigned int group = group_size(items);
 		const dim3 grid(ceil_div(items, group));
-		const typename Traits<T>::compute padv = host_scalar<T>(padding_value);
-		const bool narrow = items < (1ull << 31) && static_cast<uint64_t>(H) * W * C < (1ull << 31);
 #define AVHIP_LAUNCH_INPUT(WIDTH, IDX) hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, IDX>), grid, dim3(group), 0, s, static_cast<const T*>(x), \
 		static_cast<TM*>(Vm), N, H, W, C, Th, Tw, pad_h, pad_w, padv)
-		const bool buffered = padv == static_cast<typename Traits<T>::compute>(0) && static_cast<uint64_t>(N) * H * W * C * sizeof(T) < (1ull << 31);
-		if (V > 1 && narrow && buffered)
-		{
-			constexpr int WIDTH = VecOf<M, R, T, TM>::value;
-			if constexpr (WIDTH > 1 && (sizeof(T) * WIDTH == 4 || sizeof(T) * WIDTH == 8 || sizeof(T) * WIDTH == 16))
-				hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, uint32_t, true>), grid, dim3(group), 0, s, static_cast<const T*>(x), static_cast<TM*>(Vm), N, H, W,
-						C, Th, Tw, pad_h, pad_w, padv);
-			else
-				AVHIP_LAUNCH_INPUT(WIDTH, uint32_t);
-		}
-		else if (V > 1 && narrow)
+		if (V > 1 && narrow)
 			AVHIP_LAUNCH_INPUT((VecOf<M, R, T, TM>::value), uint32_t);
 		else if (V > 1)
 			AVHIP_LAUNCH_INPUT((VecOf<M, R, T, TM>::value), size_t);
@@ -600,20 +623,27 @@ namespace
 	{
 		const int Th = (H + M - 1) / M, Tw = (W + M - 1) / M;
 		const int V = pick_vec<M, R, T, TM>(K, dy, Mx);
-		const size_t items = static_cast<size_t>(N) * Th * Tw * ((K + V - 1) / V);
-		const unsigned int group = group_size(items);
-		const dim3 grid(ceil_div(items, group));
-		const bool narrow = items < (1ull << 31);
+		const bool narrow = static_cast<size_t>(N) * Th * Tw * ((K + V - 1) / V) < (1ull << 31);
 		const bool buffered = static_cast<uint64_t>(N) * H * W * K * sizeof(T) < (1ull << 31);
-#define AVHIP_LAUNCH_GRADIENT(WIDTH, ...) hipLaunchKernelGGL((k_gradient_transform<M, R, T, TM, WIDTH, __VA_ARGS__>), grid, dim3(group), 0, s, \
-		static_cast<const T*>(dy), static_cast<TM*>(Mx), N, H, W, K, Th, Tw)
 		constexpr int WIDTH = VecOf<M, R, T, TM>::value;
-		if constexpr (WIDTH > 1 && (sizeof(T) * WIDTH == 4 || sizeof(T) * WIDTH == 8 || sizeof(T) * WIDTH == 16))
-			if (V > 1 && narrow && buffered)
+#define AVHIP_LAUNCH_GRADIENT(WIDTH, ...) hipLaunchKernelGGL((k_gradient_transform<M, R, T, TM, WIDTH, __VA_ARGS__>), dim3(ceil_div(items, group)), dim3(group), 0, s, \
+		static_cast<const T*>(dy), static_cast<TM*>(Mx), N, H, W, K, Th, Tw)
+		if constexpr (buffer_run<T, 1>)
+			if (narrow && buffered)
 			{
-				AVHIP_LAUNCH_GRADIENT(WIDTH, uint32_t, true);
+				const int width = run_of_items<M, R, T, TM>(V, static_cast<size_t>(N) * Th * Tw * K);
+				const size_t items = static_cast<size_t>(N) * Th * Tw * (K / width);
+				const unsigned int group = group_size(items);
+				if (width == 1)
+					AVHIP_LAUNCH_GRADIENT(1, uint32_t, true);
+				else if (width == WIDTH)
+					AVHIP_LAUNCH_GRADIENT(WIDTH, uint32_t, true);
+				else
+					AVHIP_LAUNCH_GRADIENT(2, uint32_t, true);
 				return 0;
 			}
+		const size_t items = static_cast<size_t>(N) * Th * Tw * ((K + V - 1) / V);
+		const unsigned int group = group_size(items);
 		if (V > 1)
 			AVHIP_LAUNCH_GRADIENT(WIDTH, size_t);
 		else if (narrow)
