@@ -4,20 +4,22 @@
  * (16 or 36 of them) and both operands are contiguous along m and n, not along k.
  *
  * No transpose is made.  For fp32 the operand layout of v_mfma_f32_32x32x2_f32 (lane l: row l % 32, k l / 32) is exactly a
- * coalesced load of two rows of A.  For 16-bit types a lane loads one dword (two neighbouring m) of eight consecutive k
- * rows and separates them with eight v_perm_b32 into the operand chunks of two MFMA tiles, one of the even and one of the
- * odd m; what cannot be read in pairs (odd sizes) is loaded element by element.  k rows and m, n outside the matrices come
- * back as zeros from the buffer loads, so the loop has no branch.
+ * coalesced load of two rows of A, and the eight k that a lane has of a stage are an operand of a bf16 product too: with tiles of 64 x 64 the
+ * values are cut into three bf16 pieces that add up to them exactly, in registers, and six of the nine products of pieces are taken.  (The cutting costs
+ * as much as the products save with 32 x 32: 12.6 against 11.1 us below.)  For 16-bit types a lane loads one dword (two neighbouring m) of four or eight
+ * k rows and separates them with v_perm_b32 into the operand chunks of two MFMA tiles, one of the even and one of the odd m, or exchanges one
+ * of the two with the sixteen lanes beside it; what cannot be read in pairs (odd sizes) is loaded element by element.  k rows and m, n
+ * outside the matrices come back as zeros from the buffer loads, so the loop has no branch.
  *
- * Workgroup = 8 wavefronts on ONE tile of C (64 x 64 or 32 x 32): each takes every eighth stage of 16 k rows, three or four
+ * Workgroup = 8 wavefronts on ONE tile of C (64 x 64 or 32 x 32): each takes every eighth stage of 16 k rows, two to four
  * stages in flight in registers, nothing shared in the loop and no barrier; the eight partial tiles are added through LDS at
  * the end, in a fixed order.  The split along k inside the workgroup is what fills the chip: a gradient of 128 x 128
- * channels has 144 tiles of 64 x 64 (F(4x4, 3x3)), 1152 wavefronts for 1024 SIMDs.
+ * channels has 144 tiles of 64 x 64 (F(4x4, 3x3)), 1152 wavefronts for 1024 SIMDs.  Sixteen wavefronts on a tile of 32 x 32 were slower at every size.
  *
- * Measured (36 products 128 x 128 over k = 512, fp32, operands from L2 / the last-level cache): 12.6 us, of which the
- * matrix cores need 3.9 and the 18.9 MB of operands 3.4; 74 us in the generic kernel that ran before.  fp16, 16 products
- * 227 x 256 over 650: 8.9 us.  What bounds it at these sizes is the chain of one launch: first loads, one or two waves of
- * MFMAs, the sum through LDS; about 8.5 us however small the product.
+ * Measured (36 products 128 x 128 over k = 512, fp32, operands from L2 / the last-level cache): 9.5 us, of which the
+ * 18.9 MB of operands need 3.4 and the matrix cores 1.5; 11.1 with fp32 products, 74 in the generic kernel.  16-bit, tiles of 32 x 32, pairs against single
+ * elements: 16 products 72 x 96 over 15561 43.1 -> 38.7 us, 32 x 32 over 4608 12.2 -> 8.4, 64 x 80 over 750 5.9 -> 4.6.  What bounds it at small
+ * sizes is the chain of one launch: first loads, one or two waves of MFMAs, the sum through LDS.
  */
 #include <type_traits>
 
@@ -41,28 +43,32 @@ namespace
 		float alpha, beta;
 	};
 
-	/* The 16 k rows of one operand that a wavefront holds for one stage: T MFMA tiles of 32 rows.  PAIRS (16-bit types): tile t
-	 * holds the elements 2 * (lane % 32) + t of the 64, otherwise tile t holds 32 t + lane % 32. */
+	/* The 16 k rows of one operand that a wavefront holds for one stage: T MFMA tiles of 32 rows.  PAIRS (16-bit types): a lane loads two neighbouring
+	 * elements at once; tile t of two holds the elements 2 * (lane % 32) + t of the 64, one tile alone the even ones in lanes 0 to 15 and the odd ones
+	 * in 16 to 31.  Otherwise tile t holds 32 t + lane % 32. */
 	template<typename TE, int T, bool PAIRS>
 	struct Operand
 	{
-		static constexpr bool WIDE = sizeof(TE) == 4;
-		static constexpr int WORDS = PAIRS ? 8 : 8 * T;
+		static constexpr bool WIDE = sizeof(TE) == 4, ONE_OF_PAIRS = PAIRS && T == 1;
+		static constexpr int ROWS = ONE_OF_PAIRS ? 4 : 8; /* loads of a lane for one tile or pair of tiles, of one k row each */
+		static constexpr int WORDS = PAIRS ? ROWS : 8 * T;
 		unsigned int v[WORDS];
 		__device__ static __forceinline__ int element(int tile, int r)
 		{
-			return PAIRS ? 2 * r + tile : 32 * tile + r;
+			return ONE_OF_PAIRS ? 2 * (r & 15) + (r >> 4) : PAIRS ? 2 * r + tile : 32 * tile + r;
 		}
-		/* byte offset of this lane's first element in the stage (k row 0 of its half) */
-		__device__ static __forceinline__ unsigned int origin(int first, unsigned int pitch, int lane)
+		/* byte offset of this lane's element in its load j of a stage */
+		__device__ static __forceinline__ unsigned int origin(int first, unsigned int pitch, int lane, int j)
 		{
 			const unsigned int half = lane >> 5;
-			return (WIDE ? half : 8 * half) * pitch + (first + element(0, lane & 31)) * sizeof(TE);
+			if (ONE_OF_PAIRS) /* four k rows a load */
+				return (4 * j + (lane >> 4)) * pitch + (first + 2 * (lane & 15)) * sizeof(TE);
+			return (WIDE ? 2 * j + half : j + 8 * half) * pitch + (first + element(0, lane & 31)) * sizeof(TE);
 		}
-		__device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t rsrc, const unsigned int (&rows)[8])
+		__device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t rsrc, const unsigned int (&rows)[ROWS])
 		{
 #pragma unroll
-			for (int j = 0; j < 8; j++)
+			for (int j = 0; j < ROWS; j++)
 			{
 				if constexpr (WIDE)
 				{
@@ -84,17 +90,50 @@ namespace
 		__device__ __forceinline__ Chunk chunk(int t) const
 		{
 			unsigned int w[4];
-#pragma unroll
-			for (int q = 0; q < 4; q++)
+			if constexpr (ONE_OF_PAIRS)
 			{
-				if constexpr (PAIRS)
-					w[q] = __builtin_amdgcn_perm(v[2 * q + 1], v[2 * q], t ? 0x07060302u : 0x05040100u);
-				else
-					w[q] = (v[(2 * q) * T + t] & 0xFFFFu) | (v[(2 * q + 1) * T + t] << 16);
+				/* sixteen lanes keep the even elements and take those of their neighbours' k rows, which keep the odd ones */
+#pragma unroll
+				for (int q = 0; q < 2; q++)
+				{
+					const auto s = __builtin_amdgcn_permlane16_swap(__builtin_amdgcn_perm(v[2 * q + 1], v[2 * q], 0x05040100u),
+							__builtin_amdgcn_perm(v[2 * q + 1], v[2 * q], 0x07060302u), false, false);
+					w[2 * q] = s[0];
+					w[2 * q + 1] = s[1];
+				}
+			}
+			else
+			{
+#pragma unroll
+				for (int q = 0; q < 4; q++)
+				{
+					if constexpr (PAIRS)
+						w[q] = __builtin_amdgcn_perm(v[2 * q + 1], v[2 * q], t ? 0x07060302u : 0x05040100u);
+					else
+						w[q] = (v[(2 * q) * T + t] & 0xFFFFu) | (v[(2 * q + 1) * T + t] << 16);
+				}
 			}
 			Chunk c;
 			c.u = make_uint4(w[0], w[1], w[2], w[3]);
 			return c;
+		}
+		/* fp32: the eight values of tile t as three bf16 pieces that add up to them exactly (8 + 8 + 8 bits, each the rest of the one before rounded to the nearest) */
+		__device__ __forceinline__ void cut(int t, Chunk (&piece)[3]) const
+		{
+#pragma unroll
+			for (int q = 0; q < 4; q++)
+			{
+				float value[2] = { __builtin_bit_cast(float, v[(2 * q) * T + t]), __builtin_bit_cast(float, v[(2 * q + 1) * T + t]) };
+#pragma unroll
+				for (int p = 0; p < 3; p++)
+				{
+					piece[p].bf[2 * q] = static_cast<__bf16>(value[0]);
+					piece[p].bf[2 * q + 1] = static_cast<__bf16>(value[1]);
+					const unsigned int both = q == 0 ? piece[p].u.x : q == 1 ? piece[p].u.y : q == 2 ? piece[p].u.z : piece[p].u.w;
+					value[0] -= __builtin_bit_cast(float, both << 16);
+					value[1] -= __builtin_bit_cast(float, both & 0xFFFF0000u);
+				}
+			}
 		}
 	};
 
@@ -104,7 +143,7 @@ namespace
 		typedef Operand<TE, T, PAIRS> Op;
 		constexpr int SIDE = 32 * T;
 		constexpr int QUADS = T * T * 4; /* 16-byte runs a lane holds of the tile */
-		constexpr int DEPTH = T == 1 ? 4 : 3; /* stages in flight */
+		constexpr int DEPTH = T == 1 ? 4 : Op::WIDE ? 2 : 3; /* stages in flight */
 		typedef float quad_t __attribute__((ext_vector_type(4)));
 		__shared__ quad_t sums[4][QUADS][64];
 
@@ -118,13 +157,12 @@ namespace
 		const char *a = reinterpret_cast<const char*>(A + batch * g.a_batch);
 		const char *b = reinterpret_cast<const char*>(B + batch * g.b_batch);
 
-		unsigned int rows_a[8], rows_b[8];
+		unsigned int rows_a[Op::ROWS], rows_b[Op::ROWS];
 #pragma unroll
-		for (int j = 0; j < 8; j++)
+		for (int j = 0; j < Op::ROWS; j++)
 		{
-			const unsigned int k = Op::WIDE ? 2 * j : j;
-			rows_a[j] = Op::origin(m0, g.a_pitch, lane) + k * g.a_pitch;
-			rows_b[j] = Op::origin(n0, g.b_pitch, lane) + k * g.b_pitch;
+			rows_a[j] = Op::origin(m0, g.a_pitch, lane, j);
+			rows_b[j] = Op::origin(n0, g.b_pitch, lane, j);
 		}
 		/* the descriptor moves with the stage and shrinks to what is left of the matrix: nothing, behind the last stage */
 		auto remaining = [](const char *base, unsigned int extent, int64_t skip)
@@ -138,16 +176,9 @@ namespace
 			ob[d].fetch(remaining(b, g.b_extent, static_cast<int64_t>(stage) * STAGE * g.b_pitch), rows_b);
 		};
 		f32x16_t acc[T][T];
-#pragma unroll
-		for (int i = 0; i < T; i++)
-#pragma unroll
-			for (int j = 0; j < T; j++)
-#pragma unroll
-				for (int v = 0; v < 16; v++)
-					acc[i][j][v] = 0.0f;
-		auto multiply = [&](const Op &x, const Op &y) __attribute__((always_inline))
+		auto multiply = [&](const Op &x, const Op &y, auto exact) __attribute__((always_inline))
 		{
-			if constexpr (Op::WIDE)
+			if constexpr (Op::WIDE && (T == 1 || exact.value))
 			{
 #pragma unroll
 				for (int p = 0; p < 8; p++)
@@ -157,6 +188,26 @@ namespace
 						for (int j = 0; j < T; j++)
 							acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, x.v[p * T + i]), __builtin_bit_cast(float, y.v[p * T + j]),
 									acc[i][j], 0, 0, 0);
+			}
+			else if constexpr (Op::WIDE)
+			{
+				/* six of the nine products of pieces, the smallest first; what is left out is less than 2^-24 of the whole */
+				constexpr int A_OF[6] = { 2, 0, 1, 1, 0, 0 }, B_OF[6] = { 0, 2, 1, 0, 1, 0 };
+				Chunk ca[T][3];
+#pragma unroll
+				for (int i = 0; i < T; i++)
+					x.cut(i, ca[i]);
+#pragma unroll
+				for (int j = 0; j < T; j++)
+				{
+					Chunk cb[3];
+					y.cut(j, cb);
+#pragma unroll
+					for (int p = 0; p < 6; p++)
+#pragma unroll
+						for (int i = 0; i < T; i++)
+							Mma<bf16_t>::run(ca[i][A_OF[p]], cb[B_OF[p]], acc[i][j]);
+				}
 			}
 			else
 			{
@@ -177,17 +228,41 @@ namespace
 
 		const int stages = (g.K + STAGE - 1) / STAGE;
 		const int mine = (stages - wave + WAVES - 1) / WAVES; /* stages wave, wave + 8, ... */
-#pragma unroll
-		for (int d = 0; d < DEPTH; d++)
-			fetch(d, wave + d * WAVES);
-		for (int s = 0; s < mine; s += DEPTH)
+		auto walk = [&](auto exact) __attribute__((always_inline))
 		{
 #pragma unroll
+			for (int i = 0; i < T; i++)
+#pragma unroll
+				for (int j = 0; j < T; j++)
+#pragma unroll
+					for (int v = 0; v < 16; v++)
+						acc[i][j][v] = 0.0f;
+#pragma unroll
 			for (int d = 0; d < DEPTH; d++)
+				fetch(d, wave + d * WAVES);
+			for (int s = 0; s < mine; s += DEPTH)
 			{
-				multiply(oa[d], ob[d]); /* zeros behind the last stage */
-				fetch(d, wave + (s + DEPTH + d) * WAVES);
+#pragma unroll
+				for (int d = 0; d < DEPTH; d++)
+				{
+					multiply(oa[d], ob[d], exact); /* zeros behind the last stage */
+					fetch(d, wave + (s + DEPTH + d) * WAVES);
+				}
 			}
+		};
+		walk(std::false_type());
+		if constexpr (Op::WIDE && T == 2)
+		{
+			/* An infinity, a NaN or a value that rounds to an infinity in bf16 has no pieces, and their sums are NaN or infinite then: the wavefront
+			 * takes its share of k once more with fp32 products, whatever these give. */
+			bool odd = false;
+#pragma unroll
+			for (int t = 0; t < T * T; t++)
+#pragma unroll
+				for (int v = 0; v < 16; v++)
+					odd |= !(__builtin_fabsf(acc[t / T][t % T][v]) < __builtin_inff());
+			if (__builtin_amdgcn_ballot_w64(odd) != 0)
+				walk(std::true_type());
 		}
 
 		/* eight partial tiles: 4..7 onto 0..3 in registers, then every wavefront adds its share of the four copies */
@@ -277,11 +352,12 @@ namespace avhip
 		g.c_batch = strideC;
 		g.alpha = alpha;
 		g.beta = beta;
-		/* Tiles of 32 x 32 while those of 64 x 64 leave the chip short of work.  fp32 is bound by its sixteen-pass MFMAs, which
-		 * 144 large tiles cannot spread over 256 CUs (12.6 : 16.8 us; equal at 432 tiles, 26 us), 16-bit types by their operand
-		 * loads, which large tiles halve (25.1 : 30.8 us at 48 large tiles, 8.7 : 8.6 at 128, 9.4 : 8.5 at 192, 15.4 : 8.9 at 256). */
+		/* Tiles of 32 x 32 while those of 64 x 64 leave the chip short of work.  16-bit types are bound by their operand loads, which large tiles halve
+		 * (at 64 large tiles 18 to 54 % slower than small ones, at 160 to 256 equal, above faster).  fp32: small tiles have fp32 products, large
+		 * ones bf16 pieces (36 products of 128 x 128 over 512, 144 large tiles: 9.5 : 11.1 us, 128 x 248 over 2080, 288: 24.4 : 28.1; 16 of 104 x 192
+		 * over 7128, 96 large tiles: 66 : 59). */
 		const int64_t large_tiles = static_cast<int64_t>(ceil_div(M, 64)) * ceil_div(N, 64) * batch;
-		const bool small = large_tiles < (SZ == 4 ? 512 : 128);
+		const bool small = large_tiles < 128;
 		const int side = small ? 32 : 64;
 		g.row_tiles = static_cast<int>(ceil_div(M, side));
 		g.col_tiles = static_cast<int>(ceil_div(N, side));
@@ -295,9 +371,12 @@ namespace avhip
 		{
 			/* pairs: every dword of a row aligned and inside it */
 			const bool pairs = M % 2 == 0 && N % 2 == 0 && lda % 2 == 0 && ldb % 2 == 0 && strideA % 2 == 0 && strideB % 2 == 0 && aligned_to(A, 4) && aligned_to(B, 4);
-			if (!small && pairs)
+			if (pairs)
 			{
-				hipLaunchKernelGGL((k_gemm_tn<TE, TC, 2, true>), grid, block, 0, stream, a, b, c, g);
+				if (small)
+					hipLaunchKernelGGL((k_gemm_tn<TE, TC, 1, true>), grid, block, 0, stream, a, b, c, g);
+				else
+					hipLaunchKernelGGL((k_gemm_tn<TE, TC, 2, true>), grid, block, 0, stream, a, b, c, g);
 				return true;
 			}
 		}
