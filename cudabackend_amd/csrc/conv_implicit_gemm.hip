@@ -452,7 +452,7 @@ namespace
 		PixelLoader<TE, FAST> la(x, g, padv, (vec_ok & 1) != 0, p0);
 		FilterLoader<TE, FAST> lb(w, g, (vec_ok & 1) != 0, filter_block * BLOCK_N);
 		typename Mma<TE>::acc_t acc[2][2];
-		block_mma<TE>(lds, g.R * g.S * g.steps_per_tap, la, lb, acc);
+		block_mma<TE, FAST>(lds, g.R * g.S * g.steps_per_tap, la, lb, acc);
 
 		auto row_out = [&](int r, const typename Epi::scalar_t (&v)[4], int) __attribute__((always_inline))
 		{
@@ -484,7 +484,7 @@ namespace
 		PackedPixelLoader<TE, PB> la(x, g, p0);
 		PackedFilterLoader<TE, PB> lb(w, g, filter_block * BLOCK_N);
 		typename Mma<TE>::acc_t acc[2][2];
-		block_mma<TE>(lds, (g.R * g.S * g.C * static_cast<int>(sizeof(TE)) + STEP_BYTES - 1) / STEP_BYTES, la, lb, acc);
+		block_mma<TE, false>(lds, (g.R * g.S * g.C * static_cast<int>(sizeof(TE)) + STEP_BYTES - 1) / STEP_BYTES, la, lb, acc);
 
 		drain_tile<TE, 2, 2>(lds, acc, [&](int r, const typename Epi::scalar_t (&v)[4], int) __attribute__((always_inline))
 		{
@@ -518,7 +518,7 @@ namespace
 		la.seek(first);
 		lb.seek(first);
 		typename Mma<TE>::acc_t acc[2][2];
-		block_mma<TE>(lds, steps, la, lb, acc);
+		block_mma<TE, true>(lds, steps, la, lb, acc);
 
 		float *part = partial + static_cast<int64_t>(blockIdx.z) * g.pixels * g.K;
 		drain_tile<TE, 2, 2>(lds, acc, [&](int r, const float (&v)[4], int) __attribute__((always_inline))
@@ -708,7 +708,9 @@ namespace
 		/* stride-1 filters with more than one tap first try the kernel that keeps an image tile resident in LDS */
 		/* (that kernel has no limit on the number of taps) */
 		const bool fast_tile = fast || (fast_path_ok<TE>(s, flags, padding_value, false) && is_simple_activation(epi.activation) && (flags & 2) != 0);
-		if (fast_tile && s.R * s.S > 1 && conv_tile_launch<TE, Epi>(st, s, x, w, epi))
+		/* (fp32: the gather kernel multiplies twice as fast, but has tiles of 128 filters where that one has 64) */
+		const bool gather = sizeof(TE) == 4 && fast && conv_small_threshold() > 0 && conv_gather_before_image_tiles(s);
+		if (fast_tile && !gather && s.R * s.S > 1 && conv_tile_launch<TE, Epi>(st, s, x, w, epi))
 			return 0;
 		if (fast)
 			hipLaunchKernelGGL((k_conv_igemm<TE, true, Epi>), grid, dim3(256), 0, st, static_cast<const TE*>(x), static_cast<const TE*>(w), g, padv, flags, epi);

@@ -9,6 +9,10 @@
  * Where the channels of a tap are no whole number of chunks the last chunk of a tap is cut off in registers, and 16-bit or 8-bit
  * rows that start between two dwords are loaded as the dwords around them and shifted.
  *
+ * fp32 with 64 x 64: products of bf16 pieces (struct Pieces of mfma_core.hpp), cut by the wavefront that multiplies; with 32 x 32 the cutting takes as long as the
+ * products save.  96 -> 64 5x5 on 21 images of 57 x 53 290 -> 141 us, 352 -> 112 3x3 stride 2 on 76 of 35 x 35 with an ELU 240 -> 154, 128 -> 128 3x3 on 31 of
+ * 19 x 19 41 -> 34.
+ *
  * What bounds it: the 64 bytes per clock that a compute unit loads (128 clocks per stage of a 32 x 32 tile, 256 per stage of a
  * 64 x 64 tile, which needs half as much per product), for fp32 the matrix cores, and for the smallest problems the latency of
  * one launch.  Operands loaded straight in MFMA layout (32 lines per load instruction) took 55 to 60 clocks a kilobyte here, by
@@ -104,6 +108,7 @@ namespace
 		constexpr int SLOTS = QUADS * PITCH > 2 * SIDE * 8 ? QUADS * PITCH : 2 * SIDE * 8;
 		constexpr int DEPTH = T == 1 ? 2 : 1; /* stages in flight */
 		constexpr bool VEC = ACT == ACT_SIMPLE;
+		constexpr bool BY_PIECES = std::is_same<TE, float>::value && T == 2; /* (with 32 x 32 the cutting costs what the products save) */
 		typedef typename Epi::scalar_t scalar_t;
 		typedef Pack<scalar_t, 4> quad_t;
 		/* each wavefront its own part: rows of the stage being multiplied, then its partial tile */
@@ -163,14 +168,6 @@ namespace
 		const unsigned int w_origin = static_cast<unsigned int>(k0 + load_row) * filter_bytes; /* filters past the last lie outside the buffer */
 
 		typename Mma<TE>::acc_t acc[T][T]; /* [filters][pixels] */
-#pragma unroll
-		for (int i = 0; i < T; i++)
-#pragma unroll
-			for (int j = 0; j < T; j++)
-#pragma unroll
-				for (int v = 0; v < 16; v++)
-					acc[i][j][v] = 0;
-
 		/* k = the 16-byte chunks of (tap, channel) in a row, eight a stage; each wavefront takes a contiguous share of the stages */
 		const int chunks = g.R * g.S * g.chunks_per_tap;
 		const int stages = (chunks + 7) / 8;
@@ -178,7 +175,7 @@ namespace
 		const int first = wave * share;
 		const int count = stages - first < share ? stages - first : share; /* may be negative: nothing left for this wavefront */
 		const unsigned int chunks_mine = count > 0 ? (chunks < 8 * (first + count) ? chunks : 8 * (first + count)) : 0;
-		unsigned int chunk = 8 * first + load_chunk;
+		unsigned int chunk;
 		struct Stage
 		{
 			Piece<ROW> xs[LOADS], ws[LOADS];
@@ -211,9 +208,21 @@ namespace
 				to.ws[q].fetch(rw, live ? w_at + 8 * q * filter_bytes : OUT_OF_RANGE);
 		};
 		Stage stage[DEPTH];
+		auto begin = [&]() __attribute__((always_inline))
+		{
 #pragma unroll
-		for (int d = 0; d < DEPTH; d++)
-			fetch(stage[d]);
+			for (int i = 0; i < T; i++)
+#pragma unroll
+				for (int j = 0; j < T; j++)
+#pragma unroll
+					for (int v = 0; v < 16; v++)
+						acc[i][j][v] = 0;
+			chunk = 8 * first + load_chunk;
+#pragma unroll
+			for (int d = 0; d < DEPTH; d++)
+				fetch(stage[d]);
+		};
+		begin();
 
 		/* what the epilogue needs is requested behind the first operands and arrives with them */
 		constexpr int ROWS = 64 * KW / QUADS; /* pixels handed over in one pass of the workgroup */
@@ -239,41 +248,96 @@ namespace
 		 * stage may be written as soon as the reads of this one are issued: no barrier. */
 		const int put = load_row * 8 + (load_chunk ^ (load_row >> 1)); /* rows 8 i + load_row, i even; i odd: column ^ 4 */
 		const int r = lane & 31, half = lane >> 5;
-		for (int s = 0; s < count; s += DEPTH)
+		auto walk = [&](auto exact) __attribute__((always_inline))
 		{
-#pragma unroll
-			for (int d = 0; d < DEPTH; d++)
+			for (int s = 0; s < count; s += DEPTH)
 			{
-				/* both operands, so that what lies behind a row (an infinity of the next pixel or tap) counts as nothing */
-				uint4 keep = make_uint4(0, 0, 0, 0);
-				if (ROW != ROWS_OF_CHUNKS)
-					keep = make_uint4(keep_bits(stage[d].left), keep_bits(stage[d].left - 4), keep_bits(stage[d].left - 8), keep_bits(stage[d].left - 12));
 #pragma unroll
-				for (int q = 0; q < LOADS; q++)
+				for (int d = 0; d < DEPTH; d++)
 				{
-					mine[64 * q + (q & 1 ? put ^ 4 : put)] = stage[d].xs[q].get(origin[q].x + stage[d].x_tap, keep);
-					mine[8 * SIDE + 64 * q + (q & 1 ? put ^ 4 : put)] = stage[d].ws[q].get(stage[d].w_at + 8 * q * filter_bytes, keep);
-				}
-				wave_order();
-				fetch(stage[d]); /* nothing behind the last stage */
+					/* both operands, so that what lies behind a row (an infinity of the next pixel or tap) counts as nothing */
+					uint4 keep = make_uint4(0, 0, 0, 0);
+					if (ROW != ROWS_OF_CHUNKS)
+						keep = make_uint4(keep_bits(stage[d].left), keep_bits(stage[d].left - 4), keep_bits(stage[d].left - 8), keep_bits(stage[d].left - 12));
 #pragma unroll
-				for (int slab = 0; slab < 4; slab++)
-				{
-					Chunk cw[T], cx[T];
-					const int get = r * 8 + ((2 * slab + half) ^ ((r >> 1) & 7));
-#pragma unroll
-					for (int t = 0; t < T; t++)
+					for (int q = 0; q < LOADS; q++)
 					{
-						cx[t].u = mine[256 * t + get];
-						cw[t].u = mine[8 * SIDE + 256 * t + get];
+						mine[64 * q + (q & 1 ? put ^ 4 : put)] = stage[d].xs[q].get(origin[q].x + stage[d].x_tap, keep);
+						mine[8 * SIDE + 64 * q + (q & 1 ? put ^ 4 : put)] = stage[d].ws[q].get(stage[d].w_at + 8 * q * filter_bytes, keep);
 					}
+					wave_order();
+					fetch(stage[d]); /* nothing behind the last stage */
+					auto plain = [&]() __attribute__((always_inline))
+					{
 #pragma unroll
-					for (int i = 0; i < T; i++)
+						for (int slab = 0; slab < 4; slab++)
+						{
+							Chunk cw[T], cx[T];
+							const int get = r * 8 + ((2 * slab + half) ^ ((r >> 1) & 7));
 #pragma unroll
-						for (int j = 0; j < T; j++)
-							Mma<TE>::run(cw[i], cx[j], acc[i][j]);
+							for (int t = 0; t < T; t++)
+							{
+								cx[t].u = mine[256 * t + get];
+								cw[t].u = mine[8 * SIDE + 256 * t + get];
+							}
+#pragma unroll
+							for (int i = 0; i < T; i++)
+#pragma unroll
+								for (int j = 0; j < T; j++)
+									Mma<TE>::run(cw[i], cx[j], acc[i][j]);
+						}
+					};
+					if constexpr (BY_PIECES)
+					{
+						if constexpr (exact.value)
+							plain();
+						else
+						{
+#pragma unroll
+							for (int slab = 0; slab < 4; slab += 2)
+							{
+								Chunk cw[2][T], cx[2][T];
+#pragma unroll
+								for (int i = 0; i < 2; i++)
+#pragma unroll
+									for (int t = 0; t < T; t++)
+									{
+										const int get = r * 8 + ((2 * (slab + i) + half) ^ ((r >> 1) & 7));
+										cx[i][t].u = mine[256 * t + get];
+										cw[i][t].u = mine[8 * SIDE + 256 * t + get];
+									}
+								Pieces pw[T];
+#pragma unroll
+								for (int i = 0; i < T; i++)
+									pw[i].cut(cw[0][i], cw[1][i]);
+#pragma unroll
+								for (int j = 0; j < T; j++)
+								{
+									Pieces px;
+									px.cut(cx[0][j], cx[1][j]);
+#pragma unroll
+									for (int n = 0; n < PIECE_PRODUCTS; n++)
+#pragma unroll
+										for (int i = 0; i < T; i++)
+											Mma<bf16_t>::run(pw[i].p[PIECE_OF_A[n]], px.p[PIECE_OF_B[n]], acc[i][j]);
+								}
+							}
+						}
+					}
+					else
+						plain();
+					wave_order();
 				}
-				wave_order();
+			}
+		};
+		walk(std::false_type());
+		if constexpr (BY_PIECES)
+		{
+			/* sums that are not finite: this wavefront's share of k once more with fp32 products (struct Pieces) */
+			if (__builtin_amdgcn_ballot_w64(!all_finite(acc)) != 0)
+			{
+				begin();
+				walk(std::true_type());
 			}
 		}
 
@@ -344,9 +408,11 @@ namespace
 	 * columns, 16 to 512 channels and filters, 1x1 to 5x5, up to 12 GFLOP; root mean square error 6 to 14 %).  fp32: the root of the sum of
 	 * their squares, fitted to 222 layers timed with every plan (up to 6 GFLOP): the plan chosen is 0.5 % slower than the best of the four
 	 * on average and 15 % at most, with the larger of the two 1.2 % and 36 % (52 -> 408 1x1 on 637 pixels: 7.2 us with four wavefronts, which that chose,
-	 * 5.5 with one). */
+	 * 5.5 with one).  The tiles of 64 x 64, whose products are of bf16 pieces, to 260 layers (6 %), and
+	 * 6 % and 0.6 us more than that: then none of the 43 that get them is slower than with what it got before (1.28 times as fast on average; without
+	 * that 56, four of them slower). */
 	constexpr Pace PACE_16[] = { { 4.99, 0.303, 0.107, 0.20 }, { 3.34, 0.409, 0.084, 0.90 }, { 2.64, 0.173, 0.091, 2.40 }, { 3.41, 0.88, 0.182, 1.86 } };
-	constexpr Pace PACE_32[] = { { 3.80, 0.647, 0.143, 0.37 }, { 3.19, 0.490, 0.149, 1.00 }, { 2.34, 0.162, 0.165, 2.98 }, { 2.56, 1.48, 0.46, 2.79 } };
+	constexpr Pace PACE_32[] = { { 3.80, 0.647, 0.143, 0.37 }, { 3.19, 0.490, 0.149, 1.00 }, { 2.34, 0.162, 0.165, 2.98 }, { 4.34, 1.13, 0.371, 3.14 } };
 
 	/* The kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles: launch, a round of 512 workgroups (two to a compute unit), and
 	 * a k-step of one that has a compute unit to itself or shares it.  The last round, if it is of up to 256, goes at the pace of the former.
@@ -357,9 +423,25 @@ namespace
 	{
 		double launch, round, alone, shared;
 	};
-	enum { IMAGE_TILES, GATHER, GATHER_BY_ELEMENTS, GATHER_ACTIVATION };
+	enum { IMAGE_TILES, GATHER, GATHER_BY_ELEMENTS, GATHER_ACTIVATION, GATHER_GENERAL };
 	constexpr TilePace TILES_16[] = { { 0.0, 4.0, 0.42, 0.68 }, { 1.7, 7.7, 0.70, 0.90 }, { 0.0, 13.5, 0.69, 0.96 }, { 4.4, 15.9, 0.67, 0.88 } };
-	constexpr TilePace TILES_32[] = { { 3.0, 4.1, 1.94, 3.84 }, { 2.0, 8.8, 2.17, 4.20 }, { 0.3, 17.3, 1.96, 4.04 }, { 4.7, 18.0, 2.07, 3.92 } };
+	/* (fp32 in the gather kernel: products of bf16 pieces, 144 layers without a residual, 5 % with rounds of 9.2 us; not in its general instance, which takes an activation and filters in no whole
+	 * vectors at once) */
+	constexpr TilePace TILES_32[] = { { 3.0, 4.1, 1.94, 3.84 }, { 2.5, 11.5, 1.67, 2.50 }, { 0.3, 17.3, 1.67, 2.50 }, { 4.7, 18.0, 1.67, 2.50 }, { 4.7, 18.0, 2.07, 3.92 } };
+
+	double tile_kernel_us(const avhipConvShape &s, int element_bytes, int kernel)
+	{
+		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
+		const double steps = static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 127) / 128);
+		const TilePace &pace = (element_bytes == 4 ? TILES_32 : TILES_16)[kernel];
+		const double workgroups = kernel == IMAGE_TILES ? static_cast<double>(s.N) * ((s.K + 63) / 64) * ((s.Ho * s.Wo + 255) / 256)
+				: std::ceil(pixels / 128.0) * ((s.K + 127) / 128);
+		const double rounds = std::floor(workgroups / 512.0), rest = workgroups - 512.0 * rounds;
+		double us = pace.launch + rounds * (pace.round + pace.shared * steps);
+		if (rest > 0.0)
+			us += pace.round + (rest <= 256.0 ? pace.alone : pace.shared) * steps;
+		return us;
+	}
 
 	/* What the layer takes in them.  `one_tap_us`: the estimate of the persistent one-tap kernels where they take the layer, or 0: what they
 	 * decline (filters in no whole runs of 16 bytes) is the gather kernel's and no less than 9 us (bf16 32 -> 20 on 8360 pixels, with a
@@ -368,19 +450,14 @@ namespace
 	{
 		if (hand_over == HandOver::PLAIN && one_tap_us > 0.0)
 			return one_tap_us;
-		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
-		const double steps = static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 127) / 128);
 		const bool dense = s.stride_h == 1 && s.stride_w == 1 && s.dil_h == 1 && s.dil_w == 1;
 		const bool image_tiles = hand_over == HandOver::PLAIN && dense && s.R * s.S > 1 && s.K % 8 == 0 && s.Ho * s.Wo >= 128;
-		const int kernel = image_tiles ? IMAGE_TILES : hand_over == HandOver::PLAIN ? GATHER : hand_over == HandOver::ELEMENTS ? GATHER_BY_ELEMENTS : GATHER_ACTIVATION;
-		const TilePace &pace = (element_bytes == 4 ? TILES_32 : TILES_16)[kernel];
-		const double workgroups = image_tiles ? static_cast<double>(s.N) * ((s.K + 63) / 64) * ((s.Ho * s.Wo + 255) / 256)
-				: std::ceil(pixels / 128.0) * ((s.K + 127) / 128);
-		const double rounds = std::floor(workgroups / 512.0), rest = workgroups - 512.0 * rounds;
-		double us = pace.launch + rounds * (pace.round + pace.shared * steps);
-		if (rest > 0.0)
-			us += pace.round + (rest <= 256.0 ? pace.alone : pace.shared) * steps;
-		return us;
+		const int kernel = hand_over == HandOver::PLAIN ? GATHER : hand_over == HandOver::ELEMENTS ? GATHER_BY_ELEMENTS : GATHER_ACTIVATION;
+		if (element_bytes == 4 && kernel == GATHER_ACTIVATION && s.K % 4 != 0)
+			return tile_kernel_us(s, element_bytes, GATHER_GENERAL);
+		if (image_tiles && !(element_bytes == 4 && conv_gather_before_image_tiles(s)))
+			return tile_kernel_us(s, element_bytes, IMAGE_TILES);
+		return tile_kernel_us(s, element_bytes, kernel);
 	}
 }
 
@@ -445,6 +522,10 @@ namespace avhip
 		const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
 		return tiles < threshold && small_factor(element_bytes, hand_over, one_tap_us) * conv_small_plan(s, element_bytes).us
 				< workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
+	}
+	bool conv_gather_before_image_tiles(const avhipConvShape &s)
+	{
+		return tile_kernel_us(s, 4, GATHER) < tile_kernel_us(s, 4, IMAGE_TILES);
 	}
 	double conv_without_ring_us(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
 	{

@@ -135,7 +135,7 @@ namespace
 		RowLoader<TE, FAST> la(A + batch * strideA, M, K, lda, m0, (vec_ok & 1) != 0);
 		RowLoader<TE, FAST> lb(B + batch * strideB, N, K, ldb, n0, (vec_ok & 1) != 0);
 		typename Mma<TE>::acc_t acc[2][2];
-		block_mma<TE>(lds, (K + KE - 1) / KE, la, lb, acc);
+		block_mma<TE, FAST>(lds, (K + KE - 1) / KE, la, lb, acc);
 
 		TC *c = C + batch * strideC;
 		const bool vec_c = (vec_ok & 2) != 0;

@@ -14,6 +14,8 @@
  *   steps ahead of the MFMAs (two register sets) and LDS is double buffered, so there is one barrier per step;
  *   LDS rows are padded from 128 to 144 bytes so that the 32 rows a wavefront reads with one ds_read_b128 spread over banks;
  *   two workgroups fit the 160 KB of LDS of a CU.
+ * fp32 (loaders that can be copied): products of bf16 pieces (struct Pieces), cut from LDS by the wavefront that multiplies: 256 workgroups two to a compute
+ * unit 4.2 -> 2.5 us for two k-steps, one alone 2.2 -> 1.7 (its cutting and its products follow each other).
  * MFMA shapes: v_mfma_f32_32x32x16_{f16,bf16}, v_mfma_i32_32x32x32_i8, v_mfma_f32_32x32x2_f32 (four per 16-byte chunk).
  * Lane l of a wavefront supplies row (l % 32) of the operand tile and the k-chunk (l / 32); it receives, for output column
  * (l % 32), the 16 rows 8*i + 4*(l / 32) + j (i, j < 4).
@@ -105,6 +107,49 @@ namespace avhip
 				c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.f[i], b.f[i], c, 0, 0, 0);
 		}
 	};
+
+	/*
+	 * fp32 products on the bf16 matrix cores, sixteen times as fast as the fp32 ones: eight values (two chunks) as three pieces each that add up to them
+	 * exactly (8 + 8 + 8 bits, each the rest of the one before rounded to the nearest), and of the nine products of pieces the six that matter
+	 * in 32 bits; what is left out is less than 2^-24 of the whole.  An infinity, a NaN and a value that rounds to an infinity have no
+	 * such pieces: their sums are NaN or infinite, and the caller takes such a tile once more with Mma<float>.
+	 */
+	struct Pieces
+	{
+		Chunk p[3];
+		__device__ __forceinline__ void cut(const Chunk &lo, const Chunk &hi)
+		{
+#pragma unroll
+			for (int q = 0; q < 4; q++)
+			{
+				float value[2] = { q < 2 ? lo.f[2 * q] : hi.f[2 * q - 4], q < 2 ? lo.f[2 * q + 1] : hi.f[2 * q - 3] };
+#pragma unroll
+				for (int n = 0; n < 3; n++)
+				{
+					p[n].bf[2 * q] = static_cast<__bf16>(value[0]);
+					p[n].bf[2 * q + 1] = static_cast<__bf16>(value[1]);
+					const unsigned int both = q == 0 ? p[n].u.x : q == 1 ? p[n].u.y : q == 2 ? p[n].u.z : p[n].u.w;
+					value[0] -= __builtin_bit_cast(float, both << 16);
+					value[1] -= __builtin_bit_cast(float, both & 0xFFFF0000u);
+				}
+			}
+		}
+	};
+	constexpr int PIECE_PRODUCTS = 6; /* the smallest first */
+	constexpr int PIECE_OF_A[PIECE_PRODUCTS] = { 2, 0, 1, 1, 0, 0 }, PIECE_OF_B[PIECE_PRODUCTS] = { 0, 2, 1, 0, 1, 0 };
+	template<int TM, int TN>
+	__device__ __forceinline__ bool all_finite(const f32x16_t (&acc)[TM][TN])
+	{
+		bool odd = false;
+#pragma unroll
+		for (int i = 0; i < TM; i++)
+#pragma unroll
+			for (int j = 0; j < TN; j++)
+#pragma unroll
+				for (int v = 0; v < 16; v++)
+					odd |= !(__builtin_fabsf(acc[i][j][v]) < __builtin_inff());
+		return !odd;
+	}
 
 	/* Fetches 16 bytes starting at p; only the first `valid` elements exist (valid <= 0: all zero).  `vector_ok` says
 	 * that p is 16-byte aligned whenever the chunk is complete. */
@@ -218,8 +263,8 @@ namespace avhip
 	 * so a global load has the MFMAs of two iterations (2 x 16 x 32 cycles per wavefront) to land before it is needed.
 	 * acc[tm][tn] is the (tm, tn) 32 x 32 tile of this wavefront's 64 x 64 quadrant.
 	 */
-	template<typename TE, typename LoadA, typename LoadB>
-	__device__ __forceinline__ void block_mma(char *lds, int steps, LoadA &load_a, LoadB &load_b, typename Mma<TE>::acc_t (&acc)[2][2])
+	template<typename TE, bool PIECES, typename LoadA, typename LoadB>
+	__device__ __forceinline__ void block_walk(char *lds, int steps, LoadA &load_a, LoadB &load_b, typename Mma<TE>::acc_t (&acc)[2][2])
 	{
 		const int tid = threadIdx.x;
 		const int lane = tid & 63;
@@ -278,6 +323,30 @@ namespace avhip
 					rb_[i].u = *reinterpret_cast<const uint4*>(sb + rd_b + i * 32 * LDS_ROW + slab * 32);
 				}
 			};
+			if constexpr (PIECES)
+			{
+#pragma unroll
+				for (int slab = 0; slab < SLABS; slab += 2)
+				{
+					read(slab, a[0], b[0]);
+					read(slab + 1, a[1], b[1]);
+					Pieces pa[2], pb[2];
+#pragma unroll
+					for (int i = 0; i < 2; i++)
+					{
+						pa[i].cut(a[0][i], a[1][i]);
+						pb[i].cut(b[0][i], b[1][i]);
+					}
+#pragma unroll
+					for (int n = 0; n < PIECE_PRODUCTS; n++)
+#pragma unroll
+						for (int i = 0; i < 2; i++)
+#pragma unroll
+							for (int j = 0; j < 2; j++)
+								Mma<bf16_t>::run(pa[i].p[PIECE_OF_A[n]], pb[j].p[PIECE_OF_B[n]], acc[i][j]);
+				}
+				return;
+			}
 			read(0, a[0], b[0]);
 #pragma unroll
 			for (int slab = 0; slab < SLABS; slab++)
@@ -315,6 +384,22 @@ namespace avhip
 			multiply(1);
 			stash(0, ra[0], rb[0]);
 		}
+	}
+
+	/* PIECES: fp32 by pieces (the loaders are copied for the second time, which those with many registers cannot afford) */
+	template<typename TE, bool PIECES, typename LoadA, typename LoadB>
+	__device__ __forceinline__ void block_mma(char *lds, int steps, LoadA &load_a, LoadB &load_b, typename Mma<TE>::acc_t (&acc)[2][2])
+	{
+		if constexpr (PIECES && std::is_same<TE, float>::value)
+		{
+			LoadA again_a = load_a;
+			LoadB again_b = load_b;
+			block_walk<TE, true>(lds, steps, load_a, load_b, acc);
+			if (__syncthreads_or(!all_finite(acc)) != 0)
+				block_walk<TE, false>(lds, steps, again_a, again_b, acc);
+		}
+		else
+			block_walk<TE, false>(lds, steps, load_a, load_b, acc);
 	}
 
 	/*
