@@ -1094,7 +1094,7 @@ namespace
 	}
 	/* The same transform in one kernel (conv_winograd_f4.hip), weights in its operand layout from the cache (kind 6): for the layers of
 	 * the non-fused plan, so that the sums are those of F(4x4,3x3) where they were before.  A workgroup takes 32 tiles x 64 filters and a
-	 * compute unit for about 14 us (first loads, results) and 4.1 us per 16 channels, so it pays on all but
+	 * compute unit for about 15 us (first loads, results) and 4.1 us per 16 channels, so it pays on all but
 	 * the layers of a few workgroups and many channels: on 19 layers of 130 to 1760 workgroups and 64 to 256 channels, of full and of hardly begun rounds, it
 	 * took 0.49 to 0.64 of the time of the three passes (51 x 33 x 33, 96 -> 64 33 us against 76, 145 x 20 x 20, 160 -> 256 111 against 188).  The other side:
 	 * their matrices written and read at 5 TB/s and the products with filters filled up to 128, which holds within a fifth up to 128 channels
@@ -1109,7 +1109,7 @@ namespace
 				|| (x < y + y_bytes && y < x + x_bytes)) /* written while others still read: only the plan in three passes may work in place */
 			return false;
 		const av_int64 workgroups = (static_cast<av_int64>(plan.tiles) + 31) / 32 * ((s.K + 63) / 64);
-		const double one = static_cast<double>((workgroups + 255) / 256) * (14.0 + 4.1 * ((s.C + 15) / 16));
+		const double one = static_cast<double>((workgroups + 255) / 256) * (15.0 + 4.1 * ((s.C + 15) / 16));
 		const double products = 2.0 * 36.0 * plan.tiles * s.C * ((s.K + 127) / 128 * 128.0);
 		const double three = 5.0 + (2.0 * static_cast<double>(plan.total) + static_cast<double>(x_bytes) + (c.z != nullptr ? 2.0 : 1.0) * static_cast<double>(y_bytes)) / 5.0e6
 				+ products / 2.5e8;

@@ -5,8 +5,9 @@
  * M in memory: for 256 images of 15 x 15 with 128 channels these are 75 MB each, written and read once, and that traffic and not the
  * 4.8 GFLOP of the products was what bounded the plan (16 + 56 + 18 us).
  *
- * The products run on the bf16 matrix cores, which are sixteen times as fast as the fp32 ones: every value is cut into three bf16 pieces that
- * add up to it exactly (8 + 8 + 8 bits of the 24), and of the nine products of pieces the six that matter in 32 bits are taken.
+ * The products run on the bf16 matrix cores, which are sixteen times as fast as the fp32 ones: every value is cut into three bf16 pieces
+ * (struct Pieces of mfma_core.hpp), and of the nine products of pieces the six that matter in 32 bits are taken.  A workgroup that finds sums which
+ * are no numbers takes its tiles once more with fp32 products.
  *
  *   workgroup = 32 tiles (of 4 x 4 output pixels, in the order of the images) x 64 filters, eight wavefronts: four groups of nine
  *               transform points x two halves of the filters; a wavefront keeps its nine 32 x 32 products in 144 registers over the
@@ -19,11 +20,13 @@
  *
  * What bounds it: a stage takes 4.1 us and its parts 1.6 (products, 3456 clocks), 1.4 (500 vector instructions of each of two wavefronts on a SIMD), 1.3
  * (LDS) and 2.2 (63 loads per wavefront) of them, one more in the way of the other than they should be with two wavefronts per SIMD;
- * around the stages 13 us of first loads and results.  All values of a stage must stay in registers: one in scratch makes every load in flight be
+ * around the stages 14 us of first loads, results and (one of them) the look at the sums.  All values of a stage must stay in registers: one in scratch makes every load in flight be
  * waited for (in-order counter), which cost a fifth.  The two passes of the output are a loop, for the same reason: written out they kept 24
  * registers in scratch and the kernel took 8 us longer.
- * Measured, fp32 products and now, one layer again and again: 256 x 15 x 15 x 128 -> 128 61 -> 46 us (three passes through memory 87), 64 channels 36 -> 24 us,
- * a tower of 20 of them in turn behind a first layer 1421 -> 1058 us.  Relative error against 64 bits 1.1e-6 to 2.4e-6, with fp32 products 1.2e-6 to 2.9e-6.
+ * Measured, fp32 products and now, one layer again and again: 256 x 15 x 15 x 128 -> 128 61 -> 47 us (three passes through memory 87), 64 channels 36 -> 25 us,
+ * a tower of 20 of them in turn behind a first layer 1421 -> 1070 us (1050 with pieces cut off and not rounded, and sums not looked at: equal operands of 1 +
+ * 2^-7 - 2^-23 then had an error of 4.7e-7, now below 2^-24, and those below 2^-110 lost their lower pieces).  Relative error against 64 bits 1.1e-6 to
+ * 2.4e-6, with fp32 products 1.2e-6 to 2.9e-6.
  */
 #include <type_traits>
 
@@ -53,6 +56,35 @@ namespace
 		int stages, filter_blocks;
 	};
 
+	/* A weight that has no pieces (an infinity, a NaN, or too large) is kept as this NaN and its own bits, the upper half first: its sums are NaN, and the
+	 * workgroup that finds them takes the value from there. */
+	constexpr unsigned int NO_PIECES = 0x7FC0u;
+	constexpr float MOST_IN_PIECES = 0x1p127f;
+	/* The highest piece of two values, as a pair; what is left of them in their place. */
+	__device__ __forceinline__ unsigned int cut_pair(float (&value)[2])
+	{
+		typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
+		const pair_t piece = { static_cast<__bf16>(value[0]), static_cast<__bf16>(value[1]) };
+		unsigned int both = __builtin_bit_cast(unsigned int, piece);
+		asm("" : "+v"(both)); /* or one of the two is converted a second time, alone */
+		value[0] -= __builtin_bit_cast(float, both << 16);
+		value[1] -= __builtin_bit_cast(float, both & 0xFFFF0000u);
+		return both;
+	}
+	/* weight i of eight in pieces, as it was */
+	__device__ __forceinline__ float joined(const Chunk (&u)[3], int i)
+	{
+		unsigned int bits[3];
+#pragma unroll
+		for (int n = 0; n < 3; n++)
+		{
+			const unsigned int pair = i < 2 ? u[n].u.x : i < 4 ? u[n].u.y : i < 6 ? u[n].u.z : u[n].u.w;
+			bits[n] = i % 2 ? pair & 0xFFFF0000u : pair << 16;
+		}
+		const float sum = __builtin_bit_cast(float, bits[0]) + (__builtin_bit_cast(float, bits[1]) + __builtin_bit_cast(float, bits[2]));
+		return bits[0] == NO_PIECES << 16 ? __builtin_bit_cast(float, bits[1] | bits[2] >> 16) : sum * (1.0f / PIECE_SCALE);
+	}
+
 	/* an offset beyond every tensor the launcher accepts (below 2^29 bytes), with the offset of a pixel added too */
 	constexpr unsigned int NO_PIXEL = 0x80000000u;
 
@@ -66,6 +98,19 @@ namespace
 		d2 = a - b;
 		d3 = e + 0.5f * c;
 		d4 = 0.5f * c - e;
+		d5 = o5;
+	}
+	/* the same times PIECE_SCALE: a power of two, so that the results are those above in every bit, with three instructions more */
+	__device__ __forceinline__ void scaled_input_line(float &d0, float &d1, float &d2, float &d3, float &d4, float &d5)
+	{
+		constexpr float S = PIECE_SCALE;
+		const float a = d2 - 0.25f * d4, b = S * (d1 - 0.25f * d3), c = d4 - d2, e = S * (d3 - d1);
+		const float o0 = S * ((d0 + 0.25f * c) - d2), o5 = (0.25f * S) * (d5 - d3) - e;
+		d0 = o0;
+		d1 = S * a + b;
+		d2 = S * a - b;
+		d3 = e + (0.5f * S) * c;
+		d4 = (0.5f * S) * c - e;
 		d5 = o5;
 	}
 	/* A^T m along one direction: [1 1 1 1/4 1/4 0; 0 1 -1 1/2 -1/2 0; 0 1 1 1 1 0; 0 1 -1 2 -2 2] */
@@ -86,6 +131,7 @@ namespace
 		constexpr int M_BYTES = POINTS * 32 * TILES * 4;
 		static_assert(2 * V_PART <= M_BYTES, "the products of half of the filters take the place of the two parts");
 		__shared__ __attribute__((aligned(16))) char lds[M_BYTES];
+		__shared__ __attribute__((aligned(16))) int odd_waves[8];
 
 		const int tid = threadIdx.x, lane = tid & 63;
 		const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -135,30 +181,21 @@ namespace
 		};
 		auto transform_row = [&](int a) __attribute__((always_inline))
 		{
-			input_line(d[6 * a], d[6 * a + 1], d[6 * a + 2], d[6 * a + 3], d[6 * a + 4], d[6 * a + 5]);
+			scaled_input_line(d[6 * a], d[6 * a + 1], d[6 * a + 2], d[6 * a + 3], d[6 * a + 4], d[6 * a + 5]);
 		};
-		/* Two values of V, in pieces: the sixteen highest bits of a float are a bf16, and these are stored of v, of v less that, and of the rest.
-		 * (med3: no rest of an infinity, and not NaN.)  Eight lanes beside the eight that have the first eight channels have the others of the
+		/* Two values of V, in pieces.  Eight lanes beside the eight that have the first eight channels have the others of the
 		 * same tile: they exchange values, so that each has both channels of a pair for one of the points, and write dwords: stores of single
 		 * pieces took the LDS longer than the products take the matrix cores. */
 		auto store_pieces = [&](int part, int buffer, int e) __attribute__((always_inline))
 		{
 			constexpr int ROW_ROTATE_8 = 0x128;
 			const int e0 = __builtin_bit_cast(int, d[12 * part + e]), e1 = __builtin_bit_cast(int, d[12 * part + e + 1]);
-			unsigned int value[2] = { static_cast<unsigned int>(__builtin_amdgcn_update_dpp(e0, e1, ROW_ROTATE_8, 15, 12, false)),
-					static_cast<unsigned int>(__builtin_amdgcn_update_dpp(e1, e0, ROW_ROTATE_8, 15, 3, false)) };
+			float value[2] = { __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(e0, e1, ROW_ROTATE_8, 15, 12, false)),
+					__builtin_bit_cast(float, __builtin_amdgcn_update_dpp(e1, e0, ROW_ROTATE_8, 15, 3, false)) };
 			unsigned int *to = reinterpret_cast<unsigned int*>(lds + buffer * V_PART + put + e * V_POINT);
 #pragma unroll
 			for (int piece = 0; piece < 3; piece++)
-			{
-				to[piece * V_PIECE / 4] = __builtin_amdgcn_perm(value[1], value[0], 0x07060302u);
-#pragma unroll
-				for (int i = 0; i < 2; i++)
-				{
-					const float rest = __builtin_bit_cast(float, value[i]) - __builtin_bit_cast(float, value[i] & 0xFFFF0000u);
-					value[i] = __builtin_bit_cast(unsigned int, piece == 0 ? __builtin_amdgcn_fmed3f(rest, rest, 0.0f) : rest);
-				}
-			}
+				to[piece * V_PIECE / 4] = cut_pair(value);
 		};
 		/* A part is two rows of V: made in 18 pieces of work, one in front of each product of the part before; then their places in the
 		 * registers are loaded with pixels of the next stage.  (Columns are transformed for the first part, as late as its work allows: its last
@@ -210,14 +247,18 @@ namespace
 				u[q][piece].u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ru, lane * 16, at + 1024 * piece, 0));
 		};
 		Mma<float>::acc_t acc[MY_POINTS]; /* [filters][tiles] */
+		auto clear = [&]() __attribute__((always_inline))
+		{
 #pragma unroll
-		for (int p = 0; p < MY_POINTS; p++)
+			for (int p = 0; p < MY_POINTS; p++)
 #pragma unroll
-			for (int v = 0; v < 16; v++)
-				acc[p][v] = 0;
+				for (int v = 0; v < 16; v++)
+					acc[p][v] = 0;
+		};
+		clear();
 		const int r = lane & 31, half = lane >> 5;
 		const int get = my_points * V_POINT + half * V_HALF + r * 16;
-		/* One part: its products, v w of the pieces h + m + l with the smallest products first (what is left out, m l and below, is less than 2^-22 of
+		/* One part: its products, v w of the pieces h + m + l with the smallest products first (what is left out, m l and below, is less than 2^-24 of
 		 * the whole), and between them the work on the next part. */
 		auto step = [&](int stage, int part, int buffer) __attribute__((always_inline))
 		{
@@ -264,6 +305,58 @@ namespace
 			step(s, 0, odd);
 			step(s, 1, odd ^ 1);
 			step(s, 2, odd);
+		}
+
+		/* Sums that are no numbers, or so large that the output transform (which adds up to 361 of them) may leave the range of a float: an infinity, a NaN
+		 * or a value that has no pieces is among the operands, or products reach 2^87.  The workgroup takes its tiles once more with fp32 products; so it
+		 * does where alpha1 is so small that it cannot take the scale of the pieces back. */
+		float size[4] = {}; /* finite if all sums are below 2^119 (comparisons hand their results to the scalar unit one by one, which took 0.6 us longer) */
+#pragma unroll
+		for (int p = 0; p < MY_POINTS; p++)
+#pragma unroll
+			for (int v = 0; v < 16; v++)
+				size[v % 4] += 0x1p9f * __builtin_fabsf(acc[p][v]);
+		const bool odd_wave = __builtin_amdgcn_ballot_w64(!((size[0] + size[1]) + (size[2] + size[3]) < __builtin_inff())) != 0
+				|| (epi.alpha1 != 0.0f && __builtin_fabsf(epi.alpha1) < 0x1p-90f);
+		if (lane == 0)
+			odd_waves[wave] = odd_wave ? 1 : 0;
+		__syncthreads();
+		const int4 first_odd = *reinterpret_cast<const int4*>(odd_waves), last_odd = *reinterpret_cast<const int4*>(odd_waves + 4);
+		const bool once_more = __builtin_amdgcn_readfirstlane(first_odd.x | first_odd.y | first_odd.z | first_odd.w | last_odd.x | last_odd.y | last_odd.z | last_odd.w) != 0;
+		epi.alpha1 *= once_more ? 1.0f : 1.0f / (PIECE_SCALE * PIECE_SCALE);
+		if (once_more)
+		{
+			clear();
+			/* [point][channel, in the order of the weights][tile] */
+			float *v_exact = reinterpret_cast<float*>(lds);
+			const int place = 2 * (channel & 7) + (channel >> 3);
+#pragma unroll 1
+			for (int s = 0; s <= last; s++)
+			{
+#pragma unroll
+				for (int a = 0; a < 6; a++)
+					load_row(s, a);
+#pragma unroll
+				for (int b = 0; b < 6; b++)
+					transform_column(b);
+#pragma unroll
+				for (int a = 0; a < 6; a++)
+					input_line(d[6 * a], d[6 * a + 1], d[6 * a + 2], d[6 * a + 3], d[6 * a + 4], d[6 * a + 5]);
+				__syncthreads();
+#pragma unroll
+				for (int p = 0; p < POINTS; p++)
+					v_exact[(p * CHANNELS + place) * TILES + tile] = d[p];
+				__syncthreads();
+#pragma unroll
+				for (int p = 0; p < MY_POINTS; p++)
+				{
+					const int point = PART_POINTS * (p / MY_PART) + my_points + p % MY_PART;
+					load_weights(s, p / MY_PART, p % MY_PART);
+#pragma unroll
+					for (int i = 0; i < 8; i++)
+						acc[p] = __builtin_amdgcn_mfma_f32_32x32x2f32(joined(u[p % MY_PART], i), v_exact[(point * CHANNELS + 8 * half + i) * TILES + r], acc[p], 0, 0, 0);
+				}
+			}
 		}
 
 		/* two filters of a tile per work-item: its place among 16 neighbours is the pair, so that runs of 128 bytes leave */
@@ -391,16 +484,14 @@ namespace
 			for (int j = 0; j < 6; j++)
 			{
 				unsigned short *piece = to + static_cast<int64_t>(6 * i + j) * slabs * 1536;
-				float rest = u[j];
+				float rest[2] = { u[j] * PIECE_SCALE, 0.0f };
+				const unsigned int bits = __builtin_bit_cast(unsigned int, u[j]);
+				const bool whole = fabsf(rest[0]) >= MOST_IN_PIECES || !(fabsf(u[j]) < INFINITY);
 #pragma unroll
 				for (int n = 0; n < 3; n++)
 				{
-					unsigned int bits = __builtin_bit_cast(unsigned int, rest);
-					rest = fabsf(rest) < INFINITY ? rest - __builtin_bit_cast(float, bits & 0xFFFF0000u) : 0.0f;
-					/* no piece is zero where u is not (and large against what takes the zero's place): the product with an infinity stays one */
-					if (bits << 1 == 0 && fabsf(u[j]) > 0x1p-80f)
-						bits = (__builtin_bit_cast(unsigned int, u[j]) & 0x80000000u) | 0x00800000u;
-					piece[512 * n] = static_cast<unsigned short>(bits >> 16);
+					const unsigned int cut = cut_pair(rest);
+					piece[512 * n] = static_cast<unsigned short>(!whole ? cut : n == 0 ? NO_PIECES : n == 1 ? bits >> 16 : bits);
 				}
 			}
 		}

@@ -13,8 +13,8 @@ extern "C"
 	 * number of channels, K a multiple of four, y and z aligned to 16 bytes, x below 512 MiB, U below 768 MiB and y below 2 GiB, beta = 0, LINEAR or RELU,
 	 * y apart from x; AVHIP_NOT_SUPPORTED for other layers, with nothing launched.  Stands where the reference calls its non-fused
 	 * kernels one after another, src/winograd_nonfused.cu:609-877.  U is what avhip_winograd_f4_weight_transform wrote (taps reversed when
-	 * `invert`): avhip_winograd_f4_weight_bytes(K, C) bytes, [K / 32][36][C / 16][3 pieces][64 lanes][8] bf16, the pieces adding up to the value, K and
-	 * C filled up to multiples of 64 and 16 with zeros. */
+	 * `invert`): avhip_winograd_f4_weight_bytes(K, C) bytes, [K / 32][36][C / 16][3 pieces][64 lanes][8] bf16, the pieces adding up to 2^16 times the
+	 * value or, where it is no number or too large, a NaN and the value's own bits; K and C filled up to multiples of 64 and 16 with zeros. */
 	AVHIP_API int avhip_conv2d_winograd_f4(void *stream, const avhipConvShape *shape, const void *x, const void *U, const void *bias, const void *z, void *y,
 			double alpha1, double alpha2, double beta, int activation);
 	AVHIP_API int avhip_winograd_f4_weight_transform(void *stream, int invert, const void *w, void *U, int K, int C);

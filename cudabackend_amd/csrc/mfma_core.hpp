@@ -113,6 +113,8 @@ namespace avhip
 	 * exactly (8 + 8 + 8 bits, each the rest of the one before rounded to the nearest), and of the nine products of pieces the six that matter
 	 * in 32 bits; what is left out is less than 2^-24 of the whole.  An infinity, a NaN and a value that rounds to an infinity have no
 	 * such pieces: their sums are NaN or infinite, and the caller takes such a tile once more with Mma<float>.
+	 * The lowest bits of a float are 2^-149 and those of a bf16 2^-133: times PIECE_SCALE every float below 2^111 has its three pieces, without it those
+	 * from 2^-110 on.
 	 */
 	struct Pieces
 	{
@@ -135,6 +137,7 @@ namespace avhip
 			}
 		}
 	};
+	constexpr float PIECE_SCALE = 0x1p16f;
 	constexpr int PIECE_PRODUCTS = 6; /* the smallest first */
 	constexpr int PIECE_OF_A[PIECE_PRODUCTS] = { 2, 0, 1, 1, 0, 0 }, PIECE_OF_B[PIECE_PRODUCTS] = { 0, 2, 1, 0, 1, 0 };
 	template<int TM, int TN>
