@@ -262,8 +262,14 @@ namespace
 #pragma unroll
 					for (int q = 0; q < LOADS; q++)
 					{
-						mine[64 * q + (q & 1 ? put ^ 4 : put)] = stage[d].xs[q].get(origin[q].x + stage[d].x_tap, keep);
-						mine[8 * SIDE + 64 * q + (q & 1 ? put ^ 4 : put)] = stage[d].ws[q].get(stage[d].w_at + 8 * q * filter_bytes, keep);
+						uint4 xs = stage[d].xs[q].get(origin[q].x + stage[d].x_tap, keep), ws = stage[d].ws[q].get(stage[d].w_at + 8 * q * filter_bytes, keep);
+						if constexpr (BY_PIECES && !exact.value)
+						{
+							xs = scaled(xs);
+							ws = scaled(ws);
+						}
+						mine[64 * q + (q & 1 ? put ^ 4 : put)] = xs;
+						mine[8 * SIDE + 64 * q + (q & 1 ? put ^ 4 : put)] = ws;
 					}
 					wave_order();
 					fetch(stage[d]); /* nothing behind the last stage */
@@ -334,7 +340,7 @@ namespace
 		if constexpr (BY_PIECES)
 		{
 			/* sums that are not finite: this wavefront's share of k once more with fp32 products (struct Pieces) */
-			if (__builtin_amdgcn_ballot_w64(!all_finite(acc)) != 0)
+			if (__builtin_amdgcn_ballot_w64(!finish_pieces(acc)) != 0)
 			{
 				begin();
 				walk(std::true_type());
@@ -624,4 +630,17 @@ namespace avhip
 	AVHIP_INSTANTIATE(int8_t, Int8Epilogue<I8_FLOAT_I8>)
 	AVHIP_INSTANTIATE(int8_t, Int8Epilogue<I8_FLOAT_F32>)
 #undef AVHIP_INSTANTIATE
+}
+
+/* The tile that a layer of more than one tap (of fp32, or one that the ring kernel leaves alone) gets in this kernel: MFMA tiles of 32 x 32 a side times 16
+ * plus wavefronts, or 0 where it goes to another.  `hand_over`: HandOver.  Exported so that a test can ask which instance it is about to run. */
+extern "C" AVHIP_API int avhip_conv2d_small_plan(int x_dtype, const avhipConvShape *shape, int hand_over)
+{
+	if (shape == nullptr || hand_over < 0 || hand_over > 2)
+		return 0;
+	const int element_bytes = x_dtype == DT_INT8 ? 1 : x_dtype == DT_FLOAT32 ? 4 : 2;
+	if (!conv_small_preferred(*shape, element_bytes, static_cast<HandOver>(hand_over), 0.0))
+		return 0;
+	const SmallPlan plan = conv_small_plan(*shape, element_bytes);
+	return 16 * plan.tiles + plan.waves;
 }

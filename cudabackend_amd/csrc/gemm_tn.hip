@@ -5,7 +5,7 @@
  *
  * No transpose is made.  For fp32 the operand layout of v_mfma_f32_32x32x2_f32 (lane l: row l % 32, k l / 32) is exactly a
  * coalesced load of two rows of A, and the eight k that a lane has of a stage are an operand of a bf16 product too: with tiles of 64 x 64 the
- * values are cut into three bf16 pieces that add up to them exactly, in registers, and six of the nine products of pieces are taken.  (The cutting costs
+ * values are cut into three bf16 pieces in registers (struct Pieces of mfma_core.hpp), and six of the nine products of pieces are taken.  (The cutting costs
  * as much as the products save with 32 x 32: 12.6 against 11.1 us below.)  For 16-bit types a lane loads one dword (two neighbouring m) of four or eight
  * k rows and separates them with v_perm_b32 into the operand chunks of two MFMA tiles, one of the even and one of the odd m, or exchanges one
  * of the two with the sixteen lanes beside it; what cannot be read in pairs (odd sizes) is loaded element by element.  k rows and m, n
@@ -117,23 +117,12 @@ namespace
 			c.u = make_uint4(w[0], w[1], w[2], w[3]);
 			return c;
 		}
-		/* fp32: the eight values of tile t as three bf16 pieces that add up to them exactly (8 + 8 + 8 bits, each the rest of the one before rounded to the nearest) */
-		__device__ __forceinline__ void cut(int t, Chunk (&piece)[3]) const
+		/* fp32: the eight values of tile t */
+		__device__ __forceinline__ void cut(int t, Pieces &pieces) const
 		{
 #pragma unroll
 			for (int q = 0; q < 4; q++)
-			{
-				float value[2] = { __builtin_bit_cast(float, v[(2 * q) * T + t]), __builtin_bit_cast(float, v[(2 * q + 1) * T + t]) };
-#pragma unroll
-				for (int p = 0; p < 3; p++)
-				{
-					piece[p].bf[2 * q] = static_cast<__bf16>(value[0]);
-					piece[p].bf[2 * q + 1] = static_cast<__bf16>(value[1]);
-					const unsigned int both = q == 0 ? piece[p].u.x : q == 1 ? piece[p].u.y : q == 2 ? piece[p].u.z : piece[p].u.w;
-					value[0] -= __builtin_bit_cast(float, both << 16);
-					value[1] -= __builtin_bit_cast(float, both & 0xFFFF0000u);
-				}
-			}
+				pieces.cut(q, PIECE_SCALE * __builtin_bit_cast(float, v[(2 * q) * T + t]), PIECE_SCALE * __builtin_bit_cast(float, v[(2 * q + 1) * T + t]));
 		}
 	};
 
@@ -191,22 +180,20 @@ namespace
 			}
 			else if constexpr (Op::WIDE)
 			{
-				/* six of the nine products of pieces, the smallest first; what is left out is less than 2^-24 of the whole */
-				constexpr int A_OF[6] = { 2, 0, 1, 1, 0, 0 }, B_OF[6] = { 0, 2, 1, 0, 1, 0 };
-				Chunk ca[T][3];
+				Pieces ca[T];
 #pragma unroll
 				for (int i = 0; i < T; i++)
 					x.cut(i, ca[i]);
 #pragma unroll
 				for (int j = 0; j < T; j++)
 				{
-					Chunk cb[3];
+					Pieces cb;
 					y.cut(j, cb);
 #pragma unroll
-					for (int p = 0; p < 6; p++)
+					for (int p = 0; p < PIECE_PRODUCTS; p++)
 #pragma unroll
 						for (int i = 0; i < T; i++)
-							Mma<bf16_t>::run(ca[i][A_OF[p]], cb[B_OF[p]], acc[i][j]);
+							Mma<bf16_t>::run(ca[i].p[PIECE_OF_A[p]], cb.p[PIECE_OF_B[p]], acc[i][j]);
 				}
 			}
 			else
@@ -253,15 +240,8 @@ namespace
 		walk(std::false_type());
 		if constexpr (Op::WIDE && T == 2)
 		{
-			/* An infinity, a NaN or a value that rounds to an infinity in bf16 has no pieces, and their sums are NaN or infinite then: the wavefront
-			 * takes its share of k once more with fp32 products, whatever these give. */
-			bool odd = false;
-#pragma unroll
-			for (int t = 0; t < T * T; t++)
-#pragma unroll
-				for (int v = 0; v < 16; v++)
-					odd |= !(__builtin_fabsf(acc[t / T][t % T][v]) < __builtin_inff());
-			if (__builtin_amdgcn_ballot_w64(odd) != 0)
+			/* sums that are no numbers: this wavefront's share of k once more with fp32 products, whatever these give (struct Pieces) */
+			if (__builtin_amdgcn_ballot_w64(!finish_pieces(acc)) != 0)
 				walk(std::true_type());
 		}
 

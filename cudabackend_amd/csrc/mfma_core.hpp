@@ -113,45 +113,62 @@ namespace avhip
 	 * exactly (8 + 8 + 8 bits, each the rest of the one before rounded to the nearest), and of the nine products of pieces the six that matter
 	 * in 32 bits; what is left out is less than 2^-24 of the whole.  An infinity, a NaN and a value that rounds to an infinity have no
 	 * such pieces: their sums are NaN or infinite, and the caller takes such a tile once more with Mma<float>.
-	 * The lowest bits of a float are 2^-149 and those of a bf16 2^-133: times PIECE_SCALE every float below 2^111 has its three pieces, without it those
-	 * from 2^-110 on.
+	 * The lowest bits of a float are 2^-149 and those of a bf16 2^-133: times PIECE_SCALE every float below 2^111 has its three pieces, without it only those
+	 * from 2^-110 on (at 2^-118 an error of 9e-6, at 2^-138 of 1).  The scale and its way back cost the kernels that cut 3 to 4 %.
 	 */
+	constexpr float PIECE_SCALE = 0x1p16f;
+	__device__ __forceinline__ uint4 scaled(const uint4 &chunk)
+	{
+		Chunk c;
+		c.u = chunk;
+#pragma unroll
+		for (int e = 0; e < 4; e++)
+			c.f[e] *= PIECE_SCALE;
+		return c.u;
+	}
 	struct Pieces
 	{
 		Chunk p[3];
-		__device__ __forceinline__ void cut(const Chunk &lo, const Chunk &hi)
+		/* elements 2 q and 2 q + 1 of the eight, scaled */
+		__device__ __forceinline__ void cut(int q, float first, float second)
 		{
+			float value[2] = { first, second };
 #pragma unroll
-			for (int q = 0; q < 4; q++)
+			for (int n = 0; n < 3; n++)
 			{
-				float value[2] = { q < 2 ? lo.f[2 * q] : hi.f[2 * q - 4], q < 2 ? lo.f[2 * q + 1] : hi.f[2 * q - 3] };
-#pragma unroll
-				for (int n = 0; n < 3; n++)
-				{
-					p[n].bf[2 * q] = static_cast<__bf16>(value[0]);
-					p[n].bf[2 * q + 1] = static_cast<__bf16>(value[1]);
-					const unsigned int both = q == 0 ? p[n].u.x : q == 1 ? p[n].u.y : q == 2 ? p[n].u.z : p[n].u.w;
-					value[0] -= __builtin_bit_cast(float, both << 16);
-					value[1] -= __builtin_bit_cast(float, both & 0xFFFF0000u);
-				}
+				p[n].bf[2 * q] = static_cast<__bf16>(value[0]);
+				p[n].bf[2 * q + 1] = static_cast<__bf16>(value[1]);
+				const unsigned int both = q == 0 ? p[n].u.x : q == 1 ? p[n].u.y : q == 2 ? p[n].u.z : p[n].u.w;
+				value[0] -= __builtin_bit_cast(float, both << 16);
+				value[1] -= __builtin_bit_cast(float, both & 0xFFFF0000u);
 			}
 		}
+		__device__ __forceinline__ void cut(const Chunk &lo, const Chunk &hi)
+		{
+			cut(0, lo.f[0], lo.f[1]);
+			cut(1, lo.f[2], lo.f[3]);
+			cut(2, hi.f[0], hi.f[1]);
+			cut(3, hi.f[2], hi.f[3]);
+		}
 	};
-	constexpr float PIECE_SCALE = 0x1p16f;
 	constexpr int PIECE_PRODUCTS = 6; /* the smallest first */
 	constexpr int PIECE_OF_A[PIECE_PRODUCTS] = { 2, 0, 1, 1, 0, 0 }, PIECE_OF_B[PIECE_PRODUCTS] = { 0, 2, 1, 0, 1, 0 };
+	/* Takes the scale of both operands out of the sums.  False where one of them is no number (or above 2^96, which the scale makes infinite). */
 	template<int TM, int TN>
-	__device__ __forceinline__ bool all_finite(const f32x16_t (&acc)[TM][TN])
+	__device__ __forceinline__ bool finish_pieces(f32x16_t (&acc)[TM][TN])
 	{
-		bool odd = false;
+		float size[4] = {}; /* (comparisons would hand their results to the scalar unit one by one) */
 #pragma unroll
 		for (int i = 0; i < TM; i++)
 #pragma unroll
 			for (int j = 0; j < TN; j++)
 #pragma unroll
 				for (int v = 0; v < 16; v++)
-					odd |= !(__builtin_fabsf(acc[i][j][v]) < __builtin_inff());
-		return !odd;
+				{
+					size[v % 4] += 1.0f / (16 * TM * TN) * __builtin_fabsf(acc[i][j][v]);
+					acc[i][j][v] *= 1.0f / (PIECE_SCALE * PIECE_SCALE);
+				}
+		return (size[0] + size[1]) + (size[2] + size[3]) < __builtin_inff();
 	}
 
 	/* Fetches 16 bytes starting at p; only the first `valid` elements exist (valid <= 0: all zero).  `vector_ok` says
@@ -307,8 +324,8 @@ namespace avhip
 #pragma unroll
 			for (int q = 0; q < FETCH_PASSES; q++)
 			{
-				*reinterpret_cast<uint4*>(sa + st_off + q * FETCH_ROWS * LDS_ROW) = a[q];
-				*reinterpret_cast<uint4*>(sb + st_off + q * FETCH_ROWS * LDS_ROW) = b[q];
+				*reinterpret_cast<uint4*>(sa + st_off + q * FETCH_ROWS * LDS_ROW) = PIECES ? scaled(a[q]) : a[q];
+				*reinterpret_cast<uint4*>(sb + st_off + q * FETCH_ROWS * LDS_ROW) = PIECES ? scaled(b[q]) : b[q];
 			}
 		};
 		auto multiply = [&](int buffer)
@@ -398,7 +415,7 @@ namespace avhip
 			LoadA again_a = load_a;
 			LoadB again_b = load_b;
 			block_walk<TE, true>(lds, steps, load_a, load_b, acc);
-			if (__syncthreads_or(!all_finite(acc)) != 0)
+			if (__syncthreads_or(!finish_pieces(acc)) != 0)
 				block_walk<TE, false>(lds, steps, again_a, again_b, acc);
 		}
 		else
