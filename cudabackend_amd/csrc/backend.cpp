@@ -977,8 +977,9 @@ namespace
 		return from_launcher(rc);
 	}
 
-	/* Whether the implicit-GEMM kernel with a ring of LDS buffers (conv_ring.hip) is estimated to need less than `us` for a 16-bit layer.  A kernel
-	 * with one workgroup per compute unit and fixed tiles pays a whole round for the first workgroup beyond the last full one. */
+	/* Whether the implicit-GEMM kernel with a ring of LDS buffers (conv_ring.hip) takes a 16-bit layer of whole vectors with LINEAR or RELU, and is estimated
+	 * to need less than `us`.  A kernel with one workgroup per compute unit and fixed tiles pays a whole round for the first workgroup beyond the
+	 * last full one. */
 	bool ring_is_faster(const ConvCall &c, double us)
 	{
 		const avhipConvShape &s = c.problem.shape;
@@ -986,7 +987,11 @@ namespace
 		const int64_t x_bytes = 2ll * s.N * s.H * s.W * s.C, y_bytes = 2ll * s.N * s.Ho * s.Wo * s.K;
 		if (x < y + y_bytes && y < x + x_bytes) /* it takes no calls in place */
 			return false;
-		return avhip::ring_choice(s, 2, 2, 0, c.z != nullptr).us < us;
+		/* and reads both operands as they lie */
+		if (reinterpret_cast<uintptr_t>(c.x->data) % 16 != 0 || reinterpret_cast<uintptr_t>(c.w->data) % 16 != 0)
+			return false;
+		const double ring = avhip_conv2d_ring_us(c.problem.x_dtype, c.problem.y_dtype, &s, 0, c.z != nullptr ? 1 : 0);
+		return ring > 0.0 && ring < us;
 	}
 
 	/* 3x3 stride-2 layers of 16-bit tensors through the parity-plane kernel (conv_strided.hip), weights in its operand layout from

@@ -319,20 +319,68 @@ namespace
 	}
 }
 
+namespace
+{
+	struct RingPlan
+	{
+		int pixels, filters, per_cu; /* of a tile; workgroups that share a compute unit */
+		/* microseconds: of a launch, of a stage per workgroup on the compute unit, of a workgroup's beginning and end, more for results element by
+		 * element and for those with a call per activation, and per megabyte of results and residuals */
+		double launch, stage, tile, elements, activation, megabyte;
+	};
+	/* Fitted to 410 layers of 16-bit and 8-bit types (36 to 500000 pixels, 16 to 1024 channels and filters, 1x1 to 5x5, strides 1 and 2), each timed with
+	 * every plan; root mean square error 9 to 12 %.  The four are needed: the best plan is each of them on a fifth of the layers at least, without
+	 * the second the mean gain falls from 12 to 11 %, without the first from 12 to 10. */
+	constexpr RingPlan RING_PLANS[] = { { 256, 128, 1, 0.0, 0.63, 5.5, 7.4, 10.0, 0.07 }, { 128, 128, 1, 1.1, 0.38, 3.5, 3.8, 4.6, 0.045 },
+			{ 128, 64, 2, 2.1, 0.265, 2.0, 1.8, 2.8, 0.04 }, { 64, 64, 3, 2.5, 0.165, 1.7, 1.7, 2.6, 0.0 } };
+
+	struct RingChoice
+	{
+		int plan;
+		double us;
+	};
+	/* `hand_over`: 0 whole vectors, 1 element by element, 2 any activation (HandOver of conv_small.hpp) */
+	RingChoice ring_choice(const avhipConvShape &s, int element_bytes, int out_bytes, int hand_over, bool residual)
+	{
+		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
+		const double stages = std::ceil(static_cast<double>(s.R) * s.S * (s.C * element_bytes / 16) / 8.0);
+		const double megabytes = pixels * s.K * out_bytes * (residual ? 2.0e-6 : 1.0e-6);
+		RingChoice best = { -1, 0.0 };
+		for (int i = 0; i < 4; i++)
+		{
+			const RingPlan &p = RING_PLANS[i];
+			const double tile = p.tile + (hand_over == 1 ? p.elements : hand_over == 2 ? p.activation : 0.0);
+			const double loads = std::ceil(pixels / p.pixels) * ((s.K + p.filters - 1) / p.filters) / 256.0; /* of workgroups, one per compute unit each */
+			const double rounds = std::floor(loads / p.per_cu), rest = std::ceil(loads - rounds * p.per_cu);
+			const double us = p.launch + (rounds + (rest > 0.0 ? 1.0 : 0.0)) * tile + (rounds * p.per_cu + rest) * p.stage * stages + p.megabyte * megabytes;
+			if (best.plan < 0 || us < best.us)
+				best = { i, us };
+		}
+		return best;
+	}
+
+	/* The tile that the layer gets and its estimate, or no plan where it is left to the other kernels */
+	RingChoice ring_route(const avhipConvShape &s, int element_bytes, int out_bytes, HandOver hand_over, double one_tap_us, bool residual)
+	{
+		const RingChoice none = { -1, 0.0 };
+		/* (the switch of the small tiles is this kernel's too: at 0 the kernels with fixed tiles of 128 x 128 are asked for, below it small ones) */
+		if (element_bytes > 2 || static_cast<int64_t>(s.C) * element_bytes % 16 != 0 || !conv_small_possible(s, element_bytes) || conv_small_threshold() <= 0)
+			return none;
+		/* of 8-bit one-tap layers the persistent kernels are a fifth to a third faster than they are estimated (17 layers) */
+		if (element_bytes == 1 && one_tap_us > 0.0)
+			return none;
+		/* 15 % below the others' estimates, which are the coarser ones: of the 410 layers one is then slower than before (bf16, a filter count that is no
+		 * multiple of four), and the mean gain is 11.7 of the 13.9 % that the best choice for each would have */
+		const RingChoice choice = ring_choice(s, element_bytes, out_bytes, static_cast<int>(hand_over), residual);
+		return choice.us < 0.85 * conv_without_ring_us(s, element_bytes, hand_over, one_tap_us) ? choice : none;
+	}
+}
+
 namespace avhip
 {
 	double conv_ring_us(const avhipConvShape &s, int element_bytes, int out_bytes, HandOver hand_over, double one_tap_us, bool residual)
 	{
-		/* (the switch of the small tiles is this kernel's too: at 0 the kernels with fixed tiles of 128 x 128 are asked for, below it small ones) */
-		if (element_bytes > 2 || static_cast<int64_t>(s.C) * element_bytes % 16 != 0 || !conv_small_possible(s, element_bytes) || conv_small_threshold() <= 0)
-			return 0.0;
-		/* of 8-bit one-tap layers the persistent kernels are a fifth to a third faster than they are estimated (17 layers) */
-		if (element_bytes == 1 && one_tap_us > 0.0)
-			return 0.0;
-		/* 15 % below the others' estimates, which are the coarser ones: of the 410 layers one is then slower than before (bf16, a filter count that is no
-		 * multiple of four), and the mean gain is 11.7 of the 13.9 % that the best choice for each would have */
-		const double us = ring_choice(s, element_bytes, out_bytes, static_cast<int>(hand_over), residual).us;
-		return us < 0.85 * conv_without_ring_us(s, element_bytes, hand_over, one_tap_us) ? us : 0.0;
+		return ring_route(s, element_bytes, out_bytes, hand_over, one_tap_us, residual).us;
 	}
 
 	template<typename TE, typename Epi>
@@ -343,10 +391,9 @@ namespace avhip
 		const bool simple = epi.vec && is_simple_activation(epi.activation);
 		const HandOver hand_over = simple ? HandOver::PLAIN : is_simple_activation(epi.activation) ? HandOver::ELEMENTS : HandOver::ACTIVATION;
 		const bool residual = epi.z != nullptr;
-		if (conv_ring_us(s, SZ, Epi::out_bytes, hand_over, simple ? conv_pointwise_us<TE>(s, epi) : 0.0, residual) == 0.0
-				|| in_place(s, x, SZ, epi.y, Epi::out_bytes))
+		const int plan = ring_route(s, SZ, Epi::out_bytes, hand_over, simple ? conv_pointwise_us<TE>(s, epi) : 0.0, residual).plan;
+		if (plan < 0 || in_place(s, x, SZ, epi.y, Epi::out_bytes))
 			return false;
-		const int plan = ring_choice(s, SZ, Epi::out_bytes, static_cast<int>(hand_over), residual).plan;
 		const int px = RING_PLANS[plan].pixels, ft = RING_PLANS[plan].filters;
 		const int64_t pixel_tiles = (pixels + px - 1) / px, filter_tiles = (static_cast<int64_t>(s.K) + ft - 1) / ft;
 		if (pixel_tiles * 512 >= (1ll << 32) /* work-items of a launch along one direction */ || filter_tiles > 65535 || pixel_tiles * filter_tiles > 0x7FFFFFFFll || pixels >= (1ll << 31) - 256)
@@ -417,6 +464,14 @@ namespace avhip
 #undef AVHIP_INSTANTIATE
 }
 
+extern "C" double avhip_conv2d_ring_us(int x_dtype, int y_dtype, const avhipConvShape *shape, int hand_over, int residual)
+{
+	if (shape == nullptr || hand_over < 0 || hand_over > 2 || (x_dtype != DT_FLOAT16 && x_dtype != DT_BFLOAT16 && x_dtype != DT_INT8))
+		return 0.0;
+	const int element_bytes = x_dtype == DT_INT8 ? 1 : 2, out_bytes = y_dtype == DT_INT8 ? 1 : x_dtype == DT_INT8 ? 4 : 2;
+	return conv_ring_us(*shape, element_bytes, out_bytes, static_cast<HandOver>(hand_over), 0.0, residual != 0);
+}
+
 /* The tile that a layer with whole vectors of results and LINEAR or RELU gets: 0 to 3, or -1 where the layer goes to another of the implicit-GEMM
  * kernels.  Exported so that a test can ask which tile it is about to run. */
 extern "C" AVHIP_API int avhip_conv2d_ring_plan(int x_dtype, int y_dtype, const avhipConvShape *shape)
@@ -424,7 +479,5 @@ extern "C" AVHIP_API int avhip_conv2d_ring_plan(int x_dtype, int y_dtype, const 
 	if (shape == nullptr || (x_dtype != DT_FLOAT16 && x_dtype != DT_BFLOAT16 && x_dtype != DT_INT8))
 		return -1;
 	const int element_bytes = x_dtype == DT_INT8 ? 1 : 2, out_bytes = y_dtype == DT_INT8 ? 1 : x_dtype == DT_INT8 ? 4 : 2;
-	if (conv_ring_us(*shape, element_bytes, out_bytes, HandOver::PLAIN, 0.0, false) == 0.0)
-		return -1;
-	return ring_choice(*shape, element_bytes, out_bytes, 0, false).plan;
+	return ring_route(*shape, element_bytes, out_bytes, HandOver::PLAIN, 0.0, false).plan;
 }

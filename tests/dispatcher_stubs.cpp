@@ -16,6 +16,8 @@ namespace
 {
 	std::map<std::string, int> calls;
 	bool malloc_fails = false, capturing = false;
+	int strided_workgroups = 0;
+	double ring_us = 0.0;
 	int called(const char *name, int result = 0)
 	{
 		calls[name]++;
@@ -30,6 +32,12 @@ extern "C"
 		malloc_fails = malloc_fails_now != 0;
 		capturing = capturing_now != 0;
 		calls.clear();
+	}
+	/* the parity-plane kernel's workgroups (0: it takes nothing) and what the ring kernel answers for every layer (0: it takes nothing) */
+	AVHIP_API void stub_set_strided(int workgroups, double ring_us_now)
+	{
+		strided_workgroups = workgroups;
+		ring_us = ring_us_now;
 	}
 	AVHIP_API int stub_calls(const char *name)
 	{
@@ -96,7 +104,19 @@ extern "C"
 		return called("implicit_gemm");
 	}
 	int avhip_conv2d_winograd_rows_plan(int, const avhipConvShape*, int*, int*) { return AVHIP_NOT_SUPPORTED; }
-	int avhip_conv2d_strided_plan(int, const avhipConvShape*, int*, int*) { return AVHIP_NOT_SUPPORTED; }
+	int avhip_conv2d_strided_plan(int, const avhipConvShape*, int *workgroups, int *rows_used)
+	{
+		*workgroups = strided_workgroups;
+		*rows_used = 224;
+		return strided_workgroups > 0 ? 0 : AVHIP_NOT_SUPPORTED;
+	}
+	int64_t avhip_conv2d_strided_weight_bytes(int K, int C) { return 18ll * K * C; }
+	int avhip_conv2d_strided_weight_layout(void*, int, int, const void*, void*, int, int) { return called("strided_weights"); }
+	int avhip_conv2d_strided(void*, int, const avhipConvShape*, const void*, const void*, const void*, const void*, void*, double, double, double, int)
+	{
+		return called("strided");
+	}
+	double avhip_conv2d_ring_us(int, int, const avhipConvShape*, int, int) { return ring_us; }
 	int avhip_conv2d_pointwise_block_plan(int, const avhipConvShape*, int*, int*) { return AVHIP_NOT_SUPPORTED; }
 }
 
@@ -110,9 +130,6 @@ STUB_UNUSED(avhip_conv2d_implicit_gemm_split_k)
 STUB_UNUSED(avhip_conv2d_pointwise_block)
 STUB_UNUSED(avhip_conv2d_pointwise_block_weight_bytes)
 STUB_UNUSED(avhip_conv2d_pointwise_block_weight_layout)
-STUB_UNUSED(avhip_conv2d_strided)
-STUB_UNUSED(avhip_conv2d_strided_weight_bytes)
-STUB_UNUSED(avhip_conv2d_strided_weight_layout)
 STUB_UNUSED(avhip_conv2d_winograd_fused)
 STUB_UNUSED(avhip_conv2d_winograd_rows)
 STUB_UNUSED(avhip_im2row)

@@ -27,6 +27,7 @@ def lib(tmp_path_factory):
         fn = getattr(dll, name)
         fn.restype, fn.argtypes = res, args
     dll.stub_calls.argtypes = [C.c_char_p]
+    dll.stub_set_strided.argtypes = [C.c_int, C.c_double]
     return dll
 
 
@@ -98,3 +99,46 @@ def test_capture_uses_what_is_cached(layer):
     assert layer.forward(capturing=True) == ("SUCCESS", THREE_PASSES)
     layer.forward()
     assert layer.forward(capturing=True) == ("SUCCESS", F4)
+
+
+class StridedLayer(Layer):
+    """bf16 3x3 stride 2, 192 -> 512 on 24 images of 34 x 34: 256 workgroups of the parity-plane kernel, some 29 us by its estimate."""
+
+    def __init__(self, lib):
+        self.lib = lib
+        lib.stub_set(0, 0)
+        self.context = self.made(lib.cudaCreateContextDescriptor, 0)
+        self.conv = self.made(lib.cudaCreateConvolutionDescriptor)
+        cb.check(lib.cudaSetConvolutionDescriptor(self.conv, cb.CONVOLUTION_MODE, 2, (C.c_int * 2)(-1, -1), (C.c_int * 2)(2, 2), None, 1, None))
+        self.x, self.w, self.y = (self.tensor(*shape) for shape in ((24, 34, 34, 192), (512, 3, 3, 192), (24, 17, 17, 512)))
+        self.space = 0
+
+    def tensor(self, *shape, offset=0):
+        desc, size = self.made(self.lib.cudaCreateTensorDescriptor), 2
+        cb.check(self.lib.cudaSetTensorDescriptor(desc, cb.DTYPE_BFLOAT16, 4, (C.c_int * 4)(*shape)))
+        for n in shape:
+            size *= n
+        whole = self.made(self.lib.cudaCreateMemoryDescriptor, 0, size + offset)
+        return desc, self.made(self.lib.cudaCreateMemoryView, whole, size, offset) if offset else whole
+
+    def route(self, ring_us, **tensors):
+        self.lib.stub_set_strided(256, ring_us)
+        for name, t in tensors.items():
+            setattr(self, name, t)
+        status, _ = self.forward()
+        self.lib.stub_set_strided(0, 0.0)
+        assert status == "SUCCESS"
+        return [n for n in ("strided", "implicit_gemm") if self.lib.stub_calls(n.encode())]
+
+
+def test_stride_2_layers_go_to_the_ring_kernel_where_that_takes_them(lib):
+    """The parity-plane kernel has a layout of its own of the weights, from any address; the ring kernel reads them as they lie, and a layer that
+    it declines ends in a kernel that is slower than both."""
+    layer = StridedLayer(lib)
+    assert layer.route(15.0) == ["implicit_gemm"]
+    assert layer.route(40.0) == ["strided"], "slower"
+    assert layer.route(0.0) == ["strided"], "declined: switched off, or not far enough below the other kernels"
+    assert layer.route(15.0, w=layer.tensor(512, 3, 3, 192, offset=8)) == ["strided"], "weights that are not aligned to 16 bytes"
+    layer = StridedLayer(lib)
+    images = layer.tensor(24, 34, 34, 192)
+    assert layer.route(15.0, x=images, y=(layer.y[0], images[1])) == ["strided"], "in place"
