@@ -654,13 +654,11 @@ namespace
 		const dim3 grid(ceil_div(g.pixels, BLOCK_M), ceil_div(s.K, BLOCK_N));
 		/* the branch-free instances also store whole 4-filter vectors (streaming stores): K % 4 == 0 and y, z aligned (bit 1) */
 		const bool fast = fast_path_ok<TE>(s, flags, padding_value) && is_simple_activation(epi.activation) && (flags & 2) != 0;
-		/* few input channels: pack (tap, channel) into the k-steps instead of spending a step per tap.  Below 64 bytes per pixel:
-		 * at 64 (half a k-step per tap) the kernels below are the faster ones, measured on 3x3 layers of 64 int8 / 32 bf16 / 16 fp32
-		 * channels (12 against 28 us, 21 against 52 us, 82 against 113 us); at 48 and 32 bytes these are (16 against 22 us, 13 against 22 us) */
+		/* few input channels: pack (tap, channel) into the k-steps instead of spending a step per tap */
 		const int pixel_bytes = s.C * static_cast<int>(sizeof(TE));
 		/* channels that are no whole number of 16-byte chunks: of the kernels below the few-channel ones and that of small tiles take them */
 		const bool ragged = pixel_bytes % 16 != 0 && aligned_to(x, 16) && aligned_to(w, 16) && fast_path_ok<TE>(s, 1, padding_value);
-		if (pixel_bytes < STEP_BYTES / 2 && s.R * s.S > 1 && fast_path_ok<TE>(s, 1, padding_value, false) && is_simple_activation(epi.activation)
+		if (conv_few_channels(s, static_cast<int>(sizeof(TE))) && fast_path_ok<TE>(s, 1, padding_value, false) && is_simple_activation(epi.activation)
 				&& (flags & 2) != 0)
 		{
 			/* a pixel of exactly 8 bytes and a small filter: operands straight into registers, no k loop */

@@ -363,6 +363,9 @@ namespace
 	RingChoice ring_route(const avhipConvShape &s, int element_bytes, int out_bytes, HandOver hand_over, double one_tap_us, bool residual)
 	{
 		const RingChoice none = { -1, 0.0 };
+		/* layers that the few-channel kernels have taken before this one is asked */
+		if (hand_over == HandOver::PLAIN && conv_few_channels(s, element_bytes))
+			return none;
 		/* (the switch of the small tiles is this kernel's too: at 0 the kernels with fixed tiles of 128 x 128 are asked for, below it small ones) */
 		if (element_bytes > 2 || static_cast<int64_t>(s.C) * element_bytes % 16 != 0 || !conv_small_possible(s, element_bytes) || conv_small_threshold() <= 0)
 			return none;
@@ -464,20 +467,47 @@ namespace avhip
 #undef AVHIP_INSTANTIATE
 }
 
-extern "C" double avhip_conv2d_ring_us(int x_dtype, int y_dtype, const avhipConvShape *shape, int hand_over, int residual)
+namespace
 {
-	if (shape == nullptr || hand_over < 0 || hand_over > 2 || (x_dtype != DT_FLOAT16 && x_dtype != DT_BFLOAT16 && x_dtype != DT_INT8))
-		return 0.0;
-	const int element_bytes = x_dtype == DT_INT8 ? 1 : 2, out_bytes = y_dtype == DT_INT8 ? 1 : x_dtype == DT_INT8 ? 4 : 2;
-	return conv_ring_us(*shape, element_bytes, out_bytes, static_cast<HandOver>(hand_over), 0.0, residual != 0);
+	/* as the launcher asks for a call with this epilogue, tensors at address 16 */
+	template<typename TE, typename Epi>
+	RingChoice route_of_call(const avhipConvShape &s, int hand_over, int residual)
+	{
+		Epi epi { };
+		epi.vec = hand_over == 0;
+		if (residual != 0)
+			epi.z = reinterpret_cast<decltype(epi.z)>(16);
+		return ring_route(s, static_cast<int>(sizeof(TE)), Epi::out_bytes, static_cast<HandOver>(hand_over), hand_over == 0 ? conv_pointwise_us<TE>(s, epi) : 0.0,
+				residual != 0);
+	}
+	RingChoice route_of_call(int x_dtype, int y_dtype, const avhipConvShape *shape, int hand_over, int residual)
+	{
+		if (shape == nullptr || hand_over < 0 || hand_over > 2)
+			return { -1, 0.0 };
+		switch (x_dtype)
+		{
+			case DT_FLOAT16:
+				return route_of_call<f16_t, FloatEpilogue<f16_t>>(*shape, hand_over, residual);
+			case DT_BFLOAT16:
+				return route_of_call<bf16_t, FloatEpilogue<bf16_t>>(*shape, hand_over, residual);
+			case DT_INT8:
+				if (y_dtype == DT_INT8)
+					return route_of_call<int8_t, Int8Epilogue<I8_REQUANT>>(*shape, hand_over, residual);
+				if (y_dtype == DT_INT32)
+					return route_of_call<int8_t, Int8Epilogue<I8_EXACT>>(*shape, hand_over, residual);
+				return route_of_call<int8_t, Int8Epilogue<I8_FLOAT_F32>>(*shape, hand_over, residual);
+			default:
+				return { -1, 0.0 };
+		}
+	}
 }
 
-/* The tile that a layer with whole vectors of results and LINEAR or RELU gets: 0 to 3, or -1 where the layer goes to another of the implicit-GEMM
- * kernels.  Exported so that a test can ask which tile it is about to run. */
-extern "C" AVHIP_API int avhip_conv2d_ring_plan(int x_dtype, int y_dtype, const avhipConvShape *shape)
+extern "C" double avhip_conv2d_ring_us(int x_dtype, int y_dtype, const avhipConvShape *shape, int hand_over, int residual)
 {
-	if (shape == nullptr || (x_dtype != DT_FLOAT16 && x_dtype != DT_BFLOAT16 && x_dtype != DT_INT8))
-		return -1;
-	const int element_bytes = x_dtype == DT_INT8 ? 1 : 2, out_bytes = y_dtype == DT_INT8 ? 1 : x_dtype == DT_INT8 ? 4 : 2;
-	return ring_route(*shape, element_bytes, out_bytes, HandOver::PLAIN, 0.0, false).plan;
+	return route_of_call(x_dtype, y_dtype, shape, hand_over, residual).us;
+}
+
+extern "C" int avhip_conv2d_ring_plan(int x_dtype, int y_dtype, const avhipConvShape *shape, int hand_over, int residual)
+{
+	return route_of_call(x_dtype, y_dtype, shape, hand_over, residual).plan;
 }

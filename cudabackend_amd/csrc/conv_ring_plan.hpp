@@ -12,6 +12,8 @@ extern "C"
 	 * aligned x and w below 2 GiB, a zero padding value and y apart from x.  `hand_over`: 0 LINEAR or RELU in whole aligned vectors of four
 	 * filters, 1 those element by element, 2 any other activation; `residual`: whether there is a z. */
 	AVHIP_API double avhip_conv2d_ring_us(int x_dtype, int y_dtype, const avhipConvShape *shape, int hand_over, int residual);
+	/* The tile that such a call gets, pixels x filters: 0 256 x 128, 1 128 x 128, 2 128 x 64, 3 64 x 64, or -1 where it goes to another kernel. */
+	AVHIP_API int avhip_conv2d_ring_plan(int x_dtype, int y_dtype, const avhipConvShape *shape, int hand_over, int residual);
 }
 
 #endif /* AVHIP_CONV_RING_PLAN_HPP_ */

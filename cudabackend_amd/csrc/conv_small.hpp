@@ -46,6 +46,15 @@ namespace avhip
 		return in < out + y_bytes && out < in + x_bytes;
 	}
 
+	/* Layers of few input channels, below 64 bytes per pixel, whose (tap, channel) pairs are worth packing into the k-steps instead of spending a step
+	 * per tap, given whole aligned vectors of results and LINEAR or RELU.  At 64 (half a k-step per tap) the other kernels are the faster ones, measured on
+	 * 3x3 layers of 64 int8 / 32 bf16 / 16 fp32 channels (12 against 28 us, 21 against 52 us, 82 against 113 us); at 48 and 32 bytes those
+	 * that pack are (16 against 22 us, 13 against 22 us). */
+	inline bool conv_few_channels(const avhipConvShape &s, int element_bytes)
+	{
+		return static_cast<int64_t>(s.C) * element_bytes < 64 && s.R * s.S > 1;
+	}
+
 	/* tiles x tiles MFMA tiles of 32 x 32, `waves` wavefronts sharing the k range, and the estimated microseconds */
 	struct SmallPlan
 	{
