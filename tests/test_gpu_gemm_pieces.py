@@ -37,4 +37,4 @@ def test_short_fp32_values_without_pieces():
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
     assert np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
     rows = np.abs(want).max(axis=2, keepdims=True, where=finite, initial=1.0)
-    assert (np.abs(got - want)[finite] <= (2e-5 * np.broadcast_to(rows, want.shape))[finite]).all()
+    assert (np.abs(got[finite] - want[finite]) <= 2e-5 * np.broadcast_to(rows, want.shape)[finite]).all()
