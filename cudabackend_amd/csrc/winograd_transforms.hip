@@ -481,7 +481,7 @@ namespace
 		static constexpr int wider = sizeof(T) > sizeof(TM) ? sizeof(T) : sizeof(TM);
 		static constexpr int wide = 4 * sizeof(float) / wider;
 		static constexpr int cap = (M + R - 1 >= 6) ? AVHIP_WINOGRAD_WIDTH_T6 : AVHIP_WINOGRAD_WIDTH_T4;
-		static constexpr int value = wide > cap ? cap : wide;
+		static constexpr int value = wide > cap ? cap : wide, half = value > 1 ? value / 2 : 1;
 	};
 	/* The width to launch with: VecOf's when every access of a [.., C] tensor stays aligned to it, else 1. */
 	template<int M, int R, typename T, typename TM>
@@ -503,10 +503,13 @@ namespace
 	}
 
 	/* Channels per work-item of the input and gradient transforms: `widest` (what pick_vec allows), or half of it, dwords at least, where that leaves
-	 * fewer than two wavefronts per SIMD, each of which would do its loads, its arithmetic and its stores one after the other (fp32 F(2x2, 3x3)
-	 * gradient of 41 images of 12 x 12, 240 -> 32, all four launches: 32.7 -> 31.1 us; of 61 x 21 x 24, 96 -> 140: 65.3 -> 61.9). */
+	 * fewer than two wavefronts per SIMD, each of which would do its loads, its arithmetic and its stores one after the other.  All four launches of a weight
+	 * gradient, against the widest: fp32 F(2x2, 3x3) of 41 images of 12 x 12, 240 -> 32 33.0 -> 31.4 us, F(4x4, 3x3) of 25 x 19 x 19, 248 -> 192
+	 * 49.0 -> 45.5; on 39 of them 3.7 % (fp32 F(4x4, 3x3)), 1.8 (fp32 F(2x2, 3x3)), 2.3 (fp16) and 0.8 (bf16) on average; forward stages 1 % either
+	 * way.  One transform again and again by itself gains 5 to 9 % up to a third of the line and loses as much above it (fp32 F(4x4, 3x3) of 36 x
+	 * 18 x 18 x 232 7.7 -> 8.7), but a line there loses 0.4 to 1.1 % of the gradients. */
 	constexpr size_t TWO_WAVES_PER_SIMD = 2 * 4 * 256 * 64;
-	template<int M, int R, typename T, typename TM>
+	template<typename T>
 	int run_of_items(int widest, size_t elements)
 	{
 		return widest > 1 && sizeof(T) * widest > 4 && elements / widest < TWO_WAVES_PER_SIMD ? widest / 2 : widest;
@@ -543,7 +546,7 @@ namespace
 		if constexpr (buffer_run<T, 1>)
 			if (narrow && buffered)
 			{
-				const int width = run_of_items<M, R, T, TM>(V, static_cast<size_t>(N) * Th * Tw * C);
+				const int width = run_of_items<T>(V, static_cast<size_t>(N) * Th * Tw * C);
 				const size_t items = static_cast<size_t>(N) * Th * Tw * (C / width);
 				const unsigned int group = group_size(items);
 #define AVHIP_LAUNCH_INPUT_BUFFER(WIDTH) hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, uint32_t, true>), dim3(ceil_div(items, group)), dim3(group), 0, s, \
@@ -553,7 +556,7 @@ namespace
 				else if (width == VecOf<M, R, T, TM>::value)
 					AVHIP_LAUNCH_INPUT_BUFFER((VecOf<M, R, T, TM>::value));
 				else
-					AVHIP_LAUNCH_INPUT_BUFFER(2);
+					AVHIP_LAUNCH_INPUT_BUFFER((VecOf<M, R, T, TM>::half));
 #undef AVHIP_LAUNCH_INPUT_BUFFER
 				return 0;
 			}
@@ -631,7 +634,7 @@ namespace
 		if constexpr (buffer_run<T, 1>)
 			if (narrow && buffered)
 			{
-				const int width = run_of_items<M, R, T, TM>(V, static_cast<size_t>(N) * Th * Tw * K);
+				const int width = run_of_items<T>(V, static_cast<size_t>(N) * Th * Tw * K);
 				const size_t items = static_cast<size_t>(N) * Th * Tw * (K / width);
 				const unsigned int group = group_size(items);
 				if (width == 1)
@@ -639,7 +642,7 @@ namespace
 				else if (width == WIDTH)
 					AVHIP_LAUNCH_GRADIENT(WIDTH, uint32_t, true);
 				else
-					AVHIP_LAUNCH_GRADIENT(2, uint32_t, true);
+					AVHIP_LAUNCH_GRADIENT((VecOf<M, R, T, TM>::half), uint32_t, true);
 				return 0;
 			}
 		const size_t items = static_cast<size_t>(N) * Th * Tw * ((K + V - 1) / V);

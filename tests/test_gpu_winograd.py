@@ -42,6 +42,15 @@ def test_input_transform(oracle, dtype, m, r, shape):
     assert oracle.rel_l2(got, want) < TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype,m", [("f16", 2), ("bf16", 2), ("f32", 2), ("f32", 4)])
+def test_input_transform_of_whole_runs(oracle, dtype, m):
+    """131072 work-items and more of the widest runs of channels (fewer are given half of them), the last row and column of tiles cut off."""
+    g = h.rng(11)
+    x = h.rounded(oracle, g.standard_normal((40 * m // 2, 29, 31, 64)), dtype)
+    got = h.winograd_input_transform(x, (21, 3, 3, 64), dtype, m, (-1, -1))
+    assert oracle.rel_l2(got, oracle.winograd_input_transform(x, m, 3, (-1, -1))) < TOL[dtype]
+
+
 def test_input_transform_padding_value_and_offsets(oracle):
     g = h.rng(3)
     x = h.rounded(oracle, g.standard_normal((2, 9, 7, 12)), "f32")
