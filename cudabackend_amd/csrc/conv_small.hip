@@ -232,7 +232,7 @@ namespace
 		typename Epi::Columns columns;
 		epi.load_columns(kcol, columns);
 		typename Epi::template Residual<4> residual[PASSES];
-		if (VEC)
+		auto request_residual = [&]() __attribute__((always_inline))
 		{
 #pragma unroll
 			for (int pass = 0; pass < PASSES; pass++)
@@ -241,7 +241,9 @@ namespace
 				if (row < SIDE && p0 + row < g.pixels && kcol < g.K)
 					epi.template load_residual<4>(static_cast<int64_t>(p0 + row) * g.K + kcol, residual[pass]);
 			}
-		}
+		};
+		if (VEC && !BY_PIECES) /* (where the pieces take the registers: behind the products, or it waits in scratch memory) */
+			request_residual();
 
 		/* LDS rows of 128 bytes, filters behind pixels; chunk c of row r lies in column c ^ (r / 2) % 8: conflict-free to write by rows
 		 * and to read by columns.  A wavefront's LDS accesses are done in their order and nobody else touches its part, so the next
@@ -345,6 +347,8 @@ namespace
 				begin();
 				walk(std::true_type());
 			}
+			if (VEC)
+				request_residual();
 		}
 
 		/* a lane holds, of pixel r of each pixel tile, the filters 8 v + 4 (lane / 32) .. + 3 of each filter tile */
