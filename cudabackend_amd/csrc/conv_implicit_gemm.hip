@@ -900,12 +900,14 @@ namespace
 		 * split, 16.8 in small tiles) and an fp32 layer's sums would be of another kind (that layer's error against 64 bits: 2.1e-7 split, 3.1e-7 in
 		 * small tiles, 3.1e-6 through F(4x4, 3x3)). */
 		/* (at eight k-steps and more the one-tap kernels take nothing) */
-		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), HandOver::PLAIN, 0.0) && split_us(s, plan, static_cast<int>(sizeof(TE))) > 0.95 * conv_small_plan(s, static_cast<int>(sizeof(TE))).us
+		SmallPlan small;
+		const double split = split_us(s, plan, static_cast<int>(sizeof(TE)));
+		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), HandOver::PLAIN, 0.0, small) && split > 0.95 * small.us
 				&& !in_place(s, x, sizeof(TE), y, sizeof(TE)))
 			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
 		/* Nor is it where the ring kernel is: bf16 480 -> 128 5x5 stride 2 on 155 images of 9 x 9, 34.5 us in nine parts. */
 		const double ring = is_simple_activation(activation) ? conv_ring_us(s, static_cast<int>(sizeof(TE)), static_cast<int>(sizeof(TE)), HandOver::PLAIN, 0.0, z != nullptr) : 0.0;
-		if (ring > 0.0 && ring < 0.9 * split_us(s, plan, static_cast<int>(sizeof(TE))) && !in_place(s, x, sizeof(TE), y, sizeof(TE)))
+		if (ring > 0.0 && ring < 0.9 * split && !in_place(s, x, sizeof(TE), y, sizeof(TE)))
 			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
 		const ConvGeom g = make_geom<TE>(s);
 		const dim3 grid(ceil_div(g.pixels, BLOCK_M), ceil_div(s.K, BLOCK_N), static_cast<unsigned int>(plan.splits));

@@ -520,18 +520,18 @@ namespace avhip
 	{
 		return hand_over != HandOver::PLAIN ? (element_bytes == 4 ? 1.1 : 1.2) : one_tap_us > 0.0 ? 1.05 : 1.0;
 	}
-	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
+	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us, SmallPlan &plan)
 	{
 		if (!conv_small_possible(s, element_bytes))
 			return false;
+		plan = conv_small_plan(s, element_bytes);
 		const int threshold = conv_small_threshold();
 		if (threshold < 0) /* asked for by name (tests): whatever the kernel can run */
 			return true;
 		if (!whole_chunks(s, element_bytes)) /* otherwise the general gather kernel, element by element: 2.2 to 17 times slower on all of 14 layers of 1152 to 627200 pixels */
 			return threshold != 0;
 		const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
-		return tiles < threshold && small_factor(element_bytes, hand_over, one_tap_us) * conv_small_plan(s, element_bytes).us
-				< workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
+		return tiles < threshold && small_factor(element_bytes, hand_over, one_tap_us) * plan.us < workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
 	}
 	bool conv_gather_before_image_tiles(const avhipConvShape &s)
 	{
@@ -539,7 +539,8 @@ namespace avhip
 	}
 	double conv_without_ring_us(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
 	{
-		return conv_small_preferred(s, element_bytes, hand_over, one_tap_us) ? small_factor(element_bytes, hand_over, 0.0) * conv_small_plan(s, element_bytes).us
+		SmallPlan plan;
+		return conv_small_preferred(s, element_bytes, hand_over, one_tap_us, plan) ? small_factor(element_bytes, hand_over, 0.0) * plan.us
 				: workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
 	}
 
@@ -551,9 +552,9 @@ namespace avhip
 		/* whole 4-filter vectors and LINEAR / RELU, or anything (the integer epilogues know no other activation) */
 		const bool simple = epi.vec && is_simple_activation(epi.activation);
 		const HandOver hand_over = simple ? HandOver::PLAIN : is_simple_activation(epi.activation) ? HandOver::ELEMENTS : HandOver::ACTIVATION;
-		if (!conv_small_preferred(s, SZ, hand_over, simple ? conv_pointwise_us<TE>(s, epi) : 0.0) || in_place(s, x, SZ, epi.y, Epi::out_bytes))
+		SmallPlan plan;
+		if (!conv_small_preferred(s, SZ, hand_over, simple ? conv_pointwise_us<TE>(s, epi) : 0.0, plan) || in_place(s, x, SZ, epi.y, Epi::out_bytes))
 			return false;
-		const SmallPlan plan = conv_small_plan(s, SZ);
 		const int side = SMALL_TILE * plan.tiles;
 		const int64_t pixel_tiles = (pixels + side - 1) / side, filter_tiles = (static_cast<int64_t>(s.K) + side - 1) / side;
 		if (pixel_tiles * 64 * plan.waves >= (1ll << 32) /* work-items of a launch along one direction */ || filter_tiles > 65535
@@ -643,8 +644,8 @@ extern "C" AVHIP_API int avhip_conv2d_small_plan(int x_dtype, const avhipConvSha
 	if (shape == nullptr || hand_over < 0 || hand_over > 2)
 		return 0;
 	const int element_bytes = x_dtype == DT_INT8 ? 1 : x_dtype == DT_FLOAT32 ? 4 : 2;
-	if (!conv_small_preferred(*shape, element_bytes, static_cast<HandOver>(hand_over), 0.0))
+	SmallPlan plan;
+	if (!conv_small_preferred(*shape, element_bytes, static_cast<HandOver>(hand_over), 0.0, plan))
 		return 0;
-	const SmallPlan plan = conv_small_plan(*shape, element_bytes);
 	return 16 * plan.tiles + plan.waves;
 }

@@ -69,8 +69,8 @@ namespace avhip
 	{
 		PLAIN, ELEMENTS, ACTIVATION
 	};
-	/* Whether the launcher sends the layer to that kernel, given the conditions above.  `one_tap_us`: conv_pointwise_us. */
-	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us);
+	/* Whether the launcher sends the layer to that kernel, given the conditions above, and with which plan.  `one_tap_us`: conv_pointwise_us. */
+	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us, SmallPlan &plan);
 	/* fp32 layers that the image-tile kernel takes: whether the gather kernel, whose fp32 products are of bf16 pieces, is estimated to be faster. */
 	bool conv_gather_before_image_tiles(const avhipConvShape &s);
 	/* What the layer is estimated to take in that kernel or, where it is not preferred, in those with large tiles: microseconds. */
