@@ -317,9 +317,10 @@ namespace
 			const int64_t row_blocks = ceil_div(M, ROWS), col_blocks = ceil_div(N, BLOCK_N);
 			const int64_t tiles = row_blocks * col_blocks * batch;
 			/* fp32 with three or four steps: the one-tile kernel multiplies in bf16 pieces (64 x 64 for a wavefront, which pays for the cutting; the rows
-			 * of 32 here do not), and is the faster one once its tiles are more than a round of the 512 workgroups that are resident: 648
-			 * tiles and more 1.03 to 1.27 times (36 products 4096 x 128 x 128 47 -> 41 us, 10890 x 192 x 96 by sixteen 95 -> 79), 576 tiles 0.93 to
-			 * 1.15, 288 0.92 to 1.0, 36 0.7 to 0.8.  With two steps its start costs what the pieces save (0.81 to 1.08).  A grid has at most 65535 along z. */
+			 * of 32 here do not), and is the faster one once its tiles are more than a round of the 512 workgroups that are resident: on 57 products of
+			 * 608 to 2520 tiles 1.3 times as fast on average (36 products 4096 x 128 x 128 46.5 -> 42.7 us, 10890 x 192 x 96 by sixteen 96.5 -> 76.8), on
+			 * two of them slower (1294 x 240 x 92 28.9 -> 32.5, 1318 x 160 x 100 28.5 -> 29.7); 576 tiles 0.93 to 1.15 times as fast, 288 0.92 to 1.0,
+			 * 36 0.7 to 0.8.  With two steps its start costs what the pieces save (0.81 to 1.08).  A grid has at most 65535 along z. */
 			if (sizeof(TE) == 4 && steps > 2 && batch <= 65535 && ceil_div(M, BLOCK_M) * col_blocks * batch >= 600)
 				return false;
 			if (sA < 0 || sB < 0 || a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31) || tiles >= (1ll << 31) - 1024)

@@ -6,7 +6,7 @@
  * No transpose is made.  For fp32 the operand layout of v_mfma_f32_32x32x2_f32 (lane l: row l % 32, k l / 32) is exactly a
  * coalesced load of two rows of A, and the eight k that a lane has of a stage are an operand of a bf16 product too: with tiles of 64 x 64 the
  * values are cut into three bf16 pieces in registers (struct Pieces of mfma_core.hpp), and six of the nine products of pieces are taken.  (The cutting costs
- * as much as the products save with 32 x 32: 12.6 against 11.1 us below.)  For 16-bit types a lane loads one dword (two neighbouring m) of four or eight
+ * as much as the products save with 32 x 32: 12.6 against 11.4 us below.)  For 16-bit types a lane loads one dword (two neighbouring m) of four or eight
  * k rows and separates them with v_perm_b32 into the operand chunks of two MFMA tiles, one of the even and one of the odd m, or exchanges one
  * of the two with the sixteen lanes beside it; what cannot be read in pairs (odd sizes) is loaded element by element.  k rows and m, n
  * outside the matrices come back as zeros from the buffer loads, so the loop has no branch.
@@ -16,11 +16,12 @@
  * the end, in a fixed order.  The split along k inside the workgroup is what fills the chip: a gradient of 128 x 128
  * channels has 144 tiles of 64 x 64 (F(4x4, 3x3)), 1152 wavefronts for 1024 SIMDs.  Sixteen wavefronts on a tile of 32 x 32 were slower at every size.
  *
- * Measured (36 products 128 x 128 over k = 512, fp32, operands from L2 / the last-level cache): 9.5 us, of which the
- * 18.9 MB of operands need 3.4 and the matrix cores 1.5; 11.1 with fp32 products, 74 in the generic kernel.  16-bit, tiles of 32 x 32, pairs against single
+ * Measured (36 products 128 x 128 over k = 512, fp32, operands from L2 / the last-level cache): 9.8 us, of which the
+ * 18.9 MB of operands need 3.4 and the matrix cores 1.5; 11.4 with fp32 products, 74 in the generic kernel.  16-bit, tiles of 32 x 32, pairs against single
  * elements: 16 products 72 x 96 over 15561 43.1 -> 38.7 us, 32 x 32 over 4608 12.2 -> 8.4, 64 x 80 over 750 5.9 -> 4.6.  What bounds it at small
  * sizes is the chain of one launch: first loads, one or two waves of MFMAs, the sum through LDS.
  */
+#include <cmath>
 #include <type_traits>
 
 #include "gemm_tn.hpp"
@@ -307,6 +308,33 @@ namespace
 	}
 }
 
+namespace
+{
+	/* The side of a tile of C: 32 while tiles of 64 leave the chip short of work.  16-bit types are bound by their operand loads, which large tiles halve
+	 * (at 64 large tiles 18 to 54 % slower than small ones, at 160 to 256 equal, above faster).  fp32: small tiles have fp32 products and four of
+	 * them share a compute unit, large ones have bf16 pieces and a compute unit each, so that 288 of them are two rounds and cost what 512 do.
+	 * Microseconds of the two, fitted to 115 products with both (16 or 36 of 32 to 256 a side over 60 to 7128; root mean square error 10 and 7 %);
+	 * with the large ones 5 % below, the one taken is 0.2 % slower than the faster one on average and 7 % at most (80 x 224 over 2150, 36 of them, 288 large tiles:
+	 * 54.7 : 36.6 us, 216 x 32 over 1716 22.7 : 15.5; 128 x 128 over 512, 144 large tiles 9.8 : 11.4, 168 x 128 over 273, 216 8.5 : 14.1). */
+	int tn_side(int element_bytes, int batch, int M, int N, int K)
+	{
+		auto tiles = [&](int side) { return static_cast<int64_t>(ceil_div(M, side)) * ceil_div(N, side) * batch; };
+		if (element_bytes != 4)
+			return tiles(64) < 128 ? 32 : 64;
+		if (tiles(32) * 64 * WAVES >= (1ll << 32)) /* more work-items than a launch takes along one direction */
+			return 64;
+		const int stages = static_cast<int>(ceil_div(ceil_div(K, STAGE), WAVES)); /* of a wavefront; large tiles have them in flight in pairs */
+		auto on_a_unit = [&](int side) { return std::ceil(static_cast<double>(tiles(side)) / 256.0); };
+		const double small = 2.4 + on_a_unit(32) * (1.8 + 0.51 * stages), large = 0.7 + on_a_unit(64) * (4.1 + 0.86 * stages + 0.80 * ((stages + 1) / 2));
+		return large < 0.95 * small ? 64 : 32;
+	}
+}
+
+extern "C" int avhip_gemm_tn_side(int element_bytes, int batch, int M, int N, int K)
+{
+	return tn_side(element_bytes, batch, M, N, K);
+}
+
 namespace avhip
 {
 	template<typename TE, typename TC>
@@ -332,13 +360,8 @@ namespace avhip
 		g.c_batch = strideC;
 		g.alpha = alpha;
 		g.beta = beta;
-		/* Tiles of 32 x 32 while those of 64 x 64 leave the chip short of work.  16-bit types are bound by their operand loads, which large tiles halve
-		 * (at 64 large tiles 18 to 54 % slower than small ones, at 160 to 256 equal, above faster).  fp32: small tiles have fp32 products, large
-		 * ones bf16 pieces (36 products of 128 x 128 over 512, 144 large tiles: 9.5 : 11.1 us, 128 x 248 over 2080, 288: 24.4 : 28.1; 16 of 104 x 192
-		 * over 7128, 96 large tiles: 66 : 59). */
-		const int64_t large_tiles = static_cast<int64_t>(ceil_div(M, 64)) * ceil_div(N, 64) * batch;
-		const bool small = large_tiles < 128;
-		const int side = small ? 32 : 64;
+		const int side = tn_side(SZ, batch, M, N, K);
+		const bool small = side == 32;
 		g.row_tiles = static_cast<int>(ceil_div(M, side));
 		g.col_tiles = static_cast<int>(ceil_div(N, side));
 		const int64_t tiles = static_cast<int64_t>(g.row_tiles) * g.col_tiles * batch;

@@ -6,6 +6,12 @@
 
 #include "common.hpp"
 
+extern "C"
+{
+	/* The side of the tiles of C that a product is taken in, 32 or 64 (fp32: the latter in bf16 pieces).  Exported for tests. */
+	AVHIP_API int avhip_gemm_tn_side(int element_bytes, int batch, int M, int N, int K);
+}
+
 namespace avhip
 {
 	/* Launches the (T, N) product C[b][m][n] = alpha * sum_k A[b][k][m] * B[b][k][n] + beta * C[b][m][n] (row-major, fp32

@@ -90,7 +90,7 @@ def test_gemm_batched_other_forms(oracle, opA, opB):
                                    (130, 64, 64, 130), (129, 63, 64, 127), (515, 60, 33, 33)])
 def test_gemm_batched_tn(oracle, dtype, c_dtype, shape):
     """C[b] = A[b]^T B[b], the product of the weight gradient: 32 x 32 tiles for the small ones, 64 x 64 tiles from 128
-    of them on, in pairs of elements where M and N are even; k below, at and above one stage of 16 rows and one round of the
+    of them on (16-bit) or by estimate (fp32), in pairs of elements where M and N are even; k below, at and above one stage of 16 rows and one round of the
     eight wavefronts (128).  Bars as for the (N, T) form: one fp32 sum of at most 513 products, one rounding on store."""
     g = h.rng(14)
     batch, M, N, K = shape

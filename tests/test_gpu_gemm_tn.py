@@ -3,6 +3,7 @@ have no such pieces; 16-bit pairs in tiles of 32 x 32."""
 import numpy as np
 import pytest
 
+import cudabackend_amd as cb
 import helpers as h
 
 pytestmark = pytest.mark.gpu
@@ -15,9 +16,10 @@ def product(A, B):
 @pytest.mark.parametrize("scale", [1.0, 2.0 ** -60, 2.0 ** 55])
 @pytest.mark.parametrize("shape", [(130, 64, 64, 130), (36, 128, 97, 1031), (33, 100, 126, 17)])
 def test_fp32_pieces_are_no_less_precise(shape, scale):
-    """Tiles of 64 x 64 (128 of them or more).  What is dropped is below 2^-24 of a product, so the error stays that of a 32-bit sum: at most
+    """Tiles of 64 x 64.  What is dropped is below 2^-24 of a product, so the error stays that of a 32-bit sum: at most
     sqrt(K) roundings of 2^-24 as they add up at random, with a factor of two; measured 1e-7 to 2e-7."""
     batch, M, N, K = shape
+    assert cb.load_library().avhip_gemm_tn_side(4, *shape) == 64
     g = h.rng(31)
     A, B = ((g.standard_normal((batch, K, n)) * scale).astype(np.float32) for n in (M, N))
     got = h.gemm(A, B, np.zeros((batch, M, N), np.float32), "f32", True, False, batched=True)
@@ -27,7 +29,8 @@ def test_fp32_pieces_are_no_less_precise(shape, scale):
 
 def test_fp32_values_without_pieces():
     """Infinities, NaN and the largest numbers (no bf16 near them): the sums are those of fp32 products."""
-    batch, M, N, K = 128, 64, 64, 300
+    batch, M, N, K = 130, 64, 64, 300
+    assert cb.load_library().avhip_gemm_tn_side(4, batch, M, N, K) == 64
     g = h.rng(32)
     A, B = (g.standard_normal((batch, K, n)).astype(np.float32) for n in (M, N))
     A[3, 7, 5], A[4, 250, 63], B[5, 0, 0], A[6, 20, 20] = np.inf, np.nan, -np.inf, np.finfo(np.float32).max

@@ -28,7 +28,8 @@ def check(got, want, k):
 
 @pytest.mark.parametrize("scales", SCALES)
 def test_tn_product(scales):
-    """64 x 64 tiles: 130 of them."""
+    """Tiles of 64 x 64."""
+    assert cb.load_library().avhip_gemm_tn_side(4, 130, 64, 60, 200) == 64
     A, B = operands([(130, 200, 64), (130, 200, 60)], scales)
     got = h.gemm(A, B, np.zeros((130, 64, 60), np.float32), "f32", True, False, batched=True)
     check(got, np.matmul(A.astype(np.float64).transpose(0, 2, 1), B.astype(np.float64)), 200)
