@@ -671,7 +671,8 @@ namespace
 			while (pb > 1 && (pixel_bytes % pb != 0 || !aligned_to(x, pb) || !aligned_to(w, pb)))
 				pb /= 2;
 			pb = (pb < static_cast<int>(sizeof(TE)) || s.R * s.S > 32) ? 0 : pb; /* the gather kernel's tap mask has 32 bits */
-			if (ragged && small_before_packed(s, sizeof(TE), pb, epi.z != nullptr) && conv_small_launch<TE, Epi>(st, s, x, w, epi))
+			if (ragged && small_before_packed(s, sizeof(TE), pb, epi.z != nullptr) 
+					&& conv_small_launch<TE, Epi>(st, s, x, w, epi, conv_small_choice<TE>(s, epi)))
 				return 0;
 #define AVHIP_PACKED(PB) hipLaunchKernelGGL((k_conv_igemm_packed<TE, PB, Epi>), grid, dim3(256), 0, st, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi)
 			switch (pb)
@@ -693,13 +694,18 @@ namespace
 			}
 #undef AVHIP_PACKED
 		}
-		/* operands through a ring of LDS buffers, where that is estimated to be faster than what follows */
-		if constexpr (sizeof(TE) < 4)
-			if (fast_path_ok<TE>(s, flags, padding_value) && conv_ring_launch<TE, Epi>(st, s, x, w, epi))
+		const bool chunks = fast_path_ok<TE>(s, flags, padding_value);
+		if (ragged || chunks)
+		{
+			const SmallChoice small = conv_small_choice<TE>(s, epi);
+			/* operands through a ring of LDS buffers, where that is estimated to be faster than what follows */
+			if constexpr (sizeof(TE) < 4)
+				if (chunks && conv_ring_launch<TE, Epi>(st, s, x, w, epi, small))
+					return 0;
+			/* a problem that does not fill the chip with big tiles goes to the kernel with small ones and k shared by wavefronts */
+			if (conv_small_launch<TE, Epi>(st, s, x, w, epi, small))
 				return 0;
-		/* a problem that does not fill the chip with big tiles goes to the kernel with small ones and k shared by wavefronts */
-		if ((ragged || fast_path_ok<TE>(s, flags, padding_value)) && conv_small_launch<TE, Epi>(st, s, x, w, epi))
-			return 0;
+		}
 		/* one-tap filters are plain matrix products with a short k: a persistent kernel pipelines across tiles */
 		if (fast && s.R * s.S == 1 && conv_pointwise_launch<TE, Epi>(st, s, x, w, epi))
 			return 0;
@@ -900,13 +906,14 @@ namespace
 		 * split, 16.8 in small tiles) and an fp32 layer's sums would be of another kind (that layer's error against 64 bits: 2.1e-7 split, 3.1e-7 in
 		 * small tiles, 3.1e-6 through F(4x4, 3x3)). */
 		/* (at eight k-steps and more the one-tap kernels take nothing) */
-		SmallPlan small;
-		const double split = split_us(s, plan, static_cast<int>(sizeof(TE)));
-		if (conv_small_preferred(s, static_cast<int>(sizeof(TE)), HandOver::PLAIN, 0.0, small) && split > 0.95 * small.us
+		constexpr int SZ = static_cast<int>(sizeof(TE));
+		const SmallChoice small = conv_small_choice(s, SZ, HandOver::PLAIN, 0.0);
+		const double split = split_us(s, plan, SZ);
+		if (small.preferred && split > 0.95 * small.plan.us
 				&& !in_place(s, x, sizeof(TE), y, sizeof(TE)))
 			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
 		/* Nor is it where the ring kernel is: bf16 480 -> 128 5x5 stride 2 on 155 images of 9 x 9, 34.5 us in nine parts. */
-		const double ring = is_simple_activation(activation) ? conv_ring_us(s, static_cast<int>(sizeof(TE)), static_cast<int>(sizeof(TE)), HandOver::PLAIN, 0.0, z != nullptr) : 0.0;
+		const double ring = is_simple_activation(activation) ? conv_ring_us(s, SZ, SZ, small, z != nullptr) : 0.0;
 		if (ring > 0.0 && ring < 0.9 * split && !in_place(s, x, sizeof(TE), y, sizeof(TE)))
 			return launch_float<TE>(st, s, x, w, bias, z, y, padding_value, alpha1, alpha2, beta, activation);
 		const ConvGeom g = make_geom<TE>(s);

@@ -19,7 +19,6 @@
 #include <cmath>
 #include <type_traits>
 
-#include "conv_pointwise.hpp"
 #include "conv_ring.hpp"
 #include "conv_ring_plan.hpp"
 #include "conv_small.hpp"
@@ -334,22 +333,32 @@ namespace
 	constexpr RingPlan RING_PLANS[] = { { 256, 128, 1, 0.0, 0.63, 5.5, 7.4, 10.0, 0.07 }, { 128, 128, 1, 1.1, 0.38, 3.5, 3.8, 4.6, 0.045 },
 			{ 128, 64, 2, 2.1, 0.265, 2.0, 1.8, 2.8, 0.04 }, { 64, 64, 3, 2.5, 0.165, 1.7, 1.7, 2.6, 0.0 } };
 
+	/* no layer is estimated below a workgroup of the fastest pace, beginning and end */
+	constexpr double ring_at_least_us(double stages)
+	{
+		double fixed = RING_PLANS[0].launch + RING_PLANS[0].tile, stage = RING_PLANS[0].stage;
+		for (const RingPlan &p : RING_PLANS)
+		{
+			fixed = p.launch + p.tile < fixed ? p.launch + p.tile : fixed;
+			stage = p.stage < stage ? p.stage : stage;
+		}
+		return fixed + stage * stages;
+	}
+
 	struct RingChoice
 	{
 		int plan;
 		double us;
 	};
-	/* `hand_over`: 0 whole vectors, 1 element by element, 2 any activation (HandOver of conv_small.hpp) */
-	RingChoice ring_choice(const avhipConvShape &s, int element_bytes, int out_bytes, int hand_over, bool residual)
+	RingChoice ring_choice(const avhipConvShape &s, double stages, int out_bytes, HandOver hand_over, bool residual)
 	{
 		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
-		const double stages = std::ceil(static_cast<double>(s.R) * s.S * (s.C * element_bytes / 16) / 8.0);
 		const double megabytes = pixels * s.K * out_bytes * (residual ? 2.0e-6 : 1.0e-6);
 		RingChoice best = { -1, 0.0 };
 		for (int i = 0; i < 4; i++)
 		{
 			const RingPlan &p = RING_PLANS[i];
-			const double tile = p.tile + (hand_over == 1 ? p.elements : hand_over == 2 ? p.activation : 0.0);
+			const double tile = p.tile + (hand_over == HandOver::ELEMENTS ? p.elements : hand_over == HandOver::ACTIVATION ? p.activation : 0.0);
 			const double loads = std::ceil(pixels / p.pixels) * ((s.K + p.filters - 1) / p.filters) / 256.0; /* of workgroups, one per compute unit each */
 			const double rounds = std::floor(loads / p.per_cu), rest = std::ceil(loads - rounds * p.per_cu);
 			const double us = p.launch + (rounds + (rest > 0.0 ? 1.0 : 0.0)) * tile + (rounds * p.per_cu + rest) * p.stage * stages + p.megabyte * megabytes;
@@ -360,41 +369,43 @@ namespace
 	}
 
 	/* The tile that the layer gets and its estimate, or no plan where it is left to the other kernels */
-	RingChoice ring_route(const avhipConvShape &s, int element_bytes, int out_bytes, HandOver hand_over, double one_tap_us, bool residual)
+	RingChoice ring_route(const avhipConvShape &s, int element_bytes, int out_bytes, const SmallChoice &small, bool residual)
 	{
 		const RingChoice none = { -1, 0.0 };
 		/* layers that the few-channel kernels have taken before this one is asked */
-		if (hand_over == HandOver::PLAIN && conv_few_channels(s, element_bytes))
+		if (small.hand_over == HandOver::PLAIN && conv_few_channels(s, element_bytes))
 			return none;
 		/* (the switch of the small tiles is this kernel's too: at 0 the kernels with fixed tiles of 128 x 128 are asked for, below it small ones) */
 		if (element_bytes > 2 || static_cast<int64_t>(s.C) * element_bytes % 16 != 0 || !conv_small_possible(s, element_bytes) || conv_small_threshold() <= 0)
 			return none;
 		/* of 8-bit one-tap layers the persistent kernels are a fifth to a third faster than they are estimated (17 layers) */
-		if (element_bytes == 1 && one_tap_us > 0.0)
+		if (element_bytes == 1 && small.one_tap_us > 0.0)
 			return none;
 		/* 15 % below the others' estimates, which are the coarser ones: of the 410 layers one is then slower than before (bf16, a filter count that is no
 		 * multiple of four), and the mean gain is 11.7 of the 13.9 % that the best choice for each would have */
-		const RingChoice choice = ring_choice(s, element_bytes, out_bytes, static_cast<int>(hand_over), residual);
-		return choice.us < 0.85 * conv_without_ring_us(s, element_bytes, hand_over, one_tap_us) ? choice : none;
+		const double limit = 0.85 * small.us, stages = std::ceil(static_cast<double>(s.R) * s.S * (s.C * element_bytes / 16) / 8.0);
+		/* one workgroup takes longer than that, whatever its tile: the smallest layers, whose calls cost the host no less than the GPU */
+		if (ring_at_least_us(stages) >= limit)
+			return none;
+		const RingChoice choice = ring_choice(s, stages, out_bytes, small.hand_over, residual);
+		return choice.us < limit ? choice : none;
 	}
 }
 
 namespace avhip
 {
-	double conv_ring_us(const avhipConvShape &s, int element_bytes, int out_bytes, HandOver hand_over, double one_tap_us, bool residual)
+	double conv_ring_us(const avhipConvShape &s, int element_bytes, int out_bytes, const SmallChoice &small, bool residual)
 	{
-		return ring_route(s, element_bytes, out_bytes, hand_over, one_tap_us, residual).us;
+		return ring_route(s, element_bytes, out_bytes, small, residual).us;
 	}
 
 	template<typename TE, typename Epi>
-	bool conv_ring_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi)
+	bool conv_ring_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi, const SmallChoice &small)
 	{
 		constexpr int SZ = static_cast<int>(sizeof(TE));
 		const int64_t pixels = static_cast<int64_t>(s.N) * s.Ho * s.Wo;
-		const bool simple = epi.vec && is_simple_activation(epi.activation);
-		const HandOver hand_over = simple ? HandOver::PLAIN : is_simple_activation(epi.activation) ? HandOver::ELEMENTS : HandOver::ACTIVATION;
-		const bool residual = epi.z != nullptr;
-		const int plan = ring_route(s, SZ, Epi::out_bytes, hand_over, simple ? conv_pointwise_us<TE>(s, epi) : 0.0, residual).plan;
+		const bool simple = small.hand_over == HandOver::PLAIN;
+		const int plan = ring_route(s, SZ, Epi::out_bytes, small, epi.z != nullptr).plan;
 		if (plan < 0 || in_place(s, x, SZ, epi.y, Epi::out_bytes))
 			return false;
 		const int px = RING_PLANS[plan].pixels, ft = RING_PLANS[plan].filters;
@@ -456,7 +467,7 @@ namespace avhip
 		return true;
 	}
 
-#define AVHIP_INSTANTIATE(TE, EPI) template bool conv_ring_launch<TE, EPI>(hipStream_t, const avhipConvShape&, const void*, const void*, const EPI&);
+#define AVHIP_INSTANTIATE(TE, EPI) template bool conv_ring_launch<TE, EPI>(hipStream_t, const avhipConvShape&, const void*, const void*, const EPI&, const SmallChoice&);
 	AVHIP_INSTANTIATE(f16_t, FloatEpilogue<f16_t>)
 	AVHIP_INSTANTIATE(bf16_t, FloatEpilogue<bf16_t>)
 	AVHIP_INSTANTIATE(int8_t, Int8Epilogue<I8_EXACT>)
@@ -475,10 +486,10 @@ namespace
 	{
 		Epi epi { };
 		epi.vec = hand_over == 0;
+		epi.activation = hand_over == 2 ? ACT_ELU : ACT_LINEAR;
 		if (residual != 0)
 			epi.z = reinterpret_cast<decltype(epi.z)>(16);
-		return ring_route(s, static_cast<int>(sizeof(TE)), Epi::out_bytes, static_cast<HandOver>(hand_over), hand_over == 0 ? conv_pointwise_us<TE>(s, epi) : 0.0,
-				residual != 0);
+		return ring_route(s, static_cast<int>(sizeof(TE)), Epi::out_bytes, conv_small_choice<TE>(s, epi), residual != 0);
 	}
 	RingChoice route_of_call(int x_dtype, int y_dtype, const avhipConvShape *shape, int hand_over, int residual)
 	{

@@ -27,7 +27,6 @@
 #include <cmath>
 #include <type_traits>
 
-#include "conv_pointwise.hpp"
 #include "conv_small.hpp"
 #include "mfma_core.hpp"
 
@@ -520,40 +519,40 @@ namespace avhip
 	{
 		return hand_over != HandOver::PLAIN ? (element_bytes == 4 ? 1.1 : 1.2) : one_tap_us > 0.0 ? 1.05 : 1.0;
 	}
-	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us, SmallPlan &plan)
+	SmallChoice conv_small_choice(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
 	{
+		SmallChoice choice = { hand_over, one_tap_us, false, { 0, 0, 0.0 }, 0.0 };
 		if (!conv_small_possible(s, element_bytes))
-			return false;
-		plan = conv_small_plan(s, element_bytes);
+			return choice;
+		choice.plan = conv_small_plan(s, element_bytes);
 		const int threshold = conv_small_threshold();
 		if (threshold < 0) /* asked for by name (tests): whatever the kernel can run */
-			return true;
-		if (!whole_chunks(s, element_bytes)) /* otherwise the general gather kernel, element by element: 2.2 to 17 times slower on all of 14 layers of 1152 to 627200 pixels */
-			return threshold != 0;
-		const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
-		return tiles < threshold && small_factor(element_bytes, hand_over, one_tap_us) * plan.us < workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
+			choice.preferred = true;
+		else if (!whole_chunks(s, element_bytes)) /* otherwise the general gather kernel, element by element: 2.2 to 17 times slower on all of 14 layers of 1152 to 627200 pixels */
+			choice.preferred = threshold != 0;
+		else
+		{
+			choice.us = workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
+			const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
+			choice.preferred = tiles < threshold && small_factor(element_bytes, hand_over, one_tap_us) * choice.plan.us < choice.us;
+		}
+		if (choice.preferred)
+			choice.us = small_factor(element_bytes, hand_over, 0.0) * choice.plan.us;
+		return choice;
 	}
 	bool conv_gather_before_image_tiles(const avhipConvShape &s)
 	{
 		return tile_kernel_us(s, 4, GATHER) < tile_kernel_us(s, 4, IMAGE_TILES);
 	}
-	double conv_without_ring_us(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
-	{
-		SmallPlan plan;
-		return conv_small_preferred(s, element_bytes, hand_over, one_tap_us, plan) ? small_factor(element_bytes, hand_over, 0.0) * plan.us
-				: workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
-	}
 
 	template<typename TE, typename Epi>
-	bool conv_small_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi)
+	bool conv_small_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi, const SmallChoice &choice)
 	{
 		constexpr int SZ = static_cast<int>(sizeof(TE));
 		const int64_t pixels = static_cast<int64_t>(s.N) * s.Ho * s.Wo;
-		/* whole 4-filter vectors and LINEAR / RELU, or anything (the integer epilogues know no other activation) */
-		const bool simple = epi.vec && is_simple_activation(epi.activation);
-		const HandOver hand_over = simple ? HandOver::PLAIN : is_simple_activation(epi.activation) ? HandOver::ELEMENTS : HandOver::ACTIVATION;
-		SmallPlan plan;
-		if (!conv_small_preferred(s, SZ, hand_over, simple ? conv_pointwise_us<TE>(s, epi) : 0.0, plan) || in_place(s, x, SZ, epi.y, Epi::out_bytes))
+		const SmallPlan &plan = choice.plan;
+		const bool simple = choice.hand_over == HandOver::PLAIN;
+		if (!choice.preferred || in_place(s, x, SZ, epi.y, Epi::out_bytes))
 			return false;
 		const int side = SMALL_TILE * plan.tiles;
 		const int64_t pixel_tiles = (pixels + side - 1) / side, filter_tiles = (static_cast<int64_t>(s.K) + side - 1) / side;
@@ -625,7 +624,7 @@ namespace avhip
 		return true;
 	}
 
-#define AVHIP_INSTANTIATE(TE, EPI) template bool conv_small_launch<TE, EPI>(hipStream_t, const avhipConvShape&, const void*, const void*, const EPI&);
+#define AVHIP_INSTANTIATE(TE, EPI) template bool conv_small_launch<TE, EPI>(hipStream_t, const avhipConvShape&, const void*, const void*, const EPI&, const SmallChoice&);
 	AVHIP_INSTANTIATE(float, FloatEpilogue<float>)
 	AVHIP_INSTANTIATE(f16_t, FloatEpilogue<f16_t>)
 	AVHIP_INSTANTIATE(bf16_t, FloatEpilogue<bf16_t>)
@@ -644,8 +643,6 @@ extern "C" AVHIP_API int avhip_conv2d_small_plan(int x_dtype, const avhipConvSha
 	if (shape == nullptr || hand_over < 0 || hand_over > 2)
 		return 0;
 	const int element_bytes = x_dtype == DT_INT8 ? 1 : x_dtype == DT_FLOAT32 ? 4 : 2;
-	SmallPlan plan;
-	if (!conv_small_preferred(*shape, element_bytes, static_cast<HandOver>(hand_over), 0.0, plan))
-		return 0;
-	return 16 * plan.tiles + plan.waves;
+	const SmallChoice choice = conv_small_choice(*shape, element_bytes, static_cast<HandOver>(hand_over), 0.0);
+	return choice.preferred ? 16 * choice.plan.tiles + choice.plan.waves : 0;
 }

@@ -5,6 +5,7 @@
 #define AVHIP_CONV_SMALL_HPP_
 
 #include "conv_epilogue.hpp"
+#include "conv_pointwise.hpp"
 
 namespace avhip
 {
@@ -28,13 +29,6 @@ namespace avhip
 		result.factor = static_cast<unsigned int>(((1ull << (31 + result.shift)) + d - 1) / d);
 		return result;
 	}
-
-	/* Launches the kernel and returns true when its estimate for the problem is below that of the kernels with 128 x 128 (or
-	 * 256 x 64) workgroup tiles; returns false without side effects otherwise.  The caller has established the conditions of the
-	 * branch-free loaders (16-byte aligned tensors below 2 GiB, zero padding value);
-	 * any activation and number of filters.  Calls that work in place are left to the other kernels. */
-	template<typename TE, typename Epi>
-	bool conv_small_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi);
 
 	/* Whether the call writes y where x lies.  No header promises that, but it works where the sums are complete before the first result
 	 * is written (k split through the workspace, the three passes of non-fused Winograd) and where a workgroup alone reads the pixels that
@@ -69,12 +63,32 @@ namespace avhip
 	{
 		PLAIN, ELEMENTS, ACTIVATION
 	};
-	/* Whether the launcher sends the layer to that kernel, given the conditions above, and with which plan.  `one_tap_us`: conv_pointwise_us. */
-	bool conv_small_preferred(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us, SmallPlan &plan);
+	/* What the launchers of this kernel and of the ring kernel (conv_ring.hip) both ask about a call.  Its caller has it worked out once, as it is a good part of
+	 * what a call of the smallest layers costs the host: by each of them for itself 0.14 us of some 5, so 5 us.  */
+	struct SmallChoice
+	{
+		HandOver hand_over;
+		double one_tap_us; /* conv_pointwise_us */
+		bool preferred; /* whether the layer is sent to this kernel: its estimate is below that of the kernels with 128 x 128 (or 256 x 64) workgroup tiles */
+		SmallPlan plan;
+		double us; /* estimate of the layer in this kernel or, where it is not preferred, in those (0: it cannot run the layer) */
+	};
+	SmallChoice conv_small_choice(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us);
+	template<typename TE, typename Epi>
+	SmallChoice conv_small_choice(const avhipConvShape &s, const Epi &epi)
+	{
+		/* whole 4-filter vectors and LINEAR / RELU, or anything (the integer epilogues know no other activation) */
+		const bool simple = is_simple_activation(epi.activation);
+		const HandOver hand_over = !simple ? HandOver::ACTIVATION : epi.vec ? HandOver::PLAIN : HandOver::ELEMENTS;
+		return conv_small_choice(s, static_cast<int>(sizeof(TE)), hand_over, hand_over == HandOver::PLAIN ? conv_pointwise_us<TE>(s, epi) : 0.0);
+	}
+	/* Launches the kernel and returns true where it is preferred; returns false without side effects otherwise.  The caller has established the conditions of
+	 * the branch-free loaders (16-byte aligned tensors below 2 GiB, zero padding value); any activation and number of filters.  Calls
+	 * that work in place are left to the other kernels. */
+	template<typename TE, typename Epi>
+	bool conv_small_launch(hipStream_t stream, const avhipConvShape &s, const void *x, const void *w, const Epi &epi, const SmallChoice &choice);
 	/* fp32 layers that the image-tile kernel takes: whether the gather kernel, whose fp32 products are of bf16 pieces, is estimated to be faster. */
 	bool conv_gather_before_image_tiles(const avhipConvShape &s);
-	/* What the layer is estimated to take in that kernel or, where it is not preferred, in those with large tiles: microseconds. */
-	double conv_without_ring_us(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us);
 }
 
 #endif /* AVHIP_CONV_SMALL_HPP_ */
