@@ -12,7 +12,8 @@
  * Loads in a row behind the barrier stalled their wavefronts in the queue of the memory pipeline; one by one between the products they
  * do not (a 64 x 64 tile with a compute unit to itself: 0.24 -> 0.21 us a stage, 256 x 128: 38.7 -> 34.3 us on the second layer below).
  * Measured, before (the kernel that took the layer then: gather, image tiles or small tiles) and now: bf16 192 -> 384 3x3 stride 2 on 25 images of 58 x 58 and its
- * 1x1 384 -> 768 73 -> 56 us, fp16 224 -> 112 3x3 on 79 x 26 x 26 48 -> 34, int8 144 -> 80 3x3 on 81 x 39 x 39 43.5 -> 27, bf16 256 -> 512 3x3 stride 2
+ * 1x1 384 -> 768 73 -> 56 us, fp16 224 -> 112 3x3 on 79 x 26 x 26 with an ELU 54 -> 43.5 (with LINEAR or
+ * RELU the estimates keep it in image tiles, 49), int8 144 -> 80 3x3 on 81 x 39 x 39 43.5 -> 27, bf16 256 -> 512 3x3 stride 2
  * on 23 x 35 x 35 34 -> 21, bf16 192 -> 384 3x3 stride 2 on 11 x 41 x 41 15.3 -> 11.5.
  */
 #include <algorithm>
@@ -381,8 +382,9 @@ namespace
 		/* of 8-bit one-tap layers the persistent kernels are a fifth to a third faster than they are estimated (17 layers) */
 		if (element_bytes == 1 && small.one_tap_us > 0.0)
 			return none;
-		/* 15 % below the others' estimates, which are the coarser ones: of the 410 layers one is then slower than before (bf16, a filter count that is no
-		 * multiple of four), and the mean gain is 11.7 of the 13.9 % that the best choice for each would have */
+		/* 15 % below the others' estimates, which are the coarser ones (those of image tiles and one-tap kernels up to 1.9 and 1.7 times too low where filters fill no
+		 * blocks of 64 or channels no 128 bytes: 32 -> 440 3x3 on 4 x 61 x 64 takes 19.6 us there against 13.2 here, and stays there): of the
+		 * 410 layers one is then slower than before (bf16, a filter count that is no multiple of four), and the mean gain is 11.7 of the 13.9 % that the best choice for each would have */
 		const double limit = 0.85 * small.us, stages = std::ceil(static_cast<double>(s.R) * s.S * (s.C * element_bytes / 16) / 8.0);
 		/* one workgroup takes longer than that, whatever its tile: the smallest layers, whose calls cost the host no less than the GPU */
 		if (ring_at_least_us(stages) >= limit)

@@ -10,8 +10,7 @@
  * rows that start between two dwords are loaded as the dwords around them and shifted.
  *
  * fp32 with 64 x 64: products of bf16 pieces (struct Pieces of mfma_core.hpp), cut by the wavefront that multiplies; with 32 x 32 the cutting takes as long as the
- * products save.  96 -> 64 5x5 on 21 images of 57 x 53 290 -> 141 us, 352 -> 112 3x3 stride 2 on 76 of 35 x 35 with an ELU 240 -> 154, 128 -> 128 3x3 on 31 of
- * 19 x 19 41 -> 34.
+ * products save.  96 -> 64 5x5 on 21 images of 57 x 53 287 -> 131 us (image tiles before), 352 -> 112 3x3 stride 2 on 76 of 35 x 35 with an ELU 235 -> 169 (32 x 32).
  *
  * What bounds it: the 64 bytes per clock that a compute unit loads (128 clocks per stage of a 32 x 32 tile, 256 per stage of a
  * 64 x 64 tile, which needs half as much per product), for fp32 the matrix cores, and for the smallest problems the latency of
@@ -427,7 +426,9 @@ namespace
 	 * a k-step of one that has a compute unit to itself or shares it.  The last round, if it is of up to 256, goes at the pace of the former.
 	 * Microseconds, fitted to 448 layers (2000 to 130000 pixels, 16 to 512 channels and filters; root mean square error 6 to 13 %).  With every
 	 * round of the same length a 517th workgroup seemed to double the time: fp16 128 -> 128 3x3 on 129 images of 18 x 18 went to small tiles
-	 * and took 29.3 us, 25.5 in the image-tile kernel. */
+	 * and took 29.3 us, 25.5 in the image-tile kernel.  The image tiles' figures hold where filters fill blocks of 64 and channels 128 bytes; of 18 layers
+	 * where they do not, seven take 1.3 to 1.9 times as long (fp16 224 -> 112 3x3 on 79 x 26 x 26 28.5 : 49 us), and int8
+	 * layers up to a third longer (128 -> 128 on 128 x 20 x 20 10.1 : 13). */
 	struct TilePace
 	{
 		double launch, round, alone, shared;

@@ -114,7 +114,8 @@ namespace avhip
 	 * in 32 bits; what is left out is less than 2^-24 of the whole.  An infinity, a NaN and a value that rounds to an infinity have no
 	 * such pieces: their sums are NaN or infinite, and the caller takes such a tile once more with Mma<float>.
 	 * The lowest bits of a float are 2^-149 and those of a bf16 2^-133: times PIECE_SCALE every float below 2^111 has its three pieces, without it only those
-	 * from 2^-110 on (at 2^-118 an error of 9e-6, at 2^-138 of 1).  The scale and its way back cost the kernels that cut 3 to 4 %.
+	 * from 2^-110 on (at 2^-118 an error of 9e-6, at 2^-138 of 1).  The scale and its way back cost 0.5 %
+	 * on average over 45 layers, 4 % at most.
 	 */
 	constexpr float PIECE_SCALE = 0x1p16f;
 	__device__ __forceinline__ uint4 scaled(const uint4 &chunk)
