@@ -385,7 +385,12 @@ namespace
 		/* 15 % below the others' estimates, which are the coarser ones (those of image tiles and one-tap kernels up to 1.9 and 1.7 times too low where filters fill no
 		 * blocks of 64 or channels no 128 bytes: 32 -> 440 3x3 on 4 x 61 x 64 takes 19.6 us there against 13.2 here, and stays there): of the
 		 * 410 layers one is then slower than before (bf16, a filter count that is no multiple of four), and the mean gain is 11.7 of the 13.9 % that the best choice for each would have */
-		const double limit = 0.85 * small.us, stages = std::ceil(static_cast<double>(s.R) * s.S * (s.C * element_bytes / 16) / 8.0);
+		/* Small tiles of fewer than 32 filters of a 16-bit layer take down to three quarters of their estimate, which counts the filters that do not exist as loaded.
+		 * Of 140 layers of 8 to 64 filters 32 leave the ring for that, 15 of them 2 to 24 % slower in it (fp16 512 -> 13 1x1 on 187 x 10 x 11 7.7 : 10.2 us, bf16 400 -> 10
+		 * 3x3 on 94 x 30 x 30 58 : 70.5), the others 11 % faster at most; of 70 that the rule was not made from 32, 0.70 to 1.16 times as fast in
+		 * it and 0.97 on average, where the 38 that stay are 1.10 times as fast.  8-bit layers stay (25 of them 1.02 times as fast in the ring). */
+		const double others = element_bytes == 2 && small.preferred && s.K < 32 ? (0.75 + 0.25 / 32.0 * s.K) * small.us : small.us;
+		const double limit = 0.85 * others, stages = std::ceil(static_cast<double>(s.R) * s.S * (s.C * element_bytes / 16) / 8.0);
 		/* one workgroup takes longer than that, whatever its tile: the smallest layers, whose calls cost the host no less than the GPU */
 		if (ring_at_least_us(stages) >= limit)
 			return none;

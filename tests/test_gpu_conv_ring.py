@@ -52,22 +52,22 @@ class Layer:
 FLOAT_CASES = {
     "relu": [
         (0, 25, 37, 37, 32, 68, 3, 1, 1, 0), (0, 19, 42, 44, 16, 100, 1, 1, 1, 0), (0, 30, 33, 35, 144, 68, 1, 1, 1, 0), (1, 33, 23, 24, 32, 76, 3, 1, 1, 1),
-        (1, 35, 23, 22, 40, 68, 3, 1, 2, 1), (1, 11, 41, 40, 48, 72, 3, 1, 2, 1), (2, 32, 26, 27, 32, 16, 3, 1, 1, 1), (2, 28, 28, 30, 16, 20, 1, 1, 1, 0),
-        (2, 30, 47, 46, 160, 16, 1, 2, 1, 0), (3, 3, 37, 37, 32, 36, 3, 1, 1, 1), (3, 9, 44, 43, 16, 40, 1, 2, 1, 0), (3, 37, 15, 15, 152, 20, 1, 1, 1, 0),
+        (1, 35, 23, 22, 40, 68, 3, 1, 2, 1), (1, 11, 41, 40, 48, 72, 3, 1, 2, 1), (2, 32, 26, 27, 32, 36, 3, 1, 1, 1), (2, 28, 28, 30, 16, 20, 1, 1, 1, 0),
+        (2, 30, 47, 46, 160, 36, 1, 2, 1, 0), (3, 3, 37, 37, 32, 36, 3, 1, 1, 1), (3, 9, 44, 43, 16, 40, 1, 2, 1, 0), (3, 37, 15, 15, 152, 36, 1, 1, 1, 0),
     ],
     "relu_residual": [
         (0, 28, 35, 37, 40, 72, 3, 1, 2, 1), (0, 40, 36, 38, 16, 84, 1, 1, 1, 0), (0, 31, 32, 34, 72, 68, 1, 1, 1, 0), (1, 22, 34, 33, 32, 68, 3, 1, 1, 1),
-        (1, 9, 44, 44, 48, 68, 3, 1, 2, 0), (1, 14, 44, 43, 40, 76, 3, 1, 2, 0), (2, 27, 27, 28, 40, 16, 3, 1, 1, 0), (2, 38, 23, 22, 24, 16, 1, 1, 1, 0),
-        (2, 13, 37, 37, 80, 16, 1, 1, 1, 0), (3, 31, 17, 18, 32, 16, 3, 1, 1, 0), (3, 39, 16, 17, 16, 20, 1, 1, 1, 0), (3, 27, 27, 26, 136, 36, 1, 2, 1, 0),
+        (1, 9, 44, 44, 48, 68, 3, 1, 2, 0), (1, 14, 44, 43, 40, 76, 3, 1, 2, 0), (2, 27, 27, 28, 40, 36, 3, 1, 1, 0), (2, 38, 23, 22, 24, 16, 1, 1, 1, 0),
+        (2, 13, 37, 37, 80, 16, 1, 1, 1, 0), (3, 31, 17, 18, 32, 36, 3, 1, 1, 0), (3, 39, 16, 17, 16, 36, 1, 1, 1, 0), (3, 27, 27, 26, 136, 36, 1, 2, 1, 0),
     ],
     "elements": [
         (0, 31, 39, 41, 24, 66, 5, 1, 2, 1), (0, 27, 44, 44, 72, 66, 3, 1, 1, 1), (1, 19, 31, 30, 160, 65, 3, 1, 2, 0), (1, 25, 26, 28, 168, 69, 3, 1, 1, 1),
-        (1, 30, 45, 47, 64, 73, 5, 2, 1, 0), (2, 17, 38, 40, 16, 13, 3, 1, 1, 0), (2, 23, 36, 35, 16, 13, 1, 1, 1, 0), (2, 27, 30, 32, 88, 13, 1, 1, 1, 0),
-        (3, 25, 35, 37, 32, 37, 3, 2, 1, 0), (3, 27, 26, 28, 16, 143, 1, 2, 1, 0), (3, 25, 40, 41, 152, 14, 1, 1, 1, 0),
+        (1, 30, 45, 47, 64, 73, 5, 2, 1, 0), (2, 17, 38, 40, 16, 33, 3, 1, 1, 0), (2, 19, 36, 35, 16, 33, 1, 1, 1, 0), (2, 27, 30, 32, 88, 33, 1, 1, 1, 0),
+        (3, 25, 35, 37, 32, 37, 3, 2, 1, 0), (3, 27, 26, 28, 16, 143, 1, 2, 1, 0), (3, 25, 40, 41, 152, 33, 1, 1, 1, 0),
     ],
     "elu_residual": [
         (0, 40, 36, 36, 72, 80, 3, 1, 1, 1), (1, 21, 29, 29, 168, 68, 3, 1, 1, 1), (1, 20, 28, 30, 160, 76, 3, 1, 1, 1),
-        (1, 15, 40, 42, 120, 72, 3, 1, 1, 1), (2, 14, 43, 43, 16, 16, 5, 1, 2, 1), (2, 39, 36, 37, 80, 36, 1, 1, 1, 0), (2, 31, 45, 45, 192, 16, 1, 1, 1, 0),
+        (1, 15, 40, 42, 120, 72, 3, 1, 1, 1), (2, 14, 43, 43, 16, 36, 5, 1, 2, 1), (2, 39, 36, 37, 80, 36, 1, 1, 1, 0), (2, 31, 45, 45, 192, 36, 1, 1, 1, 0),
         (3, 12, 43, 43, 16, 44, 3, 1, 1, 0), (3, 22, 36, 37, 16, 40, 1, 1, 1, 0), (3, 19, 35, 35, 88, 36, 1, 1, 1, 0),
     ],
 }
