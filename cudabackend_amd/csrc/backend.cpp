@@ -27,6 +27,7 @@
 
 #include "../../include/avocado_hip_backend.h"
 #include "../../include/avocado_hip_kernels.h"
+#include "conv_estimates.hpp"
 #include "conv_ring_plan.hpp"
 #include "conv_winograd_f4.hpp"
 
@@ -943,6 +944,20 @@ namespace
 		const int rc = avhip_conv2d_winograd_fused(c.ctx.stream, p.x_dtype, &p.shape, c.x->data, U, c.bias, c.z, c.y->data, c.alpha1, c.alpha2, c.beta,
 				activation);
 		return from_launcher(rc);
+	}
+
+	/* fp32: whether the direct sums (small tiles, or 128 x 128 tiles with products in bf16 pieces) are estimated to be faster than the fused kernel.  That walks rounds of 256
+	 * workgroups of 256 pixels x 128 filters, filled up, 14 us and 43.5 us per 64 channels a round (58 us at 32 channels, 104 at 128, 362 at 472, ten layers within a tenth), 8 more
+	 * with a residual and 25 with an activation by a call.  Of 65 layers that went to it, 32 to 448 channels and 32 to 512 filters, 160 to 2151 workgroups, every one is faster in
+	 * direct sums: 1.3 to 6.3 times, 2.4 on average (32 -> 32 on 34 x 40 x 43 118 -> 19 us, 256 -> 256 on 114 x 12 x 12 202 -> 156).  What is left to it are full rounds of 128 channels
+	 * and filters without a workspace: 128 -> 128 on 256 x 15 x 15 104 us by both. */
+	bool direct_before_fused(const ConvCall &c, avActivationType_t activation, av_int64 fused_workgroups)
+	{
+		const avhipConvShape &s = c.problem.shape;
+		const bool simple = activation == AVOCADO_ACTIVATION_LINEAR || activation == AVOCADO_ACTIVATION_RELU;
+		const double fused = static_cast<double>((fused_workgroups + 255) / 256) * (14.0 + 43.5 * ((s.C + 63) / 64) + (c.z != nullptr ? 8.0 : 0.0) + (simple ? 0.0 : 25.0));
+		const double direct = std::min(avhip::conv_small_plan(s, 4).us, avhip::tile_kernel_us(s, 4, simple ? avhip::GATHER : avhip::GATHER_ACTIVATION));
+		return direct < 0.95 * fused;
 	}
 
 	/* Row-wise Winograd F(2,3) for 16-bit 3x3 layers whose image bands fit a compute unit's LDS (conv_winograd_rows.hip): two
@@ -2188,7 +2203,8 @@ namespace avocado
 			else if (fused_winograd_applicable(p) && p.x_dtype == AVOCADO_DTYPE_FLOAT32 && bias_fp32 && p.shape.C >= 32 && p.shape.K >= 32
 					&& p.shape.Ho == p.shape.H && p.shape.Wo == p.shape.W && fused_pays)
 			{
-				const avStatus_t fs = run_fused_winograd(call, wMem, yMem, activation);
+				const avStatus_t fs = direct_before_fused(call, activation, fused_workgroups) ? run_implicit_gemm(call, yMem, activation, nullptr)
+						: run_fused_winograd(call, wMem, yMem, activation);
 				if (fs != AVOCADO_STATUS_NOT_SUPPORTED && fs != AVOCADO_STATUS_BAD_ALLOC)
 					return fs;
 				if (fs == AVOCADO_STATUS_NOT_SUPPORTED && nonfused_ready)

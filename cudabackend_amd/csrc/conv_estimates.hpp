@@ -1,0 +1,98 @@
+/*
+ * conv_estimates.hpp -- what the implicit-GEMM kernels of small tiles (conv_small.hip) and of 128 x 128 tiles are estimated to take: host arithmetic on a shape, for their
+ * launchers and for the dispatcher, which weighs other plans against them.
+ */
+#ifndef AVHIP_CONV_ESTIMATES_HPP_
+#define AVHIP_CONV_ESTIMATES_HPP_
+
+#include <algorithm>
+#include <cmath>
+#include <stdint.h>
+
+#include "../../include/avocado_hip_kernels.h"
+
+namespace avhip
+{
+	/* tiles x tiles MFMA tiles of 32 x 32, `waves` wavefronts sharing the k range, and the estimated microseconds */
+	struct SmallPlan
+	{
+		int tiles, waves;
+		double us;
+	};
+	inline constexpr int SMALL_TILE = 32; /* side of the MFMA tile */
+	inline constexpr SmallPlan PLANS[] = { { 1, 1, 0.0 }, { 1, 4, 0.0 }, { 1, 8, 0.0 }, { 2, 4, 0.0 } };
+
+	struct Pace
+	{
+		double launch, chain, stage, tile;
+	};
+	/* Microseconds: launch and first loads, one stage of a wavefront alone, one stage of a tile when its compute unit is busy, and everything
+	 * else about a tile.  Order of PLANS.  16-bit and 8-bit types: the larger of the two stage costs, fitted to 320 layers (7 to 64 rows and
+	 * columns, 16 to 512 channels and filters, 1x1 to 5x5, up to 12 GFLOP; root mean square error 6 to 14 %).  fp32: the root of the sum of
+	 * their squares, fitted to 222 layers timed with every plan (up to 6 GFLOP): the plan chosen is 0.5 % slower than the best of the four
+	 * on average and 15 % at most, with the larger of the two 1.2 % and 36 % (52 -> 408 1x1 on 637 pixels: 7.2 us with four wavefronts, which that chose,
+	 * 5.5 with one).  The tiles of 64 x 64, whose products are of bf16 pieces, to 260 layers (6 %), and
+	 * 6 % and 0.6 us more than that: then none of the 43 that get them is slower than with what it got before (1.28 times as fast on average; without
+	 * that 56, four of them slower). */
+	inline constexpr Pace PACE_16[] = { { 4.99, 0.303, 0.107, 0.20 }, { 3.34, 0.409, 0.084, 0.90 }, { 2.64, 0.173, 0.091, 2.40 }, { 3.41, 0.88, 0.182, 1.86 } };
+	inline constexpr Pace PACE_32[] = { { 3.80, 0.647, 0.143, 0.37 }, { 3.19, 0.490, 0.149, 1.00 }, { 2.34, 0.162, 0.165, 2.98 }, { 4.34, 1.13, 0.371, 3.14 } };
+
+	/* The kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles: launch, a round of 512 workgroups (two to a compute unit), and
+	 * a k-step of one that has a compute unit to itself or shares it.  The last round, if it is of up to 256, goes at the pace of the former.
+	 * Microseconds, fitted to 448 layers (2000 to 130000 pixels, 16 to 512 channels and filters; root mean square error 6 to 13 %).  With every
+	 * round of the same length a 517th workgroup seemed to double the time: fp16 128 -> 128 3x3 on 129 images of 18 x 18 went to small tiles
+	 * and took 29.3 us, 25.5 in the image-tile kernel.  The image tiles' figures hold where filters fill blocks of 64 and channels 128 bytes; of 18 layers
+	 * where they do not, seven take 1.3 to 1.9 times as long (fp16 224 -> 112 3x3 on 79 x 26 x 26 28.5 : 49 us), and int8
+	 * layers up to a third longer (128 -> 128 on 128 x 20 x 20 10.1 : 13). */
+	struct TilePace
+	{
+		double launch, round, alone, shared;
+	};
+	enum TileKernel
+	{
+		IMAGE_TILES, GATHER, GATHER_BY_ELEMENTS, GATHER_ACTIVATION, GATHER_GENERAL
+	};
+	inline constexpr TilePace TILES_16[] = { { 0.0, 4.0, 0.42, 0.68 }, { 1.7, 7.7, 0.70, 0.90 }, { 0.0, 13.5, 0.69, 0.96 }, { 4.4, 15.9, 0.67, 0.88 } };
+	/* (fp32 in the gather kernel: products of bf16 pieces, 144 layers without a residual, 5 % with rounds of 9.2 us; not in its general instance, which takes an activation and filters in no whole
+	 * vectors at once) */
+	inline constexpr TilePace TILES_32[] = { { 3.0, 4.1, 1.94, 3.84 }, { 2.5, 11.5, 1.67, 2.50 }, { 0.3, 17.3, 1.67, 2.50 }, { 4.7, 18.0, 1.67, 2.50 }, { 4.7, 18.0, 2.07, 3.92 } };
+
+	inline double tile_kernel_us(const avhipConvShape &s, int element_bytes, int kernel)
+	{
+		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
+		const double steps = static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 127) / 128);
+		const TilePace &pace = (element_bytes == 4 ? TILES_32 : TILES_16)[kernel];
+		const double workgroups = kernel == IMAGE_TILES ? static_cast<double>(s.N) * ((s.K + 63) / 64) * ((s.Ho * s.Wo + 255) / 256)
+				: std::ceil(pixels / 128.0) * ((s.K + 127) / 128);
+		const double rounds = std::floor(workgroups / 512.0), rest = workgroups - 512.0 * rounds;
+		double us = pace.launch + rounds * (pace.round + pace.shared * steps);
+		if (rest > 0.0)
+			us += pace.round + (rest <= 256.0 ? pace.alone : pace.shared) * steps;
+		return us;
+	}
+
+	/* Tile and number of wavefronts by the estimates above.  Where the lines lie: 1 wavefront for thousands of tiles with a short k
+	 * (bf16 1x1, 107632 pixels, one stage: 13.8 us against 20.0 with four), 64 x 64 tiles where they alone fill the chip (bf16 256 ->
+	 * 256 on 3800 pixels: 13.8 us against 19.2), 8 wavefronts for few tiles and a long k (fp32, 40 tiles, 325 stages: 56 us against
+	 * 68), otherwise 4. */
+	inline SmallPlan conv_small_plan(const avhipConvShape &s, int element_bytes)
+	{
+		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
+		const double stages = std::ceil(static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 15) / 16) / 8.0);
+		SmallPlan best = { 0, 0, 0.0 };
+		for (int i = 0; i < 4; i++)
+		{
+			const int side = SMALL_TILE * PLANS[i].tiles;
+			const Pace &pace = element_bytes == 4 ? PACE_32[i] : PACE_16[i];
+			const double tiles = std::ceil(pixels / side) * ((s.K + side - 1) / side);
+			const double per_cu = tiles <= 1024.0 ? std::ceil(tiles / 256.0) : tiles / 256.0;
+			const double alone = std::ceil(stages / PLANS[i].waves) * pace.chain, shared = per_cu * stages * pace.stage;
+			const double us = pace.launch + (element_bytes == 4 ? std::hypot(alone, shared) : std::max(alone, shared)) + per_cu * pace.tile;
+			if (best.tiles == 0 || us < best.us)
+				best = { PLANS[i].tiles, PLANS[i].waves, us };
+		}
+		return best;
+	}
+}
+
+#endif /* AVHIP_CONV_ESTIMATES_HPP_ */

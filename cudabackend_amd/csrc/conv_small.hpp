@@ -5,6 +5,7 @@
 #define AVHIP_CONV_SMALL_HPP_
 
 #include "conv_epilogue.hpp"
+#include "conv_estimates.hpp"
 #include "conv_pointwise.hpp"
 
 namespace avhip
@@ -49,15 +50,8 @@ namespace avhip
 		return static_cast<int64_t>(s.C) * element_bytes < 64 && s.R * s.S > 1;
 	}
 
-	/* tiles x tiles MFMA tiles of 32 x 32, `waves` wavefronts sharing the k range, and the estimated microseconds */
-	struct SmallPlan
-	{
-		int tiles, waves;
-		double us;
-	};
 	int conv_small_threshold(); /* what avhip_set_small_problem_threshold set */
 	bool conv_small_possible(const avhipConvShape &s, int element_bytes); /* taps and chunks of a tap within the kernel's arithmetic */
-	SmallPlan conv_small_plan(const avhipConvShape &s, int element_bytes);
 	/* How results leave: LINEAR or RELU in whole aligned vectors of four filters; those activations element by element; any activation */
 	enum class HandOver
 	{
