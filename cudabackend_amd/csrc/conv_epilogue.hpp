@@ -20,6 +20,9 @@ namespace avhip
 	 * and select. */
 	constexpr int ACT_SIMPLE = -2;
 	constexpr int ACT_ANY = -1;
+	/* any activation of floating tensors in whole aligned vectors: the residual is requested ahead as for ACT_SIMPLE and the activation chosen once for all values of a tile that a
+	 * work-item holds (FloatEpilogue::before_activation, activate_run, after_activation) */
+	constexpr int ACT_VECTORS = -3;
 	__host__ inline bool is_simple_activation(int activation)
 	{
 		return activation == ACT_LINEAR || activation == ACT_RELU;
@@ -141,10 +144,10 @@ namespace avhip
 				t[q] = RELU ? __builtin_fmaxf(r, 0.0f) : r;
 			}
 		}
-		/* The arithmetic of store_at without its store.  `readable`: the run exists in y and z (callers that store
+		/* alpha1 * v + bias [+ alpha2 * z], with the ReLU of ACT_SIMPLE in it.  `readable`: the run exists in y and z (callers that store
 		 * unconditionally compute rows past the end of the tensor on zeros). */
 		template<int ACT, bool VEC, int W>
-		__device__ __forceinline__ void values(float (&t)[W], bool readable, int64_t idx, int k, const float (&v)[W], const ColumnsT<W> &c,
+		__device__ __forceinline__ void before_activation(float (&t)[W], bool readable, int64_t idx, int k, const float (&v)[W], const ColumnsT<W> &c,
 				const Residual<W> *fetched) const
 		{
 			const bool vec = VEC || this->vec;
@@ -181,21 +184,60 @@ namespace avhip
 				else
 					combine<false, false, W>(t, v, c, v);
 			}
-			if (ACT != ACT_SIMPLE)
-			{
-#pragma unroll
-				for (int q = 0; q < W; q++)
-					t[q] = activation_forward<float>(activation, t[q]);
-			}
+		}
+		/* + beta * y */
+		template<bool VEC, int W>
+		__device__ __forceinline__ void after_activation(float (&t)[W], bool readable, int64_t idx, int k) const
+		{
 			if (beta != 0.0f && readable)
 			{
 				float yv[W];
-				load_vec<TE, W, float>(y + idx, valid, yv, vec);
+				load_vec<TE, W, float>(y + idx, VEC ? W : K - k, yv, VEC || this->vec);
 #pragma unroll
 				for (int q = 0; q < W; q++)
 					t[q] += beta * yv[q];
 			}
 		}
+		/* The arithmetic of store_at without its store. */
+		template<int ACT, bool VEC, int W>
+		__device__ __forceinline__ void values(float (&t)[W], bool readable, int64_t idx, int k, const float (&v)[W], const ColumnsT<W> &c,
+				const Residual<W> *fetched) const
+		{
+			before_activation<ACT, VEC, W>(t, readable, idx, k, v, c, fetched);
+			if (ACT != ACT_SIMPLE)
+				activate_run<TE, W>(activation, t);
+			after_activation<VEC, W>(t, readable, idx, k);
+		}
+		/* N runs of a work-item in whole aligned vectors, any activation: `at`(n, idx) says whether run n exists and where it starts */
+		template<int N, int W, typename At>
+		__device__ __forceinline__ void store_runs(int k, const float (&v)[N][W], const ColumnsT<W> &c, const Residual<W> (&fetched)[N], const At &at) const
+		{
+			float t[N * W];
+#pragma unroll
+			for (int n = 0; n < N; n++)
+			{
+				float run[W];
+				before_activation<ACT_VECTORS, true, W>(run, false, 0, k, v[n], c, &fetched[n]);
+#pragma unroll
+				for (int q = 0; q < W; q++)
+					t[n * W + q] = run[q];
+			}
+			activate_run<TE, N * W>(activation, t);
+#pragma unroll
+			for (int n = 0; n < N; n++)
+			{
+				int64_t idx;
+				if (!at(n, idx))
+					continue;
+				float run[W];
+#pragma unroll
+				for (int q = 0; q < W; q++)
+					run[q] = t[n * W + q];
+				after_activation<true, W>(run, true, idx, k);
+				store_vec<TE, W, float, true>(y + idx, W, run, true);
+			}
+		}
+		static constexpr bool runs = true;
 		/* idx: element index of (pixel, filter k) in y and z, for callers that keep it cheaper than p * K + k */
 		template<int ACT, bool VEC = false, int W = 4>
 		__device__ __forceinline__ void store_at(int64_t idx, int k, const float (&v)[W], const ColumnsT<W> &c, const Residual<W> *fetched = nullptr) const
@@ -442,6 +484,7 @@ namespace avhip
 				words[part] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
 			}
 		}
+		static constexpr bool runs = false;
 		/* no unconditional hand-over of runs (FloatEpilogue::store_masked) here: measured on the 1x1 layer of config 4 it
 		 * made the int32-output kernel 5 % slower and left the requantising one unchanged */
 		static constexpr bool masked_stores = false;

@@ -103,7 +103,7 @@ namespace
 		constexpr int PITCH = T == 1 ? SIDE + 2 : SIDE + 1; /* 16-byte slots between two runs of a pixel: conflict-free both ways */
 		constexpr int SLOTS = QUADS * PITCH > 2 * SIDE * 8 ? QUADS * PITCH : 2 * SIDE * 8;
 		constexpr int DEPTH = T == 1 ? 2 : 1; /* stages in flight */
-		constexpr bool VEC = ACT == ACT_SIMPLE;
+		constexpr bool VEC = ACT != ACT_ANY;
 		constexpr bool BY_PIECES = std::is_same<TE, float>::value && T == 2; /* (with 32 x 32 the cutting costs what the products save) */
 		typedef typename Epi::scalar_t scalar_t;
 		typedef Pack<scalar_t, 4> quad_t;
@@ -363,11 +363,8 @@ namespace
 					part[(8 * i + 2 * v + half) * PITCH + 32 * j + r] = q;
 				}
 		__syncthreads();
-		auto hand_over = [&](int pass) __attribute__((always_inline))
+		auto sum_of = [&](int row) __attribute__((always_inline))
 		{
-			const int row = row0 + ROWS * pass;
-			if (ROWS > SIDE && row >= SIDE)
-				return;
 			quad_t v = reinterpret_cast<const quad_t*>(lds[0])[quad * PITCH + row];
 #pragma unroll
 			for (int k = 1; k < KW; k++)
@@ -377,10 +374,38 @@ namespace
 				for (int e = 0; e < 4; e++)
 					v.v[e] += o.v[e];
 			}
+			return v;
+		};
+		auto hand_over = [&](int pass) __attribute__((always_inline))
+		{
+			const int row = row0 + ROWS * pass;
+			if (ROWS > SIDE && row >= SIDE)
+				return;
+			const quad_t v = sum_of(row);
 			if (p0 + row < g.pixels && kcol < g.K)
 				epi.template store_at<ACT, VEC, 4>(static_cast<int64_t>(p0 + row) * g.K + kcol, kcol, v.v, columns, VEC ? &residual[VEC ? pass : 0] : nullptr);
 		};
-		if constexpr (ACT == ACT_SIMPLE)
+		if constexpr (ACT == ACT_VECTORS)
+		{
+			if (ROWS > SIDE && row0 >= SIDE)
+				return;
+			float v[PASSES][4];
+#pragma unroll
+			for (int pass = 0; pass < PASSES; pass++)
+			{
+				const quad_t q = sum_of(row0 + ROWS * pass);
+#pragma unroll
+				for (int e = 0; e < 4; e++)
+					v[pass][e] = q.v[e];
+			}
+			epi.store_runs(kcol, v, columns, residual, [&](int pass, int64_t &idx) __attribute__((always_inline))
+			{
+				const int p = p0 + row0 + ROWS * pass;
+				idx = static_cast<int64_t>(p) * g.K + kcol;
+				return p < g.pixels && kcol < g.K;
+			});
+		}
+		else if constexpr (ACT == ACT_SIMPLE)
 		{
 #pragma unroll
 			for (int pass = 0; pass < PASSES; pass++)
@@ -521,6 +546,8 @@ namespace avhip
 		{ \
 			if (simple) \
 				hipLaunchKernelGGL((k_conv_small<TE, Epi, T, KW, ACT_SIMPLE, ROW>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
+			else if (Epi::runs && epi.vec && choice.hand_over == HandOver::ACTIVATION) \
+				hipLaunchKernelGGL((k_conv_small<TE, Epi, T, KW, Epi::runs ? ACT_VECTORS : ACT_ANY, ROW>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
 			else \
 				hipLaunchKernelGGL((k_conv_small<TE, Epi, T, KW, ACT_ANY, ROW>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
 		} while (0)
