@@ -24,6 +24,7 @@ SOURCES = [
     "conv_implicit_gemm.hip",
     "conv_tile.hip",
     "conv_small.hip",
+    "conv_small16.hip",
     "conv_ring.hip",
     "conv_stem.hip",
     "conv_thin.hip",

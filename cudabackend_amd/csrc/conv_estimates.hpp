@@ -13,14 +13,18 @@
 
 namespace avhip
 {
-	/* tiles x tiles MFMA tiles of 32 x 32, `waves` wavefronts sharing the k range, and the estimated microseconds */
+	/* tiles of side x side, `waves` wavefronts sharing the k range, and the estimated microseconds */
 	struct SmallPlan
 	{
-		int tiles, waves;
+		int side, waves;
 		double us;
+		double larger_us; /* of the best without tiles of 16 x 16 */
 	};
-	inline constexpr int SMALL_TILE = 32; /* side of the MFMA tile */
-	inline constexpr SmallPlan PLANS[] = { { 1, 1, 0.0 }, { 1, 4, 0.0 }, { 1, 8, 0.0 }, { 2, 4, 0.0 } };
+	struct SmallTiling
+	{
+		int side, waves;
+	};
+	inline constexpr SmallTiling PLANS[] = { { 32, 1 }, { 32, 4 }, { 32, 8 }, { 64, 4 }, { 16, 1 }, { 16, 4 }, { 16, 8 } };
 
 	struct Pace
 	{
@@ -33,9 +37,12 @@ namespace avhip
 	 * on average and 15 % at most, with the larger of the two 1.2 % and 36 % (52 -> 408 1x1 on 637 pixels: 7.2 us with four wavefronts, which that chose,
 	 * 5.5 with one).  The tiles of 64 x 64, whose products are of bf16 pieces, to 260 layers (6 %), and
 	 * 6 % and 0.6 us more than that: then none of the 43 that get them is slower than with what it got before (1.28 times as fast on average; without
-	 * that 56, four of them slower). */
-	inline constexpr Pace PACE_16[] = { { 4.99, 0.303, 0.107, 0.20 }, { 3.34, 0.409, 0.084, 0.90 }, { 2.64, 0.173, 0.091, 2.40 }, { 3.41, 0.88, 0.182, 1.86 } };
-	inline constexpr Pace PACE_32[] = { { 3.80, 0.647, 0.143, 0.37 }, { 3.19, 0.490, 0.149, 1.00 }, { 2.34, 0.162, 0.165, 2.98 }, { 4.34, 1.13, 0.371, 3.14 } };
+	 * that 56, four of them slower).  The tiles of 16 x 16 (conv_small16.hip; the root of the sum of squares in every type) to 254 layers of up to 800 tiles of 32 x 32, 6 to 8 %, and taken
+	 * where they are 5 % below the others: of 224 layers they were not fitted to the plan chosen is 1.3 % slower than the best on average, 5 are slower than they were, by 13 % at most. */
+	inline constexpr Pace PACE_16[] = { { 4.99, 0.303, 0.107, 0.20 }, { 3.34, 0.409, 0.084, 0.90 }, { 2.64, 0.173, 0.091, 2.40 }, { 3.41, 0.88, 0.182, 1.86 },
+			{ 2.75, 0.171, 0.043, 0.09 }, { 2.81, 0.144, 0.041, 0.205 }, { 2.31, 0.228, 0.035, 0.73 } };
+	inline constexpr Pace PACE_32[] = { { 3.80, 0.647, 0.143, 0.37 }, { 3.19, 0.490, 0.149, 1.00 }, { 2.34, 0.162, 0.165, 2.98 }, { 4.34, 1.13, 0.371, 3.14 },
+			{ 2.91, 0.280, 0.069, 0.05 }, { 2.83, 0.217, 0.060, 0.275 }, { 2.65, 0.260, 0.058, 0.52 } };
 
 	/* The kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles: launch, a round of 512 workgroups (two to a compute unit), and
 	 * a k-step of one that has a compute unit to itself or shares it.  The last round, if it is of up to 256, goes at the pace of the former.
@@ -74,22 +81,23 @@ namespace avhip
 	/* Tile and number of wavefronts by the estimates above.  Where the lines lie: 1 wavefront for thousands of tiles with a short k
 	 * (bf16 1x1, 107632 pixels, one stage: 13.8 us against 20.0 with four), 64 x 64 tiles where they alone fill the chip (bf16 256 ->
 	 * 256 on 3800 pixels: 13.8 us against 19.2), 8 wavefronts for few tiles and a long k (fp32, 40 tiles, 325 stages: 56 us against
-	 * 68), otherwise 4. */
+	 * 68), otherwise 4.  Tiles of 16 x 16 where those of 32 x 32 are few: from some 300 (five stages: 600) on those load less, 10.1 against 10.8 us for bf16 128 -> 128 3x3 with 572. */
 	inline SmallPlan conv_small_plan(const avhipConvShape &s, int element_bytes)
 	{
 		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
 		const double stages = std::ceil(static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 15) / 16) / 8.0);
-		SmallPlan best = { 0, 0, 0.0 };
-		for (int i = 0; i < 4; i++)
+		SmallPlan best = { 0, 0, 0.0, 0.0 };
+		const int plans = static_cast<int64_t>(s.C) * element_bytes % 16 == 0 ? 7 : 4; /* the tiles of 16 x 16 are of whole chunks */
+		for (int i = 0; i < plans; i++)
 		{
-			const int side = SMALL_TILE * PLANS[i].tiles;
+			const int side = PLANS[i].side;
 			const Pace &pace = element_bytes == 4 ? PACE_32[i] : PACE_16[i];
 			const double tiles = std::ceil(pixels / side) * ((s.K + side - 1) / side);
 			const double per_cu = tiles <= 1024.0 ? std::ceil(tiles / 256.0) : tiles / 256.0;
 			const double alone = std::ceil(stages / PLANS[i].waves) * pace.chain, shared = per_cu * stages * pace.stage;
-			const double us = pace.launch + (element_bytes == 4 ? std::hypot(alone, shared) : std::max(alone, shared)) + per_cu * pace.tile;
-			if (best.tiles == 0 || us < best.us)
-				best = { PLANS[i].tiles, PLANS[i].waves, us };
+			const double us = pace.launch + (element_bytes == 4 || side == 16 ? std::sqrt(alone * alone + shared * shared) : std::max(alone, shared)) + per_cu * pace.tile;
+			if (best.side == 0 || us < (side == 16 && best.side != 16 ? 0.95 : 1.0) * best.us)
+				best = { side, PLANS[i].waves, us, side == 16 ? best.larger_us : us };
 		}
 		return best;
 	}

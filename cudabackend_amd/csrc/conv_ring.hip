@@ -410,13 +410,16 @@ namespace
 		 * Of 140 layers of 8 to 64 filters 32 leave the ring for that, 15 of them 2 to 24 % slower in it (fp16 512 -> 13 1x1 on 187 x 10 x 11 7.7 : 10.2 us, bf16 400 -> 10
 		 * 3x3 on 94 x 30 x 30 58 : 70.5), the others 11 % faster at most; of 70 that the rule was not made from 32, 0.70 to 1.16 times as fast in
 		 * it and 0.97 on average, where the 38 that stay are 1.10 times as fast.  8-bit layers stay (25 of them 1.02 times as fast in the ring). */
-		const double others = element_bytes == 2 && small.preferred && s.K < 32 ? (0.75 + 0.25 / 32.0 * s.K) * small.us : small.us;
+		const double others = element_bytes == 2 && small.larger_preferred && s.K < 32 ? (0.75 + 0.25 / 32.0 * s.K) * small.larger_us : small.larger_us;
 		const double limit = 0.85 * others, stages = std::ceil(static_cast<double>(s.R) * s.S * (s.C * element_bytes / 16) / 8.0);
 		/* one workgroup takes longer than that, whatever its tile: the smallest layers, whose calls cost the host no less than the GPU */
 		if (ring_at_least_us(stages) >= limit)
 			return none;
 		const RingChoice choice = ring_choice(s, stages, out_bytes, small.hand_over, residual);
-		return choice.us < limit ? choice : none;
+		if (choice.us >= limit)
+			return none;
+		/* Tiles of 16 x 16 take what they are estimated to do in 0.69 of the time or less: 1x1 layers of two stages and less whose rows are few to a tile of either side. */
+		return small.preferred && small.plan.side == 16 && small.us < 0.69 * choice.us ? none : choice;
 	}
 }
 

@@ -1,7 +1,7 @@
 /*
  * conv_small.hip -- implicit-GEMM convolution for problems that do not fill the chip with 128 x 128 workgroup tiles.
  *
- * The GEMM (rows = output pixels, columns = filters, k = (tap, channel)) is cut into tiles of 32 x 32 or 64 x 64 and the k range
+ * The GEMM (rows = output pixels, columns = filters, k = (tap, channel)) is cut into tiles of 32 x 32 or 64 x 64 (of 16 x 16: conv_small16.hip) and the k range
  * of a tile is shared by the one, four or eight wavefronts of a workgroup, so that a layer of a few hundred pixels still occupies
  * the chip; the partial tiles are added through LDS in a fixed order.  There is no barrier in the k loop: each wavefront loads its
  * own operands, 128 bytes of k of every row at a time, eight lanes to a row, and brings them into MFMA layout through its own
@@ -32,17 +32,6 @@
 namespace
 {
 	using namespace avhip;
-
-	struct SmallGeom
-	{
-		int H, W, C, K, R, S, Ho, Wo, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, flip;
-		int chunks_per_tap; /* 16-byte chunks of the channels of one tap */
-		unsigned int by_chunks, by_s; /* ceil(2^32 / chunks_per_tap), ceil(2^16 / S): division by multiplication */
-		int pixels, images;
-		unsigned int pixel_tiles, filter_tiles;
-		Divisor by_wo, by_ho, by_tiles; /* by_tiles: of the faster of the two */
-		int pixels_first; /* order of the tiles: pixel tiles run fastest within an XCD (more weights than image), or filter tiles */
-	};
 
 	/* LDS accesses of a wavefront to its own part stay in this order (the hardware does them in order, without a barrier) */
 	__device__ __forceinline__ void wave_order()
@@ -97,7 +86,7 @@ namespace
 	__global__ __launch_bounds__(64 * KW, KW == 8 ? 2 : T == 1 ? 3 : 2) void k_conv_small(const TE *__restrict__ x, const TE *__restrict__ w, SmallGeom g, Epi epi)
 	{
 		constexpr unsigned int SZ = sizeof(TE);
-		constexpr int SIDE = SMALL_TILE * T;
+		constexpr int SIDE = 32 * T;
 		constexpr int LOADS = 4 * T; /* loads of 8 rows each, per operand and stage */
 		constexpr int QUADS = SIDE / 4; /* runs of four filters of a pixel */
 		constexpr int PITCH = T == 1 ? SIDE + 2 : SIDE + 1; /* 16-byte slots between two runs of a pixel: conflict-free both ways */
@@ -475,23 +464,28 @@ namespace avhip
 	}
 	SmallChoice conv_small_choice(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
 	{
-		SmallChoice choice = { hand_over, one_tap_us, false, { 0, 0, 0.0 }, 0.0 };
+		SmallChoice choice = { hand_over, one_tap_us, false, { 0, 0, 0.0, 0.0 }, 0.0, false, 0.0 };
 		if (!conv_small_possible(s, element_bytes))
 			return choice;
 		choice.plan = conv_small_plan(s, element_bytes);
 		const int threshold = conv_small_threshold();
 		if (threshold < 0) /* asked for by name (tests): whatever the kernel can run */
-			choice.preferred = true;
+			choice.preferred = choice.larger_preferred = true;
 		else if (!whole_chunks(s, element_bytes)) /* otherwise the general gather kernel, element by element: 2.2 to 17 times slower on all of 14 layers of 1152 to 627200 pixels */
-			choice.preferred = threshold != 0;
+			choice.preferred = choice.larger_preferred = threshold != 0;
 		else
 		{
-			choice.us = workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
+			choice.us = choice.larger_us = workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
 			const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
-			choice.preferred = tiles < threshold && small_factor(element_bytes, hand_over, one_tap_us) * choice.plan.us < choice.us;
+			const double limit = tiles < threshold ? choice.us / small_factor(element_bytes, hand_over, one_tap_us) : 0.0;
+			choice.preferred = choice.plan.us < limit;
+			choice.larger_preferred = choice.plan.larger_us < limit;
 		}
+		const double factor = small_factor(element_bytes, hand_over, 0.0);
 		if (choice.preferred)
-			choice.us = small_factor(element_bytes, hand_over, 0.0) * choice.plan.us;
+			choice.us = factor * choice.plan.us;
+		if (choice.larger_preferred)
+			choice.larger_us = factor * choice.plan.larger_us;
 		return choice;
 	}
 	bool conv_gather_before_image_tiles(const avhipConvShape &s)
@@ -508,39 +502,18 @@ namespace avhip
 		const bool simple = choice.hand_over == HandOver::PLAIN;
 		if (!choice.preferred || in_place(s, x, SZ, epi.y, Epi::out_bytes))
 			return false;
-		const int side = SMALL_TILE * plan.tiles;
+		const int side = plan.side;
 		const int64_t pixel_tiles = (pixels + side - 1) / side, filter_tiles = (static_cast<int64_t>(s.K) + side - 1) / side;
 		if (pixel_tiles * 64 * plan.waves >= (1ll << 32) /* work-items of a launch along one direction */ || filter_tiles > 65535
 				|| pixel_tiles * filter_tiles > 0x7FFFFFFFll || pixels >= (1ll << 31) - side)
 			return false;
-		SmallGeom g;
-		g.H = s.H;
-		g.W = s.W;
-		g.C = s.C;
-		g.K = s.K;
-		g.R = s.R;
-		g.S = s.S;
-		g.Ho = s.Ho;
-		g.Wo = s.Wo;
-		g.pad_h = s.pad_h;
-		g.pad_w = s.pad_w;
-		g.stride_h = s.stride_h;
-		g.stride_w = s.stride_w;
-		g.dil_h = s.dil_h;
-		g.dil_w = s.dil_w;
-		g.flip = s.mode != 0 ? 1 : 0;
-		g.chunks_per_tap = (s.C * SZ + 15) / 16;
-		g.by_chunks = static_cast<unsigned int>(((1ll << 32) + g.chunks_per_tap - 1) / g.chunks_per_tap); /* 1: unused */
-		g.by_s = (65536 + s.S - 1) / s.S;
-		g.pixels = static_cast<int>(pixels);
-		g.images = s.N;
-		g.pixels_first = static_cast<int64_t>(s.K) * s.R * s.S > static_cast<int64_t>(s.N) * s.H * s.W ? 1 : 0;
-		g.pixel_tiles = static_cast<unsigned int>(pixel_tiles);
-		g.filter_tiles = static_cast<unsigned int>(filter_tiles);
-		g.by_wo = divisor(s.Wo);
-		g.by_ho = divisor(s.Ho);
-		g.by_tiles = divisor(g.pixels_first ? g.pixel_tiles : g.filter_tiles);
+		const SmallGeom g = small_geometry(s, SZ, pixel_tiles, filter_tiles);
 		const dim3 grid(g.pixel_tiles, g.filter_tiles);
+		if (side == 16)
+		{
+			conv_small16_launch<TE, Epi>(stream, grid, plan.waves, x, w, g, epi, choice.hand_over);
+			return true;
+		}
 #define AVHIP_SMALL_PLAN(T, KW, ROW) \
 		do \
 		{ \
@@ -554,7 +527,7 @@ namespace avhip
 #define AVHIP_SMALL(ROW) \
 		do \
 		{ \
-			if (plan.tiles == 2) \
+			if (side == 64) \
 				AVHIP_SMALL_PLAN(2, 4, ROW); \
 			else if (plan.waves == 8) \
 				AVHIP_SMALL_PLAN(1, 8, ROW); \
@@ -592,7 +565,7 @@ namespace avhip
 #undef AVHIP_INSTANTIATE
 }
 
-/* The tile that a layer of more than one tap (of fp32, or one that the ring kernel leaves alone) gets in this kernel: MFMA tiles of 32 x 32 a side times 16
+/* The tile that a layer of more than one tap (of fp32, or one that the ring kernel leaves alone) gets in this kernel: half of its side
  * plus wavefronts, or 0 where it goes to another.  `hand_over`: HandOver.  Exported so that a test can ask which instance it is about to run. */
 extern "C" AVHIP_API int avhip_conv2d_small_plan(int x_dtype, const avhipConvShape *shape, int hand_over)
 {
@@ -600,5 +573,5 @@ extern "C" AVHIP_API int avhip_conv2d_small_plan(int x_dtype, const avhipConvSha
 		return 0;
 	const int element_bytes = x_dtype == DT_INT8 ? 1 : x_dtype == DT_FLOAT32 ? 4 : 2;
 	const SmallChoice choice = conv_small_choice(*shape, element_bytes, static_cast<HandOver>(hand_over), 0.0);
-	return choice.preferred ? 16 * choice.plan.tiles + choice.plan.waves : 0;
+	return choice.preferred ? choice.plan.side / 2 + choice.plan.waves : 0;
 }
