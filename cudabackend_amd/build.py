@@ -36,7 +36,7 @@ SOURCES = [
     "conv_pointwise_block.hip",
     "elementwise.hip",
 ]
-HEADERS = ["common.hpp", "mfma_core.hpp", "conv_epilogue.hpp", "conv_tile.hpp", "conv_small.hpp", "conv_estimates.hpp", "conv_ring.hpp", "conv_ring_plan.hpp", "conv_stem.hpp", "conv_thin.hpp", "conv_winograd_f4.hpp", "conv_pointwise.hpp", "gemm_tn.hpp", "persistent_gemm.hpp", "resident_gemm.hpp", "../../include/avocado_hip_kernels.h", "../../include/avocado_hip_backend.h",
+HEADERS = ["common.hpp", "mfma_core.hpp", "conv_epilogue.hpp", "conv_tile.hpp", "conv_small.hpp", "conv_small_rows.hpp", "conv_estimates.hpp", "conv_ring.hpp", "conv_ring_plan.hpp", "conv_stem.hpp", "conv_thin.hpp", "conv_winograd_f4.hpp", "conv_pointwise.hpp", "gemm_tn.hpp", "persistent_gemm.hpp", "resident_gemm.hpp", "../../include/avocado_hip_kernels.h", "../../include/avocado_hip_backend.h",
            "../../include/avocado_backend_defs.h"]
 
 FLAGS = ["-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

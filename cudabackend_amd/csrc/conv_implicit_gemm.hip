@@ -630,13 +630,23 @@ namespace
 		const double rounds = std::ceil(pixels / BLOCK_M) * ((s.K + BLOCK_N - 1) / BLOCK_N) / 256.0;
 		return p.launch + std::max(p.chain * steps, rounds * p.step * steps) + rounds * p.tile + p.megabyte * pixels * s.K * element_bytes * 1.0e-6 * (residual ? 2.0 : 1.0);
 	}
-	/* Whether small tiles take a layer from the packed gather (pieces of `piece` bytes, 0: it cannot run it); int8 layers always.  Rows of
-	 * elements cost them a quarter more than their estimate, which is one of whole chunks. */
+	/* Whether small tiles take a layer from the packed gather (pieces of `piece` bytes, 0: it cannot run it); int8 layers always. */
 	bool small_before_packed(const avhipConvShape &s, int element_bytes, int piece, bool residual)
 	{
 		if (piece == 0 || element_bytes == 1 || conv_small_threshold() < 0)
 			return true;
-		return conv_small_plan(s, element_bytes).us * (piece == 2 ? 1.25 : 1.0) < 0.95 * packed_us(s, element_bytes, piece, residual);
+		return conv_small_plan(s, element_bytes).us < 0.95 * packed_us(s, element_bytes, piece, residual);
+	}
+
+	/* Layers of few channels that tiles of 16 x 16 take from the kernels made for them: those take 4.0 to 4.9 us (pixels of 8 bytes, at most 12 taps), 5.9 to 9.3 (16-bit types), 7.4 and more
+	 * (int8) and 8.3 to 15 (fp32) however few their pixels are; 76 layers of up to 1200 tiles of 32 x 32: fp32 2.6 times as fast (4 -> 192 3x3 on 6 x 11 x 11 9.6 : 3.2 us), 16-bit 1.7 and 1.3 times, none slower. */
+	bool small_before_few_channels(const avhipConvShape &s, int element_bytes)
+	{
+		if (conv_small_threshold() <= 0 || !conv_small_possible(s, element_bytes))
+			return false;
+		const SmallPlan plan = conv_small_plan(s, element_bytes);
+		const bool stem = s.C * element_bytes == 8 && element_bytes < 4 && s.R * s.S <= 12;
+		return plan.side == 16 && plan.us < (stem ? 4.2 : element_bytes == 4 ? 7.5 : element_bytes == 2 ? 5.5 : 6.5);
 	}
 
 	template<typename TE, typename Epi>
@@ -661,6 +671,8 @@ namespace
 		if (conv_few_channels(s, static_cast<int>(sizeof(TE))) && fast_path_ok<TE>(s, 1, padding_value, false) && is_simple_activation(epi.activation)
 				&& (flags & 2) != 0)
 		{
+			if ((ragged || fast_path_ok<TE>(s, flags, padding_value)) && small_before_few_channels(s, sizeof(TE)) && conv_small_launch<TE, Epi>(st, s, x, w, epi, conv_small_choice<TE>(s, epi)))
+				return 0;
 			/* a pixel of exactly 8 bytes and a small filter: operands straight into registers, no k loop */
 			if (conv_stem_launch<TE, Epi>(st, s, x, w, epi))
 				return 0;

@@ -398,7 +398,7 @@ namespace
 		if (small.hand_over == HandOver::PLAIN && conv_few_channels(s, element_bytes))
 			return none;
 		/* (the switch of the small tiles is this kernel's too: at 0 the kernels with fixed tiles of 128 x 128 are asked for, below it small ones) */
-		if (element_bytes > 2 || static_cast<int64_t>(s.C) * element_bytes % 16 != 0 || !conv_small_possible(s, element_bytes) || conv_small_threshold() <= 0)
+		if (element_bytes > 2 || static_cast<int64_t>(s.C) * element_bytes % 16 != 0 || s.C * element_bytes < 32 || !conv_small_possible(s, element_bytes) || conv_small_threshold() <= 0)
 			return none;
 		/* of 8-bit one-tap layers the persistent kernels are a fifth to a third faster than they are estimated (17 layers) */
 		if (element_bytes == 1 && small.one_tap_us > 0.0)

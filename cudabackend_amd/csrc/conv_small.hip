@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "conv_small.hpp"
+#include "conv_small_rows.hpp"
 #include "mfma_core.hpp"
 
 namespace
@@ -37,48 +38,6 @@ namespace
 	__device__ __forceinline__ void wave_order()
 	{
 		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-	}
-
-	/* What the rows of channels (one pixel, one tap of a filter) are known to be: whole 16-byte chunks; dwords; elements. */
-	constexpr int ROWS_OF_CHUNKS = 0, ROWS_OF_DWORDS = 1, ROWS_OF_ELEMENTS = 2;
-
-	/* 16 bytes on their way from memory, from any byte on if ROW is ROWS_OF_ELEMENTS: then they are the aligned dwords around them */
-	template<int ROW>
-	struct Piece
-	{
-		uint4 u;
-		__device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t rsrc, unsigned int offset)
-		{
-			u = buffer_fetch(rsrc, offset);
-		}
-		/* what belongs to the row: `left` bytes of it from the first one on */
-		__device__ __forceinline__ uint4 get(unsigned int, const uint4 &keep) const
-		{
-			if (ROW == ROWS_OF_CHUNKS)
-				return u;
-			return make_uint4(u.x & keep.x, u.y & keep.y, u.z & keep.z, u.w & keep.w);
-		}
-	};
-	template<>
-	struct Piece<ROWS_OF_ELEMENTS>
-	{
-		uint4 u;
-		unsigned int next;
-		__device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t rsrc, unsigned int offset)
-		{
-			u = buffer_fetch(rsrc, offset & ~3u);
-			next = __builtin_amdgcn_raw_buffer_load_b32(rsrc, static_cast<int>((offset & ~3u) + 16), 0, 0);
-		}
-		__device__ __forceinline__ uint4 get(unsigned int offset, const uint4 &keep) const
-		{
-			return make_uint4(__builtin_amdgcn_alignbyte(u.y, u.x, offset & 3) & keep.x, __builtin_amdgcn_alignbyte(u.z, u.y, offset & 3) & keep.y,
-					__builtin_amdgcn_alignbyte(u.w, u.z, offset & 3) & keep.z, __builtin_amdgcn_alignbyte(next, u.w, offset & 3) & keep.w);
-		}
-	};
-	/* which bits of a dword belong to a row that has `left` more bytes */
-	__device__ __forceinline__ unsigned int keep_bits(int left)
-	{
-		return left >= 4 ? ~0u : left <= 0 ? 0u : (1u << (8 * left)) - 1;
 	}
 
 	/* T x T MFMA tiles of 32 x 32 per wavefront, KW wavefronts on one tile. */
@@ -454,7 +413,7 @@ namespace avhip
 	bool conv_small_possible(const avhipConvShape &s, int element_bytes)
 	{
 		const int64_t chunks = (static_cast<int64_t>(s.C) * element_bytes + 15) / 16;
-		return s.R * s.S <= 32 && (chunks >= 2 || !whole_chunks(s, element_bytes)) && chunks <= 8192;
+		return s.R * s.S <= 32 && chunks <= 8192;
 	}
 	/* The small tiles' estimates are of the plain hand-over; the others cost them up to a fifth of the whole.  Against the one-tap kernels, whose
 	 * estimate is the coarsest, they have to be 5 % below. */
@@ -479,7 +438,7 @@ namespace avhip
 			const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
 			const double limit = tiles < threshold ? choice.us / small_factor(element_bytes, hand_over, one_tap_us) : 0.0;
 			choice.preferred = choice.plan.us < limit;
-			choice.larger_preferred = choice.plan.larger_us < limit;
+			choice.larger_preferred = choice.plan.larger_us > 0.0 && choice.plan.larger_us < limit;
 		}
 		const double factor = small_factor(element_bytes, hand_over, 0.0);
 		if (choice.preferred)

@@ -122,7 +122,7 @@ namespace avhip
 		const HandOver hand_over = !simple ? HandOver::ACTIVATION : epi.vec ? HandOver::PLAIN : HandOver::ELEMENTS;
 		return conv_small_choice(s, static_cast<int>(sizeof(TE)), hand_over, hand_over == HandOver::PLAIN ? conv_pointwise_us<TE>(s, epi) : 0.0);
 	}
-	/* The kernel of 16 x 16 tiles (conv_small16.hip), for conv_small_launch: channels of whole 16-byte chunks. */
+	/* The kernel of 16 x 16 tiles (conv_small16.hip), for conv_small_launch. */
 	template<typename TE, typename Epi>
 	void conv_small16_launch(hipStream_t stream, const dim3 &grid, int waves, const void *x, const void *w, const SmallGeom &g, const Epi &epi, HandOver hand_over);
 	/* Launches the kernel and returns true where it is preferred; returns false without side effects otherwise.  The caller has established the conditions of

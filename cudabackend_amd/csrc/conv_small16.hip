@@ -9,9 +9,12 @@
  * What bounds it now: the latency of one load, the sums and the launch, 2.8 us of them for a layer of one stage.
  * Measured, before (tiles of 32 x 32) and now: that layer 6.3 -> 4.0 us, bf16 256 -> 256 3x3 on 9 x 10 x 10 8.1 -> 6.0, fp32 64 -> 64 3x3 on 8 x 15 x 15 8.2 -> 4.4, fp32 128 -> 128 on
  * 512 pixels 11.5 -> 5.9, int8 1x1 48 -> 48 on 320 pixels 3.6 -> 2.7; of 470 layers of up to 1500 tiles of 32 x 32 the mean is 1.19 times as fast in 16 bits and 1.3 in fp32.
+ * Rows of dwords and elements (any number of channels) against tiles of 32 x 32: bf16 97 -> 32 3x3 stride 2 on 360 pixels 6.9 -> 4.2 us, fp32 133 -> 32 3x3 on 640 12.0 -> 6.8; few channels against
+ * the kernels made for them: fp32 4 -> 128 3x3 on 6 x 11 x 11 9.3 -> 3.0, fp16 8 -> 80 3x3 on 860 pixels 6.3 -> 3.3, bf16 4 -> 128 on 512 4.3 -> 3.3.
  * Three or four stages in flight and sixteen wavefronts were not faster, two wavefronts in no layer by more than 5 %.
  */
 #include "conv_small.hpp"
+#include "conv_small_rows.hpp"
 #include "mfma_core.hpp"
 
 namespace
@@ -58,7 +61,7 @@ namespace
 	};
 
 	/* KW wavefronts on one tile */
-	template<typename TE, typename Epi, int KW, int ACT>
+	template<typename TE, typename Epi, int KW, int ACT, int ROW>
 	__global__ __launch_bounds__(64 * KW, 4) void k_conv_small16(const TE *__restrict__ x, const TE *__restrict__ w, SmallGeom g, Epi epi)
 	{
 		constexpr unsigned int SZ = sizeof(TE);
@@ -80,8 +83,8 @@ namespace
 		const int p0 = static_cast<int>(pixel_tile) * SIDE, k0 = static_cast<int>(filter_tile) * SIDE;
 
 		const unsigned int c_bytes = g.C * SZ, filter_bytes = g.R * g.S * c_bytes;
-		const __amdgpu_buffer_rsrc_t rx = make_buffer(x, static_cast<unsigned int>(g.images) * g.H * g.W * c_bytes);
-		const __amdgpu_buffer_rsrc_t rw = make_buffer(w, static_cast<unsigned int>(g.K) * filter_bytes);
+		const __amdgpu_buffer_rsrc_t rx = make_buffer(x, (static_cast<unsigned int>(g.images) * g.H * g.W * c_bytes + 3) & ~3u); /* a dword never crosses a page */
+		const __amdgpu_buffer_rsrc_t rw = make_buffer(w, (static_cast<unsigned int>(g.K) * filter_bytes + 3) & ~3u);
 
 		/* k = the 16-byte chunks of (tap, channel) in a row, eight a stage; each wavefront takes a contiguous share of the stages.  This lane loads chunk
 		 * (lane % 8) of the rows 8 i + lane / 8. */
@@ -95,15 +98,29 @@ namespace
 		const unsigned int chunks_mine = count > 0 ? (chunks < 8 * (first + count) ? chunks : 8 * (first + count)) : 0;
 		struct Stage
 		{
-			uint4 xs[2], ws[2];
+			Piece<ROW> xs[2], ws[2];
+			unsigned int x_tap, w_at; /* not whole chunks: where the pieces start (the lowest two bits are used) */
+			int left; /* and the bytes of the row from there */
 		};
 		Stage stage[DEPTH];
 		unsigned int w_chunk = 8 * first + load_chunk, x_chunk = w_chunk;
+		auto tap_of = [&](unsigned int chunk) __attribute__((always_inline))
+		{
+			return g.chunks_per_tap == 1 ? chunk : __umulhi(chunk, g.by_chunks); /* (one chunk a tap: the factor would be 2^32) */
+		};
 		auto fetch_w = [&](Stage &to) __attribute__((always_inline))
 		{
+			unsigned int at = w_origin + 16 * w_chunk;
+			if (ROW != ROWS_OF_CHUNKS)
+			{
+				const unsigned int tap = tap_of(w_chunk), c = w_chunk - tap * g.chunks_per_tap;
+				at = w_origin + tap * c_bytes + 16 * c;
+				to.w_at = at;
+				to.left = static_cast<int>(c_bytes - 16 * c);
+			}
 #pragma unroll
 			for (int q = 0; q < 2; q++)
-				to.ws[q] = buffer_fetch(rw, w_chunk < chunks_mine ? w_origin + 16 * w_chunk + 8 * q * filter_bytes : OUT_OF_RANGE);
+				to.ws[q].fetch(rw, w_chunk < chunks_mine ? at + 8 * q * filter_bytes : OUT_OF_RANGE);
 			w_chunk += 8;
 		};
 		/* the filters' operands are on their way while the pixels' addresses are worked out */
@@ -127,17 +144,18 @@ namespace
 		}
 		auto fetch_x = [&](Stage &to) __attribute__((always_inline))
 		{
-			const unsigned int tap = __umulhi(x_chunk, g.by_chunks);
-			const unsigned int c = x_chunk - tap * g.chunks_per_tap;
+			const unsigned int tap = tap_of(x_chunk), c = x_chunk - tap * g.chunks_per_tap;
 			const unsigned int ti = (tap * g.by_s) >> 16, tj = tap - ti * g.S;
 			const int i = static_cast<int>(g.flip ? g.R - 1 - ti : ti) * g.dil_h, j = static_cast<int>(g.flip ? g.S - 1 - tj : tj) * g.dil_w;
 			const unsigned int x_tap = static_cast<unsigned int>(i * g.W + j) * c_bytes + 16 * c;
+			if (ROW != ROWS_OF_CHUNKS)
+				to.x_tap = x_tap;
 #pragma unroll
 			for (int q = 0; q < 2; q++)
 			{
 				const bool inside = x_chunk < chunks_mine && static_cast<unsigned int>(ih0[q] + i) < static_cast<unsigned int>(g.H)
 						&& static_cast<unsigned int>(iw0[q] + j) < static_cast<unsigned int>(g.W);
-				to.xs[q] = buffer_fetch(rx, inside ? origin[q] + x_tap : OUT_OF_RANGE);
+				to.xs[q].fetch(rx, inside ? origin[q] + x_tap : OUT_OF_RANGE);
 			}
 			x_chunk += 8;
 		};
@@ -165,11 +183,15 @@ namespace
 		typename Mma16<TE>::acc_t acc = { 0, 0, 0, 0 };
 		auto bring = [&](const Stage &from) __attribute__((always_inline))
 		{
+			/* both operands, so that what lies behind a row (an infinity of the next pixel or tap) counts as nothing */
+			uint4 keep = make_uint4(0, 0, 0, 0);
+			if (ROW != ROWS_OF_CHUNKS)
+				keep = make_uint4(keep_bits(from.left), keep_bits(from.left - 4), keep_bits(from.left - 8), keep_bits(from.left - 12));
 #pragma unroll
 			for (int q = 0; q < 2; q++)
 			{
-				mine[64 * q + (q ? put ^ 4 : put)] = from.xs[q];
-				mine[8 * SIDE + 64 * q + (q ? put ^ 4 : put)] = from.ws[q];
+				mine[64 * q + (q ? put ^ 4 : put)] = from.xs[q].get(origin[q] + from.x_tap, keep);
+				mine[8 * SIDE + 64 * q + (q ? put ^ 4 : put)] = from.ws[q].get(from.w_at + 8 * q * filter_bytes, keep);
 			}
 			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 		};
@@ -248,23 +270,42 @@ namespace avhip
 	template<typename TE, typename Epi>
 	void conv_small16_launch(hipStream_t stream, const dim3 &grid, int waves, const void *x, const void *w, const SmallGeom &g, const Epi &epi, HandOver hand_over)
 	{
-#define AVHIP_SMALL16(KW) \
+#define AVHIP_SMALL16_ACT(KW, ROW, ACT) hipLaunchKernelGGL((k_conv_small16<TE, Epi, KW, ACT, ROW>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi)
+#define AVHIP_SMALL16_WAVES(KW, ROW) \
 		do \
 		{ \
 			if (hand_over == HandOver::PLAIN) \
-				hipLaunchKernelGGL((k_conv_small16<TE, Epi, KW, ACT_SIMPLE>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
+				AVHIP_SMALL16_ACT(KW, ROW, ACT_SIMPLE); \
 			else if (Epi::runs && epi.vec && hand_over == HandOver::ACTIVATION) \
-				hipLaunchKernelGGL((k_conv_small16<TE, Epi, KW, Epi::runs ? ACT_VECTORS : ACT_ANY>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
+				AVHIP_SMALL16_ACT(KW, ROW, Epi::runs ? ACT_VECTORS : ACT_ANY); \
 			else \
-				hipLaunchKernelGGL((k_conv_small16<TE, Epi, KW, ACT_ANY>), grid, dim3(64 * KW), 0, stream, static_cast<const TE*>(x), static_cast<const TE*>(w), g, epi); \
+				AVHIP_SMALL16_ACT(KW, ROW, ACT_ANY); \
 		} while (0)
-		if (waves == 8)
-			AVHIP_SMALL16(8);
-		else if (waves == 4)
-			AVHIP_SMALL16(4);
-		else
-			AVHIP_SMALL16(1);
+#define AVHIP_SMALL16(ROW) \
+		do \
+		{ \
+			if (waves == 8) \
+				AVHIP_SMALL16_WAVES(8, ROW); \
+			else if (waves == 4) \
+				AVHIP_SMALL16_WAVES(4, ROW); \
+			else \
+				AVHIP_SMALL16_WAVES(1, ROW); \
+		} while (0)
+		constexpr int SZ = static_cast<int>(sizeof(TE));
+		if (g.C * SZ % 16 == 0)
+			AVHIP_SMALL16(ROWS_OF_CHUNKS);
+		else if (g.C * SZ % 4 == 0)
+		{
+			if constexpr (SZ >= 2)
+				AVHIP_SMALL16(ROWS_OF_DWORDS);
+			else
+				AVHIP_SMALL16(ROWS_OF_ELEMENTS);
+		}
+		else if constexpr (SZ <= 2)
+			AVHIP_SMALL16(ROWS_OF_ELEMENTS);
 #undef AVHIP_SMALL16
+#undef AVHIP_SMALL16_WAVES
+#undef AVHIP_SMALL16_ACT
 	}
 
 #define AVHIP_INSTANTIATE(TE, EPI) template void conv_small16_launch<TE, EPI>(hipStream_t, const dim3&, int, const void*, const void*, const SmallGeom&, const EPI&, HandOver);

@@ -68,6 +68,46 @@ def test_against_the_oracle(oracle, case, dtype, act, z):
     assert oracle.rel_l2(got, oracle.conv2d(x, w, b, res, activation=code, **geometry)) < BAR[dtype]
 
 
+# wavefronts; images, rows, columns, channels of each type (absent: no such row); filters, their rows and columns; the rest of the geometry.  Rows of channels that are no whole chunks
+# (dwords, elements), that are one chunk, that are less than one
+ROWS = [(1, (3, 7, 5), dict(f32=9, f16=18, bf16=1, i8=36), (18, 1, 1), {}), (8, (2, 9, 7), dict(f32=33, f16=66, bf16=65, i8=131), (20, 3, 3), dict(pad=(-1, -1))),
+        (8, (1, 5, 4), dict(f32=101, f16=201, bf16=203, i8=403), (33, 3, 5), dict(pad=(-1, -2), stride=(2, 1))), (1, (3, 8, 9), dict(f32=4, f16=8, bf16=8, i8=16), (40, 1, 1), {}),
+        (1, (20, 12, 9), dict(f32=4, f16=8, bf16=2, i8=16), (36, 3, 3), dict(pad=(-1, -1))), (1, (20, 12, 9), dict(f32=3, f16=3, bf16=4, i8=5), (64, 3, 3), dict(pad=(-1, -1), mode=1)),
+        (4, (9, 13, 12), dict(f32=2, f16=3, bf16=3, i8=3), (32, 5, 5), dict(pad=(-2, -2), stride=(2, 2)))]
+
+
+@pytest.mark.parametrize("act", ["RELU", "ELU"])  # few channels: RELU by estimate, before the kernels made for them; ELU as any layer
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16", "i8"])
+@pytest.mark.parametrize("case", range(len(ROWS)))
+def test_rows_of_channels(oracle, case, dtype, act):
+    waves, (N, H, W), channels, (K, R, S), geometry = ROWS[case]
+    Cin = channels[dtype]
+    lib = cb.load_library()
+    if act == "RELU":
+        if dtype == "i8":
+            pytest.skip("integer sums: with the other activation's name")
+        lib.avhip_set_small_problem_threshold(4096)
+    (ph, pw), (sh, sw) = geometry.get("pad", (0, 0)), geometry.get("stride", (1, 1))
+    ys = (N, (H - 2 * ph - R) // sh + 1, (W - 2 * pw - S) // sw + 1, K)
+    shape = Shape(N, H, W, Cin, K, R, S, ys[1], ys[2], ph, pw, sh, sw, 1, 1, geometry.get("mode", 0))
+    code = {"f32": cb.DTYPE_FLOAT32, "f16": cb.DTYPE_FLOAT16, "bf16": cb.DTYPE_BFLOAT16, "i8": cb.DTYPE_INT8}[dtype]
+    assert lib.avhip_conv2d_small_plan(code, C.byref(shape), 0) in [8 + n for n in ((1, 4, 8) if waves == 4 else (waves,))]
+    geometry = {"pad": (0, 0), **geometry}
+    g = h.rng(800 + case)
+    if dtype == "i8":
+        x, w = g.integers(-127, 128, (N, H, W, Cin), dtype=np.int8), g.integers(-127, 128, (K, R, S, Cin), dtype=np.int8)
+        b = g.integers(-2 ** 15, 2 ** 15, K).astype(np.int32)
+        got = h.conv_forward("implicit_gemm", x, w, ys, "i8", y_dtype="i32", bias=b, bias_dtype="i32", **geometry)
+        np.testing.assert_array_equal(got, oracle.conv2d_i8(x, w, b, **geometry))
+        return
+    x = h.rounded(oracle, g.standard_normal((N, H, W, Cin)), dtype)
+    w = h.rounded(oracle, g.standard_normal((K, R, S, Cin)) * np.sqrt(2.0 / (R * S * Cin)), dtype)
+    b = g.uniform(-0.1, 0.1, K).astype(np.float32).astype(np.float64)
+    code = getattr(cb, "ACTIVATION_" + act)
+    got = h.conv_forward("implicit_gemm", x, w, ys, dtype, bias=b, activation=code, **geometry)
+    assert oracle.rel_l2(got, oracle.conv2d(x, w, b, activation=code, **geometry)) < BAR[dtype]
+
+
 def test_an_infinity_stays_with_its_pixel_and_filter():
     """Pixels outside the image, filters past the last and shares of k past the end count as zeros, whatever lies behind the tensors."""
     x, w = np.ones((1, 5, 5, 32), np.float32), np.ones((18, 3, 3, 32), np.float32)
