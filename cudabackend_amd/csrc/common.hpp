@@ -219,6 +219,27 @@ namespace avhip
 		column_block = t - row_block * gridDim.y;
 	}
 
+	/* n / d for n below 2^31 by a multiplication: with 2^shift >= d and factor = ceil(2^(31 + shift) / d), n * factor / 2^(31 + shift) is too
+	 * large by less than 1 / d.  A division by a number that only the launch knows is a chain of some twenty dependent instructions,
+	 * and three of them in a row stood before the first load of a workgroup: bf16 3x3 48 -> 48 on 3600 pixels 5.0 us a call with them, 4.4 without,
+	 * 4.6 in the kernel of one wavefront per tile that this one replaced (towers of twelve such layers; from a graph 4.3, 4.2). */
+	struct Divisor
+	{
+		unsigned int factor, shift;
+		__device__ __forceinline__ unsigned int of(unsigned int n) const
+		{
+			return __umulhi(2 * n, factor) >> shift;
+		}
+	};
+	inline Divisor divisor(unsigned int d)
+	{
+		Divisor result = { 0, 0 };
+		while ((1u << result.shift) < d)
+			result.shift++;
+		result.factor = static_cast<unsigned int>(((1ull << (31 + result.shift)) + d - 1) / d);
+		return result;
+	}
+
 	/* Forward activations, src/activations.cuh:202-425 of the reference. */
 	template<typename CT>
 	__device__ inline CT activation_forward(int act, CT x)

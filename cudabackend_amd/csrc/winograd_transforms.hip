@@ -124,6 +124,41 @@ namespace
 			}
 	}
 
+	/* What a work-item's number is divided by: channel runs of a row, tiles of an image's row, rows of tiles.  32-bit numbers by multiplications (Divisor): three divisions in a row
+	 * stood before the first load of every work-item. */
+	template<typename IDX> struct Over
+	{
+		IDX d;
+		__device__ __forceinline__ IDX of(IDX n) const
+		{
+			return n / d;
+		}
+	};
+	template<> struct Over<uint32_t>
+	{
+		uint32_t d;
+		Divisor by;
+		__device__ __forceinline__ uint32_t of(uint32_t n) const
+		{
+			return by.of(n);
+		}
+	};
+	template<typename IDX> Over<IDX> over(size_t d)
+	{
+		if constexpr (std::is_same<IDX, uint32_t>::value)
+			return { static_cast<uint32_t>(d), divisor(d > 0 ? static_cast<unsigned int>(d) : 1) };
+		else
+			return { d };
+	}
+	template<typename IDX> struct TileNumbers
+	{
+		Over<IDX> runs, tw, th;
+	};
+	template<typename IDX> TileNumbers<IDX> tile_numbers(int channels, int width, int Tw, int Th)
+	{
+		return { over<IDX>((channels + width - 1) / width), over<IDX>(Tw), over<IDX>(Th) };
+	}
+
 	template<int M, int R, typename T, typename TM, int V>
 	__global__ __launch_bounds__(256) void k_weight_transform(const T *__restrict__ w, TM *__restrict__ U, int K, int C, int invert)
 	{
@@ -131,8 +166,9 @@ namespace
 		constexpr int t = M + R - 1;
 		const int CV = (C + V - 1) / V;
 		const size_t gid = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-		const int cv = static_cast<int>(gid % CV);
-		const size_t k = gid / CV;
+		/* (numbers below 2^32: the division of 64 bits is some hundred instructions) */
+		const size_t k = gridDim.x < (1u << 24) ? static_cast<unsigned int>(gid) / static_cast<unsigned int>(CV) : gid / CV;
+		const int cv = static_cast<int>(gid - k * CV);
 		if (k >= static_cast<size_t>(K))
 			return;
 		const int c = cv * V;
@@ -189,23 +225,22 @@ namespace
 	 * channels (odd counts) likewise: bf16 159 channels on 85 images of 15 x 14 13.5 -> 9.3 us. */
 	template<int M, int R, typename T, typename TM, int V, typename IDX, bool BUF = false>
 	__global__ __launch_bounds__(256) void k_input_transform(const T *__restrict__ x, TM *__restrict__ Vm, int N, int H, int W, int C, int Th, int Tw,
-			int pad_h, int pad_w, typename Traits<T>::compute padv)
+			int pad_h, int pad_w, typename Traits<T>::compute padv, TileNumbers<IDX> by)
 	{
 		typedef typename Traits<T>::compute CT;
 		constexpr int t = M + R - 1;
 		constexpr bool FULL = V > 1 || BUF;
 		static_assert(!BUF || (buffer_run<T, V> && sizeof(IDX) == 4), "runs of 2 to 16 bytes, 32-bit offsets");
-		const IDX CV = static_cast<IDX>((C + V - 1) / V);
 		const IDX tiles = static_cast<IDX>(N) * Th * Tw;
 		/* neighbouring tiles share input pixels: consecutive runs of tiles go to one XCD, whose L2 then serves the overlap */
 		const IDX gid = static_cast<IDX>(xcd_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
-		const IDX tile = gid / CV;
-		const int cv = static_cast<int>(gid - tile * CV);
+		const IDX tile = by.runs.of(gid);
+		const int cv = static_cast<int>(gid - tile * by.runs.d);
 		if (tile >= tiles)
 			return;
-		const IDX row = tile / static_cast<IDX>(Tw);
+		const IDX row = by.tw.of(tile);
 		const int tw = static_cast<int>(tile - row * Tw);
-		const IDX n = row / static_cast<IDX>(Th);
+		const IDX n = by.th.of(row);
 		const int th = static_cast<int>(row - n * Th);
 		const int c = cv * V;
 		const int valid = FULL ? V : C - c;
@@ -276,21 +311,20 @@ namespace
 	template<int M, int R, typename T, typename TM, int V, int ACT, typename IDX>
 	__global__ __launch_bounds__(256) void k_output_transform(const TM *__restrict__ Mx, T *y, const typename Traits<T>::compute *__restrict__ bias,
 			const T *z, int N, int H, int W, int K, int Th, int Tw, typename Traits<T>::compute alpha1, typename Traits<T>::compute alpha2,
-			typename Traits<T>::compute beta, int activation)
+			typename Traits<T>::compute beta, int activation, TileNumbers<IDX> by)
 	{
 		typedef typename Traits<T>::compute CT;
 		constexpr int t = M + R - 1;
 		constexpr bool FULL = V > 1;
-		const IDX KV = static_cast<IDX>((K + V - 1) / V);
 		const IDX tiles = static_cast<IDX>(N) * Th * Tw;
 		const IDX gid = static_cast<IDX>(blockIdx.x) * 256 + threadIdx.x;
-		const IDX tile = gid / KV;
-		const int kv = static_cast<int>(gid - tile * KV);
+		const IDX tile = by.runs.of(gid);
+		const int kv = static_cast<int>(gid - tile * by.runs.d);
 		if (tile >= tiles)
 			return;
-		const IDX row = tile / static_cast<IDX>(Tw);
+		const IDX row = by.tw.of(tile);
 		const int tw = static_cast<int>(tile - row * Tw);
-		const IDX n = row / static_cast<IDX>(Th);
+		const IDX n = by.th.of(row);
 		const int th = static_cast<int>(row - n * Th);
 		const int k = kv * V;
 		const int valid = FULL ? V : K - k;
@@ -356,22 +390,21 @@ namespace
 	 * transform: with 64-bit divisions and a branch around each load it waited for its loads one after the other.  Together with
 	 * group_size below: fp32 F(4x4, 3x3) gradient of 32 x 15 x 15 x 128 -> 128, all four launches, 29.8 -> 25.2 us. */
 	template<int M, int R, typename T, typename TM, int V, typename IDX, bool BUF = false>
-	__global__ __launch_bounds__(256) void k_gradient_transform(const T *__restrict__ dy, TM *__restrict__ Mx, int N, int H, int W, int K, int Th, int Tw)
+	__global__ __launch_bounds__(256) void k_gradient_transform(const T *__restrict__ dy, TM *__restrict__ Mx, int N, int H, int W, int K, int Th, int Tw, TileNumbers<IDX> by)
 	{
 		typedef typename Traits<T>::compute CT;
 		constexpr int t = M + R - 1;
 		constexpr bool FULL = V > 1 || BUF;
-		const IDX KV = static_cast<IDX>((K + V - 1) / V);
 		const IDX tiles = static_cast<IDX>(N) * Th * Tw;
 		const IDX gid = static_cast<IDX>(blockIdx.x) * blockDim.x + threadIdx.x;
-		const IDX tile = gid / KV;
+		const IDX tile = by.runs.of(gid);
 		if (tile >= tiles)
 			return;
-		const int k = static_cast<int>(gid - tile * KV) * V;
+		const int k = static_cast<int>(gid - tile * by.runs.d) * V;
 		const int valid = FULL ? V : K - k;
-		const IDX row = tile / static_cast<IDX>(Tw);
+		const IDX row = by.tw.of(tile);
 		const int tw = static_cast<int>(tile - row * Tw);
-		const IDX n = row / static_cast<IDX>(Th);
+		const IDX n = by.th.of(row);
 		const int th = static_cast<int>(row - n * Th);
 
 		CT d[M * M][V];
@@ -427,18 +460,17 @@ namespace
 	 * [t*t, K, C] at (k, c) (src/winograd_nonfused.cu:475-519). */
 	template<int M, int R, typename T, typename TM, int V, typename IDX>
 	__global__ __launch_bounds__(256) void k_update_transform(const TM *__restrict__ Mx, T *dw, int K, int C, typename Traits<T>::compute alpha,
-			typename Traits<T>::compute beta)
+			typename Traits<T>::compute beta, Over<IDX> by_runs)
 	{
 		typedef typename Traits<T>::compute CT;
 		constexpr int t = M + R - 1;
 		constexpr bool FULL = V > 1;
-		const IDX CV = static_cast<IDX>((C + V - 1) / V);
 		const IDX gid = static_cast<IDX>(blockIdx.x) * blockDim.x + threadIdx.x;
-		const IDX row = gid / CV;
+		const IDX row = by_runs.of(gid);
 		if (row >= static_cast<IDX>(K))
 			return;
 		const size_t k = row;
-		const int c = static_cast<int>(gid - row * CV) * V;
+		const int c = static_cast<int>(gid - row * by_runs.d) * V;
 		const int valid = FULL ? V : C - c;
 
 		CT m[t * t][V];
@@ -550,7 +582,7 @@ namespace
 				const size_t items = static_cast<size_t>(N) * Th * Tw * (C / width);
 				const unsigned int group = group_size(items);
 #define AVHIP_LAUNCH_INPUT_BUFFER(WIDTH) hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, uint32_t, true>), dim3(ceil_div(items, group)), dim3(group), 0, s, \
-		static_cast<const T*>(x), static_cast<TM*>(Vm), N, H, W, C, Th, Tw, pad_h, pad_w, padv)
+		static_cast<const T*>(x), static_cast<TM*>(Vm), N, H, W, C, Th, Tw, pad_h, pad_w, padv, tile_numbers<uint32_t>(C, width, Tw, Th))
 				if (width == 1)
 					AVHIP_LAUNCH_INPUT_BUFFER(1);
 				else if (width == VecOf<M, R, T, TM>::value)
@@ -564,7 +596,7 @@ namespace
 		const unsigned int group = group_size(items);
 		const dim3 grid(ceil_div(items, group));
 #define AVHIP_LAUNCH_INPUT(WIDTH, IDX) hipLaunchKernelGGL((k_input_transform<M, R, T, TM, WIDTH, IDX>), grid, dim3(group), 0, s, static_cast<const T*>(x), \
-		static_cast<TM*>(Vm), N, H, W, C, Th, Tw, pad_h, pad_w, padv)
+		static_cast<TM*>(Vm), N, H, W, C, Th, Tw, pad_h, pad_w, padv, tile_numbers<IDX>(C, V, Tw, Th))
 		if (V > 1 && narrow)
 			AVHIP_LAUNCH_INPUT((VecOf<M, R, T, TM>::value), uint32_t);
 		else if (V > 1)
@@ -587,7 +619,7 @@ namespace
 		const dim3 grid(ceil_div(items, 256));
 #define AVHIP_LAUNCH_OUTPUT(WIDTH, ACT, IDX) hipLaunchKernelGGL((k_output_transform<M, R, T, TM, WIDTH, ACT, IDX>), grid, dim3(256), 0, s, \
 		static_cast<const TM*>(Mx), static_cast<T*>(y), static_cast<const CT*>(bias), static_cast<const T*>(z), N, H, W, K, Th, Tw, static_cast<CT>(alpha1), \
-		static_cast<CT>(alpha2), static_cast<CT>(beta), activation)
+		static_cast<CT>(alpha2), static_cast<CT>(beta), activation, tile_numbers<IDX>(K, V, Tw, Th))
 		/* LINEAR / RELU get their own instance: a nine-way switch per element makes the compiler evaluate every function */
 		const bool simple = is_simple_activation(activation);
 		const bool narrow = items < (1ull << 31) && static_cast<uint64_t>(H) * W < (1ull << 31);
@@ -603,7 +635,7 @@ namespace
 				const dim3 wide_grid(ceil_div(items / 2, 256));
 				hipLaunchKernelGGL((k_output_transform<M, R, T, TM, WIDE, ACT_SIMPLE, uint32_t>), wide_grid, dim3(256), 0, s, static_cast<const TM*>(Mx), static_cast<T*>(y),
 						static_cast<const CT*>(bias), static_cast<const T*>(z), N, H, W, K, Th, Tw, static_cast<CT>(alpha1), static_cast<CT>(alpha2), static_cast<CT>(beta),
-						activation);
+						activation, tile_numbers<uint32_t>(K, WIDE, Tw, Th));
 				return 0;
 			}
 		}
@@ -629,8 +661,8 @@ namespace
 		const bool narrow = static_cast<size_t>(N) * Th * Tw * ((K + V - 1) / V) < (1ull << 31);
 		const bool buffered = static_cast<uint64_t>(N) * H * W * K * sizeof(T) < (1ull << 31);
 		constexpr int WIDTH = VecOf<M, R, T, TM>::value;
-#define AVHIP_LAUNCH_GRADIENT(WIDTH, ...) hipLaunchKernelGGL((k_gradient_transform<M, R, T, TM, WIDTH, __VA_ARGS__>), dim3(ceil_div(items, group)), dim3(group), 0, s, \
-		static_cast<const T*>(dy), static_cast<TM*>(Mx), N, H, W, K, Th, Tw)
+#define AVHIP_LAUNCH_GRADIENT(WIDTH, IDX, BUF) hipLaunchKernelGGL((k_gradient_transform<M, R, T, TM, WIDTH, IDX, BUF>), dim3(ceil_div(items, group)), dim3(group), 0, s, \
+		static_cast<const T*>(dy), static_cast<TM*>(Mx), N, H, W, K, Th, Tw, tile_numbers<IDX>(K, WIDTH, Tw, Th))
 		if constexpr (buffer_run<T, 1>)
 			if (narrow && buffered)
 			{
@@ -648,11 +680,11 @@ namespace
 		const size_t items = static_cast<size_t>(N) * Th * Tw * ((K + V - 1) / V);
 		const unsigned int group = group_size(items);
 		if (V > 1)
-			AVHIP_LAUNCH_GRADIENT(WIDTH, size_t);
+			AVHIP_LAUNCH_GRADIENT(WIDTH, size_t, false);
 		else if (narrow)
-			AVHIP_LAUNCH_GRADIENT(1, uint32_t);
+			AVHIP_LAUNCH_GRADIENT(1, uint32_t, false);
 		else
-			AVHIP_LAUNCH_GRADIENT(1, size_t);
+			AVHIP_LAUNCH_GRADIENT(1, size_t, false);
 #undef AVHIP_LAUNCH_GRADIENT
 		return 0;
 	}
@@ -665,7 +697,7 @@ namespace
 		const unsigned int group = group_size(items);
 		const dim3 grid(ceil_div(items, group));
 #define AVHIP_LAUNCH_UPDATE(WIDTH, IDX) hipLaunchKernelGGL((k_update_transform<M, R, T, TM, WIDTH, IDX>), grid, dim3(group), 0, s, \
-		static_cast<const TM*>(Mx), static_cast<T*>(dw), K, C, static_cast<CT>(alpha), static_cast<CT>(beta))
+		static_cast<const TM*>(Mx), static_cast<T*>(dw), K, C, static_cast<CT>(alpha), static_cast<CT>(beta), over<IDX>((C + WIDTH - 1) / WIDTH))
 		constexpr int WIDTH = VecOf<M, R, T, TM>::value;
 		const bool narrow = items < (1ull << 31);
 		if (V > 1 && narrow)
