@@ -19,7 +19,8 @@
  * Measured (36 products 128 x 128 over k = 512, fp32, operands from L2 / the last-level cache): 9.8 us, of which the
  * 18.9 MB of operands need 3.4 and the matrix cores 1.5; 11.4 with fp32 products, 74 in the generic kernel.  16-bit, tiles of 32 x 32, pairs against single
  * elements: 16 products 72 x 96 over 15561 43.1 -> 38.7 us, 32 x 32 over 4608 12.2 -> 8.4, 64 x 80 over 750 5.9 -> 4.6.  What bounds it at small
- * sizes is the chain of one launch: first loads, one or two waves of MFMAs, the sum through LDS.
+ * sizes is the chain of one launch: first loads, one or two waves of MFMAs, the sum through LDS.  With a last round that requested as many stages again and multiplied zeros to its end,
+ * 120 drawn gradients took 4.5 % longer, all launches.  fp32 values loaded in pairs (half as many loads, sixteen lanes exchanged for 32 x 32) took 7 to 12 % longer.
  */
 #include <cmath>
 #include <type_traits>
@@ -228,15 +229,21 @@ namespace
 #pragma unroll
 			for (int d = 0; d < DEPTH; d++)
 				fetch(d, wave + d * WAVES);
-			for (int s = 0; s < mine; s += DEPTH)
+			int left = mine; /* may be none */
+			for (int next = wave + DEPTH * WAVES; left > DEPTH; left -= DEPTH, next += DEPTH * WAVES)
 			{
 #pragma unroll
 				for (int d = 0; d < DEPTH; d++)
 				{
-					multiply(oa[d], ob[d], exact); /* zeros behind the last stage */
-					fetch(d, wave + (s + DEPTH + d) * WAVES);
+					multiply(oa[d], ob[d], exact);
+					fetch(d, next + d * WAVES); /* zeros behind the last stage */
 				}
 			}
+			/* the last round requests nothing, and multiplies what there is */
+#pragma unroll
+			for (int d = 0; d < DEPTH; d++)
+				if (d < left)
+					multiply(oa[d], ob[d], exact);
 		};
 		walk(std::false_type());
 		if constexpr (Op::WIDE && T == 2)
