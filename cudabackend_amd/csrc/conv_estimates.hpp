@@ -22,9 +22,9 @@ namespace avhip
 	};
 	struct SmallTiling
 	{
-		int side, waves;
+		int side_bits, wave_bits; /* a side of 2^side_bits: shifts on the host, not divisions or calls that round */
 	};
-	inline constexpr SmallTiling PLANS[] = { { 32, 1 }, { 32, 4 }, { 32, 8 }, { 64, 4 }, { 16, 1 }, { 16, 4 }, { 16, 8 } };
+	inline constexpr SmallTiling PLANS[] = { { 5, 0 }, { 5, 2 }, { 5, 3 }, { 6, 2 }, { 4, 0 }, { 4, 2 }, { 4, 3 } };
 
 	struct Pace
 	{
@@ -100,8 +100,8 @@ namespace avhip
 	 * 68), otherwise 4.  Tiles of 16 x 16 where those of 32 x 32 are few: from some 300 (five stages: 600) on those load less, 10.1 against 10.8 us for bf16 128 -> 128 3x3 with 572. */
 	inline SmallPlan conv_small_plan(const avhipConvShape &s, int element_bytes)
 	{
-		const double pixels = static_cast<double>(s.N) * s.Ho * s.Wo;
-		const double stages = std::ceil(static_cast<double>(s.R) * s.S * ((s.C * element_bytes + 15) / 16) / 8.0);
+		const int64_t pixels = static_cast<int64_t>(s.N) * s.Ho * s.Wo;
+		const int64_t stages = (static_cast<int64_t>(s.R) * s.S * ((static_cast<int64_t>(s.C) * element_bytes + 15) / 16) + 7) >> 3;
 		SmallPlan best = { 0, 0, 0.0, 0.0 };
 		const int64_t row = static_cast<int64_t>(s.C) * element_bytes;
 		/* Rows of dwords or elements: two loads and a shift for a piece of elements, and bits to be cut off.  Of tiles of 16 x 16 a stage takes 1.5 and 1.9 times as long (83 layers, 6 to 16 %): with
@@ -109,16 +109,16 @@ namespace avhip
 		const double by_rows = row % 16 == 0 ? 1.0 : row % 4 == 0 ? 1.5 : 1.9;
 		for (int i = row == 16 ? 4 : 0; i < 7; i++) /* (one chunk a tap: only the tiles of 16 x 16 count taps so) */
 		{
-			const int side = PLANS[i].side;
+			const int bits = PLANS[i].side_bits, side = 1 << bits, waves = 1 << PLANS[i].wave_bits;
 			const Pace &pace = element_bytes == 4 ? PACE_32[i] : PACE_16[i];
-			const double tiles = std::ceil(pixels / side) * ((s.K + side - 1) / side);
-			const double per_cu = tiles <= 1024.0 ? std::ceil(tiles / 256.0) : tiles / 256.0;
+			const int64_t tiles = ((pixels + side - 1) >> bits) * ((static_cast<int64_t>(s.K) + side - 1) >> bits);
+			const double per_cu = tiles <= 1024 ? static_cast<double>((tiles + 255) >> 8) : static_cast<double>(tiles) / 256.0;
 			const double slower = side == 16 ? by_rows : 1.0;
-			const double alone = std::ceil(stages / PLANS[i].waves) * pace.chain * slower, shared = per_cu * stages * pace.stage * slower;
+			const double alone = static_cast<double>((stages + waves - 1) >> PLANS[i].wave_bits) * pace.chain * slower, shared = per_cu * static_cast<double>(stages) * pace.stage * slower;
 			const double us = (pace.launch + (element_bytes == 4 || side == 16 ? std::sqrt(alone * alone + shared * shared) : std::max(alone, shared)) + per_cu * pace.tile)
 					* (side != 16 && row % 4 != 0 ? 1.25 : 1.0);
 			if (best.side == 0 || us < (side == 16 && best.side != 16 ? 0.95 : 1.0) * best.us)
-				best = { side, PLANS[i].waves, us, side == 16 ? best.larger_us : us };
+				best = { side, waves, us, side == 16 ? best.larger_us : us };
 		}
 		return best;
 	}
