@@ -418,7 +418,8 @@ namespace
 		const RingChoice choice = ring_choice(s, stages, out_bytes, small.hand_over, residual);
 		if (choice.us >= limit)
 			return none;
-		/* Tiles of 16 x 16 take what they are estimated to do in 0.69 of the time or less: 1x1 layers of two stages and less whose rows are few to a tile of either side. */
+		/* Tiles of 16 x 16 take a layer from here where they are estimated at 0.69 of its time or less.  Both estimates are loose where this one is low (5 to 12 %, and 64 x 64 tiles alone on a compute unit take longer
+		 * than theirs): at 1.0 of it bf16 192 -> 192 3x3 on 14 x 11 x 11 moved the wrong way, 9.6 -> 11.5 us; what lies between stays where it was timed. */
 		return small.preferred && small.plan.side == 16 && small.us < 0.69 * choice.us ? none : choice;
 	}
 }
