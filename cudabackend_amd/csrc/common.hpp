@@ -233,9 +233,7 @@ namespace avhip
 	};
 	inline Divisor divisor(unsigned int d)
 	{
-		Divisor result = { 0, 0 };
-		while ((1u << result.shift) < d)
-			result.shift++;
+		Divisor result = { 0, d > 1 ? 32u - static_cast<unsigned int>(__builtin_clz(d - 1)) : 0u };
 		result.factor = static_cast<unsigned int>(((1ull << (31 + result.shift)) + d - 1) / d);
 		return result;
 	}
