@@ -267,33 +267,12 @@ namespace avhip
 	}
 
 	/*
-	 * The activations of a run of values, chosen once for the run and not once per value.
-	 * For 16-bit results, which are rounded to 8 or 11 bits right behind: sigmoid, tanh, ELU and SELU in 10 to 17 instructions' time, with the exponential of a product rounded once.  Their
-	 * error is 1e-6 of the value at most where that is not rounded to 0 or 1 (4 million values of all sizes, against 64 bits), that of the rounding 4.9e-4 and 3.9e-3.
-	 * For fp32 results: ELU and SELU in 18, as exact as the library's functions (9e-8 at most, 1.4e-8 on average by both); those of sigmoid and tanh are left, which are rounded
-	 * better than what is faster.
-	 * The library's functions take 30 to 60, with branches: of the 57 us of bf16 24 -> 384 3x3 on 243 x 15 x 18 an ELU's 25 million results took 30.
+	 * The activations of a run of values, chosen once for the run and not once per value: ELU and SELU in 18 instructions' time, as exact as the library's functions (9e-8 at most, 1.4e-8 on
+	 * average by both), the others by those.  16-bit results too: formulas that are good enough for their rounding (an exponential of a product rounded once, a reciprocal) have two to forty times as many results
+	 * rounded the other way, 4.7e-4 of fp16 ELUs of -0.1 to -0.0625 instead of 1e-5, 2e-4 of bf16 sigmoids of -87 to -60 instead of none.
 	 */
-	__device__ __forceinline__ float sigmoid_16(float x)
-	{
-		return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -0x1.715476p+0f));
-	}
-	__device__ __forceinline__ float tanh_16(float x)
-	{
-		const float far = __builtin_fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * 0x1.715476p+1f)), 1.0f), xx = x * x;
-		const float near = x * __builtin_fmaf(xx, __builtin_fmaf(xx, 2.0f / 15.0f, -1.0f / 3.0f), 1.0f); /* 17/315 x^6 are 2e-7 at the line */
-		return xx < 0x1p-6f ? near : far;
-	}
-	/* e^x - 1 for x < 0, x for the others */
-	__device__ __forceinline__ float elu_16(float x)
-	{
-		const float far = __builtin_amdgcn_exp2f(x * 0x1.715476p+0f) - 1.0f;
-		const float near = x * __builtin_fmaf(x, __builtin_fmaf(x, __builtin_fmaf(x, 1.0f / 24.0f, 1.0f / 6.0f), 0.5f), 1.0f); /* x^4/120 are 1.3e-7 at the line */
-		const float below = x > -0x1p-4f ? near : far;
-		return x < 0.0f ? below : x;
-	}
-	/* The same as 2^n (e^r - 1) + (2^n - 1) with |r| <= ln 2 / 2; the polynomial is (e^r - 1 - r) / r^2 fitted by least squares, to 2.5e-9 of e^r - 1 */
-	__device__ __forceinline__ float elu_32(float x)
+	/* e^x - 1 for x < 0, x for the others: as 2^n (e^r - 1) + (2^n - 1) with |r| <= ln 2 / 2; the polynomial is (e^r - 1 - r) / r^2 fitted by least squares, to 2.5e-9 of e^r - 1 */
+	__host__ __device__ __forceinline__ float elu_32(float x)
 	{
 		constexpr float SHIFT = 12582912.0f; /* 1.5 * 2^23: the sum's lowest bit is 1 */
 		float y = x < 0.0f ? x : 0.0f;
@@ -311,29 +290,16 @@ namespace avhip
 		const float below = __builtin_fmaf(scale, p, scale - 1.0f);
 		return x < 0.0f ? below : x; /* (a NaN is not below) */
 	}
-	template<typename T, int W>
+	template<int W>
 	__device__ __forceinline__ void activate_run(int act, float (&t)[W])
 	{
-		constexpr bool HALVES = sizeof(T) == 2;
-		if (HALVES && act == ACT_SIGMOID)
-		{
-#pragma unroll
-			for (int q = 0; q < W; q++)
-				t[q] = sigmoid_16(t[q]);
-		}
-		else if (HALVES && act == ACT_TANH)
-		{
-#pragma unroll
-			for (int q = 0; q < W; q++)
-				t[q] = tanh_16(t[q]);
-		}
-		else if (act == ACT_ELU || act == ACT_SELU)
+		if (act == ACT_ELU || act == ACT_SELU)
 		{
 			const float below = act == ACT_ELU ? 1.0f : 1.67326324f, all = act == ACT_ELU ? 1.0f : 1.05070098f;
 #pragma unroll
 			for (int q = 0; q < W; q++)
 			{
-				const float e = HALVES ? elu_16(t[q]) : elu_32(t[q]);
+				const float e = elu_32(t[q]);
 				t[q] = all * (t[q] < 0.0f ? below * e : e);
 			}
 		}

@@ -205,7 +205,7 @@ namespace avhip
 		{
 			before_activation<ACT, VEC, W>(t, readable, idx, k, v, c, fetched);
 			if (ACT != ACT_SIMPLE)
-				activate_run<TE, W>(activation, t);
+				activate_run<W>(activation, t);
 			after_activation<VEC, W>(t, readable, idx, k);
 		}
 		/* N runs of a work-item in whole aligned vectors, any activation: `at`(n, idx) says whether run n exists and where it starts */
@@ -222,7 +222,7 @@ namespace avhip
 				for (int q = 0; q < W; q++)
 					t[n * W + q] = run[q];
 			}
-			activate_run<TE, N * W>(activation, t);
+			activate_run<N * W>(activation, t);
 #pragma unroll
 			for (int n = 0; n < N; n++)
 			{
