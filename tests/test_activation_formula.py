@@ -51,3 +51,40 @@ def test_special_values(elu):
     want = np.array([0.0, -0.0, np.inf, -1.0, np.nan, 3.5, -1.0, -1.0, 2.0 ** -149, -2.0 ** -149, -2.0 ** -127], np.float32)
     got = elu(x)
     assert np.array_equal(got, want, equal_nan=True) and np.array_equal(np.signbit(got[:4]), np.signbit(want[:4]))
+
+
+RUNS = """#include "common.hpp"
+template<int ACT, int W> __device__ void run(float *p)
+{
+	float t[W];
+	for (int q = 0; q < W; q++)
+		t[q] = p[threadIdx.x * W + q];
+	avhip::activate_run<W>(ACT, t);
+	for (int q = 0; q < W; q++)
+		p[threadIdx.x * W + q] = t[q];
+}
+extern "C" __global__ void linear_4(float *p) { run<avhip::ACT_LINEAR, 4>(p); }
+extern "C" __global__ void linear_16(float *p) { run<avhip::ACT_LINEAR, 16>(p); }
+extern "C" __global__ void relu_4(float *p) { run<avhip::ACT_RELU, 4>(p); }
+extern "C" __global__ void relu_16(float *p) { run<avhip::ACT_RELU, 16>(p); }
+"""
+
+
+def test_linear_and_relu_are_no_loop(tmp_path):
+    """Filters in no whole vectors take LINEAR and RELU through activate_run: LINEAR leaves the values alone, RELU is straight code, however many values a run has."""
+    source = str(tmp_path / "runs.hip")
+    with open(source, "w") as f:
+        f.write(RUNS)
+    r = subprocess.run(["hipcc", *build.FLAGS, "-w", "-I" + build.CSRC, "--cuda-device-only", "-S", source, "-o", "-"], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
+    assert r.returncode == 0, r.stderr[-4000:]
+    name, code = None, {}
+    for line in r.stdout.splitlines():
+        if line.startswith(("linear_", "relu_")) and line.split(":")[0].split("_")[1].isdigit():
+            name = line.split(":")[0]
+        elif name and line.startswith("\t") and not line.startswith("\t."):
+            code.setdefault(name, []).append(line.split()[0])
+    assert sorted(code) == ["linear_16", "linear_4", "relu_16", "relu_4"]
+    for name, instructions in code.items():
+        assert not [i for i in instructions if "cbranch" in i], name
+        if name.startswith("linear"):
+            assert not [i for i in instructions if i.startswith(("v_max", "v_cmp", "v_cndmask"))], name
