@@ -290,6 +290,13 @@ namespace avhip
 		const float below = __builtin_fmaf(scale, p, scale - 1.0f);
 		return x < 0.0f ? below : x; /* (a NaN is not below) */
 	}
+	template<int ACT, int W>
+	__device__ __forceinline__ void activate_values(float (&t)[W])
+	{
+#pragma unroll
+		for (int q = 0; q < W; q++)
+			t[q] = activation_forward<float>(ACT, t[q]);
+	}
 	template<int W>
 	__device__ __forceinline__ void activate_run(int act, float (&t)[W])
 	{
@@ -299,11 +306,7 @@ namespace avhip
 		if (act == ACT_LINEAR)
 			return;
 		if (act == ACT_RELU)
-		{
-#pragma unroll
-			for (int q = 0; q < W; q++)
-				t[q] = activation_forward<float>(ACT_RELU, t[q]);
-		}
+			activate_values<ACT_RELU>(t);
 		else if (act == ACT_ELU || act == ACT_SELU)
 		{
 			const float below = act == ACT_ELU ? 1.0f : 1.67326324f, all = act == ACT_ELU ? 1.0f : 1.05070098f;
@@ -319,10 +322,25 @@ namespace avhip
 #pragma unroll 1 /* one copy of the library's functions for four values; the run is turned by four, so that no register is chosen by a number */
 			for (int n = 0; n < W; n += 4)
 			{
-				float quad[4];
-#pragma unroll
-				for (int q = 0; q < 4; q++)
-					quad[q] = activation_forward<float>(act, t[q]);
+				float quad[4] = { t[0], t[1], t[2], t[3] };
+				switch (act)
+				{
+					case ACT_SIGMOID:
+						activate_values<ACT_SIGMOID>(quad);
+						break;
+					case ACT_TANH:
+						activate_values<ACT_TANH>(quad);
+						break;
+					case ACT_EXPONENTIAL:
+						activate_values<ACT_EXPONENTIAL>(quad);
+						break;
+					case ACT_SOFTPLUS:
+						activate_values<ACT_SOFTPLUS>(quad);
+						break;
+					case ACT_SOFTSIGN:
+						activate_values<ACT_SOFTSIGN>(quad);
+						break;
+				}
 #pragma unroll
 				for (int q = 0; q + 4 < W; q++)
 					t[q] = t[q + 4];
