@@ -948,16 +948,26 @@ namespace
 
 	/* fp32: whether the direct sums (small tiles, or 128 x 128 tiles with products in bf16 pieces) are estimated to be faster than the fused kernel.  That walks rounds of 256
 	 * workgroups of 256 pixels x 128 filters, filled up, 14 us and 43.5 us per 64 channels a round (58 us at 32 channels, 104 at 128, 362 at 472, ten layers within a tenth), 8 more
-	 * with a residual and 25 with an activation by a call.  Of 65 layers that went to it, 32 to 448 channels and 32 to 512 filters, 160 to 2151 workgroups, every one is faster in
-	 * direct sums: 1.3 to 6.3 times, 2.4 on average (32 -> 32 on 34 x 40 x 43 118 -> 19 us, 256 -> 256 on 114 x 12 x 12 202 -> 156).  What is left to it are full rounds of 128 channels
-	 * and filters without a workspace: 128 -> 128 on 256 x 15 x 15 104 us by both. */
+	 * with a residual and 25 with an activation by a call.  Of 122 layers that went to it, 32 to 448 channels and 32 to 512 filters, 160 to 2151 workgroups, whole vectors and single filters, every one is faster in
+	 * direct sums: 1.07 to 7.9 times, 2.3 on average (32 -> 32 on 34 x 40 x 43 118 -> 19 us, 256 -> 256 on 114 x 12 x 12 202 -> 156).  What is left to it are full rounds of 128 channels
+	 * and filters without a workspace, 128 -> 128 on 256 x 15 x 15 104 us by both, and calls whose direct sums would be formed element by element: the fused kernel has a layout of its own of
+	 * the weights, from any address, the others read them as they lie (96 -> 192 on 11 x 39 x 39 with weights at 4 bytes 192 us so, 96 in the fused kernel). */
 	bool direct_before_fused(const ConvCall &c, avActivationType_t activation, av_int64 fused_workgroups)
 	{
 		const avhipConvShape &s = c.problem.shape;
+		const char *x = static_cast<const char*>(c.x->data), *y = static_cast<const char*>(c.y->data);
+		const int64_t x_bytes = 4ll * s.N * s.H * s.W * s.C, y_bytes = 4ll * s.N * s.Ho * s.Wo * s.K;
+		/* only what the fused kernel takes, so that the plan behind it stays the same where it declines; nothing in place, which small tiles decline */
+		if (s.C % 4 != 0 || x_bytes >= (1ll << 31) || 64ll * s.K * s.C >= (1ll << 31) || (x < y + y_bytes && y < x + x_bytes))
+			return false;
+		const auto aligned = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+		if (!aligned(x) || !aligned(c.w->data))
+			return false;
 		const bool simple = activation == AVOCADO_ACTIVATION_LINEAR || activation == AVOCADO_ACTIVATION_RELU;
+		const bool vectors = s.K % 4 == 0 && aligned(y) && aligned(c.z);
 		const double fused = static_cast<double>((fused_workgroups + 255) / 256) * (14.0 + 43.5 * ((s.C + 63) / 64) + (c.z != nullptr ? 8.0 : 0.0) + (simple ? 0.0 : 25.0));
-		const double direct = std::min(avhip::conv_small_plan(s, 4).us, avhip::tile_kernel_us(s, 4, simple ? avhip::GATHER : avhip::GATHER_ACTIVATION));
-		return direct < 0.95 * fused;
+		const double direct = avhip_conv2d_small_us(AVOCADO_DTYPE_FLOAT32, &s, !simple ? 2 : vectors ? 0 : 1);
+		return direct > 0.0 && direct < 0.95 * fused;
 	}
 
 	/* Row-wise Winograd F(2,3) for 16-bit 3x3 layers whose image bands fit a compute unit's LDS (conv_winograd_rows.hip): two

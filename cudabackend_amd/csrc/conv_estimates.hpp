@@ -11,6 +11,13 @@
 
 #include "../../include/avocado_hip_kernels.h"
 
+extern "C"
+{
+	/* Microseconds that a layer of more than one tap in 16-byte chunks of channels is estimated to take in the implicit-GEMM kernel that it is sent to, small tiles or 128 x 128 (256 x 64) ones; 0 where
+	 * neither is weighed (avhip_set_small_problem_threshold at 0 or below).  `hand_over`: HandOver of conv_small.hpp.  Defined in conv_small.hip. */
+	AVHIP_API double avhip_conv2d_small_us(int x_dtype, const avhipConvShape *shape, int hand_over);
+}
+
 namespace avhip
 {
 	/* tiles of side x side, `waves` wavefronts sharing the k range, and the estimated microseconds */

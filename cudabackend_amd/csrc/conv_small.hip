@@ -540,3 +540,11 @@ extern "C" AVHIP_API int avhip_conv2d_small_plan(int x_dtype, const avhipConvSha
 	const SmallChoice choice = conv_small_choice(*shape, element_bytes, static_cast<HandOver>(hand_over), 0.0);
 	return choice.preferred ? choice.plan.side / 2 + choice.plan.waves : 0;
 }
+
+extern "C" AVHIP_API double avhip_conv2d_small_us(int x_dtype, const avhipConvShape *shape, int hand_over)
+{
+	if (shape == nullptr || hand_over < 0 || hand_over > 2 || conv_small_threshold() <= 0)
+		return 0.0;
+	const int element_bytes = x_dtype == DT_INT8 ? 1 : x_dtype == DT_FLOAT32 ? 4 : 2;
+	return whole_chunks(*shape, element_bytes) ? conv_small_choice(*shape, element_bytes, static_cast<HandOver>(hand_over), 0.0).us : 0.0;
+}

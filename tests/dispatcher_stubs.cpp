@@ -10,6 +10,7 @@
 #include <map>
 #include <string>
 
+#include "../cudabackend_amd/csrc/conv_estimates.hpp"
 #include "../cudabackend_amd/csrc/conv_winograd_f4.hpp"
 
 namespace
@@ -17,7 +18,7 @@ namespace
 	std::map<std::string, int> calls;
 	bool malloc_fails = false, capturing = false;
 	int strided_workgroups = 0;
-	double ring_us = 0.0;
+	double ring_us = 0.0, direct_us = 0.0;
 	int called(const char *name, int result = 0)
 	{
 		calls[name]++;
@@ -38,6 +39,11 @@ extern "C"
 	{
 		strided_workgroups = workgroups;
 		ring_us = ring_us_now;
+	}
+	/* what direct sums are estimated to take, for every layer (0: not weighed) */
+	AVHIP_API void stub_set_direct(double direct_us_now)
+	{
+		direct_us = direct_us_now;
 	}
 	AVHIP_API int stub_calls(const char *name)
 	{
@@ -117,6 +123,11 @@ extern "C"
 		return called("strided");
 	}
 	double avhip_conv2d_ring_us(int, int, const avhipConvShape*, int, int) { return ring_us; }
+	double avhip_conv2d_small_us(int, const avhipConvShape*, int) { return direct_us; }
+	int avhip_conv2d_winograd_fused(void*, int, const avhipConvShape*, const void*, const void*, const void*, const void*, void*, double, double, double, int)
+	{
+		return called("fused");
+	}
 	int avhip_conv2d_pointwise_block_plan(int, const avhipConvShape*, int*, int*) { return AVHIP_NOT_SUPPORTED; }
 }
 
@@ -130,7 +141,6 @@ STUB_UNUSED(avhip_conv2d_implicit_gemm_split_k)
 STUB_UNUSED(avhip_conv2d_pointwise_block)
 STUB_UNUSED(avhip_conv2d_pointwise_block_weight_bytes)
 STUB_UNUSED(avhip_conv2d_pointwise_block_weight_layout)
-STUB_UNUSED(avhip_conv2d_winograd_fused)
 STUB_UNUSED(avhip_conv2d_winograd_rows)
 STUB_UNUSED(avhip_im2row)
 STUB_UNUSED(avhip_set_conv_strided)

@@ -28,6 +28,7 @@ def lib(tmp_path_factory):
         fn.restype, fn.argtypes = res, args
     dll.stub_calls.argtypes = [C.c_char_p]
     dll.stub_set_strided.argtypes = [C.c_int, C.c_double]
+    dll.stub_set_direct.argtypes = [C.c_double]
     return dll
 
 
@@ -142,3 +143,46 @@ def test_stride_2_layers_go_to_the_ring_kernel_where_that_takes_them(lib):
     layer = StridedLayer(lib)
     images = layer.tensor(24, 34, 34, 192)
     assert layer.route(15.0, x=images, y=(layer.y[0], images[1])) == ["strided"], "in place"
+
+
+class FusedLayer(Layer):
+    """fp32 3x3 32 -> 36 on 34 images of 40 x 43 without a workspace: 306 workgroups of the fused Winograd kernel, 115 us by its estimate."""
+
+    def __init__(self, lib):
+        self.lib = lib
+        lib.stub_set(0, 0)
+        self.context = self.made(lib.cudaCreateContextDescriptor, 0)
+        self.conv = self.made(lib.cudaCreateConvolutionDescriptor)
+        cb.check(lib.cudaSetConvolutionDescriptor(self.conv, cb.CONVOLUTION_MODE, 2, (C.c_int * 2)(-1, -1), None, None, 1, None))
+        self.x, self.w, self.y = (self.tensor(*shape) for shape in ((34, 40, 43, 32), (36, 3, 3, 32), (34, 40, 43, 36)))
+        self.space = 0
+
+    def tensor(self, *shape, offset=0):
+        desc, memory = super().tensor(*shape)
+        if not offset:
+            return desc, memory
+        size = 4 * shape[0] * shape[1] * shape[2] * shape[3]
+        return desc, self.made(self.lib.cudaCreateMemoryView, self.made(self.lib.cudaCreateMemoryDescriptor, 0, size + offset), size, offset)
+
+    def route(self, direct_us, **tensors):
+        self.lib.stub_set_direct(direct_us)
+        for name, t in tensors.items():
+            setattr(self, name, t)
+        status, _ = self.forward()
+        self.lib.stub_set_direct(0.0)
+        assert status == "SUCCESS"
+        return [n for n in ("fused", "implicit_gemm") if self.lib.stub_calls(n.encode())]
+
+
+@pytest.mark.parametrize("direct_us, tensors, want", [
+    (50.0, {}, "implicit_gemm"), (150.0, {}, "fused"), (0.0, {}, "fused"),
+    (50.0, dict(w=((36, 3, 3, 32), 4)), "fused"), (50.0, dict(w=((36, 3, 3, 32), 16)), "implicit_gemm"), (50.0, dict(x=((34, 40, 43, 32), 8)), "fused"),
+    (50.0, dict(y=((34, 40, 43, 36), 4)), "implicit_gemm"), (50.0, dict(x=((34, 40, 43, 36), 0), w=((36, 3, 3, 36), 0), y="x"), "fused")], ids=str)
+def test_direct_sums_replace_the_fused_kernel_where_they_read_the_operands(lib, direct_us, tensors, want):
+    """The fused kernel has a layout of its own of the weights, from any address; the direct kernels read them as they lie, and what they decline ends in a kernel that is slower than
+    both.  Nor do calls in place go to them, nor any where they are not weighed."""
+    layer = FusedLayer(lib)
+    made = {name: layer.tensor(*t[0], offset=t[1]) for name, t in tensors.items() if t != "x"}
+    if tensors.get("y") == "x":
+        made["y"] = made["x"]
+    assert layer.route(direct_us, **made) == [want]

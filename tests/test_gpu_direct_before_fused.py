@@ -9,9 +9,9 @@ from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
 
-# images, rows, columns, channels, filters, activation, residual: full rounds of the fused kernel's workgroups, hardly begun ones, filters that fill no block, rows in no whole vectors
+# images, rows, columns, channels, filters, activation, residual: full rounds of the fused kernel's workgroups, hardly begun ones, filters that fill no block, rows in no whole vectors, channels in no whole chunks (which the fused kernel declines)
 CASES = [(246, 13, 13, 32, 32, "relu", False), (64, 29, 29, 64, 48, "relu", False), (34, 40, 43, 32, 33, "linear", True), (45, 48, 51, 32, 32, "sigmoid", True),
-         (22, 36, 35, 96, 55, "elu", False), (11, 39, 39, 96, 192, "tanh", False)]
+         (22, 36, 35, 96, 55, "elu", False), (11, 39, 39, 96, 192, "tanh", False), (42, 31, 31, 60, 99, "relu", True), (42, 31, 31, 61, 99, "linear", False)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=str)
