@@ -25,7 +25,13 @@ namespace avhip
 	{
 		int side, waves;
 		double us;
-		double larger_us; /* of the best without tiles of 16 x 16 */
+		double larger_us; /* of the best without tiles of 16 x 16; 0: there is none */
+		int waves_16; /* and of the best with them */
+		double us_16;
+		SmallPlan of_16() const
+		{
+			return { 16, waves_16, us_16, larger_us, waves_16, us_16 };
+		}
 	};
 	struct SmallTiling
 	{
@@ -45,11 +51,22 @@ namespace avhip
 	 * 5.5 with one).  The tiles of 64 x 64, whose products are of bf16 pieces, to 260 layers (6 %), and
 	 * 6 % and 0.6 us more than that: then none of the 43 that get them is slower than with what it got before (1.28 times as fast on average; without
 	 * that 56, four of them slower).  The tiles of 16 x 16 (conv_small16.hip; the root of the sum of squares in every type) to 254 layers of up to 800 tiles of 32 x 32, 6 to 8 %, and taken
-	 * where they are 5 % below the others: of 224 layers they were not fitted to the plan chosen is 1.3 % slower than the best on average, 5 are slower than they were, by 13 % at most. */
+	 * where they are 5 % below the others; in 16 and 8 bits by margin_16. */
 	inline constexpr Pace PACE_16[] = { { 4.99, 0.303, 0.107, 0.20 }, { 3.34, 0.409, 0.084, 0.90 }, { 2.64, 0.173, 0.091, 2.40 }, { 3.41, 0.88, 0.182, 1.86 },
 			{ 2.75, 0.171, 0.043, 0.09 }, { 2.81, 0.144, 0.041, 0.205 }, { 2.31, 0.228, 0.035, 0.73 } };
 	inline constexpr Pace PACE_32[] = { { 3.80, 0.647, 0.143, 0.37 }, { 3.19, 0.490, 0.149, 1.00 }, { 2.34, 0.162, 0.165, 2.98 }, { 4.34, 1.13, 0.371, 3.14 },
 			{ 2.91, 0.280, 0.069, 0.05 }, { 2.83, 0.217, 0.060, 0.275 }, { 2.65, 0.260, 0.058, 0.52 } };
+
+	/* How far below those of larger tiles the estimate of tiles of 16 x 16 has to be: 5 %, and in 16 and 8 bits, whose larger tiles are estimated 5 to 10 % too high where their number begins a second round or k is long, 10 beyond
+	 * 768 of them or for a long k in rows that are no whole lines, 20 for many tiles of a long k.  Of 1794 16-bit layers that got tiles of 16 x 16 with 5 % everywhere, a tile beyond four in part and no look at
+	 * how rows lie, 74 were more than 3 % slower with them, by 25 at most (472 -> 192 3x3 stride 2 on 16 x 19 x 18 18.3 -> 24.4 us; 384 -> 200 5x5 stride 2 on 7 x 27 x 26, which was split before, 23.7 -> 36.2).
+	 * 1568 keep them, 9 of those more than 3 % slower, by 10 at most, and 1.26 times as fast on average. */
+	inline double margin_16(int element_bytes, bool whole_lines, int64_t tiles, int64_t stages)
+	{
+		if (element_bytes == 4 || tiles <= 256 || (tiles <= 768 && (whole_lines || stages < 90)))
+			return 0.95;
+		return tiles <= 1536 || stages < 24 ? 0.9 : 0.8;
+	}
 
 	/* The kernels with 128 x 128 (image-tile kernel: 256 x 64) workgroup tiles: launch, a round of 512 workgroups (two to a compute unit), and
 	 * a k-step of one that has a compute unit to itself or shares it.  The last round, if it is of up to 256, goes at the pace of the former.
@@ -109,24 +126,43 @@ namespace avhip
 	{
 		const int64_t pixels = static_cast<int64_t>(s.N) * s.Ho * s.Wo;
 		const int64_t stages = (static_cast<int64_t>(s.R) * s.S * ((static_cast<int64_t>(s.C) * element_bytes + 15) / 16) + 7) >> 3;
-		SmallPlan best = { 0, 0, 0.0, 0.0 };
+		SmallPlan best = { 0, 0, 0.0, 0.0, 0, 0.0 };
+		int64_t tiles_16 = 0;
 		const int64_t row = static_cast<int64_t>(s.C) * element_bytes;
 		/* Rows of dwords or elements: two loads and a shift for a piece of elements, and bits to be cut off.  Of tiles of 16 x 16 a stage takes 1.5 and 1.9 times as long (83 layers, 6 to 16 %): with
 		 * these factors the 62 that small tiles had before are 1.22 times as fast, none slower by more than 1 %. */
 		const double by_rows = row % 16 == 0 ? 1.0 : row % 4 == 0 ? 1.5 : 1.9;
+		/* and where rows are no whole lines of 128 bytes in 16 and 8 bits the 128 bytes of a load lie in two of them: 1.2 times (1.15 to 1.25 over 560 layers; larger tiles, which load half as much for a product, are not slower for it) */
+		const double across_lines = element_bytes < 4 && row % 16 == 0 && row % 128 != 0 && row >= 64 ? 1.2 : 1.0;
 		for (int i = row == 16 ? 4 : 0; i < 7; i++) /* (one chunk a tap: only the tiles of 16 x 16 count taps so) */
 		{
 			const int bits = PLANS[i].side_bits, side = 1 << bits, waves = 1 << PLANS[i].wave_bits;
 			const Pace &pace = element_bytes == 4 ? PACE_32[i] : PACE_16[i];
 			const int64_t tiles = ((pixels + side - 1) >> bits) * ((static_cast<int64_t>(s.K) + side - 1) >> bits);
-			const double per_cu = tiles <= 1024 ? static_cast<double>((tiles + 255) >> 8) : static_cast<double>(tiles) / 256.0;
-			const double slower = side == 16 ? by_rows : 1.0;
-			const double alone = static_cast<double>((stages + waves - 1) >> PLANS[i].wave_bits) * pace.chain * slower, shared = per_cu * static_cast<double>(stages) * pace.stage * slower;
+			/* (beyond four tiles of 16 x 16 to a compute unit, whose wavefronts fill it, one more takes its whole time where k is long) */
+			const double per_cu = tiles <= 1024 || (side == 16 && element_bytes < 4 && stages >= 12) ? static_cast<double>((tiles + 255) >> 8) : static_cast<double>(tiles) / 256.0;
+			const double slower = side == 16 ? by_rows : 1.0, across = side == 16 ? across_lines : 1.0;
+			const double alone = static_cast<double>((stages + waves - 1) >> PLANS[i].wave_bits) * pace.chain * slower, shared = per_cu * static_cast<double>(stages) * pace.stage * slower * across;
 			const double us = (pace.launch + (element_bytes == 4 || side == 16 ? std::sqrt(alone * alone + shared * shared) : std::max(alone, shared)) + per_cu * pace.tile)
 					* (side != 16 && row % 4 != 0 ? 1.25 : 1.0);
-			if (best.side == 0 || us < (side == 16 && best.side != 16 ? 0.95 : 1.0) * best.us)
-				best = { side, waves, us, side == 16 ? best.larger_us : us };
+			if (side == 16)
+			{
+				if (best.waves_16 == 0 || us < best.us_16)
+				{
+					best.waves_16 = waves;
+					best.us_16 = us;
+				}
+				tiles_16 = tiles;
+			}
+			else if (best.side == 0 || us < best.us)
+			{
+				best.side = side;
+				best.waves = waves;
+				best.us = best.larger_us = us;
+			}
 		}
+		if (best.side == 0 || best.us_16 < margin_16(element_bytes, row % 128 == 0, tiles_16, stages) * best.us)
+			best = best.of_16();
 		return best;
 	}
 }

@@ -640,13 +640,28 @@ namespace
 
 	/* Layers of few channels that tiles of 16 x 16 take from the kernels made for them: those take 4.0 to 4.9 us (pixels of 8 bytes, at most 12 taps), 5.9 to 9.3 (16-bit types), 7.4 and more
 	 * (int8) and 8.3 to 15 (fp32) however few their pixels are; 76 layers of up to 1200 tiles of 32 x 32: fp32 2.6 times as fast (4 -> 192 3x3 on 6 x 11 x 11 9.6 : 3.2 us), 16-bit 1.7 and 1.3 times, none slower. */
-	bool small_before_few_channels(const avhipConvShape &s, int element_bytes)
+	bool small_before_few_channels(const avhipConvShape &s, int element_bytes, const SmallPlan &plan)
 	{
-		if (conv_small_threshold() <= 0 || !conv_small_possible(s, element_bytes))
+		if (conv_small_threshold() <= 0 || plan.waves_16 == 0 || (plan.larger_us > 0.0 && plan.us_16 >= 0.95 * plan.larger_us))
 			return false;
-		const SmallPlan plan = conv_small_plan(s, element_bytes);
 		const bool stem = s.C * element_bytes == 8 && element_bytes < 4 && s.R * s.S <= 12;
-		return plan.side == 16 && plan.us < (stem ? 4.2 : element_bytes == 4 ? 7.5 : element_bytes == 2 ? 5.5 : 6.5);
+		return plan.us_16 < (stem ? 4.2 : element_bytes == 4 ? 7.5 : element_bytes == 2 ? 5.5 : 6.5);
+	}
+
+	/* What a call with LINEAR or RELU in whole aligned vectors is asked first: the tile that it gets in the kernels of small tiles, half of its side plus wavefronts, or 0 */
+	template<typename TE, typename Epi>
+	int plain_small_plan(const avhipConvShape &s)
+	{
+		Epi epi {};
+		epi.activation = ACT_RELU;
+		epi.K = s.K;
+		epi.vec = true;
+		const SmallChoice choice = conv_small_choice<TE>(s, epi);
+		if (!choice.preferred)
+			return 0;
+		if (conv_few_channels(s, static_cast<int>(sizeof(TE))))
+			return small_before_few_channels(s, sizeof(TE), choice.plan) ? 16 / 2 + choice.plan.waves_16 : 0;
+		return choice.plan.side / 2 + choice.plan.waves;
 	}
 
 	template<typename TE, typename Epi>
@@ -671,8 +686,16 @@ namespace
 		if (conv_few_channels(s, static_cast<int>(sizeof(TE))) && fast_path_ok<TE>(s, 1, padding_value, false) && is_simple_activation(epi.activation)
 				&& (flags & 2) != 0)
 		{
-			if ((ragged || fast_path_ok<TE>(s, flags, padding_value)) && small_before_few_channels(s, sizeof(TE)) && conv_small_launch<TE, Epi>(st, s, x, w, epi, conv_small_choice<TE>(s, epi)))
-				return 0;
+			if (ragged || fast_path_ok<TE>(s, flags, padding_value))
+			{
+				SmallChoice few = conv_small_choice<TE>(s, epi);
+				if (small_before_few_channels(s, sizeof(TE), few.plan))
+				{
+					few.plan = few.plan.of_16();
+					if (conv_small_launch<TE, Epi>(st, s, x, w, epi, few))
+						return 0;
+				}
+			}
 			/* a pixel of exactly 8 bytes and a small filter: operands straight into registers, no k loop */
 			if (conv_stem_launch<TE, Epi>(st, s, x, w, epi))
 				return 0;
@@ -768,6 +791,27 @@ namespace
 		const Int8Epilogue<MODE> epi { bias, z, y, scale, static_cast<float>(alpha1), static_cast<float>(alpha2), static_cast<float>(beta), activation, s.K,
 				(flags & 2) != 0 };
 		return launch<int8_t>(st, s, x, w, padding_value, flags, epi);
+	}
+}
+
+/* The tile that a call with LINEAR or RELU in whole aligned vectors gets in the kernels of small tiles before any other (the ring kernel, which takes 16- and 8-bit layers of whole chunks first, aside): half of its side plus
+ * wavefronts, or 0 where it is the kernels for few channels, one tap or large tiles that are asked.  Exported so that a test can ask which instance it is about to run. */
+extern "C" AVHIP_API int avhip_conv2d_plain_small_plan(int x_dtype, const avhipConvShape *shape)
+{
+	if (shape == nullptr || shape->K % 4 != 0)
+		return 0;
+	switch (x_dtype)
+	{
+		case DT_FLOAT32:
+			return plain_small_plan<float, FloatEpilogue<float>>(*shape);
+		case DT_FLOAT16:
+			return plain_small_plan<f16_t, FloatEpilogue<f16_t>>(*shape);
+		case DT_BFLOAT16:
+			return plain_small_plan<bf16_t, FloatEpilogue<bf16_t>>(*shape);
+		case DT_INT8:
+			return plain_small_plan<int8_t, Int8Epilogue<I8_EXACT>>(*shape);
+		default:
+			return 0;
 	}
 }
 

@@ -423,7 +423,7 @@ namespace avhip
 	}
 	SmallChoice conv_small_choice(const avhipConvShape &s, int element_bytes, HandOver hand_over, double one_tap_us)
 	{
-		SmallChoice choice = { hand_over, one_tap_us, false, { 0, 0, 0.0, 0.0 }, 0.0, false, 0.0 };
+		SmallChoice choice = { hand_over, one_tap_us, false, { 0, 0, 0.0, 0.0, 0, 0.0 }, 0.0, false, 0.0 };
 		if (!conv_small_possible(s, element_bytes))
 			return choice;
 		choice.plan = conv_small_plan(s, element_bytes);
@@ -437,8 +437,11 @@ namespace avhip
 			choice.us = choice.larger_us = workgroup_tiles_us(s, element_bytes, hand_over, one_tap_us);
 			const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
 			const double limit = tiles < threshold ? choice.us / small_factor(element_bytes, hand_over, one_tap_us) : 0.0;
-			choice.preferred = choice.plan.us < limit;
 			choice.larger_preferred = choice.plan.larger_us > 0.0 && choice.plan.larger_us < limit;
+			/* (tiles of 16 x 16 against the one-tap kernels in 16 and 8 bits, which take 4 us where they are estimated at 5.2: 20 % below; with 5 % layers of 2900 to 4200 such tiles, int8 128 -> 80 on 12600 pixels 4.1 -> 4.6 us,
+			 * bf16 64 -> 64 on 16632 4.2 -> 4.6) */
+			const bool loose = choice.plan.side == 16 && element_bytes < 4 && one_tap_us > 0.0;
+			choice.preferred = choice.plan.us < (loose ? 0.84 * limit : limit) || (choice.plan.side == 16 && choice.larger_preferred);
 		}
 		const double factor = small_factor(element_bytes, hand_over, 0.0);
 		if (choice.preferred)
