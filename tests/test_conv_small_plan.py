@@ -58,3 +58,9 @@ TIMED = [("f16", (1, 15, 15, 128, 128, 3, 1), 6.3, 4.0), ("f32", (8, 15, 15, 64,
 def test_tiles_of_16_x_16_where_they_are_faster(lib, dtype, layer, without, within):
     plan = lib.avhip_conv2d_plain_small_plan(CODE[dtype], C.byref(shape_of(*layer)))
     assert (plan in (9, 12, 16)) == (within < without), plan
+
+
+@pytest.mark.parametrize("dtype, layer", [("bf16", (32, 224, 224, 3, 64, 7, 2)), ("f32", (10, 137, 137, 3, 96, 5, 1)), ("f16", (256, 15, 15, 4, 128, 3, 1)), ("f16", (94, 25, 25, 16, 128, 3, 1)),
+                                          ("i8", (60, 28, 28, 16, 64, 3, 1)), ("f32", (64, 56, 56, 8, 64, 3, 1))])
+def test_few_channels_of_many_pixels_stay_in_the_kernels_made_for_them(lib, dtype, layer):
+    assert lib.avhip_conv2d_plain_small_plan(CODE[dtype], C.byref(shape_of(*layer))) == 0

@@ -16,7 +16,7 @@ BAR = {"f32": 1e-5, "f16": 2e-3, "bf16": 2e-3}
 
 @pytest.fixture(autouse=True, params=["wavefront_tiles", "workgroup_tiles"])
 def tiling(request):
-    """Every test runs twice: with the kernel of small tiles (32 x 32 or 64 x 64, k shared by wavefronts) forced for whatever it can run
+    """Every test runs twice: with the kernels of small tiles (16 x 16 to 64 x 64, k shared by wavefronts) forced for whatever it can run
     (the launcher itself picks it for problems that do not fill the chip with large ones), and with that kernel switched off, so that
     the same geometry goes through the 128 x 128 gather kernel, the image-tile kernel or the few-channel kernels."""
     lib = cb.load_library()
@@ -46,12 +46,12 @@ def test_implicit_gemm_config1(oracle, dtype):
 
 
 SMALL_TILE_CASES = [
-    # the four forms of the kernel with small tiles (tile side, wavefronts that share k), as its estimates pick them
+    # small tiles (side, wavefronts that share k) as the estimates pick them; those of 32 x 32 in all their forms are in test_gpu_conv_small32.py, of 16 x 16 in test_gpu_conv_small16.py
     dict(x=(40, 36, 36, 32), w=(36, 1, 1, 32), dtype="bf16"),                                              # 32, 1: thousands of tiles, one stage
     dict(x=(3, 31, 31, 136), w=(252, 3, 3, 136), pad=(-1, -1), dtype="f16", z=True, act="ELU"),            # 64, 4: ragged both ways, 20 stages
     dict(x=(3, 31, 29, 136), w=(256, 3, 3, 136), pad=(-1, -1), dtype="i8"),
-    dict(x=(1, 9, 9, 200), w=(36, 5, 5, 200), pad=(-2, -2), dtype="f32", z=True),                          # 32, 8: long k, last wavefront short
-    dict(x=(5, 9, 7, 24), w=(23, 3, 2, 24), pad=(-1, 0), dtype="f32", act="TANH", z=True),                 # 32, 4: 3 chunks left in the last stage
+    dict(x=(1, 9, 9, 200), w=(36, 5, 5, 200), pad=(-2, -2), dtype="f32", z=True),                          # 16, 8: long k, last wavefront short
+    dict(x=(5, 9, 7, 24), w=(23, 3, 2, 24), pad=(-1, 0), dtype="f32", act="TANH", z=True),                 # 16, 8: 3 chunks left in the last stage
     dict(x=(5, 13, 11, 40), w=(64, 5, 5, 40), pad=(-4, -4), stride=(2, 1), dilation=(2, 2), mode=1, dtype="bf16", z=True),
     dict(x=(2, 7, 7, 16), w=(8, 4, 8, 16), pad=(-3, -7), dtype="bf16", act="SIGMOID"),                     # 32 taps, 2 chunks each
     dict(x=(1, 3, 3, 48), w=(4, 1, 1, 48), dtype="i8"),                                                    # less than one stage, 9 pixels
@@ -68,7 +68,7 @@ SMALL_TILE_CASES = [
     dict(x=(3, 15, 13, 131), w=(65, 3, 3, 131), pad=(-1, -1), dtype="i8"),
     dict(x=(3, 15, 13, 6), w=(66, 3, 3, 6), pad=(-1, -1), dtype="i8"),
     dict(x=(40, 36, 36, 34), w=(36, 1, 1, 34), dtype="bf16", z=True),                                      # 32, 1 with rows of dwords
-    dict(x=(40, 36, 36, 33), w=(36, 1, 1, 33), dtype="f16", act="ELU"),                                    # 32, 1 with rows of elements
+    dict(x=(40, 36, 36, 33), w=(36, 1, 1, 33), dtype="f16", act="ELU"),                                    # 16, 1 with rows of elements
     dict(x=(40, 36, 36, 7), w=(36, 1, 1, 7), dtype="f32"),
 ]
 

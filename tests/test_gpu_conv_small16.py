@@ -1,5 +1,6 @@
 """Tiles of 16 x 16 (csrc/conv_small16.hip) against the oracle: one tile and many, ragged both ways, one wavefront to eight of them, shares of k from less than a stage to several rounds,
-borders, strides, dilations, flipped filters, every hand-over of results.  The plan is asked for first, so each case runs the instance that it names."""
+borders, strides, dilations, flipped filters, every hand-over of results.  The plan is asked for first, for few channels that which stands before the kernels made for them, so each case runs
+the instance that it names."""
 import ctypes as C
 
 import numpy as np
@@ -83,15 +84,15 @@ def test_rows_of_channels(oracle, case, dtype, act):
     waves, (N, H, W), channels, (K, R, S), geometry = ROWS[case]
     Cin = channels[dtype]
     lib = cb.load_library()
-    if act == "RELU":
-        if dtype == "i8":
-            pytest.skip("integer sums: with the other activation's name")
+    if act == "RELU":  # (of int8, whose sums have no activation here, the half by estimate)
         lib.avhip_set_small_problem_threshold(4096)
     (ph, pw), (sh, sw) = geometry.get("pad", (0, 0)), geometry.get("stride", (1, 1))
     ys = (N, (H - 2 * ph - R) // sh + 1, (W - 2 * pw - S) // sw + 1, K)
     shape = Shape(N, H, W, Cin, K, R, S, ys[1], ys[2], ph, pw, sh, sw, 1, 1, geometry.get("mode", 0))
     code = {"f32": cb.DTYPE_FLOAT32, "f16": cb.DTYPE_FLOAT16, "bf16": cb.DTYPE_BFLOAT16, "i8": cb.DTYPE_INT8}[dtype]
-    assert lib.avhip_conv2d_small_plan(code, C.byref(shape), 0) in [8 + n for n in ((1, 4, 8) if waves == 4 else (waves,))]
+    query = lib.avhip_conv2d_plain_small_plan if act == "RELU" and K % 4 == 0 else lib.avhip_conv2d_small_plan  # (single filters: no kernel for few channels takes them)
+    arguments = (code, C.byref(shape)) if query is lib.avhip_conv2d_plain_small_plan else (code, C.byref(shape), 2 if act == "ELU" and dtype != "i8" else 1 if K % 4 else 0)
+    assert query(*arguments) in [8 + n for n in ((1, 4, 8) if waves == 4 else (waves,))]
     geometry = {"pad": (0, 0), **geometry}
     g = h.rng(800 + case)
     if dtype == "i8":
