@@ -58,12 +58,12 @@ namespace avhip
 			{ 2.91, 0.280, 0.069, 0.05 }, { 2.83, 0.217, 0.060, 0.275 }, { 2.65, 0.260, 0.058, 0.52 } };
 
 	/* How far below those of larger tiles the estimate of tiles of 16 x 16 has to be: 5 %, and in 16 and 8 bits, whose larger tiles are estimated 5 to 10 % too high where their number begins a second round or k is long, 10 beyond
-	 * 768 of them or for a long k in rows that are no whole lines, 20 for many tiles of a long k.  Of 1794 16-bit layers that got tiles of 16 x 16 with 5 % everywhere, a tile beyond four in part and no look at
+	 * four to a compute unit (three, or a long k, in rows that are no whole lines), 20 for many tiles of a long k.  Of 1794 16-bit layers that got tiles of 16 x 16 with 5 % everywhere, a tile beyond four in part and no look at
 	 * how rows lie, 74 were more than 3 % slower with them, by 25 at most (472 -> 192 3x3 stride 2 on 16 x 19 x 18 18.3 -> 24.4 us; 384 -> 200 5x5 stride 2 on 7 x 27 x 26, which was split before, 23.7 -> 36.2).
-	 * 1568 keep them, 9 of those more than 3 % slower, by 10 at most, and 1.26 times as fast on average. */
+	 * 1584 keep them, 10 of those more than 3 % slower, by 10 at most, and 1.26 times as fast on average. */
 	inline double margin_16(int element_bytes, bool whole_lines, int64_t tiles, int64_t stages)
 	{
-		if (element_bytes == 4 || tiles <= 256 || (tiles <= 768 && (whole_lines || stages < 90)))
+		if (element_bytes == 4 || tiles <= 256 || (whole_lines ? tiles <= 1024 : tiles <= 768 && stages < 90))
 			return 0.95;
 		return tiles <= 1536 || stages < 24 ? 0.9 : 0.8;
 	}

@@ -28,4 +28,4 @@ def test_direct_sums(case):
     assert np.array_equal(got, h.conv_forward("implicit_gemm", x, w, shape, "f32", **more))
     some = slice(0, 2)  # the whole batch has been compared above; the oracle is slow
     want = orc.conv2d(x[some], w, b, z=z[some] if residual else None, activation=getattr(orc, act.upper()))
-    assert orc.rel_l2(got[some], want) < 1e-6  # direct sums 2e-7 to 4e-7, F(2x2, 3x3) in the fused kernel above
+    assert orc.rel_l2(got[some], want) < 1e-6  # direct sums 1.2e-7 to 4.3e-7 (a k of one wavefront the most), the fused kernel 1.7e-7 to 2.7e-7
