@@ -438,9 +438,9 @@ namespace avhip
 			const int64_t tiles = (static_cast<int64_t>(s.N) * s.Ho * s.Wo + 127) / 128 * ((static_cast<int64_t>(s.K) + 127) / 128);
 			const double limit = tiles < threshold ? choice.us / small_factor(element_bytes, hand_over, one_tap_us) : 0.0;
 			choice.larger_preferred = choice.plan.larger_us > 0.0 && choice.plan.larger_us < limit;
-			/* (tiles of 16 x 16 against the one-tap kernels in 16 and 8 bits, which take 4 us where they are estimated at 5.2: 13 % below; with 5 % layers of 2900 to 4200 such tiles were slower, int8 128 -> 80 on 12600 pixels 4.1 -> 4.6 us,
-			 * bf16 64 -> 64 on 16632 4.2 -> 4.6) */
-			const bool loose = choice.plan.side == 16 && element_bytes < 4 && one_tap_us > 0.0;
+			/* (tiles of 16 x 16 against the one-tap kernels in 16 and 8 bits: those take 4.0 to 4.3 us for one stage where they are estimated at 5.2, for two 4.7 to 5.2; so 13 % below for one.  With 5 % layers of 3600 to 4900
+			 * such tiles were slower, int8 80 -> 80 on 15652 pixels 4.1 -> 5.0 us, bf16 64 -> 64 on 16632 4.2 -> 4.6) */
+			const bool loose = choice.plan.side == 16 && element_bytes < 4 && one_tap_us > 0.0 && static_cast<int64_t>(s.C) * element_bytes <= 128;
 			choice.preferred = choice.plan.us < (loose ? 0.92 * limit : limit) || (choice.plan.side == 16 && choice.larger_preferred);
 		}
 		const double factor = small_factor(element_bytes, hand_over, 0.0);
