@@ -221,8 +221,8 @@ namespace avhip
 
 	/* n / d for n below 2^31 by a multiplication: with 2^shift >= d and factor = ceil(2^(31 + shift) / d), n * factor / 2^(31 + shift) is too
 	 * large by less than 1 / d.  A division by a number that only the launch knows is a chain of some twenty dependent instructions,
-	 * and three of them in a row stood before the first load of a workgroup: bf16 3x3 48 -> 48 on 3600 pixels 5.0 us a call with them, 4.4 without,
-	 * 4.6 in the kernel of one wavefront per tile that this one replaced (towers of twelve such layers; from a graph 4.3, 4.2). */
+	 * and three of them in a row stood before the first load of a workgroup in small tiles: bf16 3x3 48 -> 48 on 3600 pixels 5.0 us a call with them, 4.4 without
+	 * (towers of twelve such layers). */
 	struct Divisor
 	{
 		unsigned int factor, shift;

@@ -16,7 +16,7 @@
  * RELU the estimates keep it in image tiles, 49), int8 144 -> 80 3x3 on 81 x 39 x 39 43.5 -> 27, bf16 256 -> 512 3x3 stride 2
  * on 23 x 35 x 35 34 -> 21, bf16 192 -> 384 3x3 stride 2 on 11 x 41 x 41 15.3 -> 11.5.
  * Activations by a call: a work-item's sixteen results of a tile at once, residual requested ahead (ACT_VECTORS; four at a time in a loop before): f16 32 -> 448 3x3 on 234 x 12 x 12 with
- * a residual and an ELU 44.7 -> 35.0 us, bf16 488 -> 320 1x1 stride 2 on 22 x 54 x 55 26.2 -> 19.0, 36 such layers 1.06 to 1.4 times as fast.
+ * a residual and an ELU 43.3 -> 35.8 us, bf16 488 -> 320 1x1 stride 2 on 22 x 54 x 55 with an ELU 21.3 -> 16.8, with a sigmoid 21.4 -> 18.8, 65 such layers 1.02 to 1.37 times as fast, 1.11 on average.
  */
 #include <algorithm>
 #include <cmath>

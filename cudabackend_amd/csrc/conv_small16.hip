@@ -7,10 +7,10 @@
  * stages at a time, 0.7 us for sums and results, 1.7 us of launch.  So: tiles of a quarter, for four times as many compute units (half as many bytes each; in fp32 a quarter of the products);
  * the filters' loads before the pixels' addresses; the border by two comparisons a load and not by a mask made in loops.  One pixel quad a lane is left to hand over: the first wavefront does.
  * What bounds it now: the latency of one load, the sums and the launch, 2.8 us of them for a layer of one stage.
- * Measured, before (tiles of 32 x 32) and now: that layer 6.3 -> 4.0 us, bf16 256 -> 256 3x3 on 3 x 13 x 13 7.8 -> 6.6, fp32 64 -> 64 3x3 on 8 x 15 x 15 8.2 -> 4.4, fp32 128 -> 128 on
- * 512 pixels 11.5 -> 5.9, int8 1x1 48 -> 48 on 320 pixels 3.6 -> 2.7; of 470 layers of up to 1500 tiles of 32 x 32 the mean is 1.19 times as fast in 16 bits and 1.3 in fp32.
- * Rows of dwords and elements (any number of channels) against tiles of 32 x 32: bf16 97 -> 32 3x3 stride 2 on 360 pixels 6.9 -> 4.2 us, fp32 133 -> 32 3x3 on 640 12.0 -> 6.8; few channels against
- * the kernels made for them: fp32 4 -> 128 3x3 on 6 x 11 x 11 9.3 -> 3.0, fp16 8 -> 80 3x3 on 860 pixels 6.3 -> 3.3, bf16 4 -> 128 on 512 4.3 -> 3.3.
+ * Measured, before (tiles of 32 x 32) and now: that layer 5.9 -> 4.1 us, bf16 256 -> 256 3x3 on 3 x 13 x 13 7.8 -> 6.7, fp32 64 -> 64 3x3 on 8 x 15 x 15 8.2 -> 5.6, fp32 128 -> 128 on
+ * 512 pixels 11.3 -> 5.6, int8 1x1 48 -> 48 on 320 pixels 3.6 -> 2.7; 1584 16-bit layers that the estimates send here are 1.26 times as fast, 298 of fp32 1.48 times.
+ * Rows of dwords and elements (any number of channels) against tiles of 32 x 32: bf16 97 -> 32 3x3 stride 2 on 364 pixels 6.7 -> 4.4 us, fp32 133 -> 32 3x3 on 640 11.6 -> 6.4; few channels against
+ * the kernels made for them: fp32 4 -> 128 3x3 on 6 x 11 x 11 8.8 -> 3.3, fp16 8 -> 80 3x3 on 845 pixels 6.0 -> 3.2, bf16 4 -> 128 on 512 4.4 -> 3.4.
  * Three or four stages in flight and sixteen wavefronts were not faster, two wavefronts in no layer by more than 5 %.
  */
 #include "conv_small.hpp"
