@@ -639,7 +639,7 @@ namespace
 	}
 
 	/* Layers of few channels that tiles of 16 x 16 take from the kernels made for them: those take 4.0 to 4.9 us (pixels of 8 bytes, at most 12 taps), 5.9 to 9.3 (16-bit types), 7.4 and more
-	 * (int8) and 8.3 to 15 (fp32) however few their pixels are; 76 layers of up to 1200 tiles of 32 x 32: fp32 2.6 times as fast (4 -> 192 3x3 on 6 x 11 x 11 9.6 : 3.2 us), 16-bit 1.7 and 1.3 times, none slower. */
+	 * (int8) and 8.3 to 15 (fp32) however few their pixels are; 76 layers of up to 1200 tiles of 32 x 32: fp32 2.6 times as fast (4 -> 192 3x3 on 6 x 11 x 11 9.1 : 3.4 us), 16-bit 1.7 and 1.3 times, none slower. */
 	bool small_before_few_channels(const avhipConvShape &s, int element_bytes, const SmallPlan &plan)
 	{
 		if (conv_small_threshold() <= 0 || plan.waves_16 == 0 || (plan.larger_us > 0.0 && plan.us_16 >= 0.95 * plan.larger_us))
